@@ -285,8 +285,8 @@ def work(case):
         if kind == "mlp_forward":
             # x and the parameters once, every layer's output once
             return {"bytes": 4 * (weights + batch * sum(sizes)), "flops": products}
-        # parameters read and written; x, target in; y, dy of three layers and dx of three out
-        return {"bytes": 4 * (2 * weights + batch * (sizes[0] + sizes[3] + 2 * sum(sizes[1:]) +
+        # parameters read and written; x, target in; y and dx of three layers out
+        return {"bytes": 4 * (2 * weights + batch * (sizes[0] + sizes[3] + sum(sizes[1:]) +
                                                      sum(sizes[:3]))),
                 "flops": 3 * products}
     if kind == "spmm":
