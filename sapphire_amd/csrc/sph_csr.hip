@@ -631,9 +631,11 @@ int ExclusiveScanInPlace(uint32_t* data, uint32_t n, uint32_t* lastHost, hipStre
         // per-block totals: the caller's workspace, or a stream-ordered scratch allocation
         const bool own = sums == nullptr;
         if (own)
+        {
             ::sph::CountAllocation();
             SPH_HIP_TRY(hipMallocAsync(reinterpret_cast<void**>(&sums),
                                        blocks * sizeof(uint32_t), stream));
+        }
         hipLaunchKernelGGL(ScanBlocksKernel, dim3(blocks), dim3(kScanThreads), 0, stream, data,
                            sums, n);
         hipLaunchKernelGGL(ScanSumsKernel, dim3(1), dim3(kScanThreads), 0, stream, sums, blocks);

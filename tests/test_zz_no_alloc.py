@@ -111,3 +111,22 @@ def test_recordable_into_a_graph(dev):
     g.destroy()
     dD.release()
     dRow.release()
+
+
+def test_device_memory_in_use_does_not_grow(dev):
+    """Free device memory before and after many calls whose scan needs the block totals: a scratch
+    block of 16 KiB taken and kept by each call would add up to 32 MiB."""
+    import torch
+    M = 16000000
+    dD = capi.DeviceBuffer.from_array(np.ones(M, np.float32))
+    dRow = capi.DeviceBuffer(4 * (M + 1))
+    h.announce("sph_csr_row_offsets_noalloc_f32 x 2000, rows =", M)
+    capi.call("sph_csr_row_offsets_noalloc_f32", dRow.ptr, dD.ptr, M, 1, 1)
+    capi.sync()
+    before = torch.cuda.mem_get_info()[0]
+    for _ in range(2000):
+        capi.call("sph_csr_row_offsets_noalloc_f32", dRow.ptr, dD.ptr, M, 1, 1)
+    capi.sync()
+    assert before - torch.cuda.mem_get_info()[0] < 8 << 20
+    dD.release()
+    dRow.release()
