@@ -24,13 +24,14 @@
 // follows the entries it produces, not its width.  The same kernel runs twice: once to count
 // the entries of every row (the caller then allocates), once to write them.
 //
-// Matrices wider than two strips: rows with few products (A's row at most 64 entries, at most
-// 256 products) go to SpgemmHashKernel, which keeps the row in a hash table instead and whose
+// Matrices wider than one strip: rows with few products (A's row at most 64 entries, at most
+// 512 products) go to SpgemmLightKernel, which sorts a row's products in registers and whose
 // cost does not depend on the width; the strip kernel then takes only the remaining rows.
 //
 // Requirements on the operands: column indices of B below N and distinct within a row;
 // column indices of A below the row count of B.
 #include "sph_internal.h"
+#include "sph_place_rows.h"
 
 #include <algorithm>
 
@@ -42,14 +43,12 @@ constexpr uint32_t kStripMax = 4096;  // columns per LDS strip
 constexpr uint32_t kAhead = 8;        // rows of B whose first 64 entries are in flight together
 constexpr uint32_t kRowsPerTurnMax = 8;  // consecutive output rows a wavefront takes at a time
 constexpr uint32_t kWordsPerLaneMax = kStripMax / 32 / 64;  // bit-map words a lane owns
-// Wide matrices (more than one strip): rows with few products go through a hash table instead
-constexpr uint32_t kHashSlots = 512;            // power of two
-constexpr uint32_t kHashProducts = kHashSlots / 2;  // a row with at most this many products is "light"
+constexpr uint32_t kLightProducts = 512;  // a row with at most this many products is "light"
+constexpr uint32_t kPlaceBits = 9;        // a product's place in its row, below its column
+constexpr uint32_t kLightWaves = 4;       // wavefronts per workgroup of SpgemmLightKernel
 constexpr uint32_t kEmpty = 0xffffffffu;
-// two strips still cost less than the table and its sort (8192 columns, 8 entries per row on
-// both sides: 82 us on strips, 96 us through the table); from three strips on the table wins
-constexpr uint32_t kHashFromWidth = 2 * kStripMax;
-static_assert(kHashSlots == 512, "the hash takes the top 9 bits of a product");
+constexpr uint32_t kHeavyMark = 0xffffffffu;  // in place of a count: SpgemmRowKernel's row
+static_assert(kLightProducts <= 1u << kPlaceBits, "a key holds column and place");
 static_assert(kWordsPerLaneMax <= 4, "the sweep takes a lane's words as two pairs");
 
 struct SpgemmArgs
@@ -63,7 +62,8 @@ struct SpgemmArgs
     uint32_t M, K, N;
     uint32_t strip;  // columns per strip (multiple of 64)
     uint32_t rowsPerTurn;  // 1 .. kRowsPerTurnMax
-    uint32_t heavyOnly;    // strip kernel: leave the rows SpgemmHashKernel takes alone
+    uint32_t lightProducts;  // rows with at most this many products are SpgemmLightKernel's (0: none)
+    uint32_t heavyOnly;    // strip kernel: leave those rows alone
     // count pass: counts (M + 1 entries, counts[M] = 0).  fill pass: ROWC, VC, COLC.
     // stage pass: counts as in the count pass, and row r's entries into VC / COLC at
     // r * slot .. r * slot + slot - 1 (what does not fit is counted and dropped).
@@ -107,79 +107,257 @@ __device__ __forceinline__ uint32_t WaveSum(uint32_t v)
     return v;
 }
 
-// A row is light when A's row has at most 64 entries and the rows of B they select hold at
-// most kHashProducts entries together.  Both kernels decide from these two numbers.
-__device__ __forceinline__ bool LightRow(uint32_t entriesOfA, uint32_t products)
+// A row is light when A's row has at most 64 entries and the rows of B they select hold at most
+// kLightProducts entries together.  Both kernels decide from these two numbers; a lane counts at
+// most kLightProducts + 1 entries of its row of B, so that the sum cannot wrap.
+__device__ __forceinline__ uint32_t LightCount(uint32_t begin, uint32_t end)
 {
-    return entriesOfA <= 64 && products <= kHashProducts;
+    return end > begin ? min(end - begin, kLightProducts + 1) : 0u;
 }
 
-// Light rows of a wide product.  The strip kernel walks all products of a row once per strip
-// of 4096 columns, which is wasted on a row whose few products fall into a matrix of, say,
-// 65536 columns.  Here a wavefront keeps the row in an LDS hash table keyed by column instead
-// (the design the reference sketches, SparseGemm.cuh:16-36): the products are generated in the
-// same order as in the strip kernel -- A's entries in storage order, the entries of one row of
-// B across the lanes, so no two lanes of a step hold the same column -- a lane finds or claims
-// (compare-and-swap on the key) the slot of its column and adds into it, which keeps the sum
-// order of every element fixed.  Claimed slots are listed as they are claimed; at the end of
-// the row the listed (column, sum) pairs are sorted by column (bitonic, in LDS), sums that are
-// exactly zero are dropped, and the table is reset through the list.  The cost of a row follows
-// its products, not the width of the matrix.
-template <int MODE>
-__global__ __launch_bounds__(64) void SpgemmHashKernel(const SpgemmArgs args)
+__device__ __forceinline__ bool LightRow(const SpgemmArgs& args, uint32_t entriesOfA,
+                                         uint32_t products)
 {
-    constexpr bool FILL = MODE != kCount;    // entries are stored
-    constexpr bool COUNTS = MODE != kFill;   // counts are stored
-    if (MODE == kFill && args.overflow != nullptr && *args.overflow == 0)
-        return;  // every row is in place already
-    __shared__ uint32_t keys[kHashSlots];
-    __shared__ float sums[kHashSlots];
-    __shared__ uint32_t sortKey[kHashProducts];  // first the list of claimed slots, then columns
-    __shared__ float sortVal[kHashProducts];
-    const uint32_t lane = threadIdx.x;
-    const uint64_t below = (1ull << lane) - 1ull;
-    for (uint32_t t = lane; t < kHashSlots; t += 64)
-    {
-        keys[t] = kEmpty;
-        sums[t] = 0.0f;
-    }
+    return entriesOfA <= 64 && products <= args.lightProducts;
+}
 
-    // A wavefront takes rows blockIdx.x, blockIdx.x + gridDim.x, ... in turns of up to 64: their
-    // extents are read in one go (one row per lane), and the loads that lead to a row's
-    // products form a pipeline over the rows of the turn: while row i is multiplied, the
-    // entries of A's row i+2 and the extents of the rows of B that row i+1 selects are on
-    // their way.
-    for (uint64_t first = blockIdx.x; first < args.M; first += 64ull * gridDim.x)
+// value of lane (lane ^ MASK).  Four of the six masks are lane permutations of the vector unit
+// itself and never go through the LDS crossbar.
+template <uint32_t MASK>
+__device__ __forceinline__ uint32_t XorLane(uint32_t v)
+{
+    const int x = static_cast<int>(v);
+    if constexpr (MASK == 1)
+        return __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, true);  // quad 1 0 3 2
+    else if constexpr (MASK == 2)
+        return __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, true);  // quad 2 3 0 1
+    else if constexpr (MASK == 4)  // mirrored within 8 lanes (^ 7), then within 4 (^ 3)
+        return __builtin_amdgcn_update_dpp(
+            0, __builtin_amdgcn_update_dpp(0, x, 0x141, 0xf, 0xf, true), 0x1B, 0xf, 0xf, true);
+    else if constexpr (MASK == 8)
+        return __builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, true);  // rotate 16 by 8
+    else if constexpr (MASK == 16)
+        return __builtin_amdgcn_ds_swizzle(x, (16 << 10) | 0x1f);
+    else
+        return __shfl_xor(v, MASK, 64);
+}
+
+template <uint32_t MASK>
+__device__ __forceinline__ uint64_t XorLane(uint64_t v)
+{
+    const uint32_t lo = XorLane<MASK>(static_cast<uint32_t>(v));
+    const uint32_t hi = XorLane<MASK>(static_cast<uint32_t>(v >> 32));
+    return (static_cast<uint64_t>(hi) << 32) | lo;
+}
+
+// Bitonic sort of 64 E keys held by one wavefront, E consecutive ones per lane: the exchanges
+// from (SIZE, STRIDE) on.
+template <uint32_t E, typename Key, uint32_t SIZE = 2, uint32_t STRIDE = 1>
+__device__ __forceinline__ void SortKeys(Key (&key)[E], uint32_t lane)
+{
+    if constexpr (STRIDE < E)
     {
-        const uint64_t mine = first + static_cast<uint64_t>(lane) * gridDim.x;
-        const uint32_t rowsHere = static_cast<uint32_t>(
-            min(static_cast<uint64_t>(64), (args.M - first + gridDim.x - 1) / gridDim.x));
-        uint32_t extentBegin = 0, extentEnd = 0, outBegin = 0, outEnd = 0;
-        if (mine < args.M)
+#pragma unroll
+        for (uint32_t e = 0; e < E; ++e)
         {
-            extentBegin = args.ROWA[mine];
-            extentEnd = args.ROWA[mine + 1];
-            if (MODE == kFill)
-            {
-                outBegin = args.ROWC[mine];
-                outEnd = args.ROWC[mine + 1];
-            }
-            if (MODE == kStage)
-            {
-                outBegin = static_cast<uint32_t>(mine) * args.slot;
-                outEnd = outBegin + args.slot;
-            }
+            if ((e & STRIDE) != 0)
+                continue;
+            const bool ascending = SIZE < E ? (e & SIZE) == 0 : (lane & (SIZE / E)) == 0;
+            const Key x = key[e], y = key[e + STRIDE];
+            const bool swap = (y < x) == ascending;
+            key[e] = swap ? y : x;
+            key[e + STRIDE] = swap ? x : y;
         }
-        if (MODE == kFill && args.skipUpTo != 0 &&
-            __ballot(mine < args.M && outEnd - outBegin > args.skipUpTo) == 0)
-            continue;  // all of these rows are in place already
+    }
+    else
+    {
+        const bool smaller = ((lane & (STRIDE / E)) == 0) == ((lane & (SIZE / E)) == 0);
+#pragma unroll
+        for (uint32_t e = 0; e < E; ++e)
+        {
+            const Key other = XorLane<STRIDE / E>(key[e]);
+            key[e] = (other < key[e]) == smaller ? other : key[e];
+        }
+    }
+    if constexpr (STRIDE > 1)
+        SortKeys<E, Key, SIZE, STRIDE / 2>(key, lane);
+    else if constexpr (SIZE < 64 * E)
+        SortKeys<E, Key, SIZE * 2, SIZE>(key, lane);
+}
+
+// A wavefront's own LDS: nothing is shared between wavefronts, and the LDS operations of one
+// wavefront are executed in order.
+struct LightScratch
+{
+    float product[kLightProducts];
+    uint32_t column[kLightProducts];
+    float value[kLightProducts];
+};
+
+struct LightInput
+{
+    uint32_t entriesOfA;      // uniform, at most 64
+    uint32_t products;        // uniform, at most 64 E
+    uint32_t bBegin, before;  // of lane j: first entry of the row of B that A's entry j selects,
+    float aValue;             // products of A's entries before j, value of A's entry j
+    uint32_t rowBase, rowLimit;  // uniform: where the entries go
+};
+
+// The entries of one light row; returns their number.
+template <int MODE, uint32_t E, typename Key>
+__device__ __forceinline__ uint32_t LightRowEntries(const SpgemmArgs& args, const LightInput& in,
+                                                    LightScratch& lds, uint32_t lane)
+{
+    // product p (in the order in which the sums take them) belongs to lane p % 64
+    uint32_t base[E];
+    float a[E];
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e)
+    {
+        base[e] = 0;
+        a[e] = 0.0f;
+    }
+    for (uint32_t j = 0; j < in.entriesOfA; ++j)
+    {
+        const uint32_t start = Uniform(in.before, j);
+        const uint32_t from = Uniform(in.bBegin, j) - start;
+        const float value = Uniform(in.aValue, j);
+#pragma unroll
+        for (uint32_t e = 0; e < E; ++e)
+        {
+            const bool reached = e * 64u + lane >= start;
+            base[e] = reached ? from : base[e];
+            a[e] = reached ? value : a[e];
+        }
+    }
+    uint32_t col[E];
+    float b[E];
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e)
+    {
+        const uint32_t p = e * 64u + lane;
+        col[e] = kEmpty;
+        b[e] = 0.0f;
+        if (p < in.products)
+        {
+            col[e] = args.COLB[base[e] + p];
+            b[e] = args.VB[base[e] + p];
+        }
+    }
+    // keys: column, then place in the order of the sums; where a key starts does not matter
+    Key key[E];
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e)
+    {
+        const uint32_t p = e * 64u + lane;
+        key[e] = col[e] < args.N ? static_cast<Key>(col[e]) << kPlaceBits | p : ~static_cast<Key>(0);
+        lds.product[p] = a[e] * b[e];
+    }
+    SortKeys<E, Key>(key, lane);
+    __builtin_amdgcn_wave_barrier();
+
+    // the sorted (column, product) pairs side by side
+    const uint32_t place0 = lane * E;
+    uint32_t c[E];
+    float v[E];
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e)
+    {
+        const bool used = key[e] != ~static_cast<Key>(0);
+        c[e] = used ? static_cast<uint32_t>(key[e] >> kPlaceBits) : kEmpty;
+        v[e] = lds.product[static_cast<uint32_t>(key[e]) & (64u * E - 1)];
+    }
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e)
+    {
+        lds.column[place0 + e] = c[e];
+        lds.value[place0 + e] = v[e];
+    }
+    __builtin_amdgcn_wave_barrier();
+    // the first pair of a column sums the column's products, in their order, from +0
+    bool keep[E];
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e)
+    {
+        const uint32_t left = e != 0 ? c[e == 0 ? 0 : e - 1]
+                                     : place0 != 0 ? lds.column[place0 - 1] : kEmpty;
+        keep[e] = false;
+        if (c[e] != kEmpty && c[e] != left)
+        {
+            float sum = 0.0f + v[e];
+            for (uint32_t t = place0 + e + 1; t < 64u * E && lds.column[t] == c[e]; ++t)
+                sum = sum + lds.value[t];
+            v[e] = sum;
+            keep[e] = sum != 0.0f;  // exact zeros are not stored
+        }
+    }
+    const uint64_t below = (1ull << lane) - 1ull;
+    uint32_t before = 0, emitted = 0;
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e)
+    {
+        const uint64_t m = __ballot(keep[e]);
+        before += static_cast<uint32_t>(__popcll(m & below));
+        emitted += static_cast<uint32_t>(__popcll(m));
+    }
+    if (MODE != kCount)
+    {
+        uint32_t at = in.rowBase + before;
+#pragma unroll
+        for (uint32_t e = 0; e < E; ++e)
+            if (keep[e])
+            {
+                if (at < in.rowLimit)
+                {
+                    args.VC[at] = v[e];
+                    args.COLC[at] = c[e];
+                }
+                ++at;
+            }
+    }
+    return emitted;
+}
+
+// Light rows.  The strip kernel walks all products of a row once per strip of 4096 columns, one
+// row of B at a time with as many active lanes as that row has entries (8 of 64 on a graph with
+// 8 neighbours per node).  Here all products of a row are loaded at once, one per lane and
+// register, and sorted in registers by (column, place in the order of the sums); the first
+// product of a column then adds the following ones of the same column in that order, sums that
+// are exactly zero are dropped, and ballots give the others their output positions.  The cost of
+// a row follows its products, not the width of the matrix.
+// What bounds it is the chain of four dependent loads and the issue of the exchanges; five
+// wavefronts per SIMD are resident.  65536 rows with 8 entries on both sides: 63 us for the pass
+// (180 us with a hash table in LDS, one row of B inserted at a time); the whole call 265 -> 92 us.
+template <int MODE, typename Key>
+__global__ __launch_bounds__(kLightWaves * 64, 5) void SpgemmLightKernel(const SpgemmArgs args)
+{
+    __shared__ LightScratch scratch[kLightWaves];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t turn0 = blockIdx.x * kLightWaves + wave;
+    const uint64_t step = static_cast<uint64_t>(gridDim.x) * kLightWaves * args.rowsPerTurn;
+    // A wavefront takes rowsPerTurn consecutive rows per turn, with the loads that lead to a
+    // row's products in a pipeline over the rows of the turn, as in the strip kernel.
+    for (uint64_t turn = static_cast<uint64_t>(turn0) * args.rowsPerTurn; turn < args.M; turn += step)
+    {
+        const uint32_t first = static_cast<uint32_t>(turn);
+        const uint32_t rowsHere = min(args.rowsPerTurn, args.M - first);
+        uint32_t extentA = 0, extentC = 0;
+        if (lane <= rowsHere)
+        {
+            extentA = args.ROWA[first + lane];
+            if (MODE == kFill)
+                extentC = args.ROWC[first + lane];
+            if (MODE == kStage)
+                extentC = (first + lane) * args.slot;
+        }
         // stage 1: this lane's entry of A's row i (rows with more than 64 entries are not ours)
         auto loadStage1 = [&](uint32_t i, uint32_t& k, float& value) {
             k = kEmpty;
             value = 0.0f;
             if (i < rowsHere)
             {
-                const uint32_t begin = Uniform(extentBegin, i), end = Uniform(extentEnd, i);
+                const uint32_t begin = Uniform(extentA, i), end = Uniform(extentA, i + 1);
                 if (end - begin <= 64 && begin + lane < end)
                 {
                     k = args.COLA[begin + lane];
@@ -203,197 +381,54 @@ __global__ __launch_bounds__(64) void SpgemmHashKernel(const SpgemmArgs args)
         loadStage2(k2, nextBegin, nextEnd);
         loadStage1(1, k1, value1);
 
-      for (uint32_t i = 0; i < rowsHere; ++i)
-      {
-        const uint32_t row = static_cast<uint32_t>(first + static_cast<uint64_t>(i) * gridDim.x);
-        const uint32_t entriesOfA = Uniform(extentEnd, i) - Uniform(extentBegin, i);
-        const uint32_t bBegin = nextBegin, bEnd = nextEnd;
-        const float aValue = value2;
-        k2 = k1;
-        value2 = value1;
-        loadStage2(k2, nextBegin, nextEnd);
-        loadStage1(i + 2, k1, value1);
-        if (!LightRow(entriesOfA, WaveSum(bEnd - bBegin)))
-            continue;  // heavy: the strip kernel's row
-        if (MODE == kFill && Uniform(outEnd, i) - Uniform(outBegin, i) <= args.skipUpTo)
-            continue;  // already in place
-
-        uint32_t listed = 0;  // claimed slots so far (uniform)
-        for (uint32_t j0 = 0; j0 < entriesOfA; j0 += kAhead)
+        for (uint32_t i = 0; i < rowsHere; ++i)
         {
-            // the first 64 entries of kAhead rows of B are requested before the first is used
-            uint32_t s[kAhead], e[kAhead], col[kAhead];
-            float a[kAhead], b[kAhead];
+            LightInput in;
+            in.entriesOfA = Uniform(extentA, i + 1) - Uniform(extentA, i);
+            in.bBegin = nextBegin;
+            in.aValue = value2;
+            const uint32_t mine = LightCount(nextBegin, nextEnd);
+            k2 = k1;
+            value2 = value1;
+            loadStage2(k2, nextBegin, nextEnd);
+            loadStage1(i + 2, k1, value1);
+            uint32_t inclusive = mine;
 #pragma unroll
-            for (uint32_t u = 0; u < kAhead; ++u)
+            for (uint32_t d = 1; d < 64; d *= 2)
             {
-                const uint32_t j = min(j0 + u, 63u);
-                s[u] = Uniform(bBegin, j);
-                e[u] = j0 + u < entriesOfA ? Uniform(bEnd, j) : s[u];
-                a[u] = Uniform(aValue, j);
+                const uint32_t other = __shfl_up(inclusive, d, 64);
+                if (lane >= d)
+                    inclusive += other;
             }
-#pragma unroll
-            for (uint32_t u = 0; u < kAhead; ++u)
+            in.before = inclusive - mine;
+            in.products = Uniform(inclusive, 63);
+            if (!LightRow(args, in.entriesOfA, in.products))
             {
-                col[u] = kEmpty;
-                b[u] = 0.0f;
-                if (s[u] + lane < e[u])
-                {
-                    col[u] = args.COLB[s[u] + lane];
-                    b[u] = args.VB[s[u] + lane];
-                }
+                if (MODE != kFill && lane == 0)
+                    args.counts[first + i] = kHeavyMark;  // the strip kernel's row
+                continue;
             }
-            // one product per lane: find or claim the column's slot and add into it
-            auto insert = [&](uint32_t c, float product, bool have) {
-                bool claimed = false;
-                uint32_t h = 0;
-                if (have)
-                {
-                    h = (c * 2654435761u) >> 23;  // top 9 bits: kHashSlots = 512
-                    for (uint32_t tries = 0; tries < kHashSlots; ++tries)
-                    {
-                        const uint32_t k = keys[h];
-                        if (k == c)
-                            break;
-                        if (k == kEmpty)
-                        {
-                            const uint32_t old = atomicCAS(&keys[h], kEmpty, c);
-                            if (old == kEmpty)
-                            {
-                                claimed = true;
-                                break;
-                            }
-                            if (old == c)
-                                break;
-                        }
-                        h = (h + 1) & (kHashSlots - 1);
-                    }
-                    sums[h] = sums[h] + product;
-                }
-                const uint64_t m = __ballot(claimed);
-                if (claimed)
-                    sortKey[listed + static_cast<uint32_t>(__popcll(m & below))] = h;
-                listed += static_cast<uint32_t>(__popcll(m));
-            };
-#pragma unroll
-            for (uint32_t u = 0; u < kAhead; ++u)
+            in.rowBase = 0;
+            in.rowLimit = 0;
+            if (MODE != kCount)
             {
-                insert(col[u], a[u] * b[u], col[u] < args.N);
-                // rows of B with more than 64 entries: the rest, 64 at a time
-                for (uint32_t pb0 = s[u] + 64; pb0 < e[u]; pb0 += 64)
-                {
-                    const bool have = pb0 + lane < e[u];
-                    const uint32_t c = have ? args.COLB[pb0 + lane] : kEmpty;
-                    const float bv = have ? args.VB[pb0 + lane] : 0.0f;
-                    insert(c, a[u] * bv, have && c < args.N);
-                }
+                in.rowBase = Uniform(extentC, i);
+                in.rowLimit = Uniform(extentC, i + 1);
+                if (MODE == kFill)
+                    in.rowLimit = min(in.rowLimit, args.capacity);
             }
+            uint32_t emitted;
+            if (in.products <= 64)
+                emitted = LightRowEntries<MODE, 1, Key>(args, in, scratch[wave], lane);
+            else if (in.products <= 128)
+                emitted = LightRowEntries<MODE, 2, Key>(args, in, scratch[wave], lane);
+            else if (in.products <= 256)
+                emitted = LightRowEntries<MODE, 4, Key>(args, in, scratch[wave], lane);
+            else
+                emitted = LightRowEntries<MODE, 8, Key>(args, in, scratch[wave], lane);
+            if (MODE != kFill && lane == 0)
+                args.counts[first + i] = emitted;
         }
-
-        uint32_t emitted = 0;
-        const uint32_t rowBase = FILL ? Uniform(outBegin, i) : 0u;
-        const uint32_t rowLimit =
-            MODE == kFill ? min(Uniform(outEnd, i), args.capacity) : FILL ? Uniform(outEnd, i) : 0u;
-        if (listed <= 64)
-        {
-            // one (column, sum) pair per lane: sorted in registers with cross-lane exchanges
-            uint32_t c = kEmpty;
-            float v = 0.0f;
-            if (lane < listed)
-            {
-                const uint32_t h = sortKey[lane];
-                c = keys[h];
-                v = sums[h];
-                keys[h] = kEmpty;
-                sums[h] = 0.0f;
-            }
-#pragma unroll
-            for (uint32_t size = 2; size <= 64; size *= 2)
-#pragma unroll
-                for (uint32_t stride = size / 2; stride > 0; stride /= 2)
-                {
-                    const uint32_t oc = __shfl_xor(c, stride, 64);
-                    const float ov = __shfl_xor(v, stride, 64);
-                    // in an ascending run the lower lane of a pair keeps the smaller column
-                    const bool wantsSmaller = ((lane & stride) == 0) == ((lane & size) == 0);
-                    const bool takeOther = wantsSmaller ? oc < c : oc > c;
-                    c = takeOther ? oc : c;
-                    v = takeOther ? ov : v;
-                }
-            const bool keep = c != kEmpty && v != 0.0f;  // exact zeros are not stored
-            const uint64_t m = __ballot(keep);
-            if (FILL)
-            {
-                const uint32_t at = rowBase + static_cast<uint32_t>(__popcll(m & below));
-                if (keep && at < rowLimit)
-                {
-                    args.VC[at] = v;
-                    args.COLC[at] = c;
-                }
-            }
-            emitted = static_cast<uint32_t>(__popcll(m));
-        }
-        else
-        {
-            // the listed slots become (column, sum) pairs, and the table is empty again
-            uint32_t padded = 64;
-            while (padded < listed)
-                padded *= 2;
-            for (uint32_t q = lane; q < padded; q += 64)
-            {
-                uint32_t c = kEmpty;
-                float v = 0.0f;
-                if (q < listed)
-                {
-                    const uint32_t h = sortKey[q];
-                    c = keys[h];
-                    v = sums[h];
-                    keys[h] = kEmpty;
-                    sums[h] = 0.0f;
-                }
-                sortKey[q] = c;
-                sortVal[q] = v;
-            }
-            // bitonic sort by column; the padding (kEmpty) ends up behind the entries
-            for (uint32_t size = 2; size <= padded; size *= 2)
-                for (uint32_t stride = size / 2; stride > 0; stride /= 2)
-                    for (uint32_t t = lane; t < padded / 2; t += 64)
-                    {
-                        const uint32_t lo = 2 * t - (t & (stride - 1));  // lower index of pair t
-                        const uint32_t hi = lo + stride;
-                        const bool ascending = (lo & size) == 0;
-                        const uint32_t kLo = sortKey[lo], kHi = sortKey[hi];
-                        if ((kLo > kHi) == ascending)
-                        {
-                            const float vLo = sortVal[lo], vHi = sortVal[hi];
-                            sortKey[lo] = kHi;
-                            sortKey[hi] = kLo;
-                            sortVal[lo] = vHi;
-                            sortVal[hi] = vLo;
-                        }
-                    }
-            // entries in column order; sums that are exactly zero are not stored
-            for (uint32_t i0 = 0; i0 < listed; i0 += 64)
-            {
-                const uint32_t x = i0 + lane;
-                const float v = x < listed ? sortVal[x] : 0.0f;
-                const bool keep = v != 0.0f;
-                const uint64_t m = __ballot(keep);
-                if (FILL)
-                {
-                    const uint32_t at = rowBase + emitted + static_cast<uint32_t>(__popcll(m & below));
-                    if (keep && at < rowLimit)
-                    {
-                        args.VC[at] = v;
-                        args.COLC[at] = sortKey[x];
-                    }
-                }
-                emitted += static_cast<uint32_t>(__popcll(m));
-            }
-        }
-        if (COUNTS && lane == 0)
-            args.counts[row] = emitted;
-      }
     }
 }
 
@@ -414,19 +449,45 @@ __global__ __launch_bounds__(64) void SpgemmRowKernel(const SpgemmArgs args)
         args.counts[args.M] = 0;
     if (MODE == kStage && blockIdx.x == 0 && lane == 0)
         *args.overflow = 0;
-    // cleared once; every block that is touched is cleared again when it is swept
-    for (uint32_t x = lane; x < args.strip; x += 64)
-        strip[x] = 0.0f;
-    for (uint32_t t = lane; t < wordsInStrip; t += 64)
-        bits[t] = 0;
+    // In a wide product the counts pass has the light rows' counts by now, and the rows left for
+    // this kernel are marked.  Usually there are none or few, so the turns of a wavefront are
+    // looked through first, one per lane, and only those with a marked row are taken (walking
+    // every row for nothing took 28 us on 65536 rows).
+    // The pass after staging looks for rows that did not fit their slot in the same way.
+    const bool selective = COUNTS ? args.heavyOnly != 0 : args.skipUpTo != 0;
+    const uint32_t turns = (args.M - 1) / args.rowsPerTurn + (args.M != 0 ? 1 : 0);
+    auto wanted = [&](uint64_t t) {
+        if (t >= turns)
+            return false;
+        if (!selective)
+            return true;
+        bool any = false;
+        for (uint64_t row = t * args.rowsPerTurn; row < (t + 1) * args.rowsPerTurn; ++row)
+            any |= row < args.M && (COUNTS ? args.counts[row] == kHeavyMark
+                                           : args.ROWC[row + 1] - args.ROWC[row] > args.skipUpTo);
+        return any;
+    };
+    bool cleared = false;
 
     // A wavefront takes rowsPerTurn consecutive rows per turn.  Their extents are read in one
     // go, and the loads that lead to a row's products form a pipeline over the rows of the
     // turn: while row i is multiplied, the first 64 (column, value) pairs of A's row i+2 and
     // the extents of the rows of B that row i+1 needs are already on their way.
-    for (uint32_t turn = blockIdx.x * args.rowsPerTurn; turn < args.M;
-         turn += gridDim.x * args.rowsPerTurn)
+    for (uint64_t base = blockIdx.x; base < turns; base += 64ull * gridDim.x)
+    for (uint64_t chosen = __ballot(wanted(base + static_cast<uint64_t>(lane) * gridDim.x));
+         chosen != 0; chosen &= chosen - 1)
     {
+        if (!cleared)
+        {
+            // once; every element that is touched is cleared again when it is swept
+            for (uint32_t x = lane; x < args.strip; x += 64)
+                strip[x] = 0.0f;
+            for (uint32_t t = lane; t < wordsInStrip; t += 64)
+                bits[t] = 0;
+            cleared = true;
+        }
+        const uint32_t turn = static_cast<uint32_t>(
+            (base + static_cast<uint64_t>(__builtin_ctzll(chosen)) * gridDim.x) * args.rowsPerTurn);
         const uint32_t rowsHere = min(args.rowsPerTurn, args.M - turn);
         uint32_t extentA = 0, extentC = 0;
         if (lane <= rowsHere)
@@ -436,12 +497,6 @@ __global__ __launch_bounds__(64) void SpgemmRowKernel(const SpgemmArgs args)
                 extentC = args.ROWC[turn + lane];
             if (MODE == kStage)
                 extentC = (turn + lane) * args.slot;
-        }
-        if (MODE == kFill && args.skipUpTo != 0)
-        {
-            const uint32_t nextC = __shfl_down(extentC, 1, 64);
-            if (__ballot(lane < rowsHere && nextC - extentC > args.skipUpTo) == 0)
-                continue;  // all rows of this turn are in place already
         }
         // stage 1 (columns and values of A's row) and stage 2 (extents in B) of the pipeline
         auto loadStage1 = [&](uint32_t i, uint32_t& k, float& value) {
@@ -487,8 +542,8 @@ __global__ __launch_bounds__(64) void SpgemmRowKernel(const SpgemmArgs args)
         value2 = value1;
         loadStage2(k2, nextBegin, nextEnd);
         loadStage1(i + 2, k1, value1);
-        // in a wide product the light rows belong to SpgemmHashKernel
-        if (args.heavyOnly != 0 && LightRow(aEnd - aBegin, WaveSum(firstEnd - firstBegin)))
+        // in a wide product the light rows belong to SpgemmLightKernel
+        if (args.heavyOnly != 0 && LightRow(args, aEnd - aBegin, WaveSum(LightCount(firstBegin, firstEnd))))
             continue;
         if (MODE == kFill && rowEnd - rowBase <= args.skipUpTo)
             continue;  // already in place
@@ -684,6 +739,22 @@ __global__ __launch_bounds__(256) void SpgemmUnstageKernel(float* __restrict__ V
         }
 }
 
+// The scan of the counts and the move in one launch.
+__global__ __launch_bounds__(sph::kPlaceThreads) void SpgemmPlaceKernel(
+    float* __restrict__ VC, uint32_t* __restrict__ COLC, uint32_t* __restrict__ ROWC,
+    const uint32_t* __restrict__ counts, const float* __restrict__ stageV,
+    const uint32_t* __restrict__ stageCol, uint32_t M, uint32_t rowsPerGroup, uint32_t slot,
+    uint32_t capacity, uint32_t* overflow)
+{
+    __shared__ sph::PlaceScratch lds;
+    sph::PlaceOffsets(ROWC, counts, M, rowsPerGroup, lds);
+    sph::MoveStagedRows(VC, COLC, stageV, stageCol, M, rowsPerGroup, slot, capacity, lds,
+                        [&](uint32_t, uint32_t, uint32_t) {
+                            if ((threadIdx.x & 63u) == 0)
+                                *overflow = 1;
+                        });
+}
+
 // load[p] = entries of the row of B that entry p of A selects (the multiplications entry p
 // causes); *total (when given, zero before the launch) receives their sum.
 __global__ __launch_bounds__(256) void SpgemmLoadKernel(uint32_t* __restrict__ load,
@@ -715,6 +786,23 @@ __global__ void ClearTotalKernel(unsigned long long* total)
     *total = 0;
 }
 
+// Most products of a row that SpgemmLightKernel takes; products: the caller's bound on the
+// mean products of a row (a capacity is usually that), 0 when there is none.
+// One strip: always the strip kernel (1024 columns, 8 entries per row: 22.3 us, 26.2 us with the
+// second launch).  Two strips: the strip kernel costs little more than on one, and rows of which
+// only a part is light pay both kernels, so all have to be light (8192 columns, 8 / 10 entries
+// per row 53 / 60 -> 29 / 32 us; 16 / 22 entries 75 / 134 us with all rows up to 512 products
+// taken, 77 / 103 us on strips).  From three strips on always (9000 columns, 12 / 18 / 21
+// entries: 110 / 181 / 182 -> 40 / 107 / 160 us).
+uint32_t LightProductsFor(uint32_t N, uint32_t products)
+{
+    if (N <= kStripMax)
+        return 0;
+    if (N <= 2 * kStripMax)
+        return products != 0 && products <= 128 ? 256u : 0u;
+    return kLightProducts;
+}
+
 uint32_t StripFor(uint32_t N)
 {
     const uint32_t padded = (N + 63u) / 64u * 64u;
@@ -729,16 +817,29 @@ uint32_t RowsPerTurnFor(uint32_t M)
     return std::max<uint32_t>(1, std::min<uint32_t>(kRowsPerTurnMax, M / std::max<uint32_t>(wanted, 1)));
 }
 
-// one wavefront per workgroup, rows dealt round robin; 6 KiB of LDS each
-uint32_t HashGridFor(uint32_t M)
+// Light rows: full occupancy is eight workgroups of four wavefronts per compute unit
+template <int MODE>
+void LaunchLight(const SpgemmArgs& args, hipStream_t stream)
 {
-    const uint64_t cap = static_cast<uint64_t>(sph::ComputeUnits()) * 32;
-    return static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(M, cap)));
+    SpgemmArgs light = args;
+    const uint64_t cus = static_cast<uint64_t>(sph::ComputeUnits());
+    light.rowsPerTurn = static_cast<uint32_t>(
+        std::max<uint64_t>(1, std::min<uint64_t>(kRowsPerTurnMax, args.M / (cus * 8 * kLightWaves))));
+    const uint64_t turns = (static_cast<uint64_t>(args.M) + light.rowsPerTurn - 1) / light.rowsPerTurn;
+    const uint64_t groups = std::min<uint64_t>((turns + kLightWaves - 1) / kLightWaves, cus * 64);
+    const dim3 grid(static_cast<uint32_t>(groups)), block(kLightWaves * 64);
+    // column and place share 32 bits up to 2^23 columns (all ones stay free for "no product")
+    if (args.N < (1u << (32 - kPlaceBits)))
+        hipLaunchKernelGGL((SpgemmLightKernel<MODE, uint32_t>), grid, block, 0, stream, light);
+    else
+        hipLaunchKernelGGL((SpgemmLightKernel<MODE, uint64_t>), grid, block, 0, stream, light);
 }
 
-uint32_t GridFor(uint32_t M, uint32_t rowsPerTurn)
+// `selective`: a pass that looks for marked rows takes as many workgroups as are resident
+// (17 KiB of LDS each), each with more turns to look through
+uint32_t GridFor(uint32_t M, uint32_t rowsPerTurn, bool selective)
 {
-    const uint64_t cap = static_cast<uint64_t>(sph::ComputeUnits()) * 64;
+    const uint64_t cap = static_cast<uint64_t>(sph::ComputeUnits()) * (selective ? 9 : 64);
     const uint64_t turns = (static_cast<uint64_t>(M) + rowsPerTurn - 1) / rowsPerTurn;
     return static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(turns, cap)));
 }
@@ -772,10 +873,12 @@ int sph_spgemm_row_offsets_f32(uint32_t* ROWC, const float* VA, const uint32_t* 
     args.strip = StripFor(N);
     args.rowsPerTurn = RowsPerTurnFor(M);
     args.counts = ROWC;
-    args.heavyOnly = N > kHashFromWidth ? 1u : 0u;
+    args.lightProducts = LightProductsFor(N, 0);
+    args.heavyOnly = args.lightProducts != 0 ? 1u : 0u;
     if (args.heavyOnly != 0 && M != 0)
-        hipLaunchKernelGGL(SpgemmHashKernel<kCount>, dim3(HashGridFor(M)), dim3(64), 0, stream, args);
-    hipLaunchKernelGGL(SpgemmRowKernel<kCount>, dim3(GridFor(M, args.rowsPerTurn)), dim3(64),
+        LaunchLight<kCount>(args, stream);
+    hipLaunchKernelGGL(SpgemmRowKernel<kCount>,
+                       dim3(GridFor(M, args.rowsPerTurn, args.heavyOnly != 0)), dim3(64),
                        args.strip * sizeof(float) + args.strip / 8, stream, args);
     SPH_CHECK_LAUNCH();
     return sph::ExclusiveScanInPlace(ROWC, M + 1, nnzHost, stream);
@@ -809,10 +912,11 @@ int sph_spgemm_fill_f32(float* VC, uint32_t* COLC, const uint32_t* ROWC, const f
     args.VC = VC;
     args.COLC = COLC;
     args.capacity = 0xffffffffu;
-    args.heavyOnly = N > kHashFromWidth ? 1u : 0u;
+    args.lightProducts = LightProductsFor(N, 0);
+    args.heavyOnly = args.lightProducts != 0 ? 1u : 0u;
     if (args.heavyOnly != 0)
-        hipLaunchKernelGGL(SpgemmHashKernel<kFill>, dim3(HashGridFor(M)), dim3(64), 0, stream, args);
-    hipLaunchKernelGGL(SpgemmRowKernel<kFill>, dim3(GridFor(M, args.rowsPerTurn)), dim3(64),
+        LaunchLight<kFill>(args, stream);
+    hipLaunchKernelGGL(SpgemmRowKernel<kFill>, dim3(GridFor(M, args.rowsPerTurn, false)), dim3(64),
                        args.strip * sizeof(float) + args.strip / 8, stream, args);
     SPH_CHECK_LAUNCH();
     return SPH_OK;
@@ -889,42 +993,61 @@ int sph_spgemm_f32(float* VC, uint32_t* COLC, uint32_t* ROWC, uint32_t capacity,
     args.strip = StripFor(N);
     args.rowsPerTurn = RowsPerTurnFor(M);
     args.counts = ROWC;
-    args.heavyOnly = N > kHashFromWidth ? 1u : 0u;
-    const dim3 hashGrid(HashGridFor(M)), rowGrid(GridFor(M, args.rowsPerTurn)), wave(64);
+    args.lightProducts = LightProductsFor(N, M != 0 ? capacity / M : 0);
+    args.heavyOnly = args.lightProducts != 0 ? 1u : 0u;
+    const dim3 rowGrid(GridFor(M, args.rowsPerTurn, args.heavyOnly != 0)), wave(64);
     const size_t rowLds = args.strip * sizeof(float) + args.strip / 8;
 
-    // staging slot per row: twice the mean the capacity allows plus 64; without room for that
-    // (or without rows) the count, scan and fill passes run one after the other
-    const uint64_t slot = M != 0 ? 2 * static_cast<uint64_t>(capacity / M) + 64 : 0;
+    // staging slot per row: three times the mean the capacity allows plus 64 (twice, where
+    // that is too much); without room for that (or without rows) the count, scan and fill
+    // passes run one after the other.  Twice the mean is too little for rows whose lengths
+    // vary like those of a random graph: of 65536 rows with 64 products on average one or
+    // two did not fit, and doing those again cost 74 us.
+    const uint64_t mean = M != 0 ? capacity / M : 0;
+    uint64_t slot = M != 0 ? 3 * mean + 64 : 0;
+    if (slot * M >= (1ull << 31))
+        slot = 2 * mean + 64;
     const bool staged = M != 0 && N != 0 && capacity != 0 && slot * M < (1ull << 31);
+    const bool placed = staged && M <= sph::kPlaceMaxRows;
     float* stageV = nullptr;
     if (staged)
     {
+        // counts (16-byte aligned, when the move scans them), values, columns, one flag
+        const size_t counts = placed ? (static_cast<size_t>(M) + 4) / 4 * 4 : 0;
         ::sph::CountAllocation();
-        SPH_HIP_TRY(hipMallocAsync(reinterpret_cast<void**>(&stageV), slot * M * 8 + 4, stream));
-        args.VC = stageV;
-        args.COLC = reinterpret_cast<uint32_t*>(stageV + slot * M);
+        SPH_HIP_TRY(hipMallocAsync(reinterpret_cast<void**>(&stageV), counts * 4 + slot * M * 8 + 4,
+                                   stream));
+        if (placed)
+            args.counts = reinterpret_cast<uint32_t*>(stageV);
+        args.VC = stageV + counts;
+        args.COLC = reinterpret_cast<uint32_t*>(args.VC + slot * M);
         args.overflow = args.COLC + slot * M;
         args.slot = static_cast<uint32_t>(slot);
         if (args.heavyOnly != 0)
-            hipLaunchKernelGGL(SpgemmHashKernel<kStage>, hashGrid, wave, 0, stream, args);
+            LaunchLight<kStage>(args, stream);
         hipLaunchKernelGGL(SpgemmRowKernel<kStage>, rowGrid, wave, rowLds, stream, args);
     }
     else
     {
         if (args.heavyOnly != 0 && M != 0)
-            hipLaunchKernelGGL(SpgemmHashKernel<kCount>, hashGrid, wave, 0, stream, args);
+            LaunchLight<kCount>(args, stream);
         hipLaunchKernelGGL(SpgemmRowKernel<kCount>, rowGrid, wave, rowLds, stream, args);
     }
     hipError_t launched = hipGetLastError();
     int rc = SPH_OK;
-    if (launched == hipSuccess)
+    if (launched == hipSuccess && !placed)
         rc = sph::ExclusiveScanInPlace(ROWC, M + 1, nullptr, stream);
     if (launched == hipSuccess && rc == SPH_OK && M != 0 && N != 0 && capacity != 0)
     {
-        if (staged)
+        const uint32_t rowsPerGroup = sph::PlaceRowsPerGroup(M);
+        if (placed)
+            hipLaunchKernelGGL(SpgemmPlaceKernel, dim3((M + rowsPerGroup - 1) / rowsPerGroup),
+                               dim3(sph::kPlaceThreads), 0, stream, VC, COLC, ROWC, args.counts,
+                               args.VC, args.COLC, M, rowsPerGroup, args.slot, capacity,
+                               args.overflow);
+        else if (staged)
             hipLaunchKernelGGL(SpgemmUnstageKernel, dim3((M + 3) / 4), dim3(256), 0, stream, VC,
-                               COLC, ROWC, stageV, args.COLC, M, args.slot, capacity,
+                               COLC, ROWC, args.VC, args.COLC, M, args.slot, capacity,
                                args.overflow);
         // rows that did not fit their slot (all rows, without staging) are multiplied again
         args.ROWC = ROWC;
@@ -936,10 +1059,12 @@ int sph_spgemm_f32(float* VC, uint32_t* COLC, uint32_t* ROWC, uint32_t capacity,
         // is launched with few workgroups, which walk all rows if they must: dispatching the
         // full grid of empty workgroups alone took 15 us
         const uint32_t few = static_cast<uint32_t>(sph::ComputeUnits()) * 2;
-        const dim3 fillHashGrid(staged ? std::min(hashGrid.x, few) : hashGrid.x);
-        const dim3 fillRowGrid(staged ? std::min(rowGrid.x, few) : rowGrid.x);
-        if (args.heavyOnly != 0)
-            hipLaunchKernelGGL(SpgemmHashKernel<kFill>, fillHashGrid, wave, 0, stream, args);
+        const uint32_t fillGrid = GridFor(M, args.rowsPerTurn, false);
+        const dim3 fillRowGrid(staged ? std::min(fillGrid, few) : fillGrid);
+        if (staged)
+            args.heavyOnly = 0;  // rows that overflowed, light ones too: one launch for both
+        else if (args.heavyOnly != 0)
+            LaunchLight<kFill>(args, stream);
         hipLaunchKernelGGL(SpgemmRowKernel<kFill>, fillRowGrid, wave, rowLds, stream, args);
         launched = hipGetLastError();
     }

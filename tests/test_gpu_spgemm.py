@@ -235,3 +235,78 @@ def test_wide_product_mixes_table_rows_and_strip_rows(dev):
     assert np.array_equal(ROW, wR) and np.array_equal(COL, wC)
     assert np.array_equal(bits(V), bits(wV))
     check_one_call(A, B, M, K, N, (wV, wC, wR))
+
+
+@pytest.mark.parametrize("N,capacity_per_row", [(4097, 128), (4097, 129), (8193, 600), ((1 << 23) - 1, 600),
+                                                (1 << 23, 600)])
+def test_light_rows_at_the_edges_of_their_sort(dev, N, capacity_per_row):
+    """Rows of 63 .. 513 products (a lane sorts 1, 2, 4 or 8 of them, more go to the strips), of
+    64 and 65 entries of A, with every product in one column, with columns that cancel, with NaN,
+    infinities and -0, and rows of B in descending column order; widths on both sides of the rule
+    and of the 32-bit sort keys.  One more than the staged rows' workgroups hold rows."""
+    h.announce("sph_spgemm_* light rows at the edges", (N, capacity_per_row))
+    rng = np.random.default_rng(N)
+    counts = [1, 2, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513]
+    lists = []  # rows of B: (columns, values)
+    for n in counts:  # 0 .. 13: n entries, descending columns
+        cols = np.sort(rng.choice(N, size=n, replace=False))[::-1]
+        lists.append((cols, rng.uniform(-1, 1, n)))
+    lists.append((np.array([N - 1]), np.array([0.5])))                        # 14: last column only
+    lists.append((np.array([7, N - 1]), np.array([-0.5, -0.0])))              # 15
+    lists.append((np.array([3, 5, 7]), np.array([np.nan, np.inf, -np.inf])))  # 16
+    lists.append((np.array([], np.int64), np.array([])))                      # 17: empty
+    for k in range(18, 90):
+        cols = rng.choice(min(N, 40 + 60 * (k % 3)), size=1 + k % 8, replace=False)
+        lists.append((cols, rng.uniform(-1, 1, len(cols))))
+    K = len(lists)
+    RB = np.concatenate([[0], np.cumsum([len(c) for c, _ in lists])]).astype(np.uint32)
+    CB = np.concatenate([c for c, _ in lists]).astype(np.uint32)
+    VB = np.concatenate([v for _, v in lists]).astype(np.float32)
+    rows = [[i] for i in range(18)]                       # one row of B each
+    rows += [[3, 17, 0], [3, 0, 1], [14] * 64, [14] * 65, [14, 14, 15], [15, 16, 15], [16, 5],
+             [9, 9], [9, 9, 0], list(range(18, 82)), list(range(18, 83)), []]
+    rows += [list(rng.choice(np.arange(18, 90), size=int(rng.integers(1, 64)))) for _ in range(60)]
+    values = [rng.uniform(-1, 1, len(r)) for r in rows]
+    values[22] = np.array([1.0, -1.0, 0.25])              # the last column cancels
+    M = len(rows)
+    RA = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.uint32)
+    CA = np.concatenate([np.asarray(r, np.int64) for r in rows]).astype(np.uint32)
+    VA = np.concatenate(values).astype(np.float32)
+    A, B = (VA, CA, RA), (VB, CB, RB)
+    wV, wC, wR = po.spgemm_csr(A, B, M, K, N)
+    V, COL, ROW = gpu_spgemm(A, B, M, K, N)
+    nan = np.isnan(wV)
+    assert np.array_equal(ROW, wR) and np.array_equal(COL, wC)
+    assert np.array_equal(np.isnan(V), nan) and np.array_equal(bits(V)[~nan], bits(wV)[~nan])
+    total = int(wR[M])
+    for capacity in (capacity_per_row * M, capacity_per_row * M + M - 1, total // 2, M):
+        V, COL, ROW, nnz = gpu_spgemm_one_call(A, B, M, K, N, capacity)
+        kept = min(capacity, total)
+        assert nnz == total and np.array_equal(ROW, wR)
+        assert np.array_equal(COL[:kept], wC[:kept])
+        assert np.array_equal(np.isnan(V[:kept]), nan[:kept])
+        assert np.array_equal(bits(V[:kept])[~nan[:kept]], bits(wV[:kept])[~nan[:kept]])
+
+
+@pytest.mark.parametrize("M", [15, 16, 17, 8191, 8193, 131072, 131073])
+def test_staged_rows_find_their_place(dev, M):
+    """The offsets that every workgroup of the move adds up by itself: fewer rows than it has
+    wavefronts, one more than whole groups of rows, the last number of rows and the first that is
+    scanned by launches of its own; a row now and then overflows its slot."""
+    h.announce("sph_spgemm_f32 rows", M)
+    K = N = 300
+    rng = np.random.default_rng(M)
+    per = rng.integers(0, 4, M)
+    RA = np.concatenate([[0], np.cumsum(per)]).astype(np.uint32)
+    CA = rng.integers(0, K, int(RA[M])).astype(np.uint32)
+    VA = rng.uniform(-1, 1, len(CA)).astype(np.float32)
+    lengths = np.where(np.arange(K) == 5, 280, rng.integers(0, 3, K))
+    RB = np.concatenate([[0], np.cumsum(lengths)]).astype(np.uint32)
+    CB = np.concatenate([rng.choice(N, size=n, replace=False) for n in lengths]).astype(np.uint32)
+    VB = rng.uniform(-1, 1, len(CB)).astype(np.float32)
+    A, B = (VA, CA, RA), (VB, CB, RB)
+    wV, wC, wR = po.spgemm_csr(A, B, M, K, N)
+    total = int(wR[M])
+    V, COL, ROW, nnz = gpu_spgemm_one_call(A, B, M, K, N, total + M)
+    assert nnz == total and np.array_equal(ROW, wR) and np.array_equal(COL[:total], wC)
+    assert np.array_equal(bits(V[:total]), bits(wV))
