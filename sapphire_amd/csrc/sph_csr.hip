@@ -16,6 +16,7 @@
 // length) so that narrow matrices do not idle most of a wavefront; each lane takes 4
 // consecutive columns (16 bytes) per step.
 #include "sph_internal.h"
+#include "sph_place_rows.h"
 
 #include <algorithm>
 #include <mutex>
@@ -23,6 +24,10 @@
 namespace
 {
 constexpr int kThreads = 256;
+// 16-byte loads that a lane of the count and fill passes has in flight on long rows.  One at a
+// time a row of 8192 columns was 32 round trips to memory: 1100 x 8000 at 1 % 36 us, with four
+// 26 us (eight: 26 us), 1024 x 4096 17.7 / 14.3 us.
+constexpr uint32_t kAhead = 4;
 
 // Block totals of the row-offset scan for sph_csr_row_offsets_noalloc_f32: one 32-bit total
 // per 4096 counts, 4096 totals = 16 KiB per device for the life of the process.  In host code
@@ -40,7 +45,9 @@ struct DenseView
     uint32_t M, N, ld;
 };
 
-// 4 consecutive columns of one row; columns past N read as 0
+// 4 consecutive columns of one row; columns past N read as 0.  ONCE: the matrix is not read again
+// soon, the load asks the caches not to keep it
+template <bool ONCE = false>
 __device__ __forceinline__ float4 LoadQuad(const DenseView& d, uint32_t row, uint32_t col,
                                            bool rowOk)
 {
@@ -53,7 +60,8 @@ __device__ __forceinline__ float4 LoadQuad(const DenseView& d, uint32_t row, uin
         {
             typedef float floatx4 __attribute__((ext_vector_type(4)));
             typedef floatx4 floatx4a4 __attribute__((aligned(4)));
-            const floatx4 w = *reinterpret_cast<const floatx4a4*>(p);
+            const floatx4a4* wide = reinterpret_cast<const floatx4a4*>(p);
+            const floatx4 w = ONCE ? __builtin_nontemporal_load(wide) : *wide;
             v = make_float4(w[0], w[1], w[2], w[3]);
         }
         else
@@ -85,11 +93,23 @@ __global__ __launch_bounds__(kThreads) void CsrCountKernel(uint32_t* __restrict_
         const uint32_t row = pass * rowsPerPass + blockIdx.x * kGroups + group;
         const bool rowOk = row < d.M;
         uint32_t c = 0;
-        for (uint32_t col = lane * 4; col < d.N; col += LPR * 4)
-        {
-            const float4 v = LoadQuad(d, row, col, rowOk);
+        auto count = [&](const float4& v) {
             c += (v.x != 0.f) + (v.y != 0.f) + (v.z != 0.f) + (v.w != 0.f);
+        };
+        uint32_t col = lane * 4;
+        // long rows: kAhead loads of a lane in flight
+        for (; col - lane * 4 + kAhead * LPR * 4 <= d.N; col += kAhead * LPR * 4)
+        {
+            float4 v[kAhead];
+#pragma unroll
+            for (uint32_t u = 0; u < kAhead; ++u)
+                v[u] = LoadQuad(d, row, col + u * LPR * 4, rowOk);
+#pragma unroll
+            for (uint32_t u = 0; u < kAhead; ++u)
+                count(v[u]);
         }
+        for (; col < d.N; col += LPR * 4)
+            count(LoadQuad(d, row, col, rowOk));
 #pragma unroll
         for (int off = LPR / 2; off > 0; off >>= 1)
             c += __shfl_xor(c, off, LPR);
@@ -240,10 +260,7 @@ __global__ __launch_bounds__(kThreads) void CsrFillKernel(float* __restrict__ V,
         // a ROW that was not computed from this matrix must not make the stores run past the
         // row, and nothing is stored past the capacity of V and COL
         const uint32_t rowEnd = rowOk ? min(ROW[row + 1], capacity) : 0u;
-        for (uint32_t col0 = 0; col0 < d.N; col0 += LPR * 4)
-        {
-            const uint32_t col = col0 + lane * 4;
-            const float4 q = LoadQuad(d, row, col, rowOk);
+        auto store = [&](const float4& q, uint32_t col) {
             const float v[4] = { q.x, q.y, q.z, q.w };
             // entries are ordered by (lane, element): everything lower lanes keep comes first
             uint32_t before = 0, kept = 0;
@@ -264,7 +281,20 @@ __global__ __launch_bounds__(kThreads) void CsrFillKernel(float* __restrict__ V,
                     ++at;
                 }
             slot += kept;
+        };
+        uint32_t col0 = 0;
+        for (; col0 + kAhead * LPR * 4 <= d.N; col0 += kAhead * LPR * 4)
+        {
+            float4 q[kAhead];
+#pragma unroll
+            for (uint32_t u = 0; u < kAhead; ++u)
+                q[u] = LoadQuad(d, row, col0 + (u * LPR + lane) * 4, rowOk);
+#pragma unroll
+            for (uint32_t u = 0; u < kAhead; ++u)
+                store(q[u], col0 + (u * LPR + lane) * 4);
         }
+        for (; col0 < d.N; col0 += LPR * 4)
+            store(LoadQuad(d, row, col0 + lane * 4, rowOk), col0 + lane * 4);
     }
 }
 
@@ -282,6 +312,11 @@ __global__ __launch_bounds__(kThreads) void CsrFillKernel(float* __restrict__ V,
 // place (8 bytes read and written per entry).  A row with more than `stage` entries (the slot is
 // sized from the caller's capacity, twice the mean plus 32) is rebuilt from the dense matrix by
 // the second kernel instead, so any input converts correctly.
+//
+// The pass is bound by reading the matrix, and by what those reads push out of the caches: with
+// ordinary loads a matrix that is larger than they are replaces lines that other kernels wrote
+// and that have to go to memory first.  8192 x 8192 at 1 % after 300 MB of stores: 84 us
+// (3.2 TB/s), with loads that are not kept 46 us (5.9 TB/s; counting alone 78 and 42 us).
 // ---------------------------------------------------------------------------
 constexpr uint32_t kStageWaves = 4;  // wavefronts per workgroup
 
@@ -310,7 +345,7 @@ __global__ __launch_bounds__(kStageWaves * 64) void CsrStageKernel(
     for (int j = 0; j < QUADS; ++j)
     {
         const uint32_t col = ((part * QUADS + j) * 64 + lane) * 4;
-        q[j] = LoadQuad(d, row, col, rowOk);
+        q[j] = LoadQuad<true>(d, row, col, rowOk);
     }
     uint32_t total = 0;  // the same in every lane
 #pragma unroll
@@ -367,37 +402,15 @@ __global__ __launch_bounds__(kStageWaves * 64) void CsrStageKernel(
     }
 }
 
-// One wavefront per row: staged entries move to ROW[row] ..; a row that did not fit its staging
-// slot is read from the dense matrix again.  Nothing is stored at or past `capacity`.
-__global__ __launch_bounds__(256) void CsrUnstageKernel(float* __restrict__ V,
-                                                        uint32_t* __restrict__ COL,
-                                                        const uint32_t* __restrict__ ROW,
-                                                        const float* __restrict__ stageV,
-                                                        const uint32_t* __restrict__ stageCol,
-                                                        const uint32_t stage,
-                                                        const uint32_t capacity, const DenseView d)
+// A row that did not fit its staging slot is read from the dense matrix again, by one wavefront;
+// its entries go to `slot` onwards.  Nothing is stored at or past `capacity`.
+__device__ __forceinline__ void RebuildRow(float* __restrict__ V, uint32_t* __restrict__ COL,
+                                           uint32_t slot, const uint32_t row,
+                                           const uint32_t capacity, const DenseView& d)
 {
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= d.M)
-        return;
-    const uint32_t first = ROW[row];
-    const uint32_t count = ROW[row + 1] - first;
-    if (count <= stage)
-    {
-        const float* inV = stageV + static_cast<size_t>(row) * stage;
-        const uint32_t* inCol = stageCol + static_cast<size_t>(row) * stage;
-        for (uint32_t i = lane; i < count; i += 64)
-            if (first + i < capacity)
-            {
-                V[first + i] = inV[i];
-                COL[first + i] = inCol[i];
-            }
-        return;
-    }
     const uint64_t below = (1ull << lane) - 1ull;
-    uint32_t slot = first;
-    for (uint32_t col0 = 0; col0 < d.N; col0 += 256)
+    for (uint32_t col0 = 0; col0 < d.N && slot < capacity; col0 += 256)
     {
         const uint32_t col = col0 + lane * 4;
         const float4 q = LoadQuad(d, row, col, true);
@@ -424,6 +437,51 @@ __global__ __launch_bounds__(256) void CsrUnstageKernel(float* __restrict__ V,
             }
         slot += kept;
     }
+}
+
+// One wavefront per row: staged entries move to ROW[row] .., overfull rows are rebuilt.
+__global__ __launch_bounds__(256) void CsrUnstageKernel(float* __restrict__ V,
+                                                        uint32_t* __restrict__ COL,
+                                                        const uint32_t* __restrict__ ROW,
+                                                        const float* __restrict__ stageV,
+                                                        const uint32_t* __restrict__ stageCol,
+                                                        const uint32_t stage,
+                                                        const uint32_t capacity, const DenseView d)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= d.M)
+        return;
+    const uint32_t first = ROW[row];
+    const uint32_t count = ROW[row + 1] - first;
+    if (count > stage)
+    {
+        RebuildRow(V, COL, first, row, capacity, d);
+        return;
+    }
+    const float* inV = stageV + static_cast<size_t>(row) * stage;
+    const uint32_t* inCol = stageCol + static_cast<size_t>(row) * stage;
+    for (uint32_t i = lane; i < count; i += 64)
+        if (first + i < capacity)
+        {
+            V[first + i] = inV[i];
+            COL[first + i] = inCol[i];
+        }
+}
+
+// The scan of the counts and the move in one launch.
+__global__ __launch_bounds__(sph::kPlaceThreads) void CsrPlaceKernel(
+    float* __restrict__ V, uint32_t* __restrict__ COL, uint32_t* __restrict__ ROW,
+    const uint32_t* __restrict__ counts, const float* __restrict__ stageV,
+    const uint32_t* __restrict__ stageCol, const uint32_t rowsPerGroup, const uint32_t stage,
+    const uint32_t capacity, const DenseView d)
+{
+    __shared__ sph::PlaceScratch lds;
+    sph::PlaceOffsets(ROW, counts, d.M, rowsPerGroup, lds);
+    sph::MoveStagedRows(V, COL, stageV, stageCol, d.M, rowsPerGroup, stage, capacity, lds,
+                        [&](uint32_t row, uint32_t begin, uint32_t) {
+                            RebuildRow(V, COL, begin, row, capacity, d);
+                        });
 }
 
 // One wavefront per row, one pass over the dense matrix.  A row of at most 128 entries is
@@ -725,8 +783,9 @@ int sph_csr_from_dense_f32(float* V, uint32_t* COL, uint32_t* ROW, uint32_t capa
     // plus 32, a multiple of 4
     const uint64_t mean = M != 0 ? capacity / M : 0;
     const uint64_t stage64 = (2 * mean + 32 + 3) / 4 * 4;
-    // (below 16 Mi elements the three launches of the one-pass path cost more than the second
-    // pass over the matrix they save: 8192 x 1000 18 us against 26 us, equal at 8192 x 2048)
+    // (below 16 Mi elements the scratch allocation of the one-pass path costs more host time than
+    // the second pass over the matrix it saves: 2048 x 2048 19 us against 12 us, 8192 x 1000 23
+    // against 19 us; 4096 x 4096 20 us either way)
     if (!(M != 0 && N >= 128 && N <= 8192 && stage64 * 4 <= N &&
           static_cast<uint64_t>(M) * N >= (1ull << 24)))
     {
@@ -760,14 +819,20 @@ int sph_csr_from_dense_f32(float* V, uint32_t* COL, uint32_t* ROW, uint32_t capa
         quads *= 2;
     const uint32_t stage = static_cast<uint32_t>(stage64);
     const size_t stageEntries = static_cast<size_t>(M) * stage;
-    float* stageV = nullptr;
+    const bool placed = M <= sph::kPlaceMaxRows;
+    // counts (16-byte aligned, when the move scans them), values, columns
+    const size_t countEntries = placed ? (static_cast<size_t>(M) + 4) / 4 * 4 : 0;
+    uint32_t* block0 = nullptr;
     ::sph::CountAllocation();
-    SPH_HIP_TRY(hipMallocAsync(reinterpret_cast<void**>(&stageV), stageEntries * 8, stream));
+    SPH_HIP_TRY(hipMallocAsync(reinterpret_cast<void**>(&block0), countEntries * 4 + stageEntries * 8,
+                               stream));
+    uint32_t* counts = placed ? block0 : ROW;
+    float* stageV = reinterpret_cast<float*>(block0 + countEntries);
     uint32_t* stageCol = reinterpret_cast<uint32_t*>(stageV + stageEntries);
     const uint32_t rowsPerGroup = kStageWaves / wpr;
     const dim3 grid((M + rowsPerGroup - 1) / rowsPerGroup), block(kStageWaves * 64);
 #define SPH_STAGE(W, Q)                                                                        \
-    hipLaunchKernelGGL((CsrStageKernel<W, Q>), grid, block, 0, stream, stageV, stageCol, ROW,   \
+    hipLaunchKernelGGL((CsrStageKernel<W, Q>), grid, block, 0, stream, stageV, stageCol, counts, \
                        stage, d)
     if (wpr == 1)
         SPH_STAGE(1, 1);
@@ -784,15 +849,23 @@ int sph_csr_from_dense_f32(float* V, uint32_t* COL, uint32_t* ROW, uint32_t capa
 #undef SPH_STAGE
     hipError_t launched = hipGetLastError();
     int rc = SPH_OK;
-    if (launched == hipSuccess)
+    if (launched == hipSuccess && placed)
+    {
+        const uint32_t rowsPerPlace = sph::PlaceRowsPerGroup(M);
+        hipLaunchKernelGGL(CsrPlaceKernel, dim3((M + rowsPerPlace - 1) / rowsPerPlace),
+                           dim3(sph::kPlaceThreads), 0, stream, V, COL, ROW, counts, stageV,
+                           stageCol, rowsPerPlace, stage, capacity, d);
+        launched = hipGetLastError();
+    }
+    else if (launched == hipSuccess)
         rc = sph::ExclusiveScanInPlace(ROW, M + 1, nullptr, stream);
-    if (launched == hipSuccess && rc == SPH_OK && capacity != 0)
+    if (launched == hipSuccess && rc == SPH_OK && !placed && capacity != 0)
     {
         hipLaunchKernelGGL(CsrUnstageKernel, dim3((M + 3) / 4), dim3(256), 0, stream, V, COL, ROW,
                            stageV, stageCol, stage, capacity, d);
         launched = hipGetLastError();
     }
-    SPH_HIP_TRY(hipFreeAsync(stageV, stream));
+    SPH_HIP_TRY(hipFreeAsync(block0, stream));
     if (launched != hipSuccess)
         return sph::Fail(SPH_ERR_DEVICE, std::string("sph_csr_from_dense_f32 - launch failed with ") +
                                              hipGetErrorString(launched));

@@ -236,3 +236,30 @@ def test_sparse_linear_forward_equals_dense_layer_on_cpu(dev, dims):
     want = po.linear_forward(x, W, bias, threads=8)
     got = hl.sparse_linear_forward(x, W, bias)
     assert np.array_equal(bits(got), bits(want))
+
+
+@pytest.mark.parametrize("shape", [(131072, 128), (131073, 128), (2049, 8192), (37, 1023), (37, 1024),
+                                   (37, 1025), (5, 4100), (3, 2048)])
+def test_one_call_conversion_at_the_edges_of_its_passes(dev, shape):
+    """The last number of rows whose offsets are added up by the move itself and the first that is
+    scanned by launches of its own; a last, short group of rows; rows on both sides of whole
+    batches of loads in the two-pass kernels.  A few rows overflow their slot."""
+    M, N = shape
+    rng = np.random.default_rng(M + N)
+    dense = np.zeros((M, N), np.float32)
+    entries = 2 * M + 50
+    dense[rng.integers(0, M, entries), rng.integers(0, N, entries)] = \
+        rng.uniform(0.5, 1, entries).astype(np.float32)
+    dense[M // 2, : min(N, 120)] = 1.0
+    h.announce("sph_csr_from_dense_f32 M N =", shape)
+    rows, cols = np.nonzero(dense)
+    wantRow = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=M))]).astype(np.uint32)
+    total = len(rows)
+    for capacity in (total + 5, M // 2, 0):
+        V, COL, ROW, nnz = gpu_csr_one_call(dense, N, capacity)
+        kept = min(capacity, total)
+        assert nnz == total and np.array_equal(ROW, wantRow), capacity
+        assert np.array_equal(COL[:kept], cols[:kept]), capacity
+        assert np.array_equal(bits(V[:kept]), bits(dense[rows[:kept], cols[:kept]])), capacity
+        if capacity > total:
+            assert np.all(V[total:] == -77.0)
