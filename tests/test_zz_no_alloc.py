@@ -113,20 +113,27 @@ def test_recordable_into_a_graph(dev):
     dRow.release()
 
 
+def _free_device_memory():
+    # the HIP runtime that the library is linked with (torch brings one of its own, which cannot
+    # take the device once this one has)
+    free, total = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    assert capi.lib().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
 def test_device_memory_in_use_does_not_grow(dev):
     """Free device memory before and after many calls whose scan needs the block totals: a scratch
     block of 16 KiB taken and kept by each call would add up to 32 MiB."""
-    import torch
     M = 16000000
     dD = capi.DeviceBuffer.from_array(np.ones(M, np.float32))
     dRow = capi.DeviceBuffer(4 * (M + 1))
     h.announce("sph_csr_row_offsets_noalloc_f32 x 2000, rows =", M)
     capi.call("sph_csr_row_offsets_noalloc_f32", dRow.ptr, dD.ptr, M, 1, 1)
     capi.sync()
-    before = torch.cuda.mem_get_info()[0]
+    before = _free_device_memory()
     for _ in range(2000):
         capi.call("sph_csr_row_offsets_noalloc_f32", dRow.ptr, dD.ptr, M, 1, 1)
     capi.sync()
-    assert before - torch.cuda.mem_get_info()[0] < 8 << 20
+    assert before - _free_device_memory() < 8 << 20
     dD.release()
     dRow.release()
