@@ -1514,14 +1514,24 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF32SkinnyKernel(const GemmF32A
 // ---------------------------------------------------------------------------
 // One output row (M = 1):  out[1 x N] (+)= a[1 x K] * B[K x N], e.g. the column sums
 // ones x dy of the bias gradient.  A matrix-core tile would use one of its 32 rows; this is a
-// plain reduction bound by reading B once.  A workgroup owns 64 consecutive columns (one per
-// lane, 256-byte row segments) and splits K over its 16 wavefronts; the 16 partial sums are
-// added in wavefront order through LDS, so the result does not depend on timing.
+// plain reduction bound by reading B once.  A workgroup owns COLS consecutive columns and splits
+// K over its 16 wavefronts, whose 64 lanes read 64 / COLS rows of COLS columns at a time; the 16
+// partial sums of a lane are added in wavefront order through LDS and those of a column's lanes
+// in a fixed order after that, so the result does not depend on timing.
+// 64 columns: 256-byte row segments.  A narrow B then keeps few compute units busy (16 of 256 at
+// N = 1024), each with a chain of K / 16 rows per lane, and that chain of loads is the time of
+// the launch.  16 columns: 64-byte segments, four times the workgroups, a quarter of the chain.
+// Per call, 64 / 16 columns (a call costs the host 3.4 us): 10 x 1024 (N x K) 5.7 / 3.5 us,
+// 1024 x 1024 5.6 / 3.4, 1000 x 1001 5.7 / 3.9, 2048 x 1024 5.6 / 5.1; past half as many
+// workgroups as compute units the other way: 4096 x 1024 6.4 / 7.2 (with 4 x 4 loads in flight),
+// 8192 x 1024 7.3 / 11.9, 512 x 512 x batch 16 4.6 / 7.0.
 // ---------------------------------------------------------------------------
 constexpr int kGemvWaves = 16;
 
+template <int COLS>
 __global__ __launch_bounds__(kGemvWaves * 64) void GemvRowKernel(const GemmF32Args args)
 {
+    constexpr uint32_t kRows = 64 / COLS;  // rows of B a wavefront reads at once
     __shared__ float partial[kGemvWaves][64];
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = threadIdx.x >> 6;
@@ -1530,41 +1540,82 @@ __global__ __launch_bounds__(kGemvWaves * 64) void GemvRowKernel(const GemmF32Ar
     const float* __restrict__ B = args.B + args.strideB * static_cast<int64_t>(unit);
     float* __restrict__ out = args.out + args.strideOut * static_cast<int64_t>(unit);
     const uint32_t N = args.N, K = args.K;
-    const uint32_t col = blockIdx.x * 64 + lane;
+    const uint32_t col = blockIdx.x * COLS + lane % COLS;
     const bool colOk = col < N;
 
     const uint32_t perWave = (K + kGemvWaves - 1) / kGemvWaves;
     const uint32_t kBegin = min(wave * perWave, K);
     const uint32_t kEnd = min(kBegin + perWave, K);
-    // four independent chains keep loads in flight; they are combined in a fixed order
+    // four independent chains, combined in a fixed order
     float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
     if (colOk)
     {
-        const float* p = B + static_cast<size_t>(kBegin) * N + col;
-        uint32_t k = kBegin;
-#pragma unroll 4
-        for (; k + 4 <= kEnd; k += 4)
+        uint32_t k = kBegin + lane / COLS;
+        if constexpr (kRows > 1)
         {
-            s0 = fmaf(a[k + 0], p[0], s0);
-            s1 = fmaf(a[k + 1], p[static_cast<size_t>(N)], s1);
-            s2 = fmaf(a[k + 2], p[2 * static_cast<size_t>(N)], s2);
-            s3 = fmaf(a[k + 3], p[3 * static_cast<size_t>(N)], s3);
-            p += 4 * static_cast<size_t>(N);
+            // 16 rows of a lane in flight at once; those past its range load the last row of
+            // the range and are kept out of the sums by a select
+            constexpr int kFlight = 16;
+            const float* column = B + col;
+            for (; k < kEnd; k += kFlight * kRows)
+            {
+                float x[kFlight], y[kFlight];
+#pragma unroll
+                for (int u = 0; u < kFlight; ++u)
+                {
+                    const uint32_t at = min(k + u * kRows, kEnd - 1);
+                    x[u] = a[at];
+                    y[u] = column[static_cast<size_t>(at) * N];
+                }
+#pragma unroll
+                for (int u = 0; u < kFlight; ++u)
+                {
+                    const bool mine = k + u * kRows < kEnd;
+                    x[u] = mine ? x[u] : 0.f;
+                    y[u] = mine ? y[u] : 0.f;
+                }
+#pragma unroll
+                for (int u = 0; u < kFlight; u += 4)
+                {
+                    s0 = fmaf(x[u + 0], y[u + 0], s0);
+                    s1 = fmaf(x[u + 1], y[u + 1], s1);
+                    s2 = fmaf(x[u + 2], y[u + 2], s2);
+                    s3 = fmaf(x[u + 3], y[u + 3], s3);
+                }
+            }
         }
-        for (; k < kEnd; ++k)
+        else
         {
-            s0 = fmaf(a[k], p[0], s0);
-            p += N;
+            const float* p = B + static_cast<size_t>(k) * N + col;
+#pragma unroll 4
+            for (; k + 4 <= kEnd; k += 4)
+            {
+                s0 = fmaf(a[k + 0], p[0], s0);
+                s1 = fmaf(a[k + 1], p[static_cast<size_t>(N)], s1);
+                s2 = fmaf(a[k + 2], p[2 * static_cast<size_t>(N)], s2);
+                s3 = fmaf(a[k + 3], p[3 * static_cast<size_t>(N)], s3);
+                p += 4 * static_cast<size_t>(N);
+            }
+            for (; k < kEnd; ++k)
+            {
+                s0 = fmaf(a[k], p[0], s0);
+                p += N;
+            }
         }
     }
     partial[wave][lane] = (s0 + s1) + (s2 + s3);
     __syncthreads();
-    if (wave != 0 || !colOk)
+    if (wave != 0)
         return;
     float sum = partial[0][lane];
 #pragma unroll
     for (int w = 1; w < kGemvWaves; ++w)
         sum += partial[w][lane];
+#pragma unroll
+    for (int lanes = COLS; lanes < 64; lanes *= 2)
+        sum += __shfl_xor(sum, lanes);
+    if (!colOk || lane >= COLS)
+        return;
     float old = 0.f;
     if (args.bias != nullptr)
         old = 0.f + args.bias[col];
@@ -1932,8 +1983,15 @@ int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool o
     if (args.M == 1 && !transB && args.entries == nullptr && args.K >= 64 && units <= 65535 &&
         (args.split & 3u) == 0)
     {
-        hipLaunchKernelGGL(GemvRowKernel, dim3((args.N + 63) / 64, units), dim3(kGemvWaves * 64),
-                           0, stream, args);
+        // 16 columns per workgroup while they are at most half as many as the compute units;
+        // beyond that 64-byte segments cost more than the longer chain (figures at the kernel)
+        const uint64_t blocks16 = static_cast<uint64_t>((args.N + 15) / 16) * units;
+        if (blocks16 * 2 <= cusAll)
+            hipLaunchKernelGGL(GemvRowKernel<16>, dim3((args.N + 15) / 16, units),
+                               dim3(kGemvWaves * 64), 0, stream, args);
+        else
+            hipLaunchKernelGGL(GemvRowKernel<64>, dim3((args.N + 63) / 64, units),
+                               dim3(kGemvWaves * 64), 0, stream, args);
         SPH_CHECK_LAUNCH();
         return SPH_OK;
     }
