@@ -690,9 +690,10 @@ int ExclusiveScanInPlace(uint32_t* data, uint32_t n, uint32_t* lastHost, hipStre
         const bool own = sums == nullptr;
         if (own)
         {
-            ::sph::CountAllocation();
-            SPH_HIP_TRY(hipMallocAsync(reinterpret_cast<void**>(&sums),
-                                       blocks * sizeof(uint32_t), stream));
+            const int taken = sph::AllocScratch(reinterpret_cast<void**>(&sums),
+                                                blocks * sizeof(uint32_t), stream);
+            if (taken != SPH_OK)
+                return taken;
         }
         hipLaunchKernelGGL(ScanBlocksKernel, dim3(blocks), dim3(kScanThreads), 0, stream, data,
                            sums, n);
@@ -823,9 +824,10 @@ int sph_csr_from_dense_f32(float* V, uint32_t* COL, uint32_t* ROW, uint32_t capa
     // counts (16-byte aligned, when the move scans them), values, columns
     const size_t countEntries = placed ? (static_cast<size_t>(M) + 4) / 4 * 4 : 0;
     uint32_t* block0 = nullptr;
-    ::sph::CountAllocation();
-    SPH_HIP_TRY(hipMallocAsync(reinterpret_cast<void**>(&block0), countEntries * 4 + stageEntries * 8,
-                               stream));
+    const int taken = sph::AllocScratch(reinterpret_cast<void**>(&block0),
+                                        countEntries * 4 + stageEntries * 8, stream);
+    if (taken != SPH_OK)
+        return taken;
     uint32_t* counts = placed ? block0 : ROW;
     float* stageV = reinterpret_cast<float*>(block0 + countEntries);
     uint32_t* stageCol = reinterpret_cast<uint32_t*>(stageV + stageEntries);
@@ -990,8 +992,10 @@ int sph_csr_validate_u32(const uint32_t* COL, const uint32_t* ROW, uint32_t M, u
     if (stream == nullptr)
         return SPH_ERR_DEVICE;
     uint32_t* problems = nullptr;
-    ::sph::CountAllocation();
-    SPH_HIP_TRY(hipMallocAsync(reinterpret_cast<void**>(&problems), sizeof(uint32_t), stream));
+    const int taken = sph::AllocScratch(reinterpret_cast<void**>(&problems),
+                                        sizeof(uint32_t), stream);
+    if (taken != SPH_OK)
+        return taken;
     SPH_HIP_TRY(hipMemsetAsync(problems, 0, sizeof(uint32_t), stream));
     const uint64_t items = std::max<uint64_t>(std::max<uint64_t>(M, nnz), 1);
     const uint32_t grid = static_cast<uint32_t>(std::min<uint64_t>((items + 255) / 256, 4096));

@@ -45,6 +45,11 @@ int ResolveCsrScratch(uint32_t** scratch);
 // sph_allocation_count); called next to every hipMalloc / hipMallocAsync / hipHostMalloc.
 void CountAllocation();
 
+// Takes a stream-ordered scratch block for one call of the library (counted; given back with
+// hipFreeAsync on the same stream).  The first one on a device has the device's memory pool keep
+// up to 512 MiB of freed blocks.
+int AllocScratch(void** ptr, size_t bytes, hipStream_t stream);
+
 // True between sph_graph_begin_capture and sph_graph_end_capture on this thread.  Entry
 // points that must wait for the device or allocate refuse to run while it is set.
 bool Capturing();

@@ -24,6 +24,8 @@ std::mutex gPoolMutex;
 std::vector<hipStream_t> gIdleStreams[kMaxDevices];
 int gComputeUnits[kMaxDevices] = {};
 bool gPoolRetains[kMaxDevices] = {};
+// (same mutex) the pool has been told to keep the library's own scratch blocks
+bool gPoolKeepsScratch[kMaxDevices] = {};
 
 struct ThreadSlots
 {
@@ -54,6 +56,38 @@ namespace sph
 void CountAllocation()
 {
     gAllocations.fetch_add(1, std::memory_order_relaxed);
+}
+
+// With the pool's default threshold of zero every synchronisation hands freed blocks back to
+// the driver, and the next call maps its staging anew: a CSR x CSR product of 65536 rows
+// (139 MB of staging) that is waited for took 327 us, 87 us of them on the GPU
+// (now 100 us; dense to CSR and back, 8192 x 8192, 161 -> 123 us).  A bound keeps
+// what the library's own calls leave behind small beside the device's memory; a pool that already
+// keeps more (sph_malloc_async, or the program's own setting) is left alone.
+constexpr uint64_t kScratchKept = 512ull << 20;
+
+int AllocScratch(void** ptr, size_t bytes, hipStream_t stream)
+{
+    const int d = tlsSlots.device;
+    {
+        std::lock_guard<std::mutex> lock(gPoolMutex);
+        if (!gPoolKeepsScratch[d] && !gPoolRetains[d])
+        {
+            hipMemPool_t pool = nullptr;
+            SPH_HIP_TRY(hipDeviceGetDefaultMemPool(&pool, d));
+            uint64_t keep = 0;
+            SPH_HIP_TRY(hipMemPoolGetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep));
+            if (keep < kScratchKept)
+            {
+                keep = kScratchKept;
+                SPH_HIP_TRY(hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep));
+            }
+            gPoolKeepsScratch[d] = true;
+        }
+    }
+    CountAllocation();
+    SPH_HIP_TRY(hipMallocAsync(ptr, bytes, stream));
+    return SPH_OK;
 }
 
 int Fail(int status, const std::string& msg)

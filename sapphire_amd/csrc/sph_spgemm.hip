@@ -941,8 +941,10 @@ int sph_spgemm_load_u32(uint32_t* load, const uint32_t* COLA, const uint32_t* RO
     unsigned long long* total = nullptr;
     if (productsHost != nullptr)
     {
-        ::sph::CountAllocation();
-        SPH_HIP_TRY(hipMallocAsync(reinterpret_cast<void**>(&total), sizeof(*total), stream));
+        const int taken = sph::AllocScratch(reinterpret_cast<void**>(&total),
+                                            sizeof(*total), stream);
+        if (taken != SPH_OK)
+            return taken;
         hipLaunchKernelGGL(ClearTotalKernel, dim3(1), dim3(1), 0, stream, total);
     }
     const uint32_t blocks = static_cast<uint32_t>(std::min<uint64_t>(
@@ -1014,9 +1016,10 @@ int sph_spgemm_f32(float* VC, uint32_t* COLC, uint32_t* ROWC, uint32_t capacity,
     {
         // counts (16-byte aligned, when the move scans them), values, columns, one flag
         const size_t counts = placed ? (static_cast<size_t>(M) + 4) / 4 * 4 : 0;
-        ::sph::CountAllocation();
-        SPH_HIP_TRY(hipMallocAsync(reinterpret_cast<void**>(&stageV), counts * 4 + slot * M * 8 + 4,
-                                   stream));
+        const int taken = sph::AllocScratch(reinterpret_cast<void**>(&stageV),
+                                            counts * 4 + slot * M * 8 + 4, stream);
+        if (taken != SPH_OK)
+            return taken;
         if (placed)
             args.counts = reinterpret_cast<uint32_t*>(stageV);
         args.VC = stageV + counts;
