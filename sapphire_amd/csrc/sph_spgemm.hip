@@ -32,6 +32,7 @@
 // column indices of A below the row count of B.
 #include "sph_internal.h"
 #include "sph_place_rows.h"
+#include "sph_spgemm_plan.h"
 
 #include <algorithm>
 
@@ -455,7 +456,7 @@ __global__ __launch_bounds__(64) void SpgemmRowKernel(const SpgemmArgs args)
     // every row for nothing took 28 us on 65536 rows).
     // The pass after staging looks for rows that did not fit their slot in the same way.
     const bool selective = COUNTS ? args.heavyOnly != 0 : args.skipUpTo != 0;
-    const uint32_t turns = (args.M - 1) / args.rowsPerTurn + (args.M != 0 ? 1 : 0);
+    const uint32_t turns = sph::SpgemmTurns(args.M, args.rowsPerTurn);
     auto wanted = [&](uint64_t t) {
         if (t >= turns)
             return false;
@@ -825,7 +826,7 @@ void LaunchLight(const SpgemmArgs& args, hipStream_t stream)
     const uint64_t cus = static_cast<uint64_t>(sph::ComputeUnits());
     light.rowsPerTurn = static_cast<uint32_t>(
         std::max<uint64_t>(1, std::min<uint64_t>(kRowsPerTurnMax, args.M / (cus * 8 * kLightWaves))));
-    const uint64_t turns = (static_cast<uint64_t>(args.M) + light.rowsPerTurn - 1) / light.rowsPerTurn;
+    const uint64_t turns = sph::SpgemmTurns(args.M, light.rowsPerTurn);
     const uint64_t groups = std::min<uint64_t>((turns + kLightWaves - 1) / kLightWaves, cus * 64);
     const dim3 grid(static_cast<uint32_t>(groups)), block(kLightWaves * 64);
     // column and place share 32 bits up to 2^23 columns (all ones stay free for "no product")
@@ -840,7 +841,7 @@ void LaunchLight(const SpgemmArgs& args, hipStream_t stream)
 uint32_t GridFor(uint32_t M, uint32_t rowsPerTurn, bool selective)
 {
     const uint64_t cap = static_cast<uint64_t>(sph::ComputeUnits()) * (selective ? 9 : 64);
-    const uint64_t turns = (static_cast<uint64_t>(M) + rowsPerTurn - 1) / rowsPerTurn;
+    const uint64_t turns = sph::SpgemmTurns(M, rowsPerTurn);
     return static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(turns, cap)));
 }
 }  // namespace

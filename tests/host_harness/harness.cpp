@@ -18,6 +18,7 @@
 
 #include <sapphire_hip.h>
 #include <sph_k_partition.h>
+#include <sph_spgemm_plan.h>
 
 #include <algorithm>
 #include <chrono>
@@ -280,6 +281,13 @@ unsigned sphh_k_partition_slot(unsigned K, unsigned groupK, unsigned waves, unsi
 {
     const sph::KPartition p = sph::PartitionK(K, groupK, waves, wave, depth);
     return g == 0xffffffffu ? sph::KPartitionFirst(p, d) : sph::KPartitionNext(p, g, depth, d);
+}
+
+// Turns of rowsPerTurn rows that the CSR x CSR passes take over M rows
+// (sapphire_amd/csrc/sph_spgemm_plan.h).  No device is touched.
+unsigned sphh_spgemm_turns(unsigned M, unsigned rowsPerTurn)
+{
+    return sph::SpgemmTurns(M, rowsPerTurn);
 }
 
 // Compute::Gemm into a FRESH y (never filled, never read): the operator sees the deferred zero

@@ -34,6 +34,8 @@ def lib():
         h.sphh_k_partition.argtypes = [ctypes.c_uint] * 5 + [ctypes.POINTER(ctypes.c_uint)]
         h.sphh_k_partition_slot.argtypes = [ctypes.c_uint] * 7
         h.sphh_k_partition_slot.restype = ctypes.c_uint
+        h.sphh_spgemm_turns.argtypes = [ctypes.c_uint] * 2
+        h.sphh_spgemm_turns.restype = ctypes.c_uint
         h.sphh_transpose.argtypes = [_fp, _ip, ctypes.c_int, _fp, _ip, ctypes.c_int]
         h.sphh_mlp_forward.argtypes = [_fp, ctypes.c_int, _ip, ctypes.c_int,
                                        ctypes.POINTER(_fp), ctypes.POINTER(_fp), _fp, ctypes.c_int]
@@ -154,6 +156,10 @@ def k_partition_slot(K, group_k, waves, wave, depth, g, d):
     loaded while the round that starts at group g is multiplied."""
     return int(lib().sphh_k_partition_slot(K, group_k, waves, wave, depth,
                                            0xffffffff if g is None else g, d))
+
+
+def spgemm_turns(M, rows_per_turn):
+    return int(lib().sphh_spgemm_turns(M, rows_per_turn))
 
 
 def transpose(x, y_shape):

@@ -310,3 +310,36 @@ def test_staged_rows_find_their_place(dev, M):
     V, COL, ROW, nnz = gpu_spgemm_one_call(A, B, M, K, N, total + M)
     assert nnz == total and np.array_equal(ROW, wR) and np.array_equal(COL[:total], wC)
     assert np.array_equal(bits(V[:total]), bits(wV))
+
+
+@pytest.mark.parametrize("N", [1, 300, 4097, 8192, 8193, 70000])
+def test_no_rows(dev, N):
+    """M = 0 through every entry point, on both sides of the widths that take other kernels:
+    ROWC[0] and the count are 0, nothing behind ROWC, VC or COLC is touched."""
+    h.announce("sph_spgemm_* without rows, N =", N)
+    K = 3
+    VB = np.array([0.5, -1.0, 2.0], np.float32)
+    CB = np.array([0, N - 1, 0], np.uint32)
+    RB = np.array([0, 1, 2, 3], np.uint32)
+    bufs = [_dev(np.zeros(0, np.float32), np.float32), _dev(np.zeros(0, np.uint32), np.uint32),
+            _dev(np.zeros(1, np.uint32), np.uint32), _dev(VB, np.float32), _dev(CB, np.uint32),
+            _dev(RB, np.uint32)]
+    operands = [b.ptr for b in bufs]
+    guard = np.full(1025, 0xFFFFFFFF, np.uint32)
+    dV, dCol = (capi.DeviceBuffer.from_array(guard) for _ in range(2))
+    for entry, head in (("sph_spgemm_row_offsets_f32", []),
+                        ("sph_spgemm_f32", [dV.ptr, dCol.ptr]),):
+        for capacity in (0, 1000):
+            dRow = capi.DeviceBuffer.from_array(guard)
+            nnz = ctypes.c_uint32(0xDEADBEEF)
+            tail = [capacity] if head else []
+            capi.call(entry, *head, dRow.ptr, *tail, *operands, 0, K, N, ctypes.byref(nnz))
+            ROW = dRow.download(np.uint32, guard.shape)
+            assert nnz.value == 0 and ROW[0] == 0 and np.all(ROW[1:] == 0xFFFFFFFF), entry
+            dRow.release()
+    dRow = capi.DeviceBuffer.from_array(np.zeros(1, np.uint32))
+    capi.call("sph_spgemm_fill_f32", dV.ptr, dCol.ptr, dRow.ptr, *operands, 0, K, N)
+    for d in (dV, dCol):
+        assert np.all(d.download(np.uint32, guard.shape) == 0xFFFFFFFF)
+    for d in bufs + [dRow, dV, dCol]:
+        d.release()
