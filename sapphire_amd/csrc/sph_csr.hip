@@ -15,6 +15,7 @@
 // A row is handled by a group of LPR lanes (a power of two, 4..64, chosen from the row
 // length) so that narrow matrices do not idle most of a wavefront; each lane takes 4
 // consecutive columns (16 bytes) per step.
+#include "sph_column_walk.h"
 #include "sph_internal.h"
 #include "sph_place_rows.h"
 
@@ -75,6 +76,15 @@ __device__ __forceinline__ float4 LoadQuad(const DenseView& d, uint32_t row, uin
     return v;
 }
 
+// 16 bytes of a row, all four columns existing
+__device__ __forceinline__ float4 WholeQuad(const float* p)
+{
+    typedef float floatx4 __attribute__((ext_vector_type(4)));
+    typedef floatx4 floatx4a4 __attribute__((aligned(4)));
+    const floatx4 w = *reinterpret_cast<const floatx4a4*>(p);
+    return make_float4(w[0], w[1], w[2], w[3]);
+}
+
 // counts[r] = number of entries != 0 in row r; counts[M] = 0 (the slot the scan turns into nnz)
 template <int LPR>
 __global__ __launch_bounds__(kThreads) void CsrCountKernel(uint32_t* __restrict__ counts,
@@ -96,20 +106,23 @@ __global__ __launch_bounds__(kThreads) void CsrCountKernel(uint32_t* __restrict_
         auto count = [&](const float4& v) {
             c += (v.x != 0.f) + (v.y != 0.f) + (v.z != 0.f) + (v.w != 0.f);
         };
-        uint32_t col = lane * 4;
-        // long rows: kAhead loads of a lane in flight
-        for (; col - lane * 4 + kAhead * LPR * 4 <= d.N; col += kAhead * LPR * 4)
-        {
-            float4 v[kAhead];
+        sph::WalkColumns(
+            d.N, LPR * 4, kAhead,
+            [&](uint32_t first) {
+                // no condition between the loads: with one each they wait for each other
+                const float* p = d.data + static_cast<size_t>(row) * d.ld + first + lane * 4;
+                float4 v[kAhead];
+                if (rowOk)
+                {
 #pragma unroll
-            for (uint32_t u = 0; u < kAhead; ++u)
-                v[u] = LoadQuad(d, row, col + u * LPR * 4, rowOk);
+                    for (uint32_t u = 0; u < kAhead; ++u)
+                        v[u] = WholeQuad(p + u * LPR * 4);
 #pragma unroll
-            for (uint32_t u = 0; u < kAhead; ++u)
-                count(v[u]);
-        }
-        for (; col < d.N; col += LPR * 4)
-            count(LoadQuad(d, row, col, rowOk));
+                    for (uint32_t u = 0; u < kAhead; ++u)
+                        count(v[u]);
+                }
+            },
+            [&](uint32_t first) { count(LoadQuad(d, row, first + lane * 4, rowOk)); });
 #pragma unroll
         for (int off = LPR / 2; off > 0; off >>= 1)
             c += __shfl_xor(c, off, LPR);
@@ -282,19 +295,20 @@ __global__ __launch_bounds__(kThreads) void CsrFillKernel(float* __restrict__ V,
                 }
             slot += kept;
         };
-        uint32_t col0 = 0;
-        for (; col0 + kAhead * LPR * 4 <= d.N; col0 += kAhead * LPR * 4)
-        {
-            float4 q[kAhead];
+        sph::WalkColumns(
+            d.N, LPR * 4, kAhead,
+            [&](uint32_t first) {
+                float4 q[kAhead];
 #pragma unroll
-            for (uint32_t u = 0; u < kAhead; ++u)
-                q[u] = LoadQuad(d, row, col0 + (u * LPR + lane) * 4, rowOk);
+                for (uint32_t u = 0; u < kAhead; ++u)
+                    q[u] = LoadQuad(d, row, first + (u * LPR + lane) * 4, rowOk);
 #pragma unroll
-            for (uint32_t u = 0; u < kAhead; ++u)
-                store(q[u], col0 + (u * LPR + lane) * 4);
-        }
-        for (; col0 < d.N; col0 += LPR * 4)
-            store(LoadQuad(d, row, col0 + lane * 4, rowOk), col0 + lane * 4);
+                for (uint32_t u = 0; u < kAhead; ++u)
+                    store(q[u], first + (u * LPR + lane) * 4);
+            },
+            [&](uint32_t first) {
+                store(LoadQuad(d, row, first + lane * 4, rowOk), first + lane * 4);
+            });
     }
 }
 
@@ -724,6 +738,7 @@ int sph_csr_row_offsets_f32(uint32_t* ROW, const float* dense, uint32_t M, uint3
 {
     SPH_REQUIRE(ROW != nullptr, "ROW is null");
     SPH_REQUIRE(ld >= N, "row pitch is shorter than a row");
+    SPH_REQUIRE(N <= sph::kMaxColumns, "rows of more than 2^32 - 256 columns");
     SPH_REQUIRE(M < 0xffffffffu, "too many rows");
     SPH_REQUIRE(M == 0 || N == 0 || dense != nullptr, "dense is null");
     if (sph::ScanWaitsOrAllocates(M + 1, nnzHost))
@@ -745,6 +760,7 @@ int sph_csr_row_offsets_noalloc_f32(uint32_t* ROW, const float* dense, uint32_t 
 {
     SPH_REQUIRE(ROW != nullptr, "ROW is null");
     SPH_REQUIRE(ld >= N, "row pitch is shorter than a row");
+    SPH_REQUIRE(N <= sph::kMaxColumns, "rows of more than 2^32 - 256 columns");
     SPH_REQUIRE(M == 0 || N == 0 || dense != nullptr, "dense is null");
     SPH_REQUIRE(M < static_cast<uint64_t>(kNoAllocMaxBlocks) * kScanPerBlock,
                 "more than 16777215 rows exceed the fixed scratch array");
@@ -771,6 +787,7 @@ int sph_csr_from_dense_f32(float* V, uint32_t* COL, uint32_t* ROW, uint32_t capa
 {
     SPH_REQUIRE(ROW != nullptr, "ROW is null");
     SPH_REQUIRE(ld >= N, "row pitch is shorter than a row");
+    SPH_REQUIRE(N <= sph::kMaxColumns, "rows of more than 2^32 - 256 columns");
     SPH_REQUIRE(M < 0xffffffffu, "too many rows");
     SPH_REQUIRE(M == 0 || N == 0 || dense != nullptr, "dense is null");
     SPH_REQUIRE(capacity == 0 || (V != nullptr && COL != nullptr), "V or COL is null");
@@ -889,6 +906,7 @@ int sph_csr_fill_f32(float* V, uint32_t* COL, const uint32_t* ROW, const float* 
         return SPH_OK;
     SPH_REQUIRE(ROW != nullptr && dense != nullptr, "null pointer");
     SPH_REQUIRE(ld >= N, "row pitch is shorter than a row");
+    SPH_REQUIRE(N <= sph::kMaxColumns, "rows of more than 2^32 - 256 columns");
     // V and COL may be null only for a matrix without entries; the kernel then writes nothing
     hipStream_t stream = sph::CurrentStream();
     if (stream == nullptr)

@@ -17,6 +17,7 @@
 #include <Sapphire/util/ResourceManager.hpp>
 
 #include <sapphire_hip.h>
+#include <sph_column_walk.h>
 #include <sph_k_partition.h>
 #include <sph_spgemm_plan.h>
 
@@ -281,6 +282,35 @@ unsigned sphh_k_partition_slot(unsigned K, unsigned groupK, unsigned waves, unsi
 {
     const sph::KPartition p = sph::PartitionK(K, groupK, waves, wave, depth);
     return g == 0xffffffffu ? sph::KPartitionFirst(p, d) : sph::KPartitionNext(p, g, depth, d);
+}
+
+// The walk over a row's columns (sapphire_amd/csrc/sph_column_walk.h): out receives the columns
+// seen, the first column that did not come in ascending order or is not below N (~0: none) and
+// the steps taken.  Gives up (-1) after more steps than N columns make.  No device is touched.
+int sphh_column_walk(unsigned N, unsigned lanes, unsigned ahead, unsigned long long* out)
+{
+    const std::uint32_t step = lanes * 4;
+    const std::uint64_t most = (static_cast<std::uint64_t>(N) + step - 1) / step;
+    std::uint64_t wrong = ~0ull, steps = 0, next = 0;
+    auto take = [&](std::uint64_t first, std::uint64_t columns) {
+        if (++steps > most)
+            throw std::runtime_error("the walk does not end");
+        if ((first != next || next + columns > N) && wrong == ~0ull)
+            wrong = first;
+        next += columns;
+    };
+    return Guard([&] {
+        sph::WalkColumns(
+            N, step, ahead,
+            [&](std::uint32_t first) {
+                for (std::uint32_t u = 0; u < ahead; ++u)
+                    take(static_cast<std::uint64_t>(first) + u * step, step);
+            },
+            [&](std::uint32_t first) { take(first, std::min(step, N - first)); });
+        out[0] = next;
+        out[1] = wrong;
+        out[2] = steps;
+    });
 }
 
 // Turns of rowsPerTurn rows that the CSR x CSR passes take over M rows

@@ -34,6 +34,7 @@ def lib():
         h.sphh_k_partition.argtypes = [ctypes.c_uint] * 5 + [ctypes.POINTER(ctypes.c_uint)]
         h.sphh_k_partition_slot.argtypes = [ctypes.c_uint] * 7
         h.sphh_k_partition_slot.restype = ctypes.c_uint
+        h.sphh_column_walk.argtypes = [ctypes.c_uint] * 3 + [ctypes.POINTER(ctypes.c_ulonglong)]
         h.sphh_spgemm_turns.argtypes = [ctypes.c_uint] * 2
         h.sphh_spgemm_turns.restype = ctypes.c_uint
         h.sphh_transpose.argtypes = [_fp, _ip, ctypes.c_int, _fp, _ip, ctypes.c_int]
@@ -156,6 +157,13 @@ def k_partition_slot(K, group_k, waves, wave, depth, g, d):
     loaded while the round that starts at group g is multiplied."""
     return int(lib().sphh_k_partition_slot(K, group_k, waves, wave, depth,
                                            0xffffffff if g is None else g, d))
+
+
+def column_walk(N, lanes, ahead):
+    """(columns seen, first column out of order or None, steps)"""
+    out = (ctypes.c_ulonglong * 3)()
+    _ok(lib().sphh_column_walk(N, lanes, ahead, out))
+    return int(out[0]), None if out[1] == 2**64 - 1 else int(out[1]), int(out[2])
 
 
 def spgemm_turns(M, rows_per_turn):
