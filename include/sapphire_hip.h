@@ -345,7 +345,8 @@ int sph_spmm_csr_bias_f32(float* out, const float* V, const uint32_t* COL,
  * paddedN, numMatrices) and ConvertSparseMatrixToDenseMatrix(dst, src, m, n,
  * paddedN, numMatrices) (Includes/Sapphire/compute/sparse/Sparse.hpp:150-160)
  * and defines neither; these three calls are their device work for one matrix
- * of M rows, N columns and a row pitch of ld floats (ld = paddedN).  An entry
+ * of M rows, N columns (to CSR: at most 2^32 - 256) and a row pitch of ld floats
+ * (ld = paddedN).  An entry
  * is kept when its value != 0 (-0.0 is dropped, NaN kept); a row's entries are
  * stored in ascending column order.
  *

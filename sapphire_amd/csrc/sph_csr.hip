@@ -738,7 +738,7 @@ int sph_csr_row_offsets_f32(uint32_t* ROW, const float* dense, uint32_t M, uint3
 {
     SPH_REQUIRE(ROW != nullptr, "ROW is null");
     SPH_REQUIRE(ld >= N, "row pitch is shorter than a row");
-    SPH_REQUIRE(N <= sph::kMaxColumns, "rows of more than 2^32 - 256 columns");
+    SPH_REQUIRE(M == 0 || N <= sph::kMaxColumns, "rows of more than 2^32 - 256 columns");
     SPH_REQUIRE(M < 0xffffffffu, "too many rows");
     SPH_REQUIRE(M == 0 || N == 0 || dense != nullptr, "dense is null");
     if (sph::ScanWaitsOrAllocates(M + 1, nnzHost))
@@ -760,7 +760,7 @@ int sph_csr_row_offsets_noalloc_f32(uint32_t* ROW, const float* dense, uint32_t 
 {
     SPH_REQUIRE(ROW != nullptr, "ROW is null");
     SPH_REQUIRE(ld >= N, "row pitch is shorter than a row");
-    SPH_REQUIRE(N <= sph::kMaxColumns, "rows of more than 2^32 - 256 columns");
+    SPH_REQUIRE(M == 0 || N <= sph::kMaxColumns, "rows of more than 2^32 - 256 columns");
     SPH_REQUIRE(M == 0 || N == 0 || dense != nullptr, "dense is null");
     SPH_REQUIRE(M < static_cast<uint64_t>(kNoAllocMaxBlocks) * kScanPerBlock,
                 "more than 16777215 rows exceed the fixed scratch array");
@@ -787,7 +787,7 @@ int sph_csr_from_dense_f32(float* V, uint32_t* COL, uint32_t* ROW, uint32_t capa
 {
     SPH_REQUIRE(ROW != nullptr, "ROW is null");
     SPH_REQUIRE(ld >= N, "row pitch is shorter than a row");
-    SPH_REQUIRE(N <= sph::kMaxColumns, "rows of more than 2^32 - 256 columns");
+    SPH_REQUIRE(M == 0 || N <= sph::kMaxColumns, "rows of more than 2^32 - 256 columns");
     SPH_REQUIRE(M < 0xffffffffu, "too many rows");
     SPH_REQUIRE(M == 0 || N == 0 || dense != nullptr, "dense is null");
     SPH_REQUIRE(capacity == 0 || (V != nullptr && COL != nullptr), "V or COL is null");
@@ -906,7 +906,7 @@ int sph_csr_fill_f32(float* V, uint32_t* COL, const uint32_t* ROW, const float* 
         return SPH_OK;
     SPH_REQUIRE(ROW != nullptr && dense != nullptr, "null pointer");
     SPH_REQUIRE(ld >= N, "row pitch is shorter than a row");
-    SPH_REQUIRE(N <= sph::kMaxColumns, "rows of more than 2^32 - 256 columns");
+    SPH_REQUIRE(M == 0 || N <= sph::kMaxColumns, "rows of more than 2^32 - 256 columns");
     // V and COL may be null only for a matrix without entries; the kernel then writes nothing
     hipStream_t stream = sph::CurrentStream();
     if (stream == nullptr)
