@@ -47,6 +47,9 @@ constexpr uint32_t kWordsPerLaneMax = kStripMax / 32 / 64;  // bit-map words a l
 constexpr uint32_t kLightProducts = 512;  // a row with at most this many products is "light"
 constexpr uint32_t kPlaceBits = 9;        // a product's place in its row, below its column
 constexpr uint32_t kLightWaves = 4;       // wavefronts per workgroup of SpgemmLightKernel
+constexpr uint32_t kStripGroups = 64;  // workgroups of a strip pass per compute unit, at most
+constexpr uint32_t kMarkedGroups = 9;
+constexpr uint32_t kRedoGroups = 2;
 constexpr uint32_t kEmpty = 0xffffffffu;
 constexpr uint32_t kHeavyMark = 0xffffffffu;  // in place of a count: SpgemmRowKernel's row
 static_assert(kLightProducts <= 1u << kPlaceBits, "a key holds column and place");
@@ -75,8 +78,8 @@ struct SpgemmArgs
     uint32_t slot;      // stage pass: entries per staging slot
     uint32_t skipUpTo;  // fill pass: rows with at most this many entries are left alone
     uint32_t capacity;  // fill pass: nothing is stored at or past this index
-    // stage pass: cleared; the move kernel sets it when a row did not fit its slot; a fill
-    // pass that is given it returns at once while it is zero
+    // stage pass: cleared; the move kernel sets it when a row did not fit its slot; the pass over
+    // such rows returns at once while it is zero
     uint32_t* overflow;
 };
 
@@ -433,7 +436,13 @@ __global__ __launch_bounds__(kLightWaves * 64, 5) void SpgemmLightKernel(const S
     }
 }
 
-template <int MODE>
+// Which rows a pass of the strip kernel takes.  A pass of its own for each: with the choice made at
+// run time the narrow products, which take every row, were 0.3 us slower per launch.
+constexpr int kEveryRow = 0;
+constexpr int kMarkedRows = 1;    // those that SpgemmLightKernel has marked in `counts`
+constexpr int kOverfullRows = 2;  // those with more than skipUpTo entries, if *overflow is set
+
+template <int MODE, int ROWS>
 __global__ __launch_bounds__(64) void SpgemmRowKernel(const SpgemmArgs args)
 {
     constexpr bool FILL = MODE != kCount;    // entries are stored
@@ -444,51 +453,25 @@ __global__ __launch_bounds__(64) void SpgemmRowKernel(const SpgemmArgs args)
     const uint32_t wordsInStrip = args.strip / 32;
     const uint32_t wordsPerLane = (wordsInStrip + 63) / 64;  // at most kStripMax / 2048
     const uint32_t lane = threadIdx.x;
-    if (MODE == kFill && args.overflow != nullptr && *args.overflow == 0)
+    if (ROWS == kOverfullRows && *args.overflow == 0)
         return;  // every row is in place already
     if (COUNTS && blockIdx.x == 0 && lane == 0)
         args.counts[args.M] = 0;
     if (MODE == kStage && blockIdx.x == 0 && lane == 0)
         *args.overflow = 0;
-    // In a wide product the counts pass has the light rows' counts by now, and the rows left for
-    // this kernel are marked.  Usually there are none or few, so the turns of a wavefront are
-    // looked through first, one per lane, and only those with a marked row are taken (walking
-    // every row for nothing took 28 us on 65536 rows).
-    // The pass after staging looks for rows that did not fit their slot in the same way.
-    const bool selective = COUNTS ? args.heavyOnly != 0 : args.skipUpTo != 0;
-    const uint32_t turns = sph::SpgemmTurns(args.M, args.rowsPerTurn);
-    auto wanted = [&](uint64_t t) {
-        if (t >= turns)
-            return false;
-        if (!selective)
-            return true;
-        bool any = false;
-        for (uint64_t row = t * args.rowsPerTurn; row < (t + 1) * args.rowsPerTurn; ++row)
-            any |= row < args.M && (COUNTS ? args.counts[row] == kHeavyMark
-                                           : args.ROWC[row + 1] - args.ROWC[row] > args.skipUpTo);
-        return any;
+    // once; every element that is touched is cleared again when it is swept
+    auto clear = [&] {
+        for (uint32_t x = lane; x < args.strip; x += 64)
+            strip[x] = 0.0f;
+        for (uint32_t t = lane; t < wordsInStrip; t += 64)
+            bits[t] = 0;
     };
-    bool cleared = false;
 
     // A wavefront takes rowsPerTurn consecutive rows per turn.  Their extents are read in one
     // go, and the loads that lead to a row's products form a pipeline over the rows of the
     // turn: while row i is multiplied, the first 64 (column, value) pairs of A's row i+2 and
     // the extents of the rows of B that row i+1 needs are already on their way.
-    for (uint64_t base = blockIdx.x; base < turns; base += 64ull * gridDim.x)
-    for (uint64_t chosen = __ballot(wanted(base + static_cast<uint64_t>(lane) * gridDim.x));
-         chosen != 0; chosen &= chosen - 1)
-    {
-        if (!cleared)
-        {
-            // once; every element that is touched is cleared again when it is swept
-            for (uint32_t x = lane; x < args.strip; x += 64)
-                strip[x] = 0.0f;
-            for (uint32_t t = lane; t < wordsInStrip; t += 64)
-                bits[t] = 0;
-            cleared = true;
-        }
-        const uint32_t turn = static_cast<uint32_t>(
-            (base + static_cast<uint64_t>(__builtin_ctzll(chosen)) * gridDim.x) * args.rowsPerTurn);
+    auto multiply = [&](uint32_t turn) {
         const uint32_t rowsHere = min(args.rowsPerTurn, args.M - turn);
         uint32_t extentA = 0, extentC = 0;
         if (lane <= rowsHere)
@@ -544,10 +527,11 @@ __global__ __launch_bounds__(64) void SpgemmRowKernel(const SpgemmArgs args)
         loadStage2(k2, nextBegin, nextEnd);
         loadStage1(i + 2, k1, value1);
         // in a wide product the light rows belong to SpgemmLightKernel
-        if (args.heavyOnly != 0 && LightRow(args, aEnd - aBegin, WaveSum(LightCount(firstBegin, firstEnd))))
+        if (ROWS != kOverfullRows && args.heavyOnly != 0 &&
+            LightRow(args, aEnd - aBegin, WaveSum(LightCount(firstBegin, firstEnd))))
             continue;
         if (MODE == kFill && rowEnd - rowBase <= args.skipUpTo)
-            continue;  // already in place
+            continue;  // empty, or already in place
 
         for (uint32_t c0 = 0; c0 < args.N; c0 += args.strip)
         {
@@ -706,6 +690,43 @@ __global__ __launch_bounds__(64) void SpgemmRowKernel(const SpgemmArgs args)
         if (COUNTS && lane == 0)
             args.counts[turn + i] = emitted;
       }
+    };
+
+    const uint32_t turns = sph::SpgemmTurns(args.M, args.rowsPerTurn);
+    if (ROWS == kEveryRow)
+    {
+        clear();
+        for (uint64_t t = blockIdx.x; t < turns; t += gridDim.x)
+            multiply(static_cast<uint32_t>(t) * args.rowsPerTurn);
+        return;
+    }
+    // There are usually none or few such rows, so the turns of a wavefront are looked through
+    // first, as many at once as 64 lanes have rows for, and only those with one are taken (walking
+    // every row for nothing took 28 us on 65536 rows).
+    const uint32_t rows = args.rowsPerTurn;
+    const uint32_t looked = 64 / rows;  // turns per look
+    const uint32_t turnOfLane = lane / rows;
+    bool cleared = false;
+    for (uint64_t base = blockIdx.x; base < turns; base += static_cast<uint64_t>(looked) * gridDim.x)
+    {
+        const uint64_t row =
+            (base + static_cast<uint64_t>(turnOfLane) * gridDim.x) * rows + lane % rows;
+        bool wanted = false;
+        if (turnOfLane < looked && row < args.M)
+            wanted = COUNTS ? args.counts[row] == kHeavyMark
+                            : args.ROWC[row + 1] - args.ROWC[row] > args.skipUpTo;
+        uint64_t chosen = __ballot(wanted);
+        while (chosen != 0)
+        {
+            if (!cleared)
+                clear();
+            cleared = true;
+            const uint32_t next = static_cast<uint32_t>(__builtin_ctzll(chosen)) / rows;
+            multiply(static_cast<uint32_t>((base + static_cast<uint64_t>(next) * gridDim.x) * rows));
+            // the turn's lanes, and those below them, are done
+            const uint32_t done = (next + 1) * rows;
+            chosen = done < 64 ? chosen >> done << done : 0;
+        }
     }
 }
 
@@ -836,13 +857,43 @@ void LaunchLight(const SpgemmArgs& args, hipStream_t stream)
         hipLaunchKernelGGL((SpgemmLightKernel<MODE, uint64_t>), grid, block, 0, stream, light);
 }
 
-// `selective`: a pass that looks for marked rows takes as many workgroups as are resident
-// (17 KiB of LDS each), each with more turns to look through
-uint32_t GridFor(uint32_t M, uint32_t rowsPerTurn, bool selective)
+uint32_t GridFor(uint32_t M, uint32_t rowsPerTurn, uint32_t perComputeUnit)
 {
-    const uint64_t cap = static_cast<uint64_t>(sph::ComputeUnits()) * (selective ? 9 : 64);
+    const uint64_t cap = static_cast<uint64_t>(sph::ComputeUnits()) * perComputeUnit;
     const uint64_t turns = sph::SpgemmTurns(M, rowsPerTurn);
     return static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(turns, cap)));
+}
+
+template <int MODE, int ROWS>
+void LaunchStrips(const SpgemmArgs& args, uint32_t perComputeUnit, hipStream_t stream)
+{
+    hipLaunchKernelGGL((SpgemmRowKernel<MODE, ROWS>),
+                       dim3(GridFor(args.M, args.rowsPerTurn, perComputeUnit)), dim3(64),
+                       args.strip * sizeof(float) + args.strip / 8, stream, args);
+}
+
+// The passes that count (and stage): the light rows of a wide product first, then the strips.
+// A strip pass that looks for marked rows takes as many workgroups as are resident (17 KiB of
+// LDS each), each with more turns to look through.
+template <int MODE>
+void LaunchCounting(const SpgemmArgs& args, hipStream_t stream)
+{
+    if (args.heavyOnly == 0)
+    {
+        LaunchStrips<MODE, kEveryRow>(args, kStripGroups, stream);
+        return;
+    }
+    if (args.M != 0)
+        LaunchLight<MODE>(args, stream);
+    LaunchStrips<MODE, kMarkedRows>(args, kMarkedGroups, stream);
+}
+
+// Every row's entries to their place.
+void LaunchFill(const SpgemmArgs& args, hipStream_t stream)
+{
+    if (args.heavyOnly != 0)
+        LaunchLight<kFill>(args, stream);
+    LaunchStrips<kFill, kEveryRow>(args, kStripGroups, stream);
 }
 }  // namespace
 
@@ -876,11 +927,7 @@ int sph_spgemm_row_offsets_f32(uint32_t* ROWC, const float* VA, const uint32_t* 
     args.counts = ROWC;
     args.lightProducts = LightProductsFor(N, 0);
     args.heavyOnly = args.lightProducts != 0 ? 1u : 0u;
-    if (args.heavyOnly != 0 && M != 0)
-        LaunchLight<kCount>(args, stream);
-    hipLaunchKernelGGL(SpgemmRowKernel<kCount>,
-                       dim3(GridFor(M, args.rowsPerTurn, args.heavyOnly != 0)), dim3(64),
-                       args.strip * sizeof(float) + args.strip / 8, stream, args);
+    LaunchCounting<kCount>(args, stream);
     SPH_CHECK_LAUNCH();
     return sph::ExclusiveScanInPlace(ROWC, M + 1, nnzHost, stream);
 }
@@ -915,10 +962,7 @@ int sph_spgemm_fill_f32(float* VC, uint32_t* COLC, const uint32_t* ROWC, const f
     args.capacity = 0xffffffffu;
     args.lightProducts = LightProductsFor(N, 0);
     args.heavyOnly = args.lightProducts != 0 ? 1u : 0u;
-    if (args.heavyOnly != 0)
-        LaunchLight<kFill>(args, stream);
-    hipLaunchKernelGGL(SpgemmRowKernel<kFill>, dim3(GridFor(M, args.rowsPerTurn, false)), dim3(64),
-                       args.strip * sizeof(float) + args.strip / 8, stream, args);
+    LaunchFill(args, stream);
     SPH_CHECK_LAUNCH();
     return SPH_OK;
 }
@@ -998,8 +1042,6 @@ int sph_spgemm_f32(float* VC, uint32_t* COLC, uint32_t* ROWC, uint32_t capacity,
     args.counts = ROWC;
     args.lightProducts = LightProductsFor(N, M != 0 ? capacity / M : 0);
     args.heavyOnly = args.lightProducts != 0 ? 1u : 0u;
-    const dim3 rowGrid(GridFor(M, args.rowsPerTurn, args.heavyOnly != 0)), wave(64);
-    const size_t rowLds = args.strip * sizeof(float) + args.strip / 8;
 
     // staging slot per row: three times the mean the capacity allows plus 64 (twice, where
     // that is too much); without room for that (or without rows) the count, scan and fill
@@ -1027,15 +1069,11 @@ int sph_spgemm_f32(float* VC, uint32_t* COLC, uint32_t* ROWC, uint32_t capacity,
         args.COLC = reinterpret_cast<uint32_t*>(args.VC + slot * M);
         args.overflow = args.COLC + slot * M;
         args.slot = static_cast<uint32_t>(slot);
-        if (args.heavyOnly != 0)
-            LaunchLight<kStage>(args, stream);
-        hipLaunchKernelGGL(SpgemmRowKernel<kStage>, rowGrid, wave, rowLds, stream, args);
+        LaunchCounting<kStage>(args, stream);
     }
     else
     {
-        if (args.heavyOnly != 0 && M != 0)
-            LaunchLight<kCount>(args, stream);
-        hipLaunchKernelGGL(SpgemmRowKernel<kCount>, rowGrid, wave, rowLds, stream, args);
+        LaunchCounting<kCount>(args, stream);
     }
     hipError_t launched = hipGetLastError();
     int rc = SPH_OK;
@@ -1062,14 +1100,10 @@ int sph_spgemm_f32(float* VC, uint32_t* COLC, uint32_t* ROWC, uint32_t capacity,
         // after staging this pass usually finds nothing to do (it returns at once then), so it
         // is launched with few workgroups, which walk all rows if they must: dispatching the
         // full grid of empty workgroups alone took 15 us
-        const uint32_t few = static_cast<uint32_t>(sph::ComputeUnits()) * 2;
-        const uint32_t fillGrid = GridFor(M, args.rowsPerTurn, false);
-        const dim3 fillRowGrid(staged ? std::min(fillGrid, few) : fillGrid);
         if (staged)
-            args.heavyOnly = 0;  // rows that overflowed, light ones too: one launch for both
-        else if (args.heavyOnly != 0)
-            LaunchLight<kFill>(args, stream);
-        hipLaunchKernelGGL(SpgemmRowKernel<kFill>, fillRowGrid, wave, rowLds, stream, args);
+            LaunchStrips<kFill, kOverfullRows>(args, kRedoGroups, stream);
+        else
+            LaunchFill(args, stream);
         launched = hipGetLastError();
     }
     if (stageV != nullptr)

@@ -343,3 +343,43 @@ def test_no_rows(dev, N):
         assert np.all(d.download(np.uint32, guard.shape) == 0xFFFFFFFF)
     for d in bufs + [dRow, dV, dCol]:
         d.release()
+
+
+@pytest.mark.parametrize("N", [300, 9000])
+@pytest.mark.parametrize("M", [1, 5, 2047, 7001, 14000, 40001, 300001])
+def test_rows_that_a_pass_looks_for(dev, M, N):
+    """Passes that take only some rows (those left to the strips in a wide product, those that
+    overflowed their staging slot) with 1, 3, 6 and 8 rows per turn and more turns than one look
+    of all wavefronts covers: scattered ones, a run of neighbours, the first and the last row;
+    some of each kind overflow a slot of 67 entries."""
+    h.announce("sph_spgemm_* rows looked for, M N", (M, N))
+    K = 200
+    rng = np.random.default_rng(M + N)
+    lengths = np.where(np.arange(K) < 4, 90, rng.integers(0, 3, K))
+    RB = np.concatenate([[0], np.cumsum(lengths)]).astype(np.uint32)
+    CB = np.concatenate([rng.choice(N, size=n, replace=False) for n in lengths]).astype(np.uint32)
+    VB = rng.uniform(-1, 1, len(CB)).astype(np.float32)
+    kind = np.zeros(M, np.int64)                   # 0: one short row of B
+    kind[rng.integers(0, M, M // 97 + 1)] = 1      # 1: 70 entries of A
+    kind[rng.integers(0, M, M // 89 + 1)] = 2      # 2: two long rows of B, 180 products
+    kind[M // 2:M // 2 + 20] = 1
+    kind[[0, M - 1]] = 1, 2
+    per = np.array([1, 70, 2])[kind]
+    RA = np.concatenate([[0], np.cumsum(per)]).astype(np.uint32)
+    CA = rng.integers(4, K, int(RA[M]))
+    for row in np.nonzero(kind)[0]:
+        low, high = (4, K) if kind[row] == 1 else (0, 4)
+        CA[RA[row]:RA[row + 1]] = low + rng.choice(high - low, size=per[row], replace=False)
+    CA = CA.astype(np.uint32)
+    VA = rng.uniform(-1, 1, len(CA)).astype(np.float32)
+    A, B = (VA, CA, RA), (VB, CB, RB)
+    wV, wC, wR = po.spgemm_csr(A, B, M, K, N)
+    V, COL, ROW = gpu_spgemm(A, B, M, K, N)
+    assert np.array_equal(ROW, wR) and np.array_equal(COL, wC) and np.array_equal(bits(V), bits(wV))
+    total = int(wR[M])
+    for capacity in (M, total + 5):
+        V, COL, ROW, nnz = gpu_spgemm_one_call(A, B, M, K, N, capacity)
+        kept = min(capacity, total)
+        assert nnz == total and np.array_equal(ROW, wR), capacity
+        assert np.array_equal(COL[:kept], wC[:kept]), capacity
+        assert np.array_equal(bits(V[:kept]), bits(wV[:kept])), capacity
