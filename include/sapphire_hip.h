@@ -76,10 +76,12 @@ int sph_free(void* ptr);                               /* Memory.cpp:38-44 */
  * the device's pool, not to the driver, when it is freed, so neither call
  * waits for the device.  The pool behind the reference's ResourceManager
  * (Sources/Sapphire/util/ResourceManager.cpp:38-72 calls cudaMalloc / cudaFree,
- * both of which synchronise).  The scratch blocks of the CSR calls come from the
- * same pool, which keeps up to 512 MiB of them (without a limit once
- * sph_malloc_async has been called).  sph_mem_pool_trim hands idle pool memory
- * back. */
+ * both of which synchronise).  The scratch blocks of the CSR calls come from a
+ * pool of the library's own that keeps up to 512 MiB of freed blocks (from the
+ * device's pool, where its release threshold is at least that, as it is once
+ * sph_malloc_async has been called).  sph_mem_pool_trim hands the idle memory of
+ * both back; sph_malloc and sph_malloc_async do so with the library's own pool
+ * before they report that the device is full. */
 int sph_malloc_async(void** ptr, size_t bytes);
 int sph_free_async(void* ptr);
 int sph_mem_pool_trim(void);

@@ -46,8 +46,7 @@ int ResolveCsrScratch(uint32_t** scratch);
 void CountAllocation();
 
 // Takes a stream-ordered scratch block for one call of the library (counted; given back with
-// hipFreeAsync on the same stream).  The first one on a device has the device's memory pool keep
-// up to 512 MiB of freed blocks.
+// hipFreeAsync on the same stream), from a pool that keeps up to 512 MiB of freed blocks.
 int AllocScratch(void** ptr, size_t bytes, hipStream_t stream);
 
 // True between sph_graph_begin_capture and sph_graph_end_capture on this thread.  Entry

@@ -24,8 +24,10 @@ std::mutex gPoolMutex;
 std::vector<hipStream_t> gIdleStreams[kMaxDevices];
 int gComputeUnits[kMaxDevices] = {};
 bool gPoolRetains[kMaxDevices] = {};
-// (same mutex) the pool has been told to keep the library's own scratch blocks
-bool gPoolKeepsScratch[kMaxDevices] = {};
+// (same mutex) the devices' default pools, and the library's own pools for the scratch blocks of
+// its calls, created on first use and kept until the process ends
+hipMemPool_t gDefaultPools[kMaxDevices] = {};
+hipMemPool_t gScratchPools[kMaxDevices] = {};
 
 struct ThreadSlots
 {
@@ -58,35 +60,82 @@ void CountAllocation()
     gAllocations.fetch_add(1, std::memory_order_relaxed);
 }
 
-// With the pool's default threshold of zero every synchronisation hands freed blocks back to
-// the driver, and the next call maps its staging anew: a CSR x CSR product of 65536 rows
-// (139 MB of staging) that is waited for took 327 us, 87 us of them on the GPU
-// (now 100 us; dense to CSR and back, 8192 x 8192, 161 -> 123 us).  A bound keeps
-// what the library's own calls leave behind small beside the device's memory; a pool that already
-// keeps more (sph_malloc_async, or the program's own setting) is left alone.
+// With a release threshold of zero, the default of a device's pool, every synchronisation hands
+// freed blocks back to the driver, and the next call maps its staging anew: a CSR x CSR product of
+// 65536 rows (139 MB of staging) that is waited for took 384 us, 87 us of them on the GPU (now
+// 96 us; dense to CSR, 8192 x 4096, 58 -> 38 us).  So the blocks come from a pool of the
+// library's own that keeps a bounded amount: the device's default pool belongs to the program,
+// whose threshold and whose other users are left alone.  Where the program has the default pool
+// keep at least as much itself (sph_malloc_async does), that pool is used.
 constexpr uint64_t kScratchKept = 512ull << 20;
+
+namespace
+{
+int ScratchPool(hipMemPool_t* pool)
+{
+    const int d = tlsSlots.device;
+    std::lock_guard<std::mutex> lock(gPoolMutex);
+    if (gDefaultPools[d] == nullptr)
+        SPH_HIP_TRY(hipDeviceGetDefaultMemPool(&gDefaultPools[d], d));
+    *pool = gDefaultPools[d];
+    uint64_t keep = 0;  // the program may change it at any time
+    SPH_HIP_TRY(hipMemPoolGetAttribute(*pool, hipMemPoolAttrReleaseThreshold, &keep));
+    if (keep >= kScratchKept)
+        return SPH_OK;
+    if (gScratchPools[d] == nullptr)
+    {
+        hipMemPoolProps props{};
+        props.allocType = hipMemAllocationTypePinned;
+        props.handleTypes = hipMemHandleTypeNone;
+        props.location.type = hipMemLocationTypeDevice;
+        props.location.id = d;
+        hipMemPool_t own = nullptr;
+        SPH_HIP_TRY(hipMemPoolCreate(&own, &props));
+        keep = kScratchKept;
+        const hipError_t set = hipMemPoolSetAttribute(own, hipMemPoolAttrReleaseThreshold, &keep);
+        if (set != hipSuccess)
+        {
+            (void)hipMemPoolDestroy(own);
+            SPH_HIP_TRY(set);
+        }
+        gScratchPools[d] = own;
+    }
+    *pool = gScratchPools[d];
+    return SPH_OK;
+}
+
+// Idle blocks of the library's own pool go back to the driver.
+hipError_t TrimScratch()
+{
+    std::lock_guard<std::mutex> lock(gPoolMutex);
+    hipMemPool_t own = gScratchPools[tlsSlots.device];
+    return own != nullptr ? hipMemPoolTrimTo(own, 0) : hipSuccess;
+}
+
+// An allocation that finds the device full is tried once more without the idle scratch blocks.
+template <typename Alloc>
+hipError_t AllocWithTrim(Alloc&& alloc)
+{
+    hipError_t err = alloc();
+    if (err != hipErrorOutOfMemory)
+        return err;
+    (void)hipGetLastError();  // not the next launch's error
+    if (TrimScratch() == hipSuccess)
+        err = alloc();
+    if (err == hipErrorOutOfMemory)
+        (void)hipGetLastError();
+    return err;
+}
+}  // namespace
 
 int AllocScratch(void** ptr, size_t bytes, hipStream_t stream)
 {
-    const int d = tlsSlots.device;
-    {
-        std::lock_guard<std::mutex> lock(gPoolMutex);
-        if (!gPoolKeepsScratch[d] && !gPoolRetains[d])
-        {
-            hipMemPool_t pool = nullptr;
-            SPH_HIP_TRY(hipDeviceGetDefaultMemPool(&pool, d));
-            uint64_t keep = 0;
-            SPH_HIP_TRY(hipMemPoolGetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep));
-            if (keep < kScratchKept)
-            {
-                keep = kScratchKept;
-                SPH_HIP_TRY(hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep));
-            }
-            gPoolKeepsScratch[d] = true;
-        }
-    }
+    hipMemPool_t pool = nullptr;
+    const int found = ScratchPool(&pool);
+    if (found != SPH_OK)
+        return found;
     CountAllocation();
-    SPH_HIP_TRY(hipMallocAsync(ptr, bytes, stream));
+    SPH_HIP_TRY(AllocWithTrim([&] { return hipMallocFromPoolAsync(ptr, bytes, pool, stream); }));
     return SPH_OK;
 }
 
@@ -230,7 +279,7 @@ int sph_malloc(void** ptr, size_t bytes)
     SPH_REQUIRE(ptr != nullptr, "ptr is null");
     SPH_HIP_TRY(hipSetDevice(tlsSlots.device));
     ::sph::CountAllocation();
-    SPH_HIP_TRY(hipMalloc(ptr, bytes));
+    SPH_HIP_TRY(sph::AllocWithTrim([&] { return hipMalloc(ptr, bytes); }));
     return SPH_OK;
 }
 
@@ -260,7 +309,8 @@ int sph_malloc_async(void** ptr, size_t bytes)
         }
     }
     ::sph::CountAllocation();
-    SPH_HIP_TRY(hipMallocAsync(ptr, bytes != 0 ? bytes : 1, stream));
+    SPH_HIP_TRY(sph::AllocWithTrim(
+        [&] { return hipMallocAsync(ptr, bytes != 0 ? bytes : 1, stream); }));
     return SPH_OK;
 }
 
@@ -287,6 +337,7 @@ int sph_mem_pool_trim(void)
     hipMemPool_t pool = nullptr;
     SPH_HIP_TRY(hipDeviceGetDefaultMemPool(&pool, tlsSlots.device));
     SPH_HIP_TRY(hipMemPoolTrimTo(pool, 0));
+    SPH_HIP_TRY(sph::TrimScratch());
     return SPH_OK;
 }
 
