@@ -128,15 +128,33 @@ hipError_t AllocWithTrim(Alloc&& alloc)
 }
 }  // namespace
 
-int AllocScratch(void** ptr, size_t bytes, hipStream_t stream)
+int AllocScratchIfFree(void** ptr, size_t bytes, hipStream_t stream)
 {
+    *ptr = nullptr;
     hipMemPool_t pool = nullptr;
     const int found = ScratchPool(&pool);
     if (found != SPH_OK)
         return found;
+    const hipError_t err =
+        AllocWithTrim([&] { return hipMallocFromPoolAsync(ptr, bytes, pool, stream); });
+    if (err == hipErrorOutOfMemory)
+    {
+        *ptr = nullptr;
+        return SPH_OK;
+    }
+    SPH_HIP_TRY(err);
     CountAllocation();
-    SPH_HIP_TRY(AllocWithTrim([&] { return hipMallocFromPoolAsync(ptr, bytes, pool, stream); }));
     return SPH_OK;
+}
+
+int AllocScratch(void** ptr, size_t bytes, hipStream_t stream)
+{
+    const int taken = AllocScratchIfFree(ptr, bytes, stream);
+    if (taken == SPH_OK && *ptr == nullptr)
+        return Fail(SPH_ERR_DEVICE, std::string("no room for a scratch block of ") +
+                                        std::to_string(bytes) + " bytes: " +
+                                        hipGetErrorString(hipErrorOutOfMemory));
+    return taken;
 }
 
 int Fail(int status, const std::string& msg)

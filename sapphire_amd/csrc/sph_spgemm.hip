@@ -1079,32 +1079,27 @@ int sph_spgemm_f32(float* VC, uint32_t* COLC, uint32_t* ROWC, uint32_t capacity,
     args.lightProducts = LightProductsFor(N, M != 0 ? capacity / M : 0);
     args.heavyOnly = args.lightProducts != 0 ? 1u : 0u;
 
-    // staging slot per row: three times the mean the capacity allows plus 64 (twice, where
-    // that is too much); without room for that (or without rows) the count, scan and fill
-    // passes run one after the other.  Twice the mean is too little for rows whose lengths
-    // vary like those of a random graph: of 65536 rows with 64 products on average one or
-    // two did not fit, and doing those again cost 74 us.
-    const uint64_t mean = M != 0 ? capacity / M : 0;
-    uint64_t slot = M != 0 ? 3 * mean + 64 : 0;
-    if (slot * M >= (1ull << 31))
-        slot = 2 * mean + 64;
-    const bool staged = M != 0 && N != 0 && capacity != 0 && slot * M < (1ull << 31);
-    const bool placed = staged && M <= sph::kPlaceMaxRows;
+    // staging: counts (16-byte aligned, when the move scans them), values, columns, one flag
+    const size_t counts = M <= sph::kPlaceMaxRows ? (static_cast<size_t>(M) + 4) / 4 * 4 : 0;
     float* stageV = nullptr;
+    int taken = SPH_OK;
+    const uint32_t slot = sph::TakeStagingSlot(M, N, capacity, [&](uint32_t entries) {
+        taken = sph::AllocScratchIfFree(reinterpret_cast<void**>(&stageV),
+                                        counts * 4 + static_cast<size_t>(entries) * M * 8 + 4, stream);
+        return taken != SPH_OK || stageV != nullptr;  // a full device: with less
+    });
+    if (taken != SPH_OK)
+        return taken;
+    const bool staged = slot != 0;
+    const bool placed = staged && counts != 0;
     if (staged)
     {
-        // counts (16-byte aligned, when the move scans them), values, columns, one flag
-        const size_t counts = placed ? (static_cast<size_t>(M) + 4) / 4 * 4 : 0;
-        const int taken = sph::AllocScratch(reinterpret_cast<void**>(&stageV),
-                                            counts * 4 + slot * M * 8 + 4, stream);
-        if (taken != SPH_OK)
-            return taken;
         if (placed)
             args.counts = reinterpret_cast<uint32_t*>(stageV);
         args.VC = stageV + counts;
-        args.COLC = reinterpret_cast<uint32_t*>(args.VC + slot * M);
-        args.overflow = args.COLC + slot * M;
-        args.slot = static_cast<uint32_t>(slot);
+        args.COLC = reinterpret_cast<uint32_t*>(args.VC + static_cast<size_t>(slot) * M);
+        args.overflow = args.COLC + static_cast<size_t>(slot) * M;
+        args.slot = slot;
         LaunchCounting<kStage>(args, stream);
     }
     else

@@ -19,6 +19,27 @@ SPH_PLAN_HOST_DEVICE inline uint32_t SpgemmTurns(uint32_t M, uint32_t rowsPerTur
 {
     return M / rowsPerTurn + (M % rowsPerTurn != 0 ? 1u : 0u);
 }
+
+// Staging slots, in entries per row, that the one-call product tries in turn until `take(slot)`
+// finds memory for them: three times the mean row that the capacity allows plus 64, then twice the
+// mean.  All M slots together stay below 2^31 entries.  Returns the slot taken, 0 for none: the
+// products are then counted first and computed a second time to be stored.
+// Twice the mean is too little for rows whose lengths vary like those of a random graph: of
+// 65536 rows with 64 products on average one or two did not fit and were done again.
+template <typename Take>
+uint32_t TakeStagingSlot(uint32_t M, uint32_t N, uint32_t capacity, Take&& take)
+{
+    if (M == 0 || N == 0 || capacity == 0)
+        return 0;
+    const uint64_t mean = capacity / M;
+    for (uint64_t times = 3; times >= 2; --times)
+    {
+        const uint64_t slot = times * mean + 64;
+        if (slot * M < (1ull << 31) && take(static_cast<uint32_t>(slot)))
+            return static_cast<uint32_t>(slot);
+    }
+    return 0;
+}
 }  // namespace sph
 
 #endif

@@ -320,6 +320,18 @@ unsigned sphh_spgemm_turns(unsigned M, unsigned rowsPerTurn)
     return sph::SpgemmTurns(M, rowsPerTurn);
 }
 
+// The staging slot that the one-call CSR x CSR product takes when `room` bytes are free (8 bytes
+// per entry and row), and in tried[0 .. *tries) the slots it asked for.  No device is touched.
+unsigned sphh_staging_slot(unsigned M, unsigned N, unsigned capacity, unsigned long long room,
+                           unsigned* tried, unsigned* tries)
+{
+    *tries = 0;
+    return sph::TakeStagingSlot(M, N, capacity, [&](std::uint32_t slot) {
+        tried[(*tries)++] = slot;
+        return 8ull * slot * M <= room;
+    });
+}
+
 // Compute::Gemm into a FRESH y (never filled, never read): the operator sees the deferred zero
 // state of the new buffer and stores the product.  yOut receives the result.
 int sphh_compute_gemm_fresh_y(float* yOut, const int* y, int yn, const float* aData, const int* a,

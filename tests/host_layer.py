@@ -34,6 +34,9 @@ def lib():
         h.sphh_k_partition.argtypes = [ctypes.c_uint] * 5 + [ctypes.POINTER(ctypes.c_uint)]
         h.sphh_k_partition_slot.argtypes = [ctypes.c_uint] * 7
         h.sphh_k_partition_slot.restype = ctypes.c_uint
+        h.sphh_staging_slot.argtypes = [ctypes.c_uint] * 3 + [
+            ctypes.c_ulonglong, ctypes.POINTER(ctypes.c_uint), ctypes.POINTER(ctypes.c_uint)]
+        h.sphh_staging_slot.restype = ctypes.c_uint
         h.sphh_column_walk.argtypes = [ctypes.c_uint] * 3 + [ctypes.POINTER(ctypes.c_ulonglong)]
         h.sphh_spgemm_turns.argtypes = [ctypes.c_uint] * 2
         h.sphh_spgemm_turns.restype = ctypes.c_uint
@@ -164,6 +167,13 @@ def column_walk(N, lanes, ahead):
     out = (ctypes.c_ulonglong * 3)()
     _ok(lib().sphh_column_walk(N, lanes, ahead, out))
     return int(out[0]), None if out[1] == 2**64 - 1 else int(out[1]), int(out[2])
+
+
+def staging_slot(M, N, capacity, room):
+    """(slot taken, slots asked for)"""
+    tried, tries = (ctypes.c_uint * 8)(), ctypes.c_uint(0)
+    slot = int(lib().sphh_staging_slot(M, N, capacity, room, tried, ctypes.byref(tries)))
+    return slot, [int(tried[i]) for i in range(tries.value)]
 
 
 def spgemm_turns(M, rows_per_turn):
