@@ -1525,8 +1525,12 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF32SkinnyKernel(const GemmF32A
 // 1024 x 1024 5.6 / 3.4, 1000 x 1001 5.7 / 3.9, 2048 x 1024 5.6 / 5.1; past half as many
 // workgroups as compute units the other way: 4096 x 1024 6.4 / 7.2 (with 4 x 4 loads in flight),
 // 8192 x 1024 7.3 / 11.9, 512 x 512 x batch 16 4.6 / 7.0.
+// A lane of the 16-column form asks for 16 rows whatever K is, so its launch takes 3.5 us up to
+// K = 1024; that of the 64-column form grows with K (kernel times, N = 2048, K = 64 / 128 / 256 /
+// 320 / 384 / 512: 2.5 / 2.9 / 3.2 / 3.5 / 3.6 / 4.2 us; N = 10: 1.6 .. 2.5, 2.8, 3.2 against 2.4).
 // ---------------------------------------------------------------------------
 constexpr int kGemvWaves = 16;
+constexpr uint32_t kGemvShortK = 320;  // up to here 64 columns are the faster form for any N
 
 template <int COLS>
 __global__ __launch_bounds__(kGemvWaves * 64) void GemvRowKernel(const GemmF32Args args)
@@ -1984,9 +1988,10 @@ int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool o
         (args.split & 3u) == 0)
     {
         // 16 columns per workgroup while they are at most half as many as the compute units;
-        // beyond that 64-byte segments cost more than the longer chain (figures at the kernel)
+        // beyond that 64-byte segments cost more than the longer chain.  And from the K on where
+        // the chain is the longer one (figures at the kernel)
         const uint64_t blocks16 = static_cast<uint64_t>((args.N + 15) / 16) * units;
-        if (blocks16 * 2 <= cusAll)
+        if (blocks16 * 2 <= cusAll && args.K > kGemvShortK)
             hipLaunchKernelGGL(GemvRowKernel<16>, dim3((args.N + 15) / 16, units),
                                dim3(kGemvWaves * 64), 0, stream, args);
         else

@@ -1,5 +1,5 @@
-"""fp32 products with one output row (column sums, M = 1): 16 columns per workgroup up to half
-as many workgroups as compute units (2048 columns in all on this chip), 64 above that.
+"""fp32 products with one output row (column sums, M = 1): 16 columns per workgroup from K = 321 on up
+to half as many workgroups as compute units (2048 columns in all on this chip), 64 otherwise.
 
 Bar: the same sum in 64 bits.  An output element is at most ceil(K / 16) + 3 fused multiply-adds in
 one chain, then 2 + 15 + 2 additions of partial sums and the add of the old value, each rounded
@@ -17,7 +17,10 @@ pytestmark = pytest.mark.gpu
 # with 4 rows at a time; both sides of the line between the two widths; batches at odd strides
 SHAPES = [(1, 64, 1), (15, 65, 1), (16, 1024, 1), (17, 79, 1), (63, 1001, 1), (64, 4097, 1),
           (65, 127, 1), (1023, 1024, 1), (2048, 257, 1), (2049, 70, 1), (8255, 1001, 1),
-          (37, 333, 3), (128, 130, 16), (129, 130, 16), (65, 66, 25), (65, 66, 26)]
+          (37, 333, 3), (128, 130, 16), (129, 130, 16), (65, 66, 25), (65, 66, 26),
+          # past the short K: the edges of 16 columns, of 4 rows at a time, of the two widths
+          (1, 320, 1), (1, 321, 1), (15, 337, 1), (17, 383, 1), (65, 385, 1), (2048, 321, 1),
+          (2049, 321, 1), (128, 322, 16), (129, 322, 16), (65, 324, 25), (65, 324, 26)]
 
 
 @pytest.mark.parametrize("flags", [0, capi.SPH_GEMM_OVERWRITE])
@@ -42,9 +45,10 @@ def test_one_row_against_64_bits(dev, shape, flags):
     assert np.all(np.abs(got - (old + a @ b)) <= bound)
 
 
+@pytest.mark.parametrize("K", [130, 330])
 @pytest.mark.parametrize("relu", [0, capi.SPH_LINEAR_RELU])
-def test_one_row_bias_and_relu(dev, relu):
-    N, K = 77, 130
+def test_one_row_bias_and_relu(dev, relu, K):
+    N = 77
     h.announce("sph_linear_forward_f32 one row, flags", relu)
     x, W, bias = synth.uniform(821, (1, K)), synth.uniform(822, (K, N)), synth.uniform(823, (N,))
     dy, dx, dW, db = (capi.DeviceBuffer.from_array(v)
