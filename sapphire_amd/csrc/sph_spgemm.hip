@@ -387,6 +387,13 @@ __global__ __launch_bounds__(kLightWaves * 64, 5) void SpgemmLightKernel(const S
             if (MODE == kStage)
                 extentC = (first + lane) * args.slot;
         }
+        // a row with more entries than a light row has products is the strip kernel's
+        if (MODE == kFill)
+        {
+            const uint32_t entries = __shfl_down(extentC, 1, 64) - extentC;
+            if (__ballot(lane < rowsHere && entries <= kLightProducts) == 0)
+                continue;
+        }
         // stage 1: this lane's entry of A's row i (rows with more than 64 entries are not ours)
         auto loadStage1 = [&](uint32_t i, uint32_t& k, float& value) {
             k = kEmpty;
@@ -871,7 +878,11 @@ uint32_t RowsPerTurnFor(uint32_t M)
     return std::max<uint32_t>(1, std::min<uint32_t>(kRowsPerTurnMax, M / std::max<uint32_t>(wanted, 1)));
 }
 
-// Light rows: full occupancy is eight workgroups of four wavefronts per compute unit
+// Light rows: five workgroups of four wavefronts are resident per compute unit.  Turns are as long
+// as if there were eight: enough rows per turn to overlap their loads, with more workgroups than
+// places where rows are few, which are handed out as places fall free.  Turns that make whole
+// rounds of five were slower (16384 rows x 256 products 116.4 / 120.8 us, two calls 9000 x 144
+// 59.8 / 61.3 us) except where no row is light (two calls, 9000 x 900 308 / 300 us).
 template <int MODE>
 void LaunchLight(const SpgemmArgs& args, hipStream_t stream)
 {
