@@ -1061,7 +1061,7 @@ def main():
             "count_plus_fill_ms": ms, "products": products,
             "gproducts_per_s": 2 * products / (ms * 1e-3) / 1e9,
             "algorithmic_gbs": nbytes / (ms * 1e-3) / 1e9,
-            "note": "16 strips wide: rows with few products go through the hash-table kernel"}
+            "note": "16 strips wide: rows with few products are sorted in registers"}
         ms, ms_product, nnz_w, ms_unfused = bench_sparse_linear(capi, synth, 50, 5)
         others["sparse_linear_forward_8192x8192_batch256"] = {
             "forward_ms": ms, "csr_x_dense_ms": ms_product, "launches_per_forward": 3,

@@ -452,10 +452,12 @@ int sph_spgemm_fill_f32(float* VC, uint32_t* COLC, const uint32_t* ROWC,
  * and COLC and call sph_spgemm_fill_f32 with the ROWC already there.  The
  * products are computed once instead of twice: the counting pass also writes
  * every row into a staging slot of 3 * capacity / M + 64 entries (2 * where
- * that makes more than 2^31 in all; a stream-ordered scratch allocation of 8
- * bytes per slot entry), the counts are scanned and the staged rows moved
- * into place (one kernel up to 131072 rows) and only rows that did not fit their slot are multiplied again.  nnzHost as in
- * sph_spgemm_row_offsets_f32.  Refused during graph capture.  Same ROWC, VC
+ * that makes 2^31 or more in all or the device has no room for it; a
+ * stream-ordered scratch allocation of 8 bytes per slot entry; without room
+ * for the smaller one either, the products are computed twice), the counts are
+ * scanned and the staged rows moved into place (one kernel up to 131072 rows)
+ * and only rows that did not fit their slot are multiplied again.  nnzHost as
+ * in sph_spgemm_row_offsets_f32.  Refused during graph capture.  Same ROWC, VC
  * and COLC, bit for bit, as the two calls above. */
 int sph_spgemm_f32(float* VC, uint32_t* COLC, uint32_t* ROWC,
                    uint32_t capacity, const float* VA, const uint32_t* COLA,

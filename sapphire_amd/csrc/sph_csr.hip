@@ -801,9 +801,10 @@ int sph_csr_from_dense_f32(float* V, uint32_t* COL, uint32_t* ROW, uint32_t capa
     // plus 32, a multiple of 4
     const uint64_t mean = M != 0 ? capacity / M : 0;
     const uint64_t stage64 = (2 * mean + 32 + 3) / 4 * 4;
-    // (below 16 Mi elements the scratch allocation of the one-pass path costs more host time than
-    // the second pass over the matrix it saves: 2048 x 2048 19 us against 12 us, 8192 x 1000 23
-    // against 19 us; 4096 x 4096 20 us either way)
+    // (from 16 Mi elements on.  Separate passes / one pass with scratch blocks that the pool keeps:
+    // 2048 x 2048 10.8 / 17.9 us, 4096 x 2048 14.0 / 17.6, 8192 x 1000 18.2 / 18.1, 3000 x 4096
+    // 20.5 / 17.7, 16384 x 1000 34.3 / 24.1.  The line was drawn where both were level while
+    // every call mapped its block anew, 4096 x 4096; today that is near 8192 x 1000)
     if (!(M != 0 && N >= 128 && N <= 8192 && stage64 * 4 <= N &&
           static_cast<uint64_t>(M) * N >= (1ull << 24)))
     {

@@ -10,7 +10,7 @@
 // starting from +0; results that are exactly 0 are not stored (SparseUtil.cu:55-60 deletes
 // them as well); a row's entries come out in ascending column order.
 //
-// One wavefront owns one output row.  Instead of a hash table and a sort it keeps a dense
+// One wavefront owns one output row.  Instead of a hash table and a sort it usually keeps a dense
 // strip of the row in LDS (up to 4096 columns, 16 KiB; wider matrices are done strip by
 // strip): A's entries are taken in order, the entries of the matching row of B are spread
 // over the 64 lanes and added into the strip, and because the columns of one row of B are
@@ -363,7 +363,7 @@ __device__ __forceinline__ uint32_t LightRowOfAnyLength(const SpgemmArgs& args, 
 // a row follows its products, not the width of the matrix.
 // What bounds it is the chain of four dependent loads and the issue of the exchanges; five
 // wavefronts per SIMD are resident.  65536 rows with 8 entries on both sides: 63 us for the pass
-// (180 us with a hash table in LDS, one row of B inserted at a time); the whole call 265 -> 92 us.
+// (180 us with a hash table in LDS, one row of B inserted at a time); the whole call 264 -> 87 us.
 template <int MODE, typename Key>
 __global__ __launch_bounds__(kLightWaves * 64, 5) void SpgemmLightKernel(const SpgemmArgs args)
 {

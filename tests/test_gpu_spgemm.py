@@ -198,11 +198,12 @@ def test_random_shapes_and_densities(dev, block):
         check_one_call(A, B, M, K, N, (wV, wC, wR))
 
 
-def test_wide_product_mixes_table_rows_and_strip_rows(dev):
-    """More than two strips of columns: rows with few products are kept in the hash table,
-    the others stay with the strips.  The operands mix both kinds: rows of A that select rows of
-    B longer than 64 entries, rows of A with more than 64 entries, rows with more than 256
-    products, empty rows, and a pair of entries whose contributions cancel exactly."""
+def test_wide_product_mixes_sorted_rows_and_strip_rows(dev):
+    """More than two strips of columns: rows with few products (at most 64 entries of A, at most
+    512 products) are sorted in registers, the others stay with the strips.  The operands mix
+    both kinds: rows of A that select rows of B longer than 64 entries, rows of A with more than 64
+    entries, rows with more than 512 products, empty rows, and a pair of entries whose
+    contributions cancel exactly."""
     M, K, N = 260, 300, 20000
     h.announce("sph_spgemm_* wide product with light and heavy rows", (M, K, N))
     rng = np.random.default_rng(77)
@@ -215,13 +216,13 @@ def test_wide_product_mixes_table_rows_and_strip_rows(dev):
     dA = np.zeros((M, K), np.float32)
     for m in range(M):
         kind = m % 5
-        if kind == 0:    # one or two long rows of B: light, with the 64-at-a-time tail
+        if kind == 0:    # one or two long rows of B: light, 100 or 200 products
             ks = rng.choice(10, size=1 + m % 2, replace=False)
         elif kind == 1:  # a handful of short rows of B: light
             ks = 10 + rng.choice(K - 10, size=6, replace=False)
         elif kind == 2:  # more than 64 entries: the strips' row
             ks = rng.choice(K, size=150, replace=False)
-        elif kind == 3:  # few entries, more than 256 products: the strips' row
+        elif kind == 3:  # few entries, 600 products: the strips' row
             ks = rng.choice(10, size=6, replace=False)
         else:            # empty
             ks = np.zeros(0, np.int64)
