@@ -126,25 +126,129 @@ __device__ __forceinline__ bool LightRow(const SpgemmArgs& args, uint32_t entrie
     return entriesOfA <= 64 && products <= args.lightProducts;
 }
 
-// value of lane (lane ^ MASK).  Four of the six masks are lane permutations of the vector unit
-// itself and never go through the LDS crossbar.
+// Lane operations of the vector unit itself (no LDS crossbar, no wait): DPP controls.
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppXor3 = 0x1B;  // quad permutations
+constexpr int kDppXor7 = 0x141, kDppXor15 = 0x140;  // half-row and row mirrored
+constexpr int kDppXor8 = 0x128;                     // row rotated by 8
+constexpr int kDppShr1 = 0x111, kDppShr2 = 0x112, kDppShr4 = 0x114, kDppShr8 = 0x118;
+constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;  // last lane of a row / of two rows
+constexpr int kDppWaveShr1 = 0x138;                      // the lane before, across rows
+
+// value that lanes without a source, and rows not in ROWS, get: `none`
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ uint32_t Dpp(uint32_t none, uint32_t v)
+{
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+        static_cast<int>(none), static_cast<int>(v), CTRL, ROWS, 0xf, false));
+}
+
+// a permutation: every lane has a source
+template <int CTRL>
+__device__ __forceinline__ uint32_t Permute(uint32_t v)
+{
+    return static_cast<uint32_t>(
+        __builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xf, 0xf, true));
+}
+
+// inclusive scan over the lanes; combine(0, x) is x
+template <typename Combine>
+__device__ __forceinline__ uint32_t WaveScan(uint32_t v, Combine combine)
+{
+    v = combine(v, Dpp<kDppShr1>(0, v));
+    v = combine(v, Dpp<kDppShr2>(0, v));
+    v = combine(v, Dpp<kDppShr4>(0, v));
+    v = combine(v, Dpp<kDppShr8>(0, v));
+    v = combine(v, Dpp<kDppBcast15, 0xa>(0, v));
+    return combine(v, Dpp<kDppBcast31, 0xc>(0, v));
+}
+
+struct LanePair
+{
+    uint32_t x, y;
+};
+
+// MASK 16: odd rows of 16 lanes of x change places with even rows of y; MASK 32: the upper half of
+// x with the lower half of y.  Pairs (l, l ^ MASK) of x then stand side by side in the lanes of
+// one half and those of y in the others; a second swap undoes it.
+template <uint32_t MASK>
+__device__ __forceinline__ LanePair SwapLanes(uint32_t x, uint32_t y)
+{
+    static_assert(MASK == 16 || MASK == 32, "rows of 16 or halves");
+    if constexpr (MASK == 16)
+    {
+        const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+        return { r[0], r[1] };
+    }
+    else
+    {
+        const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+        return { r[0], r[1] };
+    }
+}
+
+// value of lane (lane ^ MASK): a power of two, or one less than a power of two up to 16
 template <uint32_t MASK>
 __device__ __forceinline__ uint32_t XorLane(uint32_t v)
 {
-    const int x = static_cast<int>(v);
-    if constexpr (MASK == 1)
-        return __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, true);  // quad 1 0 3 2
+    if constexpr (MASK == 0)
+        return v;
+    else if constexpr (MASK == 1)
+        return Permute<kDppXor1>(v);
     else if constexpr (MASK == 2)
-        return __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, true);  // quad 2 3 0 1
-    else if constexpr (MASK == 4)  // mirrored within 8 lanes (^ 7), then within 4 (^ 3)
-        return __builtin_amdgcn_update_dpp(
-            0, __builtin_amdgcn_update_dpp(0, x, 0x141, 0xf, 0xf, true), 0x1B, 0xf, 0xf, true);
+        return Permute<kDppXor2>(v);
+    else if constexpr (MASK == 3)
+        return Permute<kDppXor3>(v);
+    else if constexpr (MASK == 4)
+        return Permute<kDppXor3>(Permute<kDppXor7>(v));
+    else if constexpr (MASK == 7)
+        return Permute<kDppXor7>(v);
     else if constexpr (MASK == 8)
-        return __builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, true);  // rotate 16 by 8
-    else if constexpr (MASK == 16)
-        return __builtin_amdgcn_ds_swizzle(x, (16 << 10) | 0x1f);
+        return Permute<kDppXor8>(v);
+    else if constexpr (MASK == 15)
+        return Permute<kDppXor15>(v);
     else
-        return __shfl_xor(v, MASK, 64);
+    {
+        const LanePair p = SwapLanes<MASK>(v, v);
+        return (threadIdx.x & MASK) != 0 ? p.x : p.y;
+    }
+}
+
+// the smaller of x and y where bound is 0, the larger where it is all ones (v_med3_u32)
+__device__ __forceinline__ uint32_t Med3(uint32_t x, uint32_t y, uint32_t bound)
+{
+    return max(min(x, y), min(max(x, y), bound));
+}
+
+// all ones in the lanes with that bit set
+struct LaneBits
+{
+    uint32_t bit[6];
+    __device__ __forceinline__ explicit LaneBits(uint32_t lane)
+    {
+#pragma unroll
+        for (uint32_t k = 0; k < 6; ++k)
+            bit[k] = 0u - ((lane >> k) & 1u);
+    }
+    // Keeps the compiler from working the bounds of a sort out ahead of the rows, which costs more
+    // registers than a row has to spare.
+    __device__ __forceinline__ void Pin()
+    {
+#pragma unroll
+        for (uint32_t k = 0; k < 6; ++k)
+            asm volatile("" : "+v"(bit[k]));
+    }
+};
+
+// The one of two keys that a lane keeps: the smaller where `bound` is 0, else the larger.
+__device__ __forceinline__ uint32_t Exchange(uint32_t x, uint32_t y, uint32_t bound)
+{
+    return Med3(x, y, bound);
+}
+
+// (keys of 64 bits: 2^23 columns and more, and the pass that does overflowed rows again)
+__device__ __forceinline__ uint64_t Exchange(uint64_t x, uint64_t y, uint32_t bound)
+{
+    return (y < x) == (bound == 0) ? y : x;
 }
 
 template <uint32_t MASK>
@@ -156,84 +260,133 @@ __device__ __forceinline__ uint64_t XorLane(uint64_t v)
 }
 
 // Bitonic sort of 64 E keys held by one wavefront, E consecutive ones per lane: the exchanges
-// from (SIZE, STRIDE) on.
+// from (SIZE, STRIDE) on.  An exchange of 32-bit keys is one lane operation and one v_med3_u32
+// against a bound that is 0 in the lanes that keep the smaller key and all ones in the others: no
+// condition code, and so no wait between vector and scalar unit.
+// Merges inside a row of 16 lanes begin with an exchange between a block and its mirror image,
+// which needs no blocks of opposite directions: one bound per stride serves them all.  Odd rows
+// then end up descending (`down`), and so does the upper half of the lanes, as the merges
+// across rows need it.
 template <uint32_t E, typename Key, uint32_t SIZE = 2, uint32_t STRIDE = 1>
-__device__ __forceinline__ void SortKeys(Key (&key)[E], uint32_t lane)
+__device__ __forceinline__ void SortKeys(Key (&key)[E], const LaneBits& lanes)
 {
+    constexpr bool kInRow = SIZE <= 16 * E;
+    constexpr bool kMirror = kInRow && STRIDE == SIZE / 2;
+    const uint32_t down = kInRow ? lanes.bit[4] : SIZE == 32 * E ? lanes.bit[5] : 0u;
     if constexpr (STRIDE < E)
     {
 #pragma unroll
         for (uint32_t e = 0; e < E; ++e)
         {
-            if ((e & STRIDE) != 0)
+            const uint32_t o = kMirror ? e ^ (SIZE - 1) : e ^ STRIDE;
+            if (o < e)
                 continue;
-            const bool ascending = SIZE < E ? (e & SIZE) == 0 : (lane & (SIZE / E)) == 0;
-            const Key x = key[e], y = key[e + STRIDE];
-            const bool swap = (y < x) == ascending;
-            key[e] = swap ? y : x;
-            key[e + STRIDE] = swap ? x : y;
+            const Key x = key[e], y = key[o];
+            key[e] = Exchange(x, y, down);
+            key[o] = Exchange(x, y, ~down);
+        }
+    }
+    else if constexpr (STRIDE / E >= 16 && E > 1 && sizeof(Key) == 4)
+    {
+        // two keys of a lane at once: their pairs side by side, and back
+#pragma unroll
+        for (uint32_t e = 0; e < E; e += 2)
+        {
+            const LanePair p = SwapLanes<STRIDE / E>(key[e], key[e + 1]);
+            const LanePair q =
+                SwapLanes<STRIDE / E>(Med3(p.x, p.y, down), Med3(p.x, p.y, ~down));
+            key[e] = q.x;
+            key[e + 1] = q.y;
         }
     }
     else
     {
-        const bool smaller = ((lane & (STRIDE / E)) == 0) == ((lane & (SIZE / E)) == 0);
-#pragma unroll
-        for (uint32_t e = 0; e < E; ++e)
+        constexpr uint32_t kLanes = STRIDE / E;  // a power of two
+        const uint32_t bound = lanes.bit[__builtin_ctz(kLanes)] ^ down;
+        if constexpr (kLanes >= 16 && sizeof(Key) == 4)
         {
-            const Key other = XorLane<STRIDE / E>(key[e]);
-            key[e] = (other < key[e]) == smaller ? other : key[e];
+            const LanePair p = SwapLanes<kLanes>(key[0], key[0]);
+            key[0] = Med3(p.x, p.y, bound);
+        }
+        else if constexpr (kMirror)
+        {
+            Key other[E];
+#pragma unroll
+            for (uint32_t e = 0; e < E; ++e)
+                other[e] = XorLane<SIZE / E - 1>(key[E - 1 - e]);
+#pragma unroll
+            for (uint32_t e = 0; e < E; ++e)
+                key[e] = Exchange(key[e], other[e], bound);
+        }
+        else
+        {
+#pragma unroll
+            for (uint32_t e = 0; e < E; ++e)
+                key[e] = Exchange(key[e], XorLane<kLanes>(key[e]), bound);
         }
     }
     if constexpr (STRIDE > 1)
-        SortKeys<E, Key, SIZE, STRIDE / 2>(key, lane);
+        SortKeys<E, Key, SIZE, STRIDE / 2>(key, lanes);
     else if constexpr (SIZE < 64 * E)
-        SortKeys<E, Key, SIZE * 2, SIZE>(key, lane);
+        SortKeys<E, Key, SIZE * 2, SIZE>(key, lanes);
 }
 
 // A wavefront's own LDS: nothing is shared between wavefronts, and the LDS operations of one
 // wavefront are executed in order.
 struct LightScratch
 {
+    uint32_t column[kLightProducts];  // before the sort: the entry of A that starts here
     float product[kLightProducts];
-    uint32_t column[kLightProducts];
-    float value[kLightProducts];
 };
 
 struct LightInput
 {
     uint32_t entriesOfA;      // uniform, at most 64
     uint32_t products;        // uniform, at most 64 E
-    uint32_t bBegin, before;  // of lane j: first entry of the row of B that A's entry j selects,
-    float aValue;             // products of A's entries before j, value of A's entry j
+    // of lane j: products of A's entry j, their first entry in B, products of the entries before
+    uint32_t mine, bBegin, before;
+    float aValue;             // and the value of A's entry j
     uint32_t rowBase, rowLimit;  // uniform: where the entries go
+};
+
+// four-byte aligned groups of entries, stored with one access
+template <uint32_t E, typename T>
+struct EntryGroup
+{
+    typedef T Type __attribute__((ext_vector_type(E), aligned(4)));
 };
 
 // The entries of one light row; returns their number.
 template <int MODE, uint32_t E, typename Key>
 __device__ __forceinline__ uint32_t LightRowEntries(const SpgemmArgs& args, const LightInput& in,
-                                                    LightScratch& lds, uint32_t lane)
+                                                    LightScratch& lds, uint32_t lane,
+                                                    const LaneBits& lanes)
 {
-    // product p (in the order in which the sums take them) belongs to lane p % 64
+    // Product p (in the order in which the sums take them) belongs to lane p % 64.  The entry of A
+    // it comes from: every entry that has products leaves its number + 1 at its first one, and
+    // the largest number at or before p is the one.
+#pragma unroll
+    for (uint32_t e = 0; e < E; ++e)
+        lds.column[e * 64u + lane] = 0;
+    if (in.mine != 0)
+        lds.column[in.before] = lane + 1;
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t from = in.bBegin - in.before;
     uint32_t base[E];
     float a[E];
+    uint32_t passed = 0;
 #pragma unroll
     for (uint32_t e = 0; e < E; ++e)
     {
-        base[e] = 0;
-        a[e] = 0.0f;
-    }
-    for (uint32_t j = 0; j < in.entriesOfA; ++j)
-    {
-        const uint32_t start = Uniform(in.before, j);
-        const uint32_t from = Uniform(in.bBegin, j) - start;
-        const float value = Uniform(in.aValue, j);
-#pragma unroll
-        for (uint32_t e = 0; e < E; ++e)
-        {
-            const bool reached = e * 64u + lane >= start;
-            base[e] = reached ? from : base[e];
-            a[e] = reached ? value : a[e];
-        }
+        const uint32_t entry =
+            max(passed, WaveScan(lds.column[e * 64u + lane],
+                                 [](uint32_t x, uint32_t y) { return max(x, y); }));
+        passed = Uniform(entry, 63);
+        const int source = static_cast<int>(entry * 4u - 4u);
+        base[e] = static_cast<uint32_t>(
+            __builtin_amdgcn_ds_bpermute(source, static_cast<int>(from)));
+        a[e] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(
+                                             source, __builtin_bit_cast(int, in.aValue)));
     }
     uint32_t col[E];
     float b[E];
@@ -258,43 +411,114 @@ __device__ __forceinline__ uint32_t LightRowEntries(const SpgemmArgs& args, cons
         key[e] = col[e] < args.N ? static_cast<Key>(col[e]) << kPlaceBits | p : ~static_cast<Key>(0);
         lds.product[p] = a[e] * b[e];
     }
-    SortKeys<E, Key>(key, lane);
+    LaneBits bounds = lanes;
+    bounds.Pin();
+    SortKeys<E, Key>(key, bounds);
     __builtin_amdgcn_wave_barrier();
 
     // the sorted (column, product) pairs side by side
     const uint32_t place0 = lane * E;
     uint32_t c[E];
     float v[E];
+    bool used[E];
+    uint32_t valid = 0;  // pairs of the row
 #pragma unroll
     for (uint32_t e = 0; e < E; ++e)
     {
-        const bool used = key[e] != ~static_cast<Key>(0);
-        c[e] = used ? static_cast<uint32_t>(key[e] >> kPlaceBits) : kEmpty;
+        used[e] = key[e] != ~static_cast<Key>(0);
+        c[e] = used[e] ? static_cast<uint32_t>(key[e] >> kPlaceBits) : kEmpty;
         v[e] = lds.product[static_cast<uint32_t>(key[e]) & (64u * E - 1)];
+        valid += static_cast<uint32_t>(__popcll(__ballot(used[e])));
     }
+    // does a pair have the column of the one before it?
+    bool repeats[E];
+    bool anyRepeats = false;
 #pragma unroll
     for (uint32_t e = 0; e < E; ++e)
     {
-        lds.column[place0 + e] = c[e];
-        lds.value[place0 + e] = v[e];
+        const uint32_t left = e != 0 ? c[e == 0 ? 0 : e - 1] : Dpp<kDppWaveShr1>(kEmpty, c[E - 1]);
+        repeats[e] = used[e] && c[e] == left;
+        anyRepeats = anyRepeats || repeats[e];
     }
-    __builtin_amdgcn_wave_barrier();
     // the first pair of a column sums the column's products, in their order, from +0
+    if (__ballot(anyRepeats) == 0)
+    {
+#pragma unroll
+        for (uint32_t e = 0; e < E; ++e)
+            v[e] = 0.0f + v[e];
+    }
+    else
+    {
+        __builtin_amdgcn_wave_barrier();
+        uint32_t place = place0;
+        asm volatile("" : "+v"(place));  // (or it is held in E forms through every row)
+#pragma unroll
+        for (uint32_t e = 0; e < E; ++e)
+        {
+            lds.column[place + e] = c[e];
+            lds.product[place + e] = v[e];
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (uint32_t e = 0; e < E; ++e)
+        {
+            if (used[e] && !repeats[e])
+            {
+                float sum = 0.0f + v[e];
+                for (uint32_t t = place + e + 1; t < 64u * E && lds.column[t] == c[e]; ++t)
+                    sum = sum + lds.product[t];
+                v[e] = sum;
+            }
+        }
+    }
     bool keep[E];
+    bool dropped = false;
 #pragma unroll
     for (uint32_t e = 0; e < E; ++e)
     {
-        const uint32_t left = e != 0 ? c[e == 0 ? 0 : e - 1]
-                                     : place0 != 0 ? lds.column[place0 - 1] : kEmpty;
-        keep[e] = false;
-        if (c[e] != kEmpty && c[e] != left)
+        keep[e] = used[e] && !repeats[e] && v[e] != 0.0f;  // exact zeros are not stored
+        dropped = dropped || keep[e] != used[e];
+    }
+    if (__ballot(dropped) == 0)
+    {
+        // every pair is an entry: a lane's are neighbours
+        if (MODE != kCount)
         {
-            float sum = 0.0f + v[e];
-            for (uint32_t t = place0 + e + 1; t < 64u * E && lds.column[t] == c[e]; ++t)
-                sum = sum + lds.value[t];
-            v[e] = sum;
-            keep[e] = sum != 0.0f;  // exact zeros are not stored
+            const uint32_t at = in.rowBase + place0;
+            const uint32_t room = in.rowLimit > in.rowBase ? in.rowLimit - in.rowBase : 0u;
+            const uint32_t end = min(valid, room);
+            constexpr uint32_t kGroup = E < 4 ? E : 4;
+            typedef typename EntryGroup<kGroup, float>::Type Values;
+            typedef typename EntryGroup<kGroup, uint32_t>::Type Columns;
+#pragma unroll
+            for (uint32_t g = 0; g < E; g += kGroup)
+            {
+                if (place0 + g + kGroup <= end)
+                {
+                    Values values;
+                    Columns columns;
+#pragma unroll
+                    for (uint32_t e = 0; e < kGroup; ++e)
+                    {
+                        values[e] = v[g + e];
+                        columns[e] = c[g + e];
+                    }
+                    *reinterpret_cast<Values*>(args.VC + at + g) = values;
+                    *reinterpret_cast<Columns*>(args.COLC + at + g) = columns;
+                }
+                else if (kGroup > 1 && place0 + g < end)
+                {
+#pragma unroll
+                    for (uint32_t e = 0; e < kGroup - 1; ++e)
+                        if (place0 + g + e < end)
+                        {
+                            args.VC[at + g + e] = v[g + e];
+                            args.COLC[at + g + e] = c[g + e];
+                        }
+                }
+            }
         }
+        return valid;
     }
     const uint64_t below = (1ull << lane) - 1ull;
     uint32_t before = 0, emitted = 0;
@@ -324,17 +548,10 @@ __device__ __forceinline__ uint32_t LightRowEntries(const SpgemmArgs& args, cons
 }
 
 // Prefix sum of the lanes' numbers of products; true when the row is light.
-__device__ __forceinline__ bool CountProducts(const SpgemmArgs& args, LightInput& in, uint32_t mine,
-                                              uint32_t lane)
+__device__ __forceinline__ bool CountProducts(const SpgemmArgs& args, LightInput& in, uint32_t mine)
 {
-    uint32_t inclusive = mine;
-#pragma unroll
-    for (uint32_t d = 1; d < 64; d *= 2)
-    {
-        const uint32_t other = __shfl_up(inclusive, d, 64);
-        if (lane >= d)
-            inclusive += other;
-    }
+    const uint32_t inclusive = WaveScan(mine, [](uint32_t x, uint32_t y) { return x + y; });
+    in.mine = mine;
     in.before = inclusive - mine;
     in.products = Uniform(inclusive, 63);
     return LightRow(args, in.entriesOfA, in.products);
@@ -343,15 +560,16 @@ __device__ __forceinline__ bool CountProducts(const SpgemmArgs& args, LightInput
 // The entries of one light row, with as many products per lane as it needs.
 template <int MODE, typename Key>
 __device__ __forceinline__ uint32_t LightRowOfAnyLength(const SpgemmArgs& args, const LightInput& in,
-                                                        LightScratch& lds, uint32_t lane)
+                                                        LightScratch& lds, uint32_t lane,
+                                                        const LaneBits& lanes)
 {
     if (in.products <= 64)
-        return LightRowEntries<MODE, 1, Key>(args, in, lds, lane);
+        return LightRowEntries<MODE, 1, Key>(args, in, lds, lane, lanes);
     if (in.products <= 128)
-        return LightRowEntries<MODE, 2, Key>(args, in, lds, lane);
+        return LightRowEntries<MODE, 2, Key>(args, in, lds, lane, lanes);
     if (in.products <= 256)
-        return LightRowEntries<MODE, 4, Key>(args, in, lds, lane);
-    return LightRowEntries<MODE, 8, Key>(args, in, lds, lane);
+        return LightRowEntries<MODE, 4, Key>(args, in, lds, lane, lanes);
+    return LightRowEntries<MODE, 8, Key>(args, in, lds, lane, lanes);
 }
 
 // Light rows.  The strip kernel walks all products of a row once per strip of 4096 columns, one
@@ -361,15 +579,19 @@ __device__ __forceinline__ uint32_t LightRowOfAnyLength(const SpgemmArgs& args, 
 // product of a column then adds the following ones of the same column in that order, sums that
 // are exactly zero are dropped, and ballots give the others their output positions.  The cost of
 // a row follows its products, not the width of the matrix.
-// What bounds it is the chain of four dependent loads and the issue of the exchanges; five
-// wavefronts per SIMD are resident.  65536 rows with 8 entries on both sides: 63 us for the pass
-// (180 us with a hash table in LDS, one row of B inserted at a time); the whole call 264 -> 87 us.
+// What bounds it is the issue of vector instructions (about 300 for a row of 64 products) behind a
+// chain of four dependent loads; seven wavefronts per SIMD are resident (five left 8192 rows in
+// two rounds; eight spill scalars and are level).  Against a sort by compares and selects, shuffles
+// through the LDS crossbar and a search of every product's entry of A one entry after the other:
+// 65536 rows with 8 entries on both sides 63 -> 38 us for the pass, the whole call 86 -> 59 us;
+// 8192 rows 15.8 -> 9.4 us.
 template <int MODE, typename Key>
-__global__ __launch_bounds__(kLightWaves * 64, 5) void SpgemmLightKernel(const SpgemmArgs args)
+__global__ __launch_bounds__(kLightWaves * 64, 7) void SpgemmLightKernel(const SpgemmArgs args)
 {
     __shared__ LightScratch scratch[kLightWaves];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = threadIdx.x >> 6;
+    const LaneBits lanes(lane);
     const uint32_t turn0 = blockIdx.x * kLightWaves + wave;
     const uint64_t step = static_cast<uint64_t>(gridDim.x) * kLightWaves * args.rowsPerTurn;
     // A wavefront takes rowsPerTurn consecutive rows per turn, with the loads that lead to a
@@ -424,6 +646,7 @@ __global__ __launch_bounds__(kLightWaves * 64, 5) void SpgemmLightKernel(const S
         loadStage2(k2, nextBegin, nextEnd);
         loadStage1(1, k1, value1);
 
+        uint32_t counted = 0;  // of lane i: entries of the turn's row i
         for (uint32_t i = 0; i < rowsHere; ++i)
         {
             LightInput in;
@@ -435,10 +658,9 @@ __global__ __launch_bounds__(kLightWaves * 64, 5) void SpgemmLightKernel(const S
             value2 = value1;
             loadStage2(k2, nextBegin, nextEnd);
             loadStage1(i + 2, k1, value1);
-            if (!CountProducts(args, in, mine, lane))
+            if (!CountProducts(args, in, mine))
             {
-                if (MODE != kFill && lane == 0)
-                    args.counts[first + i] = kHeavyMark;  // the strip kernel's row
+                counted = lane == i ? kHeavyMark : counted;  // the strip kernel's row
                 continue;
             }
             in.rowBase = 0;
@@ -450,10 +672,12 @@ __global__ __launch_bounds__(kLightWaves * 64, 5) void SpgemmLightKernel(const S
                 if (MODE == kFill)
                     in.rowLimit = min(in.rowLimit, args.capacity);
             }
-            const uint32_t emitted = LightRowOfAnyLength<MODE, Key>(args, in, scratch[wave], lane);
-            if (MODE != kFill && lane == 0)
-                args.counts[first + i] = emitted;
+            const uint32_t emitted =
+                LightRowOfAnyLength<MODE, Key>(args, in, scratch[wave], lane, lanes);
+            counted = lane == i ? emitted : counted;
         }
+        if (MODE != kFill && lane < rowsHere)
+            args.counts[first + lane] = counted;
     }
 }
 
@@ -565,9 +789,9 @@ __global__ __launch_bounds__(64) void SpgemmRowKernel(const SpgemmArgs args)
             in.aValue = firstValue;
             in.rowBase = rowBase;
             in.rowLimit = rowLimit;
-            if (CountProducts(args, in, LightCount(firstBegin, firstEnd), lane))
+            if (CountProducts(args, in, LightCount(firstBegin, firstEnd)))
             {
-                LightRowOfAnyLength<kFill, uint64_t>(args, in, scratch, lane);
+                LightRowOfAnyLength<kFill, uint64_t>(args, in, scratch, lane, LaneBits(lane));
                 continue;
             }
         }
@@ -849,18 +1073,21 @@ __global__ void ClearTotalKernel(unsigned long long* total)
 
 // Most products of a row that SpgemmLightKernel takes; products: the caller's bound on the
 // mean products of a row (a capacity is usually that), 0 when there is none.
-// One strip: always the strip kernel (1024 columns, 8 entries per row: 22.3 us, 26.2 us with the
-// second launch).  Two strips: the strip kernel costs little more than on one, and rows of which
-// only a part is light pay both kernels, so all have to be light (8192 columns, 8 / 10 entries
-// per row 53 / 60 -> 29 / 32 us; 16 / 22 entries 75 / 134 us with all rows up to 512 products
-// taken, 77 / 103 us on strips).  From three strips on always (9000 columns, 12 / 18 / 21
-// entries: 110 / 181 / 182 -> 40 / 107 / 160 us).
+// One strip: always the strip kernel (4096 columns, 16 / 32 entries per row: 35 / 71 us a call,
+// 40 / 80 us with all rows up to 512 products taken; with fewer products the host bounds both).
+// Two strips: the strip kernel costs little more than on one, and rows of which only a part is
+// light pay both kernels, so nearly all have to be light (6000 columns, 12 / 15 / 16 / 17 entries
+// per row 58 / 67 / 72 / 75 us on strips, 32 / 32 / 54 / 61 us here; 4200 columns, 15 / 16 / 17
+// entries 46 / 51 / 52 against 46 / 50 / 52; 8192 columns, 17 / 18 / 19 / 22 entries
+// 77 / 84 / 87 / 97 against 64 / 82 / 97 / 121: what grows there is a few rows with more than
+// 512 products, which the strips then do one by one).  From three strips on always (9000
+// columns, 12 / 18 / 21 entries: 110 / 181 / 182 us on strips).
 uint32_t LightProductsFor(uint32_t N, uint32_t products)
 {
     if (N <= kStripMax)
         return 0;
     if (N <= 2 * kStripMax)
-        return products != 0 && products <= 128 ? 256u : 0u;
+        return products != 0 && products <= 320 ? kLightProducts : 0u;
     return kLightProducts;
 }
 
@@ -878,11 +1105,9 @@ uint32_t RowsPerTurnFor(uint32_t M)
     return std::max<uint32_t>(1, std::min<uint32_t>(kRowsPerTurnMax, M / std::max<uint32_t>(wanted, 1)));
 }
 
-// Light rows: five workgroups of four wavefronts are resident per compute unit.  Turns are as long
+// Light rows: seven workgroups of four wavefronts are resident per compute unit.  Turns are as long
 // as if there were eight: enough rows per turn to overlap their loads, with more workgroups than
-// places where rows are few, which are handed out as places fall free.  Turns that make whole
-// rounds of five were slower (16384 rows x 256 products 116.4 / 120.8 us, two calls 9000 x 144
-// 59.8 / 61.3 us) except where no row is light (two calls, 9000 x 900 308 / 300 us).
+// places where rows are few, which are handed out as places fall free.
 template <int MODE>
 void LaunchLight(const SpgemmArgs& args, hipStream_t stream)
 {
