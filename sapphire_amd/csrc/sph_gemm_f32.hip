@@ -6,7 +6,7 @@
 // (Sources/Sapphire/compute/dense/naive/NaiveGemm.cpp:12-38) is the order in
 // which the K products are summed.
 //
-// Four kernels, chosen from the shape and the alignment of the operands:
+// Five kernels, chosen from the shape and the alignment of the operands:
 //   GemmF32DmaKernel     16-byte aligned bases, K >= 16, an N (an M, for A stored K x M) that
 //                        is a multiple of 4: slabs travel global -> LDS without staging
 //                        registers, several K steps ahead (the fast path; a K that is no
@@ -20,6 +20,7 @@
 //                        loads when possible, scalar predicated loads otherwise (small K,
 //                        misaligned bases, e.g. some of the reference's random test sizes,
 //                        Tests/UnitTests/Sources/FunctionTest/GemmTest.cpp:26-33);
+//   GemmF32ThinKernel    few output rows: K split over the lanes of a workgroup, vector units;
 //   GemmF32SkinnyKernel  few output tiles: 16 x 16 or 32 x 32 tiles with K split over the
 //                        wavefronts of a workgroup;
 //   GemvRowKernel        a single output row.
@@ -1383,6 +1384,36 @@ __device__ __forceinline__ void GemmF32SkinnyBody(const GemmF32Args& args, uint3
         multiply(b.w, a.w);
     };
 
+    // what the tile's sums are added to, requested by the wavefront that stores them before its
+    // share of K: behind the sum it was one more memory latency at the end of the launch
+    float old[kAcc];
+#pragma unroll
+    for (int v = 0; v < kAcc; ++v)
+        old[v] = 0.f;
+    if (wave == 0 && rowOk && (args.bias != nullptr || !args.overwrite))
+    {
+        const float* from = args.bias != nullptr ? args.bias : out + static_cast<size_t>(row) * args.ldc;
+#pragma unroll
+        for (int q = 0; q < kQuads; ++q)
+        {
+            const uint32_t c = tn * TILE + 4 * kLaneGroups * q + 4 * kh;
+            if (c + 4 <= N)
+            {
+                const floatx4 w = *reinterpret_cast<const floatx4a4*>(from + c);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    old[4 * q + e] = w[e];
+            }
+            else
+            {
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                    if (c + e < N)
+                        old[4 * q + e] = from[c + e];
+            }
+        }
+    }
+
     const uint32_t whole = part.whole;
     if (part.gBegin < part.wholeEnd)
     {
@@ -1452,7 +1483,7 @@ __device__ __forceinline__ void GemmF32SkinnyBody(const GemmF32Args& args, uint3
         }
     if (!rowOk)
         return;
-    const bool wide = args.outVec != 0;
+    const bool fused = args.bias != nullptr || args.relu != 0 || args.sgd != 0;
 #pragma unroll
     for (int q = 0; q < kQuads; ++q)
     {
@@ -1460,47 +1491,26 @@ __device__ __forceinline__ void GemmF32SkinnyBody(const GemmF32Args& args, uint3
         if (c >= N)
             continue;
         float* p = out + static_cast<size_t>(row) * args.ldc + c;
-        if (args.bias != nullptr || args.relu || args.sgd)
-        {
-            // fused epilogues: (0 + bias) + product with an optional ReLU (out not read), or the
-            // optimizer step
+        floatx4 v;
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (c + e < N)
-                {
-                    float old = 0.f;
-                    if (args.bias != nullptr)
-                        old = 0.f + args.bias[c + e];
-                    else if (!args.overwrite)
-                        old = p[e];
-                    float v = Combine(args, old, acc[4 * q + e]);
-                    if (args.relu)
-                        v = v > 0 ? v : 0;
-                    p[e] = v;
-                }
-        }
-        else if (args.overwrite)
+        for (int e = 0; e < 4; ++e)
         {
-            p[0] = acc[4 * q + 0];
-            if (c + 1 < N) p[1] = acc[4 * q + 1];
-            if (c + 2 < N) p[2] = acc[4 * q + 2];
-            if (c + 3 < N) p[3] = acc[4 * q + 3];
+            const float sum = acc[4 * q + e];
+            float before = old[4 * q + e];
+            if (args.bias != nullptr)
+                before = 0.f + before;
+            // fused epilogues: (0 + bias) + product with an optional ReLU, or the optimizer step
+            v[e] = fused || !args.overwrite ? Combine(args, before, sum) : sum;
+            if (args.relu)
+                v[e] = v[e] > 0 ? v[e] : 0;
         }
-        else if (wide)
-        {
-            float4 v = *reinterpret_cast<const float4*>(p);
-            v.x += acc[4 * q + 0];
-            v.y += acc[4 * q + 1];
-            v.z += acc[4 * q + 2];
-            v.w += acc[4 * q + 3];
-            *reinterpret_cast<float4*>(p) = v;
-        }
+        if (c + 4 <= N)
+            *reinterpret_cast<floatx4a4*>(p) = v;
         else
         {
-            p[0] += acc[4 * q + 0];
-            if (c + 1 < N) p[1] += acc[4 * q + 1];
-            if (c + 2 < N) p[2] += acc[4 * q + 2];
-            if (c + 3 < N) p[3] += acc[4 * q + 3];
+            p[0] = v[0];
+            if (c + 1 < N) p[1] = v[1];
+            if (c + 2 < N) p[2] = v[2];
         }
     }
 }
@@ -1509,6 +1519,274 @@ template <int TILE, bool TA, bool TB, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void GemmF32SkinnyKernel(const GemmF32Args args)
 {
     GemmF32SkinnyBody<TILE, TA, TB, WAVES>(args, blockIdx.x);
+}
+
+// ---------------------------------------------------------------------------
+// Few output rows (2 to 16; one, of a B stored N x K).  B is read once and decides the time, if
+// enough compute units read it: a 16 x 16 tile per workgroup gives 1024 columns to 64 of 256.
+// Here a workgroup owns 4 columns and all MR >= M rows.  Its lanes split K: lane l of wavefront w
+// takes k = 4 (64 w + l) .. + 3 and every 256 WAVES further, as 16-byte pieces whichever way B is
+// stored, keeps 4 MR sums of its own, and the sums of the lanes are added by exchanges in the
+// vector unit, those of the wavefronts through LDS.  The order of the additions depends on K only.
+// Bound by latency: launch, one round of loads, one reduction.  Kernel times with cold operands,
+// 16 x 16 tiles before: 8 x 1024 x 784 and x 1024 6.8 -> 4.9 us, 8 x 10 x 1024 5.6 -> 4.6; calls
+// in a row (a call costs the host about 4 us): 16 x 1024 x 1024 7.1 -> 4.9, 8 x 512 x 4096
+// 11.2 -> 6.9, 16 x 128 x 4096 13.4 -> 7.9, B stored N x K 8 x 1024 x 1024 8.4 -> 3.4.
+// Few output columns stay on 16 x 16 tiles: the roles swapped, with B's narrow rows taken through
+// LDS, 1024 x 10 x 1024 gains 1.4 us, its form with A stored K x M loses 0.6 and 2048 x 16 x 2048
+// goes from 9.1 to 14.0.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kThin = 16;
+constexpr uint32_t kThinShortK = 1024;  // up to here 4 wavefronts, else 8
+
+// Sum over the 64 lanes of 16 values per lane; lane l ends up with the sum of value l / 4.
+__device__ __forceinline__ float WaveSums16(float (&v)[16], uint32_t lane)
+{
+    auto bits = [](float x) { return __builtin_bit_cast(uint32_t, x); };
+    auto real = [](uint32_t x) { return __builtin_bit_cast(float, x); };
+    // a swap puts the two halves (rows of 16 lanes) of one value side by side in the lanes of one
+    // half and those of another value in the others
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+    {
+        const auto r = __builtin_amdgcn_permlane32_swap(bits(v[j]), bits(v[j + 8]), false, false);
+        v[j] = real(r[0]) + real(r[1]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+    {
+        const auto r = __builtin_amdgcn_permlane16_swap(bits(v[j]), bits(v[j + 4]), false, false);
+        v[j] = real(r[0]) + real(r[1]);
+    }
+    // inside a row: a lane keeps one of two values and gets its partner's part of it
+    auto fromLane = [&](float x, auto control) {
+        return real(static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+            0, static_cast<int>(bits(x)), decltype(control)::value, 0xf, 0xf, true)));
+    };
+    using Xor1 = std::integral_constant<int, 0xB1>;   // quad permutations
+    using Xor2 = std::integral_constant<int, 0x4E>;
+    using Xor3 = std::integral_constant<int, 0x1B>;
+    using Xor7 = std::integral_constant<int, 0x141>;  // half row mirrored
+    using Xor8 = std::integral_constant<int, 0x128>;  // row rotated by 8
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+    {
+        const bool upper = (lane & 8) != 0;
+        const float keep = upper ? v[j + 2] : v[j], give = upper ? v[j] : v[j + 2];
+        v[j] = keep + fromLane(give, Xor8{});
+    }
+    {
+        const bool upper = (lane & 4) != 0;
+        const float keep = upper ? v[1] : v[0], give = upper ? v[0] : v[1];
+        v[0] = keep + fromLane(fromLane(give, Xor7{}), Xor3{});  // lane ^ 4
+    }
+    v[0] = v[0] + fromLane(v[0], Xor2{});
+    return v[0] + fromLane(v[0], Xor1{});
+}
+
+// B_K / A_K: that operand is stored with K contiguous.
+template <int MR, bool B_K, bool A_K, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void GemmF32ThinKernel(const GemmF32Args args)
+{
+    // an A stored K x M: 4 rows per lane and one float between the lanes' pieces, so that all
+    // lanes read from banks of their own
+    __shared__ float slab[A_K ? 1 : WAVES * 64 * (4 * MR + 1)];
+    __shared__ float partial[WAVES][64];
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wave = threadIdx.x >> 6;
+    // neighbouring columns on one XCD: they share the lines of a B stored K x N
+    const uint32_t logical = (blockIdx.x & 7u) * args.perXcd + (blockIdx.x >> 3);
+    if (logical >= args.tilesTotal)
+        return;
+    const uint32_t unit = logical / args.tilesN;
+    const uint32_t x0 = (logical - unit * args.tilesN) * 4;
+    const float* __restrict__ A;
+    const float* __restrict__ B;
+    float* out;
+    if (args.entries != nullptr)
+    {
+        const SphGemmEntry e = args.entries[unit];
+        A = args.A + e.aOff;
+        B = args.B + e.bOff;
+        out = args.out + e.outOff;
+    }
+    else
+    {
+        A = args.A + args.strideA * static_cast<int64_t>(unit);
+        B = args.B + args.strideB * static_cast<int64_t>(unit);
+        out = args.out + args.strideOut * static_cast<int64_t>(unit);
+    }
+    const uint32_t M = args.M, N = args.N, K = args.K;
+
+    // wavefront 0 stores sum 4 i + x of lane l = 4 i + x: what it is added to
+    const uint32_t row = lane >> 2, col = x0 + (lane & 3);
+    const bool stores = wave == 0 && row < M && col < N;
+    float* const place = out + static_cast<size_t>(row) * args.ldc + col;
+    float old = 0.f;
+    if (stores && args.bias != nullptr)
+        old = args.bias[col];
+    else if (stores && !args.overwrite)
+        old = *place;
+
+    float acc[MR / 4][16];
+#pragma unroll
+    for (int g = 0; g < MR / 4; ++g)
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+            acc[g][j] = 0.f;
+
+    const bool wholeQuad = x0 + 4 <= N;
+    auto load4 = [](const float* p) { return *reinterpret_cast<const floatx4a4*>(p); };
+    for (uint32_t base = 0; base < K; base += 256 * WAVES)
+    {
+        const uint32_t k0 = base + 4 * (wave * 64 + lane);
+        float s[4][4], t[MR][4];  // [x][e], [i][e]: e = k - k0
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                s[x][e] = 0.f;
+#pragma unroll
+        for (int i = 0; i < MR; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                t[i][e] = 0.f;
+        if (k0 + 4 <= K)
+        {
+            if constexpr (B_K)
+            {
+#pragma unroll
+                for (int x = 0; x < 4; ++x)
+                {
+                    const floatx4 w = load4(B + static_cast<size_t>(min(x0 + x, N - 1)) * K + k0);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        s[x][e] = w[e];
+                }
+            }
+            else if (wholeQuad)
+            {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                {
+                    const floatx4 w = load4(B + static_cast<size_t>(k0 + e) * args.ldb + x0);
+#pragma unroll
+                    for (int x = 0; x < 4; ++x)
+                        s[x][e] = w[x];
+                }
+            }
+            else
+            {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int x = 0; x < 4; ++x)
+                        s[x][e] = B[static_cast<size_t>(k0 + e) * args.ldb + min(x0 + x, N - 1)];
+            }
+            if constexpr (A_K)
+            {
+#pragma unroll
+                for (int i = 0; i < MR; ++i)
+                {
+                    const floatx4 w =
+                        load4(A + static_cast<size_t>(min(static_cast<uint32_t>(i), M - 1)) * K + k0);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        t[i][e] = w[e];
+                }
+            }
+        }
+        else if (k0 < K)
+        {
+            // the piece that K ends in: element by element, zeros past K
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                if (k0 + e < K)
+                {
+#pragma unroll
+                    for (int x = 0; x < 4; ++x)
+                    {
+                        const size_t at = min(x0 + x, N - 1);
+                        s[x][e] = B_K ? B[at * K + k0 + e]
+                                      : B[static_cast<size_t>(k0 + e) * args.ldb + at];
+                    }
+#pragma unroll
+                    for (int i = 0; i < MR && A_K; ++i)
+                    {
+                        const size_t at = min(static_cast<uint32_t>(i), M - 1);
+                        t[i][e] = A[at * K + k0 + e];
+                    }
+                }
+        }
+        if constexpr (!A_K)
+        {
+            // Rows of M floats that lie one behind the other: read as they lie (pieces of a row per
+            // lane would be 64 lines per access), and taken apart by the reads from LDS.
+            const uint32_t floats = min(256u * WAVES, K - base) * M;
+            const float* from = A + static_cast<size_t>(base) * M;
+            const uint32_t perM = ((1u << 20) + M - 1) / M;  // x / M below
+            if (base != 0)
+                __syncthreads();
+            for (uint32_t q = threadIdx.x; q * 4 < floats; q += 64 * WAVES)
+            {
+                // q / M is the lane whose four rows these floats are of
+                float* to = slab + q * 4 + (q * perM >> 20);
+                if (q * 4 + 4 <= floats)
+                {
+                    const floatx4 w = load4(from + q * 4);
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        to[u] = w[u];
+                }
+                else
+                {
+                    for (uint32_t u = 0; q * 4 + u < floats; ++u)
+                        to[u] = from[q * 4 + u];
+                }
+            }
+            __syncthreads();
+            const float* own = slab + (wave * 64 + lane) * (4 * M + 1);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (k0 + e < K)
+                {
+#pragma unroll
+                    for (int i = 0; i < MR; ++i)
+                        t[i][e] = own[e * M + min(static_cast<uint32_t>(i), M - 1)];
+                }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < MR; ++i)
+#pragma unroll
+                for (int x = 0; x < 4; ++x)
+                    acc[i / 4][(i % 4) * 4 + x] =
+                        fmaf(t[i][e], s[x][e], acc[i / 4][(i % 4) * 4 + x]);
+    }
+    // sum j of group g of four rows: lanes 4 j .. 4 j + 3; the one with lane % 4 = g hands it on
+    float mine = 0.f;
+#pragma unroll
+    for (int g = 0; g < MR / 4; ++g)
+    {
+        const float sum = WaveSums16(acc[g], lane);
+        mine = (lane & 3u) == static_cast<uint32_t>(g) ? sum : mine;
+    }
+    partial[wave][(lane & 3u) * 16 + (lane >> 2)] = mine;
+    __syncthreads();
+    if (!stores)
+        return;
+    float sum = partial[0][lane];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w)
+        sum += partial[w][lane];
+    if (args.bias != nullptr)
+        old = 0.f + old;
+    const bool fused = args.bias != nullptr || args.relu != 0 || args.sgd != 0;
+    float v = fused || !args.overwrite ? Combine(args, old, sum) : sum;
+    if (args.relu)
+        v = v > 0 ? v : 0;
+    *place = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -1703,6 +1981,27 @@ void LaunchSkinny(const GemmF32Args& args, dim3 grid, uint32_t tile, bool wide, 
         LaunchSkinnyTile<16, TA, TB>(args, grid, wide, stream);
     else
         LaunchSkinnyTile<32, TA, TB>(args, grid, wide, stream);
+}
+
+template <bool B_K, bool A_K, int WAVES>
+void LaunchThinRows(const GemmF32Args& args, hipStream_t stream)
+{
+    const dim3 grid(8 * args.perXcd), block(WAVES * 64);
+    if (args.M <= 4)
+        hipLaunchKernelGGL((GemmF32ThinKernel<4, B_K, A_K, WAVES>), grid, block, 0, stream, args);
+    else if (args.M <= 8)
+        hipLaunchKernelGGL((GemmF32ThinKernel<8, B_K, A_K, WAVES>), grid, block, 0, stream, args);
+    else
+        hipLaunchKernelGGL((GemmF32ThinKernel<16, B_K, A_K, WAVES>), grid, block, 0, stream, args);
+}
+
+template <bool B_K, bool A_K>
+void LaunchThin(const GemmF32Args& args, hipStream_t stream)
+{
+    if (args.K > kThinShortK)
+        LaunchThinRows<B_K, A_K, 8>(args, stream);
+    else
+        LaunchThinRows<B_K, A_K, 4>(args, stream);
 }
 
 // `walk`: 64-tiles only, each workgroup takes several tiles
@@ -1997,6 +2296,29 @@ int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool o
         else
             hipLaunchKernelGGL(GemvRowKernel<64>, dim3((args.N + 63) / 64, units),
                                dim3(kGemvWaves * 64), 0, stream, args);
+        SPH_CHECK_LAUNCH();
+        return SPH_OK;
+    }
+
+    // Few rows: 4 columns per workgroup while that is at most one per compute unit, or two where a
+    // workgroup's A is small; beyond that 16 x 16 tiles read A less often (16 x 2048 x 1024 7.1 us
+    // on them, 6.4 here; x 2048 11.4 / 11.4; x 4096 18.7 / 19.5; 8 x 2048 x 4096 16.0 / 15.4).
+    const uint64_t thinBlocks = static_cast<uint64_t>((args.N + 3) / 4) * units;
+    if (fewTiles && args.M <= kThin && args.M <= args.N && args.K < (1u << 31) &&
+        (thinBlocks <= cusAll ||
+         (thinBlocks <= 2 * cusAll && (args.M <= 8 || args.K <= 2 * kThinShortK))))
+    {
+        args.tilesN = (args.N + 3) / 4;
+        args.tilesTotal = static_cast<uint32_t>(thinBlocks);
+        args.perXcd = (args.tilesTotal + 7) / 8;
+        if (transA && transB)
+            LaunchThin<true, false>(args, stream);
+        else if (transA)
+            LaunchThin<false, false>(args, stream);
+        else if (transB)
+            LaunchThin<true, true>(args, stream);
+        else
+            LaunchThin<false, true>(args, stream);
         SPH_CHECK_LAUNCH();
         return SPH_OK;
     }
