@@ -35,7 +35,7 @@
 //   GemmF16Tile256<..., NT = 128>  the same kernel on 256 x 128 tiles, taken while there are
 //     between 11/16 of such a tile and one tile per compute unit.
 //
-//   GemmF16Dma128   the same conditions, any M: the
+//   GemmF16Dma128   the same conditions on K, any M and N: the
 //     same ingredients on 128 x 128 tiles with 4 or 8 wavefronts (v_mfma_f32_32x32x16_f16), for
 //     shapes with too few 256-tiles to fill the chip.
 //
@@ -50,11 +50,11 @@
 // K = 32 q + r, r != 0, K >= 64 stays on the first two kernels: a last step over [K - 32, K) in
 // which the fragment positions whose k was multiplied already are cleared.
 //
-// N = 8 q + r, r != 0: the first 8 q columns go to the tiled straight-to-LDS kernels when they
-// would take that shape (the copies into LDS need no alignment, so rows of B and of out may start
-// anywhere; only a copy's 8 columns have to lie inside the row) and the last r columns to the
-// code of GemmF16Few, as do the last M % 8 rows of an A stored K x M and up to 16 rows or columns
-// just past a tile edge: as strips on the last workgroups of the body's own launch (LaunchF16).
+// The copies into LDS need no alignment, so rows of B and of out may start anywhere; the 64- and
+// 128-tile kernels take any N, and any M of an A stored K x M, from 8 up.  In front of the 256-tile
+// kernel, whose copies' 8 columns have to lie inside the row, the last N % 8 columns (M % 8 rows of
+// an A stored K x M) go to the code of GemmF16Few, as do up to 16 rows or columns just past a tile
+// edge: as strips on the last workgroups of the body's own launch (LaunchF16).
 #include "sph_internal.h"
 #include "sph_k_partition.h"
 
@@ -847,11 +847,11 @@ __global__ __launch_bounds__(512) void GemmF16Tile256(const GemmF16Args args,
 // ---------------------------------------------------------------------------
 // 128 x 128 x 32 kernel with straight-to-LDS copies, ragged M and N
 // ---------------------------------------------------------------------------
-// For shapes the 256-tile kernel does not take (M or N not a multiple of 256) as long as K is a
-// multiple of 32 (or any K from 64 up) and N of 8.  Four wavefronts (2 x 2, each 64 x 64 = 2 x 2 MFMA blocks) or eight (2 x 4, each
-// 64 x 32), four LDS stages of 16 KiB (two workgroups per compute unit), copies issued two steps
-// ahead, one barrier per step (placed, with the copies, between the MFMAs of the step's first
-// half), fragments read half a step ahead.
+// For shapes the 256-tile kernel does not take, as long as K is a multiple of 32 or at least 64.
+// Four wavefronts (2 x 2, each 64 x 64 = 2 x 2 MFMA blocks) or eight (2 x 4, each 64 x 32), four LDS
+// stages of 16 KiB (two workgroups per compute unit), copies issued two steps ahead, one barrier per
+// step (placed, with the copies, between the MFMAs of the step's first half), fragments read half
+// a step ahead.
 // A stage: 128 rows of 64 bytes, 16-byte chunk c of row x at position c ^ ((x >> 2) & 3).
 // B stage: 32 k-rows of 256 bytes, 32-byte chunks XOR-swizzled with 2*(k%4), read with the
 // transposing LDS load like the 256-tile kernel.  Rows past M and columns past N are clamped to
@@ -859,9 +859,66 @@ __global__ __launch_bounds__(512) void GemmF16Tile256(const GemmF16Args args,
 // TA (A stored K x M) / TB (B stored N x K): an operand stored the other way round simply takes
 // the other operand's stage layout and fragment read -- an A stored k-major is copied and read
 // like B, a B stored with K contiguous like A -- so the MFMAs and their order do not change.
+//
+// A k-major operand whose rows are no whole number of 8 halves (N of a B stored K x N, M of an A
+// stored K x M): a row's last chunk reaches into the next row, whose values only feed outputs that
+// are not stored, except in the last row of the matrix, where it would reach past its end.  There
+// the lane copies the 8 halves that end with the row (`back` bytes before the chunk) and moves
+// them to their places in LDS before the stage is published (LastChunk).  Such rows and columns
+// were cut off as strips before (2048 x 1533 x 1024 21.7 -> 18.3 us, 4 x 1001 x
+// 1003 x 999 26.7 -> 22.0, 900 x 901 x 903 12.6 -> 9.5, 4001 x 201 x 1001 12.6 -> 9.1).
 constexpr int kD = 128;
 constexpr int kDStages = 4;
 constexpr int kDStageBytes = 2 * kD * kTK * 2;  // A + B
+
+// First of the 8 columns a lane copies for chunk `x` (a multiple of 8) of a k-major row of `limit`
+// >= 8 columns: chunks past the edge copy the row's last 8.
+__device__ __forceinline__ uint32_t ChunkColumn(uint32_t x, uint32_t limit)
+{
+    return x < limit ? x : limit - 8;
+}
+
+// Bytes by which that chunk, in the last row of the matrix, has to begin earlier.
+__device__ __forceinline__ uint32_t LastChunkBack(uint32_t x, uint32_t limit)
+{
+    return x < limit && x + 8 > limit ? (x + 8 - limit) * 2 : 0u;
+}
+
+// What was copied `back` bytes too early to its place; what follows belongs to no column.
+__device__ __forceinline__ void MoveLastChunk(char* chunk, uint32_t back)
+{
+    const uint64_t* from = reinterpret_cast<const uint64_t*>(chunk);
+    const unsigned __int128 v =
+        (static_cast<unsigned __int128>(from[1]) << 64 | from[0]) >> (back * 8);
+    uint64_t* to = reinterpret_cast<uint64_t*>(chunk);
+    to[0] = static_cast<uint64_t>(v);
+    to[1] = static_cast<uint64_t>(v >> 64);
+}
+
+// 4 columns of a row of out from `c` on, of which those below N exist (c < N); WHOLE: all do
+template <bool WHOLE>
+__device__ __forceinline__ float4 LoadQuad(const float* p, uint32_t c, uint32_t N)
+{
+    if (WHOLE || c + 4 <= N)
+        return Load4(p);
+    float4 v = make_float4(p[0], 0.f, 0.f, 0.f);
+    if (c + 1 < N) v.y = p[1];
+    if (c + 2 < N) v.z = p[2];
+    return v;
+}
+
+template <bool WHOLE>
+__device__ __forceinline__ void StoreQuad(float* p, const float4& v, uint32_t c, uint32_t N)
+{
+    if (WHOLE || c + 4 <= N)
+    {
+        Store4(p, v);
+        return;
+    }
+    p[0] = v.x;
+    if (c + 1 < N) p[1] = v.y;
+    if (c + 2 < N) p[2] = v.z;
+}
 
 // TAIL: K = 32 q + r, 0 < r < 32: a last step over the window [K - 32, K) whose slab has the
 // positions of the 32 - r values of k already multiplied cleared in LDS.
@@ -912,8 +969,14 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF16Dma128(const GemmF16Args ar
         const uint32_t k = j * 4 + (lane >> 4);
         const uint32_t phys16 = lane & 15;
         const uint32_t logical16 = (((phys16 >> 1) ^ (2 * (k & 3))) << 1) | (phys16 & 1);
-        const uint32_t gx = min(xBase + logical16 * 8, limit - 8);
-        return (k * pitch + gx) * 2u;
+        return (k * pitch + ChunkColumn(xBase + logical16 * 8, limit)) * 2u;
+    };
+    // ... and what its chunk of the last k-row begins earlier by
+    auto laneBack = [&](uint32_t j, uint32_t xBase, uint32_t limit) {
+        const uint32_t k = j * 4 + (lane >> 4);
+        const uint32_t phys16 = lane & 15;
+        const uint32_t logical16 = (((phys16 >> 1) ^ (2 * (k & 3))) << 1) | (phys16 & 1);
+        return k == kTK - 1 ? LastChunkBack(xBase + logical16 * 8, limit) : 0u;
     };
     uint32_t aLane[kCopiesPer], bLane[kCopiesPer], aDst[kCopiesPer], bDst[kCopiesPer];
 #pragma unroll
@@ -925,6 +988,11 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF16Dma128(const GemmF16Args ar
         aDst[i] = j * 1024;
         bDst[i] = kBytesA + j * 1024;
     }
+    // the last k-row of a slab is in a wavefront's last copy
+    constexpr uint32_t kLastCopy = kCopiesPer - 1;
+    const uint32_t aBack = TA ? laneBack(wave + WAVES * kLastCopy, rowBase, M) : 0u;
+    const uint32_t bBack = TB ? 0u : laneBack(wave + WAVES * kLastCopy, colBase, N);
+    const bool moveLast = (TA && M % 8 != 0) || (!TB && N % 8 != 0);
     const size_t aStepBytes = TA ? static_cast<size_t>(kTK) * args.lda * 2 : kTK * 2;
     const size_t bStepBytes = TB ? kTK * 2 : static_cast<size_t>(kTK) * args.ldb * 2;
     const uint32_t ldsBase = LdsAddress(lds);
@@ -958,6 +1026,11 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF16Dma128(const GemmF16Args ar
             aSrc += aBytes;
             bSrc += bBytes;
             --stepsToAdvance;
+            if ((TA || !TB) && stepsToAdvance == 0)
+            {
+                aLane[kLastCopy] -= aBack;
+                bLane[kLastCopy] -= bBack;
+            }
         }
     };
 
@@ -1043,6 +1116,13 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF16Dma128(const GemmF16Args ar
             *b = *b & (TB ? contig : major);
         }
     };
+    auto moveLastChunks = [&](char* stage) {
+        const uint32_t at = (wave + WAVES * kLastCopy) * 1024 + lane * 16;
+        if (TA && aBack != 0)
+            MoveLastChunk(stage + at, aBack);
+        if (!TB && bBack != 0)
+            MoveLastChunk(stage + kBytesA + at, bBack);
+    };
     auto multiply = [&](const halfx8 (&af)[2], const halfx8 (&bf)[TN]) {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -1071,13 +1151,13 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF16Dma128(const GemmF16Args ar
                     // behind the barrier everybody's copies are visible and everybody has
                     // read the last fragment of step st-1
                     WaitVmem<(kDStages - 3) * kDCopies>();
-                    if constexpr (TAIL)
+                    if (nextIsLast && (TAIL || ((TA || !TB) && moveLast)))
                     {
-                        if (nextIsLast)
-                        {
+                        if constexpr (TAIL)
                             clearRepeated(next);
-                            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                        }
+                        if ((TA || !TB) && moveLast)
+                            moveLastChunks(next);
+                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                     }
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
@@ -1117,7 +1197,7 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF16Dma128(const GemmF16Args ar
             loadFragments(af[1], bf[1], cur, 1);
             __builtin_amdgcn_sched_barrier(0);
             multiplyAndFeed(af[0], bf[0], (u + kDStages - 1) % kDStages,
-                            TAIL && s0 + u + 2 == steps, next);
+                            s0 + u + 2 == steps, next);
             __builtin_amdgcn_sched_barrier(0);
             loadFragments(af[0], bf[0], next, 0);
             __builtin_amdgcn_sched_barrier(0);
@@ -1128,41 +1208,48 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF16Dma128(const GemmF16Args ar
     WaitVmem<0>();  // the surplus copies of the last steps still target LDS
 
     // ---- epilogue: lane holds row l%32 of a block, columns 8q + 4*(l/32) + 0..3 -----------
-    const bool accumulate = args.overwrite == 0;
-    float4 old[8 * TN];
+    auto epilogue = [&](auto whole) {
+        constexpr bool kWhole = decltype(whole)::value;
+        const bool accumulate = args.overwrite == 0;
+        float4 old[8 * TN];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+            for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-            {
-                const uint32_t r = rowBase + waveM * 64 + i * 32 + l32;
-                const uint32_t c = colBase + (waveN * TN + j) * 32 + 8 * q + 4 * khalf;
-                float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (accumulate && r < M && c < N)  // N % 8 == 0: whole quads only
-                    v = Load4(out + static_cast<size_t>(r) * args.ldc + c);
-                old[(i * TN + j) * 4 + q] = v;
-            }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-            {
-                const uint32_t r = rowBase + waveM * 64 + i * 32 + l32;
-                const uint32_t c = colBase + (waveN * TN + j) * 32 + 8 * q + 4 * khalf;
-                if (r < M && c < N)
+                for (int q = 0; q < 4; ++q)
                 {
-                    float4 v = old[(i * TN + j) * 4 + q];
-                    v.x += acc[i][j][4 * q + 0];
-                    v.y += acc[i][j][4 * q + 1];
-                    v.z += acc[i][j][4 * q + 2];
-                    v.w += acc[i][j][4 * q + 3];
-                    Store4(out + static_cast<size_t>(r) * args.ldc + c, v);
+                    const uint32_t r = rowBase + waveM * 64 + i * 32 + l32;
+                    const uint32_t c = colBase + (waveN * TN + j) * 32 + 8 * q + 4 * khalf;
+                    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (accumulate && r < M && c < N)
+                        v = LoadQuad<kWhole>(out + static_cast<size_t>(r) * args.ldc + c, c, N);
+                    old[(i * TN + j) * 4 + q] = v;
                 }
-            }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                {
+                    const uint32_t r = rowBase + waveM * 64 + i * 32 + l32;
+                    const uint32_t c = colBase + (waveN * TN + j) * 32 + 8 * q + 4 * khalf;
+                    if (r < M && c < N)
+                    {
+                        float4 v = old[(i * TN + j) * 4 + q];
+                        v.x += acc[i][j][4 * q + 0];
+                        v.y += acc[i][j][4 * q + 1];
+                        v.z += acc[i][j][4 * q + 2];
+                        v.w += acc[i][j][4 * q + 3];
+                        StoreQuad<kWhole>(out + static_cast<size_t>(r) * args.ldc + c, v, c, N);
+                    }
+                }
+    };
+    if (N % 4 == 0)
+        epilogue(std::true_type{});
+    else
+        epilogue(std::false_type{});
 }
 
 // ---------------------------------------------------------------------------
@@ -1190,7 +1277,7 @@ constexpr int kSOperandBytes = kS * kSK * 2;        // 8 KiB
 constexpr int kSStageBytes = 2 * kSOperandBytes;    // A + B
 
 template <bool TA, bool TB, bool TAIL>
-__global__ __launch_bounds__(256) void GemmF16Dma64(const GemmF16Args args,
+__global__ __launch_bounds__(256, 2) void GemmF16Dma64(const GemmF16Args args,
                                                     const GemmF16Strips strips)
 {
     constexpr int kCopiesPer = 2;            // 1 KiB copies per operand, step and wavefront
@@ -1230,8 +1317,12 @@ __global__ __launch_bounds__(256) void GemmF16Dma64(const GemmF16Args args,
     auto laneKMajor = [&](uint32_t j, uint32_t xBase, uint32_t limit, uint32_t pitch) {
         const uint32_t k = j * 8 + (lane >> 3);
         const uint32_t logical16 = (lane & 7) ^ (((k >> 1) & 1) << 2);
-        const uint32_t gx = min(xBase + logical16 * 8, limit - 8);
-        return (k * pitch + gx) * 2u;
+        return (k * pitch + ChunkColumn(xBase + logical16 * 8, limit)) * 2u;
+    };
+    auto laneBack = [&](uint32_t j, uint32_t xBase, uint32_t limit) {
+        const uint32_t k = j * 8 + (lane >> 3);
+        const uint32_t logical16 = (lane & 7) ^ (((k >> 1) & 1) << 2);
+        return k == kSK - 1 ? LastChunkBack(xBase + logical16 * 8, limit) : 0u;
     };
     const uint32_t pitchB = TB ? K : args.ldb;
     uint32_t aLane[kCopiesPer], bLane[kCopiesPer], aDst[kCopiesPer], bDst[kCopiesPer];
@@ -1244,6 +1335,11 @@ __global__ __launch_bounds__(256) void GemmF16Dma64(const GemmF16Args args,
         aDst[i] = j * 1024;
         bDst[i] = kSOperandBytes + j * 1024;
     }
+    // the last k-row of a slab is in a wavefront's last copy
+    constexpr uint32_t kLastCopy = kCopiesPer - 1;
+    const uint32_t aBack = TA ? laneBack(wave + 4 * kLastCopy, rowBase, M) : 0u;
+    const uint32_t bBack = TB ? 0u : laneBack(wave + 4 * kLastCopy, colBase, N);
+    const bool moveLast = (TA && M % 8 != 0) || (!TB && N % 8 != 0);
     const size_t aStepBytes = TA ? static_cast<size_t>(kSK) * args.lda * 2 : kSK * 2;
     const size_t bStepBytes = TB ? kSK * 2 : static_cast<size_t>(kSK) * pitchB * 2;
     const uint32_t ldsBase = LdsAddress(lds);
@@ -1277,6 +1373,11 @@ __global__ __launch_bounds__(256) void GemmF16Dma64(const GemmF16Args args,
             aSrc += aBytes;
             bSrc += bBytes;
             --stepsToAdvance;
+            if ((TA || !TB) && stepsToAdvance == 0)
+            {
+                aLane[kLastCopy] -= aBack;
+                bLane[kLastCopy] -= bBack;
+            }
         }
     };
 
@@ -1346,6 +1447,14 @@ __global__ __launch_bounds__(256) void GemmF16Dma64(const GemmF16Args args,
         }
     };
 
+    auto moveLastChunks = [&](char* stage) {
+        const uint32_t at = (wave + 4 * kLastCopy) * 1024 + lane * 16;
+        if (TA && aBack != 0)
+            MoveLastChunk(stage + at, aBack);
+        if (!TB && bBack != 0)
+            MoveLastChunk(stage + kSOperandBytes + at, bBack);
+    };
+
 #pragma unroll
     for (uint32_t p = 0; p < kSStages - 1; ++p)
     {
@@ -1380,13 +1489,13 @@ __global__ __launch_bounds__(256) void GemmF16Dma64(const GemmF16Args args,
             if (ks == 0)
             {
                 WaitVmem<(kSStages - 3) * kCopies>();
-                if constexpr (TAIL)
+                if (st + 2 == steps && (TAIL || ((TA || !TB) && moveLast)))
                 {
-                    if (st + 2 == steps)
-                    {
+                    if constexpr (TAIL)
                         clearRepeated(next);
-                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                    }
+                    if ((TA || !TB) && moveLast)
+                        moveLastChunks(next);
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 }
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
@@ -1416,32 +1525,39 @@ __global__ __launch_bounds__(256) void GemmF16Dma64(const GemmF16Args args,
     WaitVmem<0>();  // the surplus copies of the last steps still target LDS
 
     // ---- epilogue: lane holds row l % 32 of its block, columns 8 q + 4 (l / 32) + 0..3 ----------
-    const bool accumulate = args.overwrite == 0;
-    const uint32_t r = rowBase + waveM * 32 + l32;
-    float4 old[4];
+    auto epilogue = [&](auto whole) {
+        constexpr bool kWhole = decltype(whole)::value;
+        const bool accumulate = args.overwrite == 0;
+        const uint32_t r = rowBase + waveM * 32 + l32;
+        float4 old[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-    {
-        const uint32_t c = colBase + waveN * 32 + 8 * q + 4 * khalf;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (accumulate && r < M && c < N)  // N % 8 == 0: whole quads only
-            v = Load4(out + static_cast<size_t>(r) * args.ldc + c);
-        old[q] = v;
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-    {
-        const uint32_t c = colBase + waveN * 32 + 8 * q + 4 * khalf;
-        if (r < M && c < N)
+        for (int q = 0; q < 4; ++q)
         {
-            float4 v = old[q];
-            v.x += acc[4 * q + 0];
-            v.y += acc[4 * q + 1];
-            v.z += acc[4 * q + 2];
-            v.w += acc[4 * q + 3];
-            Store4(out + static_cast<size_t>(r) * args.ldc + c, v);
+            const uint32_t c = colBase + waveN * 32 + 8 * q + 4 * khalf;
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (accumulate && r < M && c < N)
+                v = LoadQuad<kWhole>(out + static_cast<size_t>(r) * args.ldc + c, c, N);
+            old[q] = v;
         }
-    }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+        {
+            const uint32_t c = colBase + waveN * 32 + 8 * q + 4 * khalf;
+            if (r < M && c < N)
+            {
+                float4 v = old[q];
+                v.x += acc[4 * q + 0];
+                v.y += acc[4 * q + 1];
+                v.z += acc[4 * q + 2];
+                v.w += acc[4 * q + 3];
+                StoreQuad<kWhole>(out + static_cast<size_t>(r) * args.ldc + c, v, c, N);
+            }
+        }
+    };
+    if (N % 4 == 0)
+        epilogue(std::true_type{});
+    else
+        epilogue(std::false_type{});
 }
 
 // ---------------------------------------------------------------------------
@@ -1974,7 +2090,8 @@ enum class F16Kernel { kTile256, kTile256x128, kDma64, kDma128, kGeneral };
 
 // The kernel that would take M x N x K with these operands.  The straight-to-LDS copies take 16
 // bytes from any 2-byte-aligned address, so the rows of a K x N matrix B may start anywhere
-// (any ldb, any base); N itself has to be a multiple of 8 because a copy is 8 columns wide.
+// (any ldb, any base).  A copy is 8 columns wide: the 256-tile kernel wants N (and M of an A
+// stored K x M) in multiples of 8, the smaller tiles take care of a row's last piece.
 // out is accessed 16 bytes at a time from 4-byte-aligned addresses.
 F16Kernel PickF16(const GemmF16Args& args, uint32_t N, uint32_t batch, const F16Layout& lay)
 {
@@ -1999,9 +2116,10 @@ F16Kernel PickF16(const GemmF16Args& args, uint32_t N, uint32_t batch, const F16
     // partly masked step (measured 4096 x 4096 x 4080, operands stored plainly: 229 us on the
     // general kernel, 175 us with the r values left to a second launch, 128 us this way)
     const bool tailInKernel = K % kTK != 0 && K >= 2 * kTK;
-    const bool dma = K >= kTK &&
-                     (K % kTK == 0 || tailInKernel) && N % 8 == 0 && N >= 8 &&
-                     (!transA || (M % 8 == 0 && M >= 8));
+    // (rows of a k-major operand in whole chunks of 8, for the 256-tile kernel)
+    const bool wholeChunks = (transB || N % 8 == 0) && (!transA || M % 8 == 0);
+    const bool copies = K >= kTK && (K % kTK == 0 || tailInKernel) && N >= 8 && (!transA || M >= 8);
+    const bool dma = copies && N % 8 == 0 && wholeChunks;
     if (dma && tiles256 >= minTiles && fills256 && offsetsFit)
         return F16Kernel::kTile256;
     // Too few 256 x 256 tiles for the chip: 256 x 128 tiles while there are between 11/16 of a
@@ -2026,9 +2144,11 @@ F16Kernel PickF16(const GemmF16Args& args, uint32_t N, uint32_t batch, const F16
     // at most half as many 128-tiles as compute units: 64 x 64 tiles with K steps of 64
     const uint64_t tiles128 =
         static_cast<uint64_t>((M + kG - 1) / kG) * ((N + kG - 1) / kG) * batch;
-    if (dma && offsets128Fit && K >= kSK && tiles128 <= cus / 2)
+    // (partial chunks are moved ahead of the last of at least two slabs)
+    const bool small = copies && offsets128Fit;
+    if (small && K >= (wholeChunks ? kSK : 2 * kSK) && tiles128 <= cus / 2)
         return F16Kernel::kDma64;
-    if (dma && offsets128Fit)
+    if (small && (wholeChunks || K >= 2 * kTK))
         return F16Kernel::kDma128;
     return F16Kernel::kGeneral;
 }
@@ -2212,11 +2332,10 @@ int LaunchF16Kernel(GemmF16Args args, uint32_t batch, F16Kernel kind, const F16L
 // of the product's last rows and columns, which the few-tile kernel's code computes (it reads any
 // rows and columns from anywhere) on the first workgroups of the body's launch.  Every output
 // element is computed once.  Cut off are
-//  - the last N % 8 columns, when a straight-to-LDS kernel then takes the rest (its copies are 8
+//  - the last N % 8 columns, when the 256-tile kernel then takes the rest (its copies are 8
 //    columns wide; row pitches of B and out stay N; measured 4096 x 4100 x 4096: 270 us on the
-//    general kernel alone, 129 us with the strip in a launch of its own);
-//  - the last M % 8 rows of an A stored K x M, likewise (it is copied 8 rows of the product at a
-//    time);
+//    general kernel alone, 129 us with the strip in a launch of its own), and the last M % 8 rows
+//    of an A stored K x M, likewise (it is copied 8 rows of the product at a time);
 //  - up to 16 rows or columns past a multiple of the tile edge, when the compute unit with the
 //    most tiles then has fewer of them (1025^3: 17 x 17 tiles of 64 are two per compute unit
 //    somewhere, 16 x 16 one everywhere).
@@ -2380,18 +2499,23 @@ void LaunchFew(const GemmF16Args& args, uint32_t blocks, uint32_t tile, bool wid
 // 7.3 against 10.6 / 11.7 / 10.3, 512^3 5.2 against 8.5, 100 x 1024 x 784 5.4 against 10.4,
 // 1024 x 10 x 1024 4.5 against 12.5, 16384 x 10 x 256 4.6 against 11.9; with two tiles per
 // compute unit (512 x 1024 x 1024) the two are level, with four the tiled kernel wins.
-// A product that the 64 x 64-tile kernel takes whole whatever its storage flags (M and N multiples
-// of 8, K >= 64) goes there from half a 32-tile per compute unit up (measured, few-tile kernel
-// against 64-tiles: 256 x 1024 x 1024 6.5 / 5.8 us, 256 x 512 x 2048 8.9 / 7.6, 128 x 1024 x 1024
-// 6.4 / 5.7; below that the few-tile kernel wins: 256^3 3.6 / 4.2, 64 x 1024 x 1024 4.8 / 5.7,
-// 256 x 256 x 4096 11.0 / 11.4).
+// A product of M and N multiples of 8 and K >= 64 goes to the 64 x 64-tile kernel from half a
+// 32-tile per compute unit up (measured, few-tile kernel against 64-tiles: 256 x 1024 x 1024
+// 6.5 / 5.8 us, 256 x 512 x 2048 8.9 / 7.6, 128 x 1024 x 1024 6.4 / 5.7; below that the few-tile
+// kernel wins: 256^3 3.6 / 4.2, 64 x 1024 x 1024 4.8 / 5.7, 256 x 256 x 4096 11.0 / 11.4).
+// Other M and N do for a K of 256 to 1536 (402 x 502 x 702 7.9 / 6.3, 401 x 501 x 701 8.8 / 7.8,
+// 401 x 501 x 301 7.0 / 6.2, 130 x 1000 x 1001 9.6 / 8.2, 4 x 181 x 183 x 1501 14.2 / 12.3): a
+// shorter one is level (501 x 501 x 129 5.5 / 5.7), and a longer one is read faster by more
+// wavefronts where rows begin at odd halves (130 x 1001 x 2001 13.6 / 15.8,
+// 401 x 501 x 2001 13.9 / 14.2).
 bool TakesFewTiles(uint32_t M, uint32_t N, uint32_t K, uint32_t batch)
 {
     const uint64_t cus = static_cast<uint64_t>(sph::ComputeUnits());
     const uint64_t blocks32 = static_cast<uint64_t>((M + 31) / 32) * ((N + 31) / 32) * batch;
     const uint64_t blocks16 = static_cast<uint64_t>((M + 15) / 16) * ((N + 15) / 16) * batch;
-    const bool tiles64Whole = M % 8 == 0 && N % 8 == 0 && K >= 64;
-    const uint64_t limit32 = tiles64Whole ? cus / 2 - 1 : cus;
+    const bool tiles64 = M % 8 == 0 && N % 8 == 0 ? K >= 64
+                                                  : M >= 8 && N >= 8 && K >= 256 && K <= 1536;
+    const uint64_t limit32 = tiles64 ? cus / 2 - 1 : cus;
     return blocks32 <= limit32 || (std::min(M, N) <= 16 && blocks16 <= 4 * cus);
 }
 
