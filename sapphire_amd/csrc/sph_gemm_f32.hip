@@ -7,10 +7,9 @@
 // which the K products are summed.
 //
 // Five kernels, chosen from the shape and the alignment of the operands:
-//   GemmF32DmaKernel     16-byte aligned bases, K >= 16, an N (an M, for A stored K x M) that
-//                        is a multiple of 4: slabs travel global -> LDS without staging
-//                        registers, several K steps ahead (the fast path; a K that is no
-//                        multiple of the step ends in a partial step);
+//   GemmF32DmaKernel     16-byte aligned bases, K >= 16, M and N >= 4: slabs travel
+//                        global -> LDS without staging registers, several K steps ahead (the
+//                        fast path; a K that is no multiple of the step ends in a partial step);
 //                        with more 64-tiles than resident workgroups each workgroup walks
 //                        several tiles and the copy stream runs across the tile boundaries;
 //                        with 65 to 128 tiles of 64 x 64, 64 x 32 tiles whose K steps are
@@ -24,9 +23,8 @@
 //   GemmF32SkinnyKernel  few output tiles: 16 x 16 or 32 x 32 tiles with K split over the
 //                        wavefronts of a workgroup;
 //   GemvRowKernel        a single output row.
-// A product for the tiled kernels is cut by the launcher into a body and up to two thin strips:
-// the last N % 4 columns, the last M % 4 rows (from 68 rows up) and up to 16 rows or columns
-// just past a tile edge.  The strips are computed by the few-tile kernel's code on the last
+// A product for the tiled kernels is cut by the launcher into a body and up to two thin strips of
+// up to 16 rows or columns just past a tile edge where that saves a round of tiles.  The strips are computed by the few-tile kernel's code on the last
 // workgroups of the body's own launch (GemmF32Strips), or by launches of their own beside a
 // register-staged body.
 // The first two share one decomposition: a workgroup (4 wavefronts, 2 x 2) owns a BM x BN tile
@@ -273,80 +271,68 @@ __device__ __forceinline__ void StoreTile(const floatx16 (&acc)[TM][TN], float* 
     // With the operands swapped, register v of lane l holds row l%32 and column
     // 8*(v/4) + 4*(l/32) + v%4 of its 32x32 block: registers 4q..4q+3 are 4
     // consecutive columns.  The old values of the whole wavefront block are requested
-    // in one batch, then added and stored.
+    // in one batch, then added and stored.  At the matrix edge the requests stay free of branches
+    // too (places past the edge read the last element that exists): behind a branch per quad each
+    // request was waited for before the next.
     constexpr int kQuads = TM * TN * 4;
     float4 old[kQuads];
+    auto each = [&](auto&& f) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+            for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-            {
-                const uint32_t r = rowBase + i * 32 + l32;
-                const uint32_t c = colBase + j * 32 + 8 * q + 4 * khalf;
-                float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (bias != nullptr)
-                {
-                    // what the K = 1 product ones x bias leaves in a zero-filled out
-                    if (c + 0 < N) v.x = 0.f + bias[c + 0];
-                    if (c + 1 < N) v.y = 0.f + bias[c + 1];
-                    if (c + 2 < N) v.z = 0.f + bias[c + 2];
-                    if (c + 3 < N) v.w = 0.f + bias[c + 3];
-                }
-                else if (accumulate && r < M && c < N)
-                {
-                    const float* p = out + static_cast<size_t>(r) * args.ldc + c;
-                    if (c + 4 <= N)
-                    {
-                        const floatx4 w = *reinterpret_cast<const floatx4a4*>(p);
-                        v = make_float4(w[0], w[1], w[2], w[3]);
-                    }
-                    else
-                    {
-                        v.x = p[0];
-                        if (c + 1 < N) v.y = p[1];
-                        if (c + 2 < N) v.z = p[2];
-                        if (c + 3 < N) v.w = p[3];
-                    }
-                }
-                old[(i * TN + j) * 4 + q] = v;
-            }
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-            {
-                const uint32_t r = rowBase + i * 32 + l32;
-                const uint32_t c = colBase + j * 32 + 8 * q + 4 * khalf;
-                if (r < M && c < N)
-                {
-                    float4 v = old[(i * TN + j) * 4 + q];
-                    v.x = Combine(args, v.x, acc[i][j][4 * q + 0]);
-                    v.y = Combine(args, v.y, acc[i][j][4 * q + 1]);
-                    v.z = Combine(args, v.z, acc[i][j][4 * q + 2]);
-                    v.w = Combine(args, v.w, acc[i][j][4 * q + 3]);
-                    if (relu)
-                    {
-                        v.x = v.x > 0 ? v.x : 0;
-                        v.y = v.y > 0 ? v.y : 0;
-                        v.z = v.z > 0 ? v.z : 0;
-                        v.w = v.w > 0 ? v.w : 0;
-                    }
-                    float* p = out + static_cast<size_t>(r) * args.ldc + c;
-                    if (c + 4 <= N)
-                        *reinterpret_cast<floatx4a4*>(p) = floatx4{ v.x, v.y, v.z, v.w };
-                    else
-                    {
-                        p[0] = v.x;
-                        if (c + 1 < N) p[1] = v.y;
-                        if (c + 2 < N) p[2] = v.z;
-                        if (c + 3 < N) p[3] = v.w;
-                    }
-                }
-            }
+                for (int q = 0; q < 4; ++q)
+                    f(i, j, q, rowBase + i * 32 + l32, colBase + j * 32 + 8 * q + 4 * khalf,
+                      old[(i * TN + j) * 4 + q]);
+    };
+    const bool inside = rowBase + TM * 32 <= M && colBase + TN * 32 <= N;
+    if (bias != nullptr)
+        // what the K = 1 product ones x bias leaves in a zero-filled out
+        each([&](int, int, int, uint32_t, uint32_t c, float4& v) {
+            v = make_float4(0.f + bias[min(c, N - 1)], 0.f + bias[min(c + 1, N - 1)],
+                            0.f + bias[min(c + 2, N - 1)], 0.f + bias[min(c + 3, N - 1)]);
+        });
+    else if (!accumulate)
+        each([&](int, int, int, uint32_t, uint32_t, float4& v) {
+            v = make_float4(0.f, 0.f, 0.f, 0.f);
+        });
+    else if (inside)
+        each([&](int, int, int, uint32_t r, uint32_t c, float4& v) {
+            const floatx4 w =
+                *reinterpret_cast<const floatx4a4*>(out + static_cast<size_t>(r) * args.ldc + c);
+            v = make_float4(w[0], w[1], w[2], w[3]);
+        });
+    else
+        each([&](int, int, int, uint32_t r, uint32_t c, float4& v) {
+            const float* row = out + static_cast<size_t>(min(r, M - 1)) * args.ldc;
+            v = make_float4(row[min(c, N - 1)], row[min(c + 1, N - 1)], row[min(c + 2, N - 1)],
+                            row[min(c + 3, N - 1)]);
+        });
+    each([&](int i, int j, int q, uint32_t r, uint32_t c, float4& v) {
+        if (!inside && (r >= M || c >= N))
+            return;
+        v.x = Combine(args, v.x, acc[i][j][4 * q + 0]);
+        v.y = Combine(args, v.y, acc[i][j][4 * q + 1]);
+        v.z = Combine(args, v.z, acc[i][j][4 * q + 2]);
+        v.w = Combine(args, v.w, acc[i][j][4 * q + 3]);
+        if (relu)
+        {
+            v.x = v.x > 0 ? v.x : 0;
+            v.y = v.y > 0 ? v.y : 0;
+            v.z = v.z > 0 ? v.z : 0;
+            v.w = v.w > 0 ? v.w : 0;
+        }
+        float* p = out + static_cast<size_t>(r) * args.ldc + c;
+        if (inside || c + 4 <= N)
+            *reinterpret_cast<floatx4a4*>(p) = floatx4{ v.x, v.y, v.z, v.w };
+        else
+        {
+            p[0] = v.x;
+            if (c + 1 < N) p[1] = v.y;
+            if (c + 2 < N) p[2] = v.z;
+        }
+    });
 }
 
 template <int BM, int BN, bool VEC, bool TA, bool TB>
@@ -588,6 +574,14 @@ struct DmaTile
 // 4 values that end at K - and the fragments are put right where they are used (zeros for
 // k >= K, for A and B alike), so the step adds what a zero-padded slab would: the same sum,
 // in the same order, as the register-staged kernel.
+// It also stands for a k-major operand whose rows are no whole number of 4-float chunks (N of a B
+// stored K x N, M of an A stored K x M), then with r = BK where K is a multiple of the step: a
+// row's last chunk reaches into the next row, whose values feed only outputs that are not stored,
+// except in the last row of the matrix, where it would reach past its end.  There the lane copies
+// the 4 floats that end with the row, and the last step reads that row's value from where it
+// then lies (lastRow).  Such rows and columns were cut off as strips of 16 x 16 tiles before, which
+// took compute units from the body and ended after it (1001^3 23.9 -> 19.6 us, 4 x 1001 x 1003 x 999
+// 81.5 -> 66.4, 3001 x 2687 x 1000 138 -> 125, 4096 x 4095 x 4096 937 -> 922).
 //
 // KSPLIT = 2: two groups of wavefronts share the tile; of the four 8-wide k blocks of a
 // 32-wide step group 0 multiplies the first two and group 1 the last two, each into a sum of
@@ -707,13 +701,17 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
         return (gx * K + k4) * 4u - 16u + kTailBias;
     };
     auto laneOffsetXContig = [&](uint32_t j, uint32_t xBase, uint32_t limit, uint32_t pitch,
-                                 uint32_t rowBytes, uint32_t valid, auto rowAtPosition) {
+                                 uint32_t rowBytes, uint32_t valid, bool ending,
+                                 auto rowAtPosition) {
         const uint32_t b = j * 1024 + lane * 16;  // byte inside the unpadded slab
         uint32_t k = rowAtPosition(b / rowBytes);
         if (k >= valid)
             k = 0;
-        const uint32_t col = (b % rowBytes) / 4;
-        const uint32_t gx = min(xBase + col, limit - 4);
+        uint32_t gx = xBase + (b % rowBytes) / 4;
+        // chunks past the edge copy the row's last 4 floats; so does one that reaches past it in
+        // the last row of the matrix
+        if (gx >= limit || (ending && k + 1 == valid))
+            gx = min(gx, limit - 4);
         return (k * pitch + gx) * 4u + kTailBias;
     };
     auto locate = [&](uint32_t logicalTile, Place& p) {
@@ -740,11 +738,12 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
         for (uint32_t i = 0; i < kCopiesA; ++i)
         {
             const uint32_t j = wave + NW * i;
-            p.aLane[i] = TA ? laneOffsetXContig(j, p.rowBase, M, args.lda, TileA::kRowBytes, BK, TileA::RowAtPosition)
+            p.aLane[i] = TA ? laneOffsetXContig(j, p.rowBase, M, args.lda, TileA::kRowBytes, BK, false,
+                                                 TileA::RowAtPosition)
                             : laneOffsetKContig(j, p.rowBase, M, BK);
             if constexpr (TAIL)
                 p.aTail[i] = TA ? laneOffsetXContig(j, p.rowBase, M, args.lda, TileA::kRowBytes,
-                                                    lastValid, TileA::RowAtPosition)
+                                                    lastValid, true, TileA::RowAtPosition)
                                 : laneOffsetKContig(j, p.rowBase, M, lastValid);
         }
 #pragma unroll
@@ -752,11 +751,12 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
         {
             const uint32_t j = wave + NW * i;
             p.bLane[i] = TB ? laneOffsetKContig(j, p.colBase, N, BK)
-                            : laneOffsetXContig(j, p.colBase, N, args.ldb, TileB::kRowBytes, BK, TileB::RowAtPosition);
+                            : laneOffsetXContig(j, p.colBase, N, args.ldb, TileB::kRowBytes, BK, false,
+                                                 TileB::RowAtPosition);
             if constexpr (TAIL)
                 p.bTail[i] = TB ? laneOffsetKContig(j, p.colBase, N, lastValid)
                                 : laneOffsetXContig(j, p.colBase, N, args.ldb, TileB::kRowBytes,
-                                                    lastValid, TileB::RowAtPosition);
+                                                    lastValid, true, TileB::RowAtPosition);
         }
     };
     // LDS offsets of this wavefront's copies inside a stage
@@ -804,21 +804,36 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
     }
     uint32_t slabsLeft = steps;  // of the tile being fetched, the one at aSrc / bSrc included
     bool haveNext = false;       // `nxt` describes a tile the copy stream has not reached yet
+    // TAIL: the lane offsets of the last slab take over when the stream reaches it.  A branch,
+    // because selects in every step hold up its matrix instructions and a copy of the loop without
+    // them is fetched anew (4096 x 4096 x 4100: selects 947 us, two loops 932, branch 923;
+    // 512 x 1024 x 1000 12.7 / 11.8 / 11.2, of which the blocks left out of the last step 0.2).
+    auto reachLast = [&]() {
+        if constexpr (TAIL)
+            if (slabsLeft == 1)
+            {
+#pragma unroll
+                for (uint32_t i = 0; i < kCopiesA; ++i)
+                    asm volatile("v_mov_b32 %0, %1" : "=v"(aLane[i]) : "v"(aLaneLast[i]));
+#pragma unroll
+                for (uint32_t i = 0; i < kCopiesB; ++i)
+                    asm volatile("v_mov_b32 %0, %1" : "=v"(bLane[i]) : "v"(bLaneLast[i]));
+            }
+    };
+    reachLast();
     auto issueOne = [&](uint32_t stage, uint32_t n) {
         const uint32_t base = ldsBase + stage * kStageBytes;
-        // TAIL: the slab at aSrc / bSrc is the tile's last one when slabsLeft is 1
-        const bool partial = TAIL && slabsLeft == 1;
         if (n < kCopiesA)
-            DmaToLds16(partial ? aLaneLast[TAIL ? n : 0] : aLane[n], aSrc, base + aDst[n]);
+            DmaToLds16(aLane[n], aSrc, base + aDst[n]);
         else
-            DmaToLds16(partial ? bLaneLast[TAIL ? n - kCopiesA : 0] : bLane[n - kCopiesA], bSrc,
-                       base + bDst[n - kCopiesA]);
+            DmaToLds16(bLane[n - kCopiesA], bSrc, base + bDst[n - kCopiesA]);
     };
     auto advance = [&]() {
         if (--slabsLeft != 0)
         {
             aSrc += aStepBytes;
             bSrc += bStepBytes;
+            reachLast();
         }
         else if (WALK && haveNext)
         {
@@ -915,10 +930,19 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
     // TAIL: what the fragments of block q would be if the last slab were zero-padded to a whole
     // step; `valid` values of k exist.  Put in where the fragments are used so that the reads
     // above stay in flight behind the MFMAs of the block before.
-    //   k-major operand: zeros for k >= valid.
+    //   k-major operand: zeros for k >= valid, and lastRow's value for k = valid - 1.
     //   K-contiguous operand: chunks that begin at or past `valid` become zeros; the chunk
     //   that reaches past it was copied from valid - 4 on, so its values are moved down by
     //   4 - valid % 4 places and followed by zeros.
+    // value of column x of a k-major slab's row `row`, the last of the matrix: in the row's last
+    // chunk, where that is a broken one, the copied 4 floats end with the row
+    auto lastRow = [&](const char* slab, uint32_t x, uint32_t base, uint32_t limit,
+                       uint32_t rowOffset) {
+        const uint32_t chunk = base + (x & ~3u);
+        const uint32_t back = base + x < limit && chunk + 4 > limit ? chunk + 4 - limit : 0u;
+        return *reinterpret_cast<const float*>(slab + rowOffset + (x + back) * 4);
+    };
+    float aLast[TM], bLast[TN];
     auto dropMissing = [&](float (&a)[TM][4], float (&b)[TN][4], uint32_t q, uint32_t valid) {
         if constexpr (TAIL)
         {
@@ -943,16 +967,16 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
                 for (uint32_t e = 0; e < 4; ++e)
                     f[e] = g[e];
             };
-            auto fixKMajor = [&](float (&f)[4]) {
+            auto fixKMajor = [&](float (&f)[4], float last) {
 #pragma unroll
                 for (uint32_t e = 0; e < 4; ++e)
-                    f[e] = k0 + e < valid ? f[e] : 0.f;
+                    f[e] = k0 + e + 1 < valid ? f[e] : (k0 + e + 1 == valid ? last : 0.f);
             };
 #pragma unroll
             for (int i = 0; i < TM; ++i)
             {
                 if constexpr (TA)
-                    fixKMajor(a[i]);
+                    fixKMajor(a[i], aLast[i]);
                 else
                     fixKContig(a[i]);
             }
@@ -962,7 +986,7 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
                 if constexpr (TB)
                     fixKContig(b[j]);
                 else
-                    fixKMajor(b[j]);
+                    fixKMajor(b[j], bLast[j]);
             }
             // all of them ahead of the block's MFMAs, which then issue back to back
             __builtin_amdgcn_sched_barrier(0);
@@ -1184,14 +1208,36 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
             // first fragments are in fa[0] / fb[0]; no copy that is still in flight targets its
             // stage.
             const char* stage = lds + ((steps - 1) % STAGES) * kStageBytes;
+            constexpr bool kMajor = TA || !TB;  // an operand whose last row may be a broken one
+            if constexpr (TA)
+            {
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+                    aLast[i] = lastRow(stage, waveM * WM + i * 32 + l32, cur.rowBase, M,
+                                       TileA::RowOffsetXContig(lastValid - 1));
+            }
+            if constexpr (!TB)
+            {
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    bLast[j] = lastRow(stage + kBytesA, waveN * WN + j * 32 + l32, cur.colBase, N,
+                                       TileB::RowOffsetXContig(lastValid - 1));
+            }
 #pragma unroll
             for (uint32_t q = 0; q < kBlocks; ++q)
             {
                 if (q + 1 < kBlocks)
                     loadFragments(fa[(q + 1) & 1], fb[(q + 1) & 1], stage, q + 1);
                 __builtin_amdgcn_sched_barrier(0);
-                dropMissing(fa[q & 1], fb[q & 1], q, lastValid);
-                multiply(fa[q & 1], fb[q & 1]);
+                // a block past K adds nothing, one before the last row of the matrix needs no
+                // selects (the rest of the step at full length cost 1 us of a launch)
+                const uint32_t first = 8 * (q + kgroup * kBlocks);
+                if (first < lastValid)
+                {
+                    if (first + 8 + (kMajor ? 1u : 0u) > lastValid)
+                        dropMissing(fa[q & 1], fb[q & 1], q, lastValid);
+                    multiply(fa[q & 1], fb[q & 1]);
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -2013,9 +2059,11 @@ void LaunchTiled(const GemmF32Args& args, const GemmF32Strips& strips, dim3 grid
                  bool vec, bool dma, bool walk, int ksplit, hipStream_t stream)
 {
     const dim3 block(kThreads);
+    // rows of a k-major operand that end in a broken chunk: the kernels with a last step of its own
+    const bool broken = (TA && args.M % 4 != 0) || (!TB && args.N % 4 != 0);
     if (dma && ksplit != 0)
     {
-        if (args.K % 32 == 0)
+        if (args.K % 32 == 0 && !broken)
             hipLaunchKernelGGL((GemmF32DmaKernel<64, 32, 32, 4, TA, TB, false, false, 2>), grid,
                                dim3(256), 0, stream, args, strips);
         else
@@ -2025,7 +2073,7 @@ void LaunchTiled(const GemmF32Args& args, const GemmF32Strips& strips, dim3 grid
     }
     if (dma)
     {
-        if (big && args.K % 16 != 0)
+        if (big && (args.K % 16 != 0 || broken))
             hipLaunchKernelGGL((GemmF32DmaKernel<128, 128, 16, 4, TA, TB, false, true>), grid,
                                block, 0, stream, args, strips);
         else if (big)
@@ -2034,10 +2082,10 @@ void LaunchTiled(const GemmF32Args& args, const GemmF32Strips& strips, dim3 grid
         else if (walk)
             hipLaunchKernelGGL((GemmF32DmaKernel<64, 64, 32, 4, TA, TB, true>), grid, block, 0,
                                stream, args, strips);
-        else if (args.K % 32 == 0)
+        else if (args.K % 32 == 0 && !broken)
             hipLaunchKernelGGL((GemmF32DmaKernel<64, 64, 32, 4, TA, TB, false>), grid, block, 0,
                                stream, args, strips);
-        else if (args.K % 16 == 0)
+        else if (args.K % 16 == 0 && !broken)
             hipLaunchKernelGGL((GemmF32DmaKernel<64, 64, 16, 6, TA, TB, false>), grid, block, 0,
                                stream, args, strips);
         else
@@ -2156,8 +2204,6 @@ int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool o
     const uint64_t cusAll = static_cast<uint64_t>(sph::ComputeUnits());
     const bool midTiled = wholeTiles64 * 4 > cusAll && wholeTiles64 * 2 <= cusAll &&
                           args.basesOk != 0 && args.K >= 64 && args.M >= 4 && args.N >= 4 &&
-                          // (rows past the last multiple of 4 are cut off from 68 rows up)
-                          (args.M % 4 == 0 || args.M >= 68) &&
                           static_cast<uint64_t>(args.M) * args.K < (1ull << 30) &&
                           static_cast<uint64_t>(args.K) * args.N < (1ull << 30);
     const bool wholeIsFewTiles = wholeTiles64 * 2 <= cusAll && args.K >= 64 && !midTiled;
@@ -2169,61 +2215,61 @@ int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool o
         args.split = midTiled ? 12u : 4u;
     // A product for the tiled kernels is cut into a body and up to two thin strips of its last
     // rows and columns, which the few-tile kernel's code computes (it reads any rows and columns
-    // from anywhere); every output element is still computed once.  Cut off are
-    //  - the last N % 4 columns: the rows of a B stored K x N are copied 4 columns at a time
-    //    (measured 4096 x 4095 x 4096: 1615 us on the register-staged kernel's 4-byte loads);
-    //  - the last M % 4 rows, from 68 rows up: an A stored K x M is copied 4 rows at a time;
-    //  - up to 16 rows or columns past a multiple of the tile edge, when the compute unit with
-    //    the most tiles then has fewer of them (1025^3: 17 x 17 tiles of 64 are two per
-    //    compute unit somewhere, 16 x 16 one everywhere; measured 44.8 -> 23.4 us).
+    // from anywhere); every output element is still computed once.  Cut off are up to 16 rows or
+    // columns past a multiple of the tile edge, when the compute unit with the most tiles then has
+    // fewer of them (1025^3: 17 x 17 tiles of 64 are two per compute unit somewhere, 16 x 16 one
+    // everywhere; measured 44.8 -> 23.4 us).
     // The cut depends on M, N, K and the batch only, not on how the operands are stored or
     // aligned, so a product's bits do not depend on that either.
     if (whole && (args.split & 4u) != 0 && args.M > 1 && args.K >= kBK)
     {
-        const uint32_t baseM = (args.M >= 68 && args.N >= 4) ? args.M % 4 : 0;
-        const uint32_t baseN = args.N > 4 ? args.N % 4 : 0;
-        uint32_t peelM = baseM, peelN = baseN;
-        if ((args.split & 8u) == 0)
-        {
-            auto candidates = [](uint32_t x, uint32_t base, bool allowed, uint32_t* list) {
-                int n = 0;
-                list[n++] = base;
-                for (uint32_t edge = 64; edge <= 128 && allowed; edge *= 2)
+        uint32_t peelM = 0, peelN = 0;
+        const bool ksplitTiles = (args.split & 8u) != 0;
+        // the compute unit with the most tiles, as TileCost counts (a 64 x 32 tile is half of 107)
+        auto bodyCost = [&](uint32_t m, uint32_t n) -> uint64_t {
+            bool big;
+            if (!ksplitTiles)
+                return TileCost(m, n, units, &big);
+            const uint64_t tiles = static_cast<uint64_t>((m + 63) / 64) * ((n + 31) / 32) * units;
+            return (tiles + cusAll - 1) / cusAll * 54;
+        };
+        auto candidates = [&](uint32_t x, bool allowed, uint32_t* list) {
+            int n = 0;
+            list[n++] = 0;
+            for (uint32_t edge = 64; edge <= 128 && allowed; edge *= 2)
+            {
+                const uint32_t r = x % edge;
+                if (r != 0 && r <= 16 && x - r >= edge && r != list[n - 1])
+                    list[n++] = r;
+            }
+            return n;
+        };
+        uint32_t listM[3], listN[3];
+        const int countM = candidates(args.M, args.N >= 4, listM);
+        const int countN = candidates(args.N, true, listN);
+        // a strip's 16 x 16 tile: a sixteenth of a 64-tile's flops at about a quarter of
+        // its rate, beside the body's tiles
+        auto stripCost = [&](uint32_t rows, uint32_t cols) {
+            const uint64_t blocks =
+                static_cast<uint64_t>((rows + 15) / 16) * ((cols + 15) / 16) * units;
+            return (blocks + cusAll - 1) / cusAll * 27;
+        };
+        uint64_t best = ~0ull;
+        for (int i = 0; i < countM; ++i)
+            for (int j = 0; j < countN; ++j)
+            {
+                uint64_t cost = bodyCost(args.M - listM[i], args.N - listN[j]);
+                if (listM[i] != 0)
+                    cost += stripCost(listM[i], args.N);
+                if (listN[j] != 0)
+                    cost += stripCost(args.M - listM[i], listN[j]);
+                if (cost < best)
                 {
-                    const uint32_t r = x % edge;
-                    if (r != 0 && r <= 16 && r > base && x - r >= edge && r != list[n - 1])
-                        list[n++] = r;
+                    best = cost;
+                    peelM = listM[i];
+                    peelN = listN[j];
                 }
-                return n;
-            };
-            uint32_t listM[3], listN[3];
-            const int countM = candidates(args.M, baseM, args.N >= 4, listM);
-            const int countN = candidates(args.N, baseN, true, listN);
-            // a strip's 16 x 16 tile: a sixteenth of a 64-tile's flops at about a quarter of
-            // its rate, beside the body's tiles
-            auto stripCost = [&](uint32_t rows, uint32_t cols) {
-                const uint64_t blocks =
-                    static_cast<uint64_t>((rows + 15) / 16) * ((cols + 15) / 16) * units;
-                return (blocks + cusAll - 1) / cusAll * 27;
-            };
-            uint64_t best = ~0ull;
-            for (int i = 0; i < countM; ++i)
-                for (int j = 0; j < countN; ++j)
-                {
-                    bool big;
-                    uint64_t cost = TileCost(args.M - listM[i], args.N - listN[j], units, &big);
-                    if (listM[i] > baseM)
-                        cost += stripCost(listM[i], args.N);
-                    if (listN[j] > baseN)
-                        cost += stripCost(args.M - listM[i], listN[j]);
-                    if (cost < best)
-                    {
-                        best = cost;
-                        peelM = listM[i];
-                        peelN = listN[j];
-                    }
-                }
-        }
+            }
         if (peelM != 0 || peelN != 0)
         {
             GemmF32Args body = args;
@@ -2363,12 +2409,10 @@ int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool o
     // straight-to-LDS pipeline: whole K steps, 16-byte chunks everywhere, at least one chunk
     // per clamped edge, and lane offsets that fit 32 bits
     // (a K that is no multiple of the step: a last, partial one).  The copies take 16 bytes from
-    // any 4-byte-aligned address, so only an operand stored k-major, which is copied 4 rows or
-    // columns of the product at a time, needs a row length that is a multiple of 4.
+    // any 4-byte-aligned address, so rows may have any length; the kernels with a last step of its
+    // own take care of the piece that would reach past the end of an operand stored k-major.
     // (unit strides and table offsets may be anything)
-    const bool dmaLayout = args.basesOk != 0 && (!transA || args.M % 4 == 0) &&
-                           (transB || args.N % 4 == 0);
-    const bool dma = dmaLayout && args.K >= kBK && args.M >= 4 && args.N >= 4 &&
+    const bool dma = args.basesOk != 0 && args.K >= kBK && args.M >= 4 && args.N >= 4 &&
                      static_cast<uint64_t>(args.M) * args.K < (1ull << 30) &&
                      static_cast<uint64_t>(args.K) * args.N < (1ull << 30);
     bool big;

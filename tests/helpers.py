@@ -146,8 +146,7 @@ F32_CUS = 256
 
 def f32_k_split_range(M, N, K, batch=1):
     tiles64 = -(-M // 64) * -(-N // 64) * batch
-    return (4 * tiles64 > F32_CUS and 2 * tiles64 <= F32_CUS and K >= 64 and M >= 4 and N >= 4
-            and (M % 4 == 0 or M >= 68))
+    return (4 * tiles64 > F32_CUS and 2 * tiles64 <= F32_CUS and K >= 64 and M >= 4 and N >= 4)
 
 
 # Small products run on the few-tile kernel: at most one 32 x 32 output tile per compute unit

@@ -1,6 +1,5 @@
-"""fp32 GEMM whose last rows and columns are cut off as thin strips: the last N % 4 columns, the
-last M % 4 rows (from 68 rows up) and up to 16 rows or columns past a multiple of the tile edge
-when that spares the busiest compute unit a tile.  The strips are computed by the few-tile
+"""fp32 GEMM whose last rows and columns are cut off as thin strips: up to 16 rows or columns past a
+multiple of the tile edge when that spares the busiest compute unit a tile.  The strips are computed by the few-tile
 kernel's code inside the launch of the body (straight-to-LDS kernels) or by launches of their own
 (register-staged kernel: operands that start off a 16-byte boundary).
 
@@ -31,7 +30,7 @@ def _stored(A, B, flags):
 
 
 # (M, N, K, batch).  17 x 17 tiles of 64 cut down to 16 x 16; one row past 16 tile rows, 4 | N;
-# 1 column past; rows and columns past by up to 16; M % 4 and N % 4 only (no tile spared);
+# 1 column past; rows and columns past by up to 16; M % 4 and N % 4 only (no tile spared, no strip);
 # 128-tiles (33 x 33 of them cut to 32 x 32 would need 4225 rows: here 9 x 9 of 128 > 4 x 64-tile
 # rounds); a batch whose units each lose a row and a column; K below one step of 32 and K = 16
 SHAPES = [(1025, 1025, 40, 1), (1025, 1024, 70, 1), (1024, 1025, 33, 1), (1040, 1036, 48, 1),
