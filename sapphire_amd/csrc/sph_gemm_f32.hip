@@ -19,7 +19,8 @@
 //                        loads when possible, scalar predicated loads otherwise (small K,
 //                        misaligned bases, e.g. some of the reference's random test sizes,
 //                        Tests/UnitTests/Sources/FunctionTest/GemmTest.cpp:26-33);
-//   GemmF32ThinKernel    few output rows: K split over the lanes of a workgroup, vector units;
+//   GemmF32ThinKernel    few output rows (or, with a long K, columns): K split over the lanes of a
+//                        workgroup, vector units;
 //   GemmF32SkinnyKernel  few output tiles: 16 x 16 or 32 x 32 tiles with K split over the
 //                        wavefronts of a workgroup;
 //   GemvRowKernel        a single output row.
@@ -82,6 +83,7 @@ struct GemmF32Args
     // when sgd is set: out = out - ((A*B) * sgdScale) * sgdRate, every operation rounded on its
     // own -- the update Scale + Sub apply to a gradient that was stored first
     uint32_t sgd;
+    uint32_t mirror;     // launcher, few columns: operands, M and N changed places, out did not
     float sgdScale, sgdRate;
     int64_t strideOut, strideA, strideB;
 };
@@ -1584,6 +1586,7 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF32SkinnyKernel(const GemmF32A
 // ---------------------------------------------------------------------------
 constexpr uint32_t kThin = 16;
 constexpr uint32_t kThinShortK = 1024;  // up to here 4 wavefronts, else 8
+constexpr uint32_t kThinColumns = 8, kThinColumnsK = 1024;  // few columns instead (LaunchPart)
 
 // Sum over the 64 lanes of 16 values per lane; lane l ends up with the sum of value l / 4.
 __device__ __forceinline__ float WaveSums16(float (&v)[16], uint32_t lane)
@@ -1652,8 +1655,8 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF32ThinKernel(const GemmF32Arg
     if (args.entries != nullptr)
     {
         const SphGemmEntry e = args.entries[unit];
-        A = args.A + e.aOff;
-        B = args.B + e.bOff;
+        A = args.A + (args.mirror ? e.bOff : e.aOff);
+        B = args.B + (args.mirror ? e.aOff : e.bOff);
         out = args.out + e.outOff;
     }
     else
@@ -1667,10 +1670,11 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF32ThinKernel(const GemmF32Arg
     // wavefront 0 stores sum 4 i + x of lane l = 4 i + x: what it is added to
     const uint32_t row = lane >> 2, col = x0 + (lane & 3);
     const bool stores = wave == 0 && row < M && col < N;
-    float* const place = out + static_cast<size_t>(row) * args.ldc + col;
+    const uint32_t outRow = args.mirror ? col : row, outCol = args.mirror ? row : col;
+    float* const place = out + static_cast<size_t>(outRow) * args.ldc + outCol;
     float old = 0.f;
     if (stores && args.bias != nullptr)
-        old = args.bias[col];
+        old = args.bias[outCol];
     else if (stores && !args.overwrite)
         old = *place;
 
@@ -2349,22 +2353,42 @@ int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool o
     // Few rows: 4 columns per workgroup while that is at most one per compute unit, or two where a
     // workgroup's A is small; beyond that 16 x 16 tiles read A less often (16 x 2048 x 1024 7.1 us
     // on them, 6.4 here; x 2048 11.4 / 11.4; x 4096 18.7 / 19.5; 8 x 2048 x 4096 16.0 / 15.4).
-    const uint64_t thinBlocks = static_cast<uint64_t>((args.N + 3) / 4) * units;
-    if (fewTiles && args.M <= kThin && args.M <= args.N && args.K < (1u << 31) &&
-        (thinBlocks <= cusAll ||
-         (thinBlocks <= 2 * cusAll && (args.M <= 8 || args.K <= 2 * kThinShortK))))
+    // A product of few columns is the same with its operands, and rows and columns, changed over:
+    // up to 8 of them from K = 1024 on, one workgroup per compute unit (few-tile kernel / this, the
+    // slowest storage beside: 1024 x 1 x 1024 7.1 / 4.1, A stored K x M 5.9 / 4.3 us; 1024 x 4 x 1500
+    // 6.8 / 4.1, 6.5 / 5.3; 1024 x 8 x 1024 6.8 / 4.9, 5.8 / 5.7; 128 x 8 x 4096 13.2 / 7.6, 12.1 / 8.9).
+    // At K = 256 the two are level, an A stored K x M of two workgroups per compute unit is read
+    // slower (2048 x 8 x 1024 5.9 / 6.8), and of 16 columns every workgroup would read too much again
+    // (128 x 16 x 1024 6.7 / 7.0, 1024 x 10 x 1024 6.8 / 6.0 but 5.9 / 6.8 with A stored K x M).
+    GemmF32Args thin = args;
+    bool thinTransA = transA, thinTransB = transB;
+    if (args.N < args.M && args.N <= kThinColumns && args.K >= kThinColumnsK &&
+        (args.split & 3u) == 0)
     {
-        args.tilesN = (args.N + 3) / 4;
-        args.tilesTotal = static_cast<uint32_t>(thinBlocks);
-        args.perXcd = (args.tilesTotal + 7) / 8;
-        if (transA && transB)
-            LaunchThin<true, false>(args, stream);
-        else if (transA)
-            LaunchThin<false, false>(args, stream);
-        else if (transB)
-            LaunchThin<true, true>(args, stream);
+        std::swap(thin.M, thin.N);
+        std::swap(thin.A, thin.B);
+        std::swap(thin.strideA, thin.strideB);
+        std::swap(thin.lda, thin.ldb);
+        thinTransA = !transB;
+        thinTransB = !transA;
+        thin.mirror = 1;
+    }
+    const uint64_t thinBlocks = static_cast<uint64_t>((thin.N + 3) / 4) * units;
+    if (fewTiles && thin.M <= kThin && thin.M <= thin.N && args.K < (1u << 31) &&
+        (thinBlocks <= cusAll ||
+         (thin.mirror == 0 && thinBlocks <= 2 * cusAll && (thin.M <= 8 || args.K <= 2 * kThinShortK))))
+    {
+        thin.tilesN = (thin.N + 3) / 4;
+        thin.tilesTotal = static_cast<uint32_t>(thinBlocks);
+        thin.perXcd = (thin.tilesTotal + 7) / 8;
+        if (thinTransA && thinTransB)
+            LaunchThin<true, false>(thin, stream);
+        else if (thinTransA)
+            LaunchThin<false, false>(thin, stream);
+        else if (thinTransB)
+            LaunchThin<true, true>(thin, stream);
         else
-            LaunchThin<false, true>(args, stream);
+            LaunchThin<false, true>(thin, stream);
         SPH_CHECK_LAUNCH();
         return SPH_OK;
     }
