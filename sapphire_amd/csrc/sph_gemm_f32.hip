@@ -359,8 +359,55 @@ __device__ __forceinline__ void StoreTile(const floatx16 (&acc)[TM][TN], float* 
     });
 }
 
-template <int BM, int BN, bool VEC, bool TA, bool TB>
-__global__ __launch_bounds__(kThreads) void GemmF32Kernel(const GemmF32Args args)
+// Sums in parts (the launcher's SumsInParts says for which products).  One chain of K additions
+// rounds K times; four chains of K / 4 have half the error.
+//   64-wide tiles: the 8-wide k blocks go to four sums in turn, added up at the end as
+//     (0 + 1) + (2 + 3).  No instruction more in the loop, 48 registers.
+//   128-wide tiles, where four sums would not fit the registers: the sum is moved to a second one
+//     after every PartSteps steps of 16.
+template <int SUMS, int TM, int TN>
+__device__ __forceinline__ void AddParts(floatx16 (&part)[SUMS][TM][TN])
+{
+    static_assert(SUMS == 1 || SUMS == 2 || SUMS == 4, "one sum, two or four");
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+        {
+            if constexpr (SUMS >= 2)
+                part[0][i][j] += part[1][i][j];
+            if constexpr (SUMS == 4)
+            {
+                part[2][i][j] += part[3][i][j];
+                part[0][i][j] += part[2][i][j];
+            }
+        }
+}
+
+// about a quarter of K, in pairs of steps of 16 (from K = 224 on no part is longer than a quarter by
+// more than 8)
+__device__ __forceinline__ uint32_t PartSteps(uint32_t K)
+{
+    return max((K + 32u) / 128u, 1u) * 2u;
+}
+
+// total += acc, acc = 0
+template <int TM, int TN>
+__device__ __forceinline__ void MoveSum(floatx16 (&total)[TM][TN], floatx16 (&acc)[TM][TN])
+{
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+        {
+            total[i][j] += acc[i][j];
+            acc[i][j] = floatx16{};
+        }
+}
+
+template <int BM, int BN, bool VEC, bool TA, bool TB, bool PARTS>
+__global__ __launch_bounds__(kThreads, PARTS && BM == 128 ? 2 : 1) void GemmF32Kernel(
+    const GemmF32Args args)
 {
     constexpr int WM = BM / 2;   // rows per wavefront
     constexpr int WN = BN / 2;   // columns per wavefront
@@ -433,14 +480,11 @@ __global__ __launch_bounds__(kThreads) void GemmF32Kernel(const GemmF32Args args
             StashXContig<BN, LDB, B_QUADS>(Bs[buf], stageB, tid);
     };
 
-    floatx16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v)
-                acc[i][j][v] = 0.f;
+    constexpr int kSums = PARTS && TM * TN == 1 ? 4 : 1;
+    constexpr bool kMoves = PARTS && TM * TN != 1;
+    floatx16 part[kSums][TM][TN] = {};
+    floatx16 total[kMoves ? TM : 1][kMoves ? TN : 1] = {};
+    floatx16 (&acc)[TM][TN] = part[0];
 
     const uint32_t steps = (K + kBK - 1) / kBK;
     if (steps > 0)
@@ -458,8 +502,9 @@ __global__ __launch_bounds__(kThreads) void GemmF32Kernel(const GemmF32Args args
     const uint32_t l32 = lane & 31;
     const uint32_t khalf = lane >> 5;
 
-    for (uint32_t s = 0; s < steps; ++s)
-    {
+    // `sums`: the sum that the step's first block goes to
+    auto step = [&](uint32_t s, auto sums) {
+        constexpr int kFirst = decltype(sums)::value;
         const int cur = s & 1;
         if (s + 1 < steps)
             fetch((s + 1) * kBK);
@@ -489,16 +534,50 @@ __global__ __launch_bounds__(kThreads) void GemmF32Kernel(const GemmF32Args args
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
+                {
                     // operands swapped: the 32x32 result block comes out indexed
                     // [column][row], which leaves 4 consecutive columns in a lane
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[slot][j], a[slot][i],
-                                                                     acc[i][j], 0, 0, 0);
+                    floatx16& sum = part[(kFirst + kk / 8) % kSums][i][j];
+                    sum = __builtin_amdgcn_mfma_f32_32x32x2f32(b[slot][j], a[slot][i], sum, 0, 0,
+                                                               0);
+                }
             __builtin_amdgcn_sched_barrier(0);
         }
 
         if (s + 1 < steps)
             stash(cur ^ 1);
         __syncthreads();
+    };
+    if constexpr (kSums == 4)
+    {
+        for (uint32_t s = 0; s < steps; s += 2)
+        {
+            step(s, std::integral_constant<int, 0>{});
+            if (s + 1 < steps)
+                step(s + 1, std::integral_constant<int, 2>{});
+        }
+        AddParts(part);
+    }
+    else
+    {
+        uint32_t moveAt = PartSteps(K);
+        for (uint32_t s = 0; s < steps; ++s)
+        {
+            step(s, std::integral_constant<int, 0>{});
+            if constexpr (kMoves)
+                if (s + 1 == moveAt && s + 1 < steps)
+                {
+                    MoveSum(total, acc);
+                    moveAt += PartSteps(K);
+                }
+        }
+        if constexpr (kMoves)
+        {
+            MoveSum(total, acc);
+            StoreTile<TM, TN>(total, out, rowBase + waveM * WM, colBase + waveN * WN, M, N, l32,
+                              khalf, args);
+            return;
+        }
     }
 
     StoreTile<TM, TN>(acc, out, rowBase + waveM * WM, colBase + waveN * WN, M, N, l32, khalf, args);
@@ -620,10 +699,10 @@ struct DmaTile
 template <int TILE, bool TA, bool TB, int WAVES>
 __device__ __forceinline__ void GemmF32SkinnyBody(const GemmF32Args& args, uint32_t block);
 
-template <int BM, int BN, int BK, int STAGES, bool TA, bool TB, bool WALK, bool TAIL = false,
-          int KSPLIT = 1>
-__global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32DmaKernel(
-    const GemmF32Args args, const GemmF32Strips strips)
+template <int BM, int BN, int BK, int STAGES, bool TA, bool TB, bool WALK, bool TAIL, int KSPLIT,
+          bool PARTS>
+__global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64, PARTS && BM == 128 ? 2 : 1) void
+GemmF32DmaKernel(const GemmF32Args args, const GemmF32Strips strips)
 {
     static_assert(BK == 16 || BK == 32, "K step of 16 or 32");
     static_assert(!(WALK && TAIL), "a walk needs whole rings of steps");
@@ -650,6 +729,11 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
     constexpr uint32_t kBlocks = BK / 8 / KSPLIT;  // 8-wide k blocks (4 MFMAs each) per step
                                                    // and wavefront
     constexpr int kQuads = TM * TN * 4;   // float4 of `out` per lane
+    // sums in parts (see AddParts): two per group of a K split, four otherwise
+    constexpr uint32_t kSums = PARTS && TM * TN == 1 ? 4 / KSPLIT : 1;
+    constexpr bool kMoves = PARTS && TM * TN != 1;
+    static_assert(kSums <= kBlocks || STAGES % (kSums / kBlocks) == 0, "blocks in turn");
+    static_assert(!kMoves || BK == 16, "PartSteps counts steps of 16");
 
     __shared__ __attribute__((aligned(1024))) char lds[STAGES * kStageBytes];
 
@@ -876,7 +960,9 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
             slabsLeft = 1;
     };
 
-    floatx16 acc[TM][TN];
+    floatx16 part[kSums][TM][TN];
+    floatx16 total[kMoves ? TM : 1][kMoves ? TN : 1] = {};
+    floatx16 (&acc)[TM][TN] = part[0];
 
     // ---- fragment addresses inside a stage -------------------------------------------------
     // K-contiguous operand: byte offset of this lane's row, chunk chosen per 8-wide k block.
@@ -1016,15 +1102,17 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    auto multiply = [&](const float (&a)[TM][4], const float (&b)[TN][4]) {
+    // `n`: the block's number, counted from any multiple of kSums
+    auto multiply = [&](const float (&a)[TM][4], const float (&b)[TN][4], uint32_t n) {
+        floatx16 (&sum)[TM][TN] = part[n % kSums];
 #pragma unroll
         for (uint32_t e = 0; e < 4; ++e)
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    acc[i][j] =
-                        __builtin_amdgcn_mfma_f32_32x32x2f32(b[j][e], a[i][e], acc[i][j], 0, 0, 0);
+                    sum[i][j] =
+                        __builtin_amdgcn_mfma_f32_32x32x2f32(b[j][e], a[i][e], sum[i][j], 0, 0, 0);
     };
 
     // ---- WALK: the values the tile's products are added to ----------------------------------
@@ -1104,8 +1192,9 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
     // matrix pipe is already busy: behind the first one the wait for step s+1's copies and the
     // barrier, behind each of the next ones one copy of step s+STAGES-1.
     static_assert(kCopiesPerWave <= 4 * TM * TN, "one copy per MFMA of the first block");
-    auto multiplyAndFeed = [&](const float (&a)[TM][4], const float (&b)[TN][4],
+    auto multiplyAndFeed = [&](const float (&a)[TM][4], const float (&b)[TN][4], uint32_t block0,
                                uint32_t fillStage, bool tileStart, bool settle) {
+        floatx16 (&sum)[TM][TN] = part[block0 % kSums];
 #pragma unroll
         for (uint32_t e = 0; e < 4; ++e)
 #pragma unroll
@@ -1114,8 +1203,8 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
                 for (int j = 0; j < TN; ++j)
                 {
                     const uint32_t n = (e * TM + i) * TN + j;
-                    acc[i][j] =
-                        __builtin_amdgcn_mfma_f32_32x32x2f32(b[j][e], a[i][e], acc[i][j], 0, 0, 0);
+                    sum[i][j] =
+                        __builtin_amdgcn_mfma_f32_32x32x2f32(b[j][e], a[i][e], sum[i][j], 0, 0, 0);
                     if (n == 0)
                     {
                         // steps up to s+1 have landed once at most the STAGES-3 later ones
@@ -1176,12 +1265,16 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
             }
         }
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+        for (uint32_t s = 0; s < kSums; ++s)
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int v = 0; v < 16; ++v)
-                    acc[i][j][v] = 0.f;
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v)
+                        part[s][i][j][v] = 0.f;
+
+        uint32_t moveAt = PartSteps(K);  // (sums in parts, 128-wide tiles)
 
         // The loop is unrolled over the ring so that every stage offset is a constant.  With
         // WALK the step count is a positive multiple of STAGES and the first trip round the
@@ -1206,12 +1299,18 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
                         loadFragments(fa[(q + 1) & 1], fb[(q + 1) & 1], next, 0);
                     __builtin_amdgcn_sched_barrier(0);
                     if (q == 0)
-                        multiplyAndFeed(fa[0], fb[0], (u + STAGES - 1) % STAGES,
+                        multiplyAndFeed(fa[0], fb[0], u * kBlocks, (u + STAGES - 1) % STAGES,
                                         kFirst && u == 0, kFirst && u == 1);
                     else
-                        multiply(fa[q & 1], fb[q & 1]);
+                        multiply(fa[q & 1], fb[q & 1], u * kBlocks + q);
                     __builtin_amdgcn_sched_barrier(0);
                 }
+                if constexpr (kMoves)
+                    if (u % 2 == 1 && s0 + u + 1 == moveAt && moveAt < steps)
+                    {
+                        MoveSum(total, acc);
+                        moveAt += PartSteps(K);
+                    }
             }
         };
         if constexpr (WALK)
@@ -1260,7 +1359,7 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
                 {
                     if (first + 8 + (kMajor ? 1u : 0u) > lastValid)
                         dropMissing(fa[q & 1], fb[q & 1], q, lastValid);
-                    multiply(fa[q & 1], fb[q & 1]);
+                    multiply(fa[q & 1], fb[q & 1], q);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -1280,6 +1379,7 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
         }
     }
     WaitVmem<0>();  // the surplus copies of the last steps still target LDS
+    AddParts(part);
 
     if constexpr (KSPLIT == 2)
     {
@@ -1318,7 +1418,13 @@ __global__ __launch_bounds__(((BN >= 64) ? 4 : 2) * KSPLIT * 64) void GemmF32Dma
                 }
     }
 
-    if constexpr (!WALK)
+    if constexpr (kMoves)
+    {
+        MoveSum(total, acc);
+        StoreTile<TM, TN>(total, cur.out, cur.rowBase + waveM * WM, cur.colBase + waveN * WN, M, N,
+                          l32, khalf, args);
+    }
+    else if constexpr (!WALK)
         StoreTile<TM, TN>(acc, cur.out, cur.rowBase + waveM * WM, cur.colBase + waveN * WN, M, N,
                           l32, khalf, args);
 }
@@ -2076,6 +2182,53 @@ void LaunchThin(const GemmF32Args& args, hipStream_t stream)
         LaunchThinRows<B_K, A_K, 4>(args, stream);
 }
 
+// Products whose sums are taken in parts: an M or N that is no multiple of 4.  Their last rows and
+// columns used to be sums of four parts, as strips of the few-tile kernel, and a chain of K
+// additions instead has twice the error (1001^3: 5.8e-7 of a sum's size against 2.8e-7 there); with
+// all sums in parts it is 2.8e-7 everywhere.  The rule looks at the sizes only, so that a
+// product's bits do not depend on how its operands are stored.  It costs up to 3 % (513 x 515 x 257
+// 5.88 -> 6.07 us, 1001 x 1024 x 784 15.0 -> 15.4, 3001 x 2687 x 1000 124.8 -> 126.2, 4096 x 4095 x 4096
+// 917 -> 923).
+bool SumsInParts(const GemmF32Args& args)
+{
+    return args.M % 4 != 0 || args.N % 4 != 0;
+}
+
+template <bool TA, bool TB, bool PARTS>
+void LaunchStaged(const GemmF32Args& args, dim3 grid, bool big, bool vec, hipStream_t stream)
+{
+    const dim3 block(kThreads);
+    if (big && vec)
+        hipLaunchKernelGGL((GemmF32Kernel<128, 128, true, TA, TB, PARTS>), grid, block, 0, stream,
+                           args);
+    else if (big)
+        hipLaunchKernelGGL((GemmF32Kernel<128, 128, false, TA, TB, PARTS>), grid, block, 0, stream,
+                           args);
+    else if (vec)
+        hipLaunchKernelGGL((GemmF32Kernel<64, 64, true, TA, TB, PARTS>), grid, block, 0, stream,
+                           args);
+    else
+        hipLaunchKernelGGL((GemmF32Kernel<64, 64, false, TA, TB, PARTS>), grid, block, 0, stream,
+                           args);
+}
+
+// one 64 x 64 tile per workgroup; `tail`: a last step of its own
+template <bool TA, bool TB, bool PARTS>
+void LaunchTiles64(const GemmF32Args& args, const GemmF32Strips& strips, dim3 grid, bool tail,
+                   hipStream_t stream)
+{
+    const dim3 block(kThreads);
+    if (tail)
+        hipLaunchKernelGGL((GemmF32DmaKernel<64, 64, 32, 4, TA, TB, false, true, 1, PARTS>), grid,
+                           block, 0, stream, args, strips);
+    else if (args.K % 32 == 0)
+        hipLaunchKernelGGL((GemmF32DmaKernel<64, 64, 32, 4, TA, TB, false, false, 1, PARTS>), grid,
+                           block, 0, stream, args, strips);
+    else
+        hipLaunchKernelGGL((GemmF32DmaKernel<64, 64, 16, 6, TA, TB, false, false, 1, PARTS>), grid,
+                           block, 0, stream, args, strips);
+}
+
 // `walk`: 64-tiles only, each workgroup takes several tiles
 // `ksplit`: 0, or 2 = K split over two groups of wavefronts on 64 x 32 tiles
 // `strips`: edge strips that ride along; only the straight-to-LDS kernels that are no walk take
@@ -2085,58 +2238,50 @@ void LaunchTiled(const GemmF32Args& args, const GemmF32Strips& strips, dim3 grid
                  bool vec, bool dma, bool walk, int ksplit, hipStream_t stream)
 {
     const dim3 block(kThreads);
+    const bool parts = SumsInParts(args);
     // rows of a k-major operand that end in a broken chunk: the kernels with a last step of its own
     const bool broken = (TA && args.M % 4 != 0) || (!TB && args.N % 4 != 0);
     if (dma && ksplit != 0)
     {
-        if (args.K % 32 == 0 && !broken)
-            hipLaunchKernelGGL((GemmF32DmaKernel<64, 32, 32, 4, TA, TB, false, false, 2>), grid,
-                               dim3(256), 0, stream, args, strips);
+        if (parts)
+            hipLaunchKernelGGL((GemmF32DmaKernel<64, 32, 32, 4, TA, TB, false, true, 2, true>),
+                               grid, dim3(256), 0, stream, args, strips);
+        else if (args.K % 32 != 0)
+            hipLaunchKernelGGL((GemmF32DmaKernel<64, 32, 32, 4, TA, TB, false, true, 2, false>),
+                               grid, dim3(256), 0, stream, args, strips);
         else
-            hipLaunchKernelGGL((GemmF32DmaKernel<64, 32, 32, 4, TA, TB, false, true, 2>), grid,
-                               dim3(256), 0, stream, args, strips);
+            hipLaunchKernelGGL((GemmF32DmaKernel<64, 32, 32, 4, TA, TB, false, false, 2, false>),
+                               grid, dim3(256), 0, stream, args, strips);
+        return;
+    }
+    if (dma && big)
+    {
+        if (parts)
+            hipLaunchKernelGGL((GemmF32DmaKernel<128, 128, 16, 4, TA, TB, false, true, 1, true>),
+                               grid, block, 0, stream, args, strips);
+        else if (args.K % 16 != 0)
+            hipLaunchKernelGGL((GemmF32DmaKernel<128, 128, 16, 4, TA, TB, false, true, 1, false>),
+                               grid, block, 0, stream, args, strips);
+        else
+            hipLaunchKernelGGL((GemmF32DmaKernel<128, 128, 16, 4, TA, TB, false, false, 1, false>),
+                               grid, block, 0, stream, args, strips);
         return;
     }
     if (dma)
     {
-        if (big && (args.K % 16 != 0 || broken))
-            hipLaunchKernelGGL((GemmF32DmaKernel<128, 128, 16, 4, TA, TB, false, true>), grid,
-                               block, 0, stream, args, strips);
-        else if (big)
-            hipLaunchKernelGGL((GemmF32DmaKernel<128, 128, 16, 4, TA, TB, false>), grid, block, 0,
-                               stream, args, strips);
-        else if (walk)
-            hipLaunchKernelGGL((GemmF32DmaKernel<64, 64, 32, 4, TA, TB, true>), grid, block, 0,
-                               stream, args, strips);
-        else if (args.K % 32 == 0 && !broken)
-            hipLaunchKernelGGL((GemmF32DmaKernel<64, 64, 32, 4, TA, TB, false>), grid, block, 0,
-                               stream, args, strips);
-        else if (args.K % 16 == 0 && !broken)
-            hipLaunchKernelGGL((GemmF32DmaKernel<64, 64, 16, 6, TA, TB, false>), grid, block, 0,
-                               stream, args, strips);
+        if (walk)
+            hipLaunchKernelGGL((GemmF32DmaKernel<64, 64, 32, 4, TA, TB, true, false, 1, false>),
+                               grid, block, 0, stream, args, strips);
+        else if (parts)
+            LaunchTiles64<TA, TB, true>(args, strips, grid, args.K % 16 != 0 || broken, stream);
         else
-            hipLaunchKernelGGL((GemmF32DmaKernel<64, 64, 32, 4, TA, TB, false, true>), grid,
-                               block, 0, stream, args, strips);
+            LaunchTiles64<TA, TB, false>(args, strips, grid, args.K % 16 != 0, stream);
         return;
     }
-    if (big)
-    {
-        if (vec)
-            hipLaunchKernelGGL((GemmF32Kernel<128, 128, true, TA, TB>), grid, block, 0, stream,
-                               args);
-        else
-            hipLaunchKernelGGL((GemmF32Kernel<128, 128, false, TA, TB>), grid, block, 0, stream,
-                               args);
-    }
+    if (parts)
+        LaunchStaged<TA, TB, true>(args, grid, big, vec, stream);
     else
-    {
-        if (vec)
-            hipLaunchKernelGGL((GemmF32Kernel<64, 64, true, TA, TB>), grid, block, 0, stream,
-                               args);
-        else
-            hipLaunchKernelGGL((GemmF32Kernel<64, 64, false, TA, TB>), grid, block, 0, stream,
-                               args);
-    }
+        LaunchStaged<TA, TB, false>(args, grid, big, vec, stream);
 }
 
 // Tile edge: the matrix pipes bound the tiled kernels, so a launch lasts as long as the compute
