@@ -2302,6 +2302,51 @@ uint64_t TileCost(uint32_t M, uint32_t N, uint32_t units, bool* big)
     return std::min(cost128, cost64);
 }
 
+// whole 64-tiles and a K that fills the ring of four 32-wide steps a whole number of times
+bool WalksTiles(uint32_t M, uint32_t N, uint32_t K)
+{
+    return M % 64 == 0 && N % 64 == 0 && K % 128 == 0;
+}
+
+// Cost of a product of which the last `peelM` rows and `peelN` columns are strips: the compute unit
+// with the most tiles, as TileCost counts (a 64 x 32 tile is half of a 64-tile).  A strip's 16 x 16
+// tile is a sixteenth of a 64-tile's flops at about a quarter of its rate, beside the body's tiles;
+// where body and strips have a compute unit for each of their workgroups it costs nothing, unless
+// the body walks its tiles (the strips are then launches of their own: 1025 x 515 x 512 12.0 us,
+// 18.0 with them).  Of cuts that are level the one that leaves M and N in multiples of 4 is
+// better, if that spares the kernel's last step (513 x 515 x 1024 11.0 us with strips, 11.4
+// without, 66 x 4097 x 1024 18.7 / 19.3; not so with K = 700: 514 x 515 9.20 / 9.06).
+uint64_t CutCost(uint32_t M, uint32_t N, uint32_t K, uint32_t units, uint32_t peelM, uint32_t peelN,
+                 bool ksplitTiles)
+{
+    const uint64_t cus = static_cast<uint64_t>(sph::ComputeUnits());
+    const uint32_t m = M - peelM, n = N - peelN;
+    auto tilesOf = [&](uint32_t rows, uint32_t columns, uint32_t bm, uint32_t bn) {
+        return static_cast<uint64_t>((rows + bm - 1) / bm) * ((columns + bn - 1) / bn) * units;
+    };
+    bool big = false;
+    uint64_t cost, tiles;
+    if (ksplitTiles)
+    {
+        tiles = tilesOf(m, n, 64, 32);
+        cost = (tiles + cus - 1) / cus * 54;
+    }
+    else
+    {
+        cost = TileCost(m, n, units, &big);
+        tiles = big ? tilesOf(m, n, 128, 128) : tilesOf(m, n, 64, 64);
+    }
+    const uint64_t bottom = peelM != 0 ? tilesOf(peelM, N, 16, 16) : 0;
+    const uint64_t right = peelN != 0 ? tilesOf(m, peelN, 16, 16) : 0;
+    const bool walks = !ksplitTiles && !big && WalksTiles(m, n, K);
+    if (tiles + bottom + right > cus || walks)
+        cost += ((bottom + cus - 1) / cus + (right + cus - 1) / cus) * 27;
+    const uint32_t broken = (m % 4 != 0 ? 1u : 0u) + (n % 4 != 0 ? 1u : 0u);
+    if (ksplitTiles)
+        return cost * 4 + (K % 32 == 0 && broken != 0 ? 1 : 0);
+    return cost * 4 + (K % 16 == 0 ? broken : 0);
+}
+
 template <bool TA, bool TB>
 void LaunchStripAlone(const GemmF32Args& strip, uint32_t blocks, hipStream_t stream)
 {
@@ -2396,44 +2441,27 @@ int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool o
     {
         uint32_t peelM = 0, peelN = 0;
         const bool ksplitTiles = (args.split & 8u) != 0;
-        // the compute unit with the most tiles, as TileCost counts (a 64 x 32 tile is half of 107)
-        auto bodyCost = [&](uint32_t m, uint32_t n) -> uint64_t {
-            bool big;
-            if (!ksplitTiles)
-                return TileCost(m, n, units, &big);
-            const uint64_t tiles = static_cast<uint64_t>((m + 63) / 64) * ((n + 31) / 32) * units;
-            return (tiles + cusAll - 1) / cusAll * 54;
-        };
         auto candidates = [&](uint32_t x, bool allowed, uint32_t* list) {
             int n = 0;
             list[n++] = 0;
-            for (uint32_t edge = 64; edge <= 128 && allowed; edge *= 2)
+            for (uint32_t edge : { 4u, 64u, 128u })
             {
                 const uint32_t r = x % edge;
-                if (r != 0 && r <= 16 && x - r >= edge && r != list[n - 1])
+                if (allowed && r != 0 && r <= 16 && x - r >= std::max(edge, 64u) &&
+                    r != list[n - 1])
                     list[n++] = r;
             }
             return n;
         };
-        uint32_t listM[3], listN[3];
+        uint32_t listM[4], listN[4];
         const int countM = candidates(args.M, args.N >= 4, listM);
         const int countN = candidates(args.N, true, listN);
-        // a strip's 16 x 16 tile: a sixteenth of a 64-tile's flops at about a quarter of
-        // its rate, beside the body's tiles
-        auto stripCost = [&](uint32_t rows, uint32_t cols) {
-            const uint64_t blocks =
-                static_cast<uint64_t>((rows + 15) / 16) * ((cols + 15) / 16) * units;
-            return (blocks + cusAll - 1) / cusAll * 27;
-        };
         uint64_t best = ~0ull;
         for (int i = 0; i < countM; ++i)
             for (int j = 0; j < countN; ++j)
             {
-                uint64_t cost = bodyCost(args.M - listM[i], args.N - listN[j]);
-                if (listM[i] != 0)
-                    cost += stripCost(listM[i], args.N);
-                if (listN[j] != 0)
-                    cost += stripCost(args.M - listM[i], listN[j]);
+                const uint64_t cost = CutCost(args.M, args.N, args.K, units, listM[i],
+                                              listN[j], ksplitTiles);
                 if (cost < best)
                 {
                     best = cost;
@@ -2643,7 +2671,7 @@ int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool o
     // (measured 4096^3: 921 -> 966 us), so it keeps one tile per workgroup.
     const uint32_t slotsPerXcd = static_cast<uint32_t>(cus / 8 * 2);
     const bool walk = dma && !big && ksplit == 0 &&
-                      args.M % 64 == 0 && args.N % 64 == 0 && args.K % 128 == 0 &&
+                      WalksTiles(args.M, args.N, args.K) &&
                       (reinterpret_cast<uintptr_t>(args.bias) & 15u) == 0;
     // strips that wait ride along with a straight-to-LDS launch that is no walk
     GemmF32Strips strips{};
