@@ -1704,13 +1704,16 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF32SkinnyKernel(const GemmF32A
 // takes k = 4 (64 w + l) .. + 3 and every 256 WAVES further, as 16-byte pieces whichever way B is
 // stored, keeps 4 MR sums of its own, and the sums of the lanes are added by exchanges in the
 // vector unit, those of the wavefronts through LDS.  The order of the additions depends on K only.
-// Bound by latency: launch, one round of loads, one reduction.  Kernel times with cold operands,
-// 16 x 16 tiles before: 8 x 1024 x 784 and x 1024 6.8 -> 4.9 us, 8 x 10 x 1024 5.6 -> 4.6; calls
-// in a row (a call costs the host about 4 us): 16 x 1024 x 1024 7.1 -> 4.9, 8 x 512 x 4096
-// 11.2 -> 6.9, 16 x 128 x 4096 13.4 -> 7.9, B stored N x K 8 x 1024 x 1024 8.4 -> 3.4.
-// Few output columns stay on 16 x 16 tiles: the roles swapped, with B's narrow rows taken through
-// LDS, 1024 x 10 x 1024 gains 1.4 us, its form with A stored K x M loses 0.6 and 2048 x 16 x 2048
-// goes from 9.1 to 14.0.
+// Bound by latency: launch, one round of loads, one reduction.  Device times, calls one after the
+// other in a graph, 16 x 16 tiles before, 1024 columns: 8 rows, K = 64 3.02 -> 2.89 us, 256 3.37 -> 3.08,
+// 784 5.10 -> 3.84, 2048 7.77 -> 5.43; 16 rows, K = 64 3.02 -> 3.08, 256 3.46 -> 3.32, 400 3.62 -> 4.07,
+// 1024 6.95 -> 4.62, 2048 9.10 -> 6.44; B stored N x K 8 and 16 rows, K = 1024 8.25 -> 3.19, 9.51 -> 3.85.
+// An A stored K x M goes through LDS, which costs more than it gains for 9 to 16 rows of a B stored
+// K x N (K = 64 3.03 -> 3.39, 256 3.48 -> 3.64, 1024 5.73 -> 6.08, 2048 7.68 -> 8.32) and for
+// few rows and a short K (8 rows, 64 3.02 -> 3.21); it is taken all the same, as the bits are to be
+// the same however A is stored.
+// Up to 8 output columns of a long K run here too, the roles of the operands changed over (LaunchPart);
+// more stay on 16 x 16 tiles.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kThin = 16;
 constexpr uint32_t kThinShortK = 1024;  // up to here 4 wavefronts, else 8
@@ -1761,16 +1764,23 @@ __device__ __forceinline__ float WaveSums16(float (&v)[16], uint32_t lane)
     return v[0] + fromLane(v[0], Xor1{});
 }
 
-// B_K / A_K: that operand is stored with K contiguous.
-template <int MR, bool B_K, bool A_K, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void GemmF32ThinKernel(const GemmF32Args args)
+// B_K / A_K: that operand is stored with K contiguous.  KW wavefronts share K, as many as have any
+// of it up to K = 1024, and GROUPS of them the rows: the same sums in the same order, but a
+// wavefront with all 16 rows holds 64 sums, and its share of an A stored K x M did not fit the
+// registers beside them, so that its pieces were waited for one by one.
+template <int MR, bool B_K, bool A_K, int KW, int GROUPS>
+__global__ __launch_bounds__(KW * GROUPS * 64) void GemmF32ThinKernel(const GemmF32Args args)
 {
+    constexpr int kRows = MR / GROUPS;  // of a wavefront
+    static_assert(kRows == 4 || KW > 1, "sums of one wavefront are handed over");
     // an A stored K x M: 4 rows per lane and one float between the lanes' pieces, so that all
     // lanes read from banks of their own
-    __shared__ float slab[A_K ? 1 : WAVES * 64 * (4 * MR + 1)];
-    __shared__ float partial[WAVES][64];
+    __shared__ float slab[A_K ? 1 : KW * 64 * (4 * MR + 1)];
+    __shared__ float partial[GROUPS][KW][64];
     const uint32_t lane = threadIdx.x & 63;
-    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t wave = GROUPS == 1 ? threadIdx.x >> 6 : (threadIdx.x >> 6) % KW;
+    const uint32_t group = GROUPS == 1 ? 0 : (threadIdx.x >> 6) / KW;
+    const uint32_t row0 = group * kRows;
     // neighbouring columns on one XCD: they share the lines of a B stored K x N
     const uint32_t logical = (blockIdx.x & 7u) * args.perXcd + (blockIdx.x >> 3);
     if (logical >= args.tilesTotal)
@@ -1795,9 +1805,12 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF32ThinKernel(const GemmF32Arg
     }
     const uint32_t M = args.M, N = args.N, K = args.K;
 
-    // wavefront 0 stores sum 4 i + x of lane l = 4 i + x: what it is added to
-    const uint32_t row = lane >> 2, col = x0 + (lane & 3);
-    const bool stores = wave == 0 && row < M && col < N;
+    // a group's wavefront 0 stores sum 4 i + x in lane l = 4 i + x, or in the first of the four lanes
+    // that have it where there are no others; what it is added to:
+    const uint32_t sumOf = KW == 1 ? lane >> 2 : lane;
+    const uint32_t row = row0 + (sumOf >> 2), col = x0 + (sumOf & 3);
+    const bool stores = wave == 0 && (KW == 1 ? (lane & 3) == 0 : lane < 4 * kRows) && row < M &&
+                        col < N;
     const uint32_t outRow = args.mirror ? col : row, outCol = args.mirror ? row : col;
     float* const place = out + static_cast<size_t>(outRow) * args.ldc + outCol;
     float old = 0.f;
@@ -1806,26 +1819,27 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF32ThinKernel(const GemmF32Arg
     else if (stores && !args.overwrite)
         old = *place;
 
-    float acc[MR / 4][16];
+    float acc[kRows / 4][16];
 #pragma unroll
-    for (int g = 0; g < MR / 4; ++g)
+    for (int g = 0; g < kRows / 4; ++g)
 #pragma unroll
         for (int j = 0; j < 16; ++j)
             acc[g][j] = 0.f;
+    auto rowOf = [&](int i) { return min(row0 + static_cast<uint32_t>(i), M - 1); };
 
     const bool wholeQuad = x0 + 4 <= N;
     auto load4 = [](const float* p) { return *reinterpret_cast<const floatx4a4*>(p); };
-    for (uint32_t base = 0; base < K; base += 256 * WAVES)
+    for (uint32_t base = 0; base < K; base += 256 * KW)
     {
         const uint32_t k0 = base + 4 * (wave * 64 + lane);
-        float s[4][4], t[MR][4];  // [x][e], [i][e]: e = k - k0
+        float s[4][4], t[kRows][4];  // [x][e], [i][e]: e = k - k0
 #pragma unroll
         for (int x = 0; x < 4; ++x)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 s[x][e] = 0.f;
 #pragma unroll
-        for (int i = 0; i < MR; ++i)
+        for (int i = 0; i < kRows; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 t[i][e] = 0.f;
@@ -1864,10 +1878,9 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF32ThinKernel(const GemmF32Arg
             if constexpr (A_K)
             {
 #pragma unroll
-                for (int i = 0; i < MR; ++i)
+                for (int i = 0; i < kRows; ++i)
                 {
-                    const floatx4 w =
-                        load4(A + static_cast<size_t>(min(static_cast<uint32_t>(i), M - 1)) * K + k0);
+                    const floatx4 w = load4(A + static_cast<size_t>(rowOf(i)) * K + k0);
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
                         t[i][e] = w[e];
@@ -1889,10 +1902,9 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF32ThinKernel(const GemmF32Arg
                                       : B[static_cast<size_t>(k0 + e) * args.ldb + at];
                     }
 #pragma unroll
-                    for (int i = 0; i < MR && A_K; ++i)
+                    for (int i = 0; i < kRows && A_K; ++i)
                     {
-                        const size_t at = min(static_cast<uint32_t>(i), M - 1);
-                        t[i][e] = A[at * K + k0 + e];
+                        t[i][e] = A[static_cast<size_t>(rowOf(i)) * K + k0 + e];
                     }
                 }
         }
@@ -1900,28 +1912,42 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF32ThinKernel(const GemmF32Arg
         {
             // Rows of M floats that lie one behind the other: read as they lie (pieces of a row per
             // lane would be 64 lines per access), and taken apart by the reads from LDS.
-            const uint32_t floats = min(256u * WAVES, K - base) * M;
-            const float* from = A + static_cast<size_t>(base) * M;
+            // All pieces are requested before the first is put down; those past the end are
+            // the last one again.
+            const uint32_t floats = min(256u * KW, K - base) * M;
             const uint32_t perM = ((1u << 20) + M - 1) / M;  // x / M below
+            const float* from = A + static_cast<size_t>(base) * M;
+            // float 4 q + u goes here: q / M is the lane whose four rows the piece is of
+            auto place = [&](uint32_t q) { return slab + q * 4 + (q * perM >> 20); };
+            constexpr int kPieces = kRows < 8 ? kRows : 8;  // (more do not fit the registers)
             if (base != 0)
                 __syncthreads();
-            for (uint32_t q = threadIdx.x; q * 4 < floats; q += 64 * WAVES)
+#pragma unroll 1
+            for (uint32_t first = threadIdx.x; first < kRows * 64 * KW * GROUPS;
+                 first += kPieces * 64 * KW * GROUPS)
             {
-                // q / M is the lane whose four rows these floats are of
-                float* to = slab + q * 4 + (q * perM >> 20);
-                if (q * 4 + 4 <= floats)
-                {
-                    const floatx4 w = load4(from + q * 4);
+                floatx4 piece[kPieces];
 #pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        to[u] = w[u];
-                }
-                else
+                for (int i = 0; i < kPieces; ++i)
                 {
-                    for (uint32_t u = 0; q * 4 + u < floats; ++u)
-                        to[u] = from[q * 4 + u];
+                    const uint32_t q = first + i * 64 * KW * GROUPS;
+                    piece[i] = load4(from + min(q * 4, floats - 4));
+                }
+#pragma unroll
+                for (int i = 0; i < kPieces; ++i)
+                {
+                    const uint32_t q = first + i * 64 * KW * GROUPS;
+                    if (q * 4 + 4 <= floats)
+                    {
+                        float* to = place(q);
+#pragma unroll
+                        for (int u = 0; u < 4; ++u)
+                            to[u] = piece[i][u];
+                    }
                 }
             }
+            if (threadIdx.x < floats % 4)  // a broken piece at the end
+                place(floats / 4)[threadIdx.x] = from[floats / 4 * 4 + threadIdx.x];
             __syncthreads();
             const float* own = slab + (wave * 64 + lane) * (4 * M + 1);
 #pragma unroll
@@ -1929,35 +1955,45 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF32ThinKernel(const GemmF32Arg
                 if (k0 + e < K)
                 {
 #pragma unroll
-                    for (int i = 0; i < MR; ++i)
-                        t[i][e] = own[e * M + min(static_cast<uint32_t>(i), M - 1)];
+                    for (int i = 0; i < kRows; ++i)
+                        t[i][e] = own[e * M + rowOf(i)];
                 }
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
-            for (int i = 0; i < MR; ++i)
+            for (int i = 0; i < kRows; ++i)
 #pragma unroll
                 for (int x = 0; x < 4; ++x)
                     acc[i / 4][(i % 4) * 4 + x] =
                         fmaf(t[i][e], s[x][e], acc[i / 4][(i % 4) * 4 + x]);
     }
-    // sum j of group g of four rows: lanes 4 j .. 4 j + 3; the one with lane % 4 = g hands it on
-    float mine = 0.f;
-#pragma unroll
-    for (int g = 0; g < MR / 4; ++g)
+    float sum;
+    if constexpr (KW == 1)
     {
-        const float sum = WaveSums16(acc[g], lane);
-        mine = (lane & 3u) == static_cast<uint32_t>(g) ? sum : mine;
+        sum = WaveSums16(acc[0], lane);
+        if (!stores)
+            return;
     }
-    partial[wave][(lane & 3u) * 16 + (lane >> 2)] = mine;
-    __syncthreads();
-    if (!stores)
-        return;
-    float sum = partial[0][lane];
+    else
+    {
+        // sum j of four rows g: lanes 4 j .. 4 j + 3; the one with lane % 4 = g hands it on
+        float mine = 0.f;
 #pragma unroll
-    for (int w = 1; w < WAVES; ++w)
-        sum += partial[w][lane];
+        for (int g = 0; g < kRows / 4; ++g)
+        {
+            const float lanes = WaveSums16(acc[g], lane);
+            mine = (lane & 3u) == static_cast<uint32_t>(g) ? lanes : mine;
+        }
+        partial[group][wave][(lane & 3u) * 16 + (lane >> 2)] = mine;
+        __syncthreads();
+        if (!stores)
+            return;
+        sum = partial[group][0][lane];
+#pragma unroll
+        for (int w = 1; w < KW; ++w)
+            sum += partial[group][w][lane];
+    }
     if (args.bias != nullptr)
         old = 0.f + old;
     const bool fused = args.bias != nullptr || args.relu != 0 || args.sgd != 0;
@@ -2161,25 +2197,54 @@ void LaunchSkinny(const GemmF32Args& args, dim3 grid, uint32_t tile, bool wide, 
         LaunchSkinnyTile<32, TA, TB>(args, grid, wide, stream);
 }
 
-template <bool B_K, bool A_K, int WAVES>
-void LaunchThinRows(const GemmF32Args& args, hipStream_t stream)
+template <int MR, bool B_K, bool A_K, int KW, int GROUPS>
+void LaunchThinAs(const GemmF32Args& args, hipStream_t stream)
 {
-    const dim3 grid(8 * args.perXcd), block(WAVES * 64);
-    if (args.M <= 4)
-        hipLaunchKernelGGL((GemmF32ThinKernel<4, B_K, A_K, WAVES>), grid, block, 0, stream, args);
-    else if (args.M <= 8)
-        hipLaunchKernelGGL((GemmF32ThinKernel<8, B_K, A_K, WAVES>), grid, block, 0, stream, args);
-    else
-        hipLaunchKernelGGL((GemmF32ThinKernel<16, B_K, A_K, WAVES>), grid, block, 0, stream, args);
+    hipLaunchKernelGGL((GemmF32ThinKernel<MR, B_K, A_K, KW, GROUPS>), dim3(8 * args.perXcd),
+                       dim3(KW * GROUPS * 64), 0, stream, args);
 }
 
+// As many wavefronts as have some of K (256 a round each; up to K = 1024 the order of the sums is the
+// same for any number).  Rows in groups where that makes a wavefront's chain shorter than reading
+// B again costs.  1024 columns, A stored M x K / K x M, four wavefronts with all rows before:
+// 16 rows, K = 64 3.57 / 4.14 -> 3.08 / 3.39 us, 256 3.60 / 4.63 -> 3.32 / 3.64,
+// 400 3.98 / 5.28 -> 4.07 / 4.41, 1024 4.60 / 7.51 -> 4.62 / 6.08 (one group 6.50);
+// 8 rows, K = 64 2.98 / 3.48 -> 2.89 / 3.21, 400 3.36 / 4.11 -> 3.33 / 4.05, 1024 3.96 / 5.33 -> 3.96 / 4.79.
 template <bool B_K, bool A_K>
 void LaunchThin(const GemmF32Args& args, hipStream_t stream)
 {
-    if (args.K > kThinShortK)
-        LaunchThinRows<B_K, A_K, 8>(args, stream);
+    const uint32_t K = args.K;
+    if (args.M <= 4)
+    {
+        if (K <= 256)
+            LaunchThinAs<4, B_K, A_K, 1, 1>(args, stream);
+        else if (K <= kThinShortK)
+            LaunchThinAs<4, B_K, A_K, 4, 1>(args, stream);
+        else
+            LaunchThinAs<4, B_K, A_K, 8, 1>(args, stream);
+    }
+    else if (args.M <= 8)
+    {
+        if (K <= 256)
+            LaunchThinAs<8, B_K, A_K, 1, 2>(args, stream);
+        else if (K <= 512)
+            LaunchThinAs<8, B_K, A_K, 2, 1>(args, stream);
+        else if (K <= kThinShortK)
+            LaunchThinAs<8, B_K, A_K, 4, 1>(args, stream);
+        else
+            LaunchThinAs<8, B_K, A_K, 8, 1>(args, stream);
+    }
     else
-        LaunchThinRows<B_K, A_K, 4>(args, stream);
+    {
+        if (K <= 256)
+            LaunchThinAs<16, B_K, A_K, 1, 4>(args, stream);
+        else if (K <= 512)
+            LaunchThinAs<16, B_K, A_K, 2, 2>(args, stream);
+        else if (K <= kThinShortK)
+            LaunchThinAs<16, B_K, A_K, 4, A_K ? 1 : 2>(args, stream);
+        else
+            LaunchThinAs<16, B_K, A_K, 8, 1>(args, stream);
+    }
 }
 
 // Products whose sums are taken in parts: an M or N that is no multiple of 4.  Their last rows and
