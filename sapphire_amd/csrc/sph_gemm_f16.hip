@@ -1276,7 +1276,11 @@ constexpr int kSStages = 4;
 constexpr int kSOperandBytes = kS * kSK * 2;        // 8 KiB
 constexpr int kSStageBytes = 2 * kSOperandBytes;    // A + B
 
-template <bool TA, bool TB, bool TAIL>
+// PARTS: M or N is no multiple of 8.  Four sums, one per quarter of a slab, added up at the end: such
+// products, or their last rows and columns, used to be the few-tile kernel's, which adds four parts,
+// and one chain of K / 16 instructions has 1.2 to 2.2 times its error (402 x 502 x 702 1.70e-7 of a
+// sum's size against 0.97e-7, with four sums 0.97e-7; 5.92 -> 6.14 us, few-tile kernel 8.07).
+template <bool TA, bool TB, bool TAIL, bool PARTS>
 __global__ __launch_bounds__(256, 2) void GemmF16Dma64(const GemmF16Args args,
                                                     const GemmF16Strips strips)
 {
@@ -1343,7 +1347,9 @@ __global__ __launch_bounds__(256, 2) void GemmF16Dma64(const GemmF16Args args,
     const size_t aStepBytes = TA ? static_cast<size_t>(kSK) * args.lda * 2 : kSK * 2;
     const size_t bStepBytes = TB ? kSK * 2 : static_cast<size_t>(kSK) * pitchB * 2;
     const uint32_t ldsBase = LdsAddress(lds);
-    const uint32_t steps = TAIL ? K / kSK + 1 : K / kSK;
+    // (written so that it cannot be 0: the loop is otherwise laid out for that, with a copy of the
+    // sums in every step, and spills with four of them)
+    const uint32_t steps = TAIL ? K / kSK + 1 : (K - 1) / kSK + 1;
     // the last window starts K % 64 values of k after the one before it
     const uint32_t kLast = K % kSK;
     const size_t aLastBytes = TA ? static_cast<size_t>(kLast) * args.lda * 2 : kLast * 2;
@@ -1421,10 +1427,8 @@ __global__ __launch_bounds__(256, 2) void GemmF16Dma64(const GemmF16Args args,
             return readKMajor(stage + bOff[ks]);
     };
 
-    floatx16 acc;
-#pragma unroll
-    for (int v = 0; v < 16; ++v)
-        acc[v] = 0.f;
+    constexpr int kSums = PARTS ? 4 : 1;
+    floatx16 part[kSums] = {};
 
     // TAIL: the positions of the last slab whose k the step before has multiplied are cleared
     // in LDS, by the lane that copied them, once the copies have landed and before the barrier
@@ -1485,7 +1489,8 @@ __global__ __launch_bounds__(256, 2) void GemmF16Dma64(const GemmF16Args args,
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks)
         {
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(PB[ks], PA[ks], acc, 0, 0, 0);
+            floatx16& sum = part[ks % kSums];
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(PB[ks], PA[ks], sum, 0, 0, 0);
             if (ks == 0)
             {
                 WaitVmem<(kSStages - 3) * kCopies>();
@@ -1523,6 +1528,9 @@ __global__ __launch_bounds__(256, 2) void GemmF16Dma64(const GemmF16Args args,
         step(std::integral_constant<uint32_t, 3>{}, s0 + 3, af[1], bf[1], af[0], bf[0]);
     }
     WaitVmem<0>();  // the surplus copies of the last steps still target LDS
+    floatx16 acc = part[0];
+    if constexpr (PARTS)
+        acc = (part[0] + part[1]) + (part[2] + part[3]);
 
     // ---- epilogue: lane holds row l % 32 of its block, columns 8 q + 4 (l / 32) + 0..3 ----------
     auto epilogue = [&](auto whole) {
@@ -2217,14 +2225,21 @@ int LaunchF16Kernel(GemmF16Args args, uint32_t batch, F16Kernel kind, const F16L
         args.totalTiles = static_cast<uint32_t>(tiles);
         strips.first = ((args.totalTiles + 7) / 8) * 8;
         const dim3 g(strips.first + strips.blocks[0] + strips.blocks[1]), b(256);
+        const bool parts = M % 8 != 0 || N % 8 != 0;
         const bool tail = K % kSK != 0;
+#define SPH_DMA64_(TA_, TB_, TAIL_, PARTS_)                                                       \
+    hipLaunchKernelGGL((GemmF16Dma64<TA_, TB_, TAIL_, PARTS_>), g, b, 0, stream, args, strips)
 #define SPH_DMA64(TA_, TB_)                                                                       \
     do                                                                                            \
     {                                                                                             \
-        if (tail)                                                                                 \
-            hipLaunchKernelGGL((GemmF16Dma64<TA_, TB_, true>), g, b, 0, stream, args, strips);            \
+        if (parts && tail)                                                                        \
+            SPH_DMA64_(TA_, TB_, true, true);                                                     \
+        else if (parts)                                                                           \
+            SPH_DMA64_(TA_, TB_, false, true);                                                    \
+        else if (tail)                                                                            \
+            SPH_DMA64_(TA_, TB_, true, false);                                                    \
         else                                                                                      \
-            hipLaunchKernelGGL((GemmF16Dma64<TA_, TB_, false>), g, b, 0, stream, args, strips);           \
+            SPH_DMA64_(TA_, TB_, false, false);                                                   \
     } while (0)
         if (transA && transB)
             SPH_DMA64(true, true);
@@ -2235,6 +2250,7 @@ int LaunchF16Kernel(GemmF16Args args, uint32_t batch, F16Kernel kind, const F16L
         else
             SPH_DMA64(false, false);
 #undef SPH_DMA64
+#undef SPH_DMA64_
     }
     else if (kind == F16Kernel::kDma128)
     {
