@@ -922,9 +922,14 @@ __device__ __forceinline__ void StoreQuad(float* p, const float4& v, uint32_t c,
 
 // TAIL: K = 32 q + r, 0 < r < 32: a last step over the window [K - 32, K) whose slab has the
 // positions of the 32 - r values of k already multiplied cleared in LDS.
-template <bool TA, bool TB, bool TAIL, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void GemmF16Dma128(const GemmF16Args args,
-                                                            const GemmF16Strips strips)
+// PARTS: N (M of an A stored K x M) is no multiple of 8.  The last columns (rows), once strips of
+// the few-tile kernel, which adds four or eight parts, had twice the error in one chain of K / 16
+// instructions (2048 x 1533 x 1024 2.05e-7 of a sum's size against 0.94e-7).  All of them are now four
+// sums, one per half of every second slab, with eight wavefronts (1.1e-7), and two, one per half
+// slab, with four, whose registers hold no more (1.4e-7).
+template <bool TA, bool TB, bool TAIL, int WAVES, bool PARTS>
+__global__ __launch_bounds__(WAVES * 64, PARTS ? 2 : 1) void GemmF16Dma128(
+    const GemmF16Args args, const GemmF16Strips strips)
 {
     static_assert(WAVES == 4 || WAVES == 8, "2 x 2 or 2 x 4 wavefronts");
     constexpr int WN = WAVES / 2;          // wavefronts across the tile
@@ -1086,14 +1091,9 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF16Dma128(const GemmF16Args ar
         }
     };
 
-    floatx16 acc[2][TN];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v)
-                acc[i][j][v] = 0.f;
+    constexpr uint32_t kSums = !PARTS ? 1 : WAVES == 8 ? 4 : 2;
+    floatx16 part[kSums][2][TN] = {};
+    floatx16 (&acc)[2][TN] = part[0];
     // TAIL: the positions of the last slab whose k the step before has multiplied are cleared
     // in LDS, by the lane that copied them, once the copies have landed and before the barrier
     // that publishes the stage, so the steps themselves carry no masks (1024 x 1024 x 784:
@@ -1123,28 +1123,31 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF16Dma128(const GemmF16Args ar
         if (!TB && bBack != 0)
             MoveLastChunk(stage + kBytesA + at, bBack);
     };
-    auto multiply = [&](const halfx8 (&af)[2], const halfx8 (&bf)[TN]) {
+    // `half`: the half slab's number, counted from any multiple of kSums
+    auto multiply = [&](const halfx8 (&af)[2], const halfx8 (&bf)[TN], uint32_t half) {
+        floatx16 (&sum)[2][TN] = part[half % kSums];
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
-                acc[i][j] =
-                    __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[j], af[i], acc[i][j], 0, 0, 0);
+                sum[i][j] =
+                    __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[j], af[i], sum[i][j], 0, 0, 0);
     };
 
     // First half of a step.  The step's housekeeping sits between its MFMAs, where the matrix
     // pipe is already busy: behind the first one the wait for the copies of step st+1 and the
     // barrier, behind every one a copy of step st+3.
     static_assert(kDCopies == 2 * TN, "one copy behind every MFMA of the first half");
-    auto multiplyAndFeed = [&](const halfx8 (&af)[2], const halfx8 (&bf)[TN], uint32_t fillStage,
-                               bool nextIsLast, char* next) {
+    auto multiplyAndFeed = [&](const halfx8 (&af)[2], const halfx8 (&bf)[TN], uint32_t half,
+                               uint32_t fillStage, bool nextIsLast, char* next) {
+        floatx16 (&sum)[2][TN] = part[half % kSums];
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
             {
-                acc[i][j] =
-                    __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[j], af[i], acc[i][j], 0, 0, 0);
+                sum[i][j] =
+                    __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[j], af[i], sum[i][j], 0, 0, 0);
                 if (i == 0 && j == 0)
                 {
                     // steps up to st+1 have landed once at most one later step is pending;
@@ -1196,16 +1199,25 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF16Dma128(const GemmF16Args ar
             char* next = lds + ((u + 1) % kDStages) * kDStageBytes;
             loadFragments(af[1], bf[1], cur, 1);
             __builtin_amdgcn_sched_barrier(0);
-            multiplyAndFeed(af[0], bf[0], (u + kDStages - 1) % kDStages,
+            multiplyAndFeed(af[0], bf[0], 2 * u, (u + kDStages - 1) % kDStages,
                             s0 + u + 2 == steps, next);
             __builtin_amdgcn_sched_barrier(0);
             loadFragments(af[0], bf[0], next, 0);
             __builtin_amdgcn_sched_barrier(0);
-            multiply(af[1], bf[1]);
+            multiply(af[1], bf[1], 2 * u + 1);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
     WaitVmem<0>();  // the surplus copies of the last steps still target LDS
+#pragma unroll
+    for (uint32_t step = 1; step < kSums; step *= 2)
+#pragma unroll
+        for (uint32_t s = 0; s < kSums; s += 2 * step)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    part[s][i][j] += part[s + step][i][j];
 
     // ---- epilogue: lane holds row l%32 of a block, columns 8q + 4*(l/32) + 0..3 -----------
     auto epilogue = [&](auto whole) {
@@ -2263,23 +2275,28 @@ int LaunchF16Kernel(GemmF16Args args, uint32_t batch, F16Kernel kind, const F16L
         const bool wide = args.totalTiles <= static_cast<uint32_t>(sph::ComputeUnits());
         const dim3 g(grid);
         const bool tail = K % kTK != 0;
-#define SPH_DMA128_(TA_, TB_, TAIL_)                                                              \
+        const bool parts = N % 8 != 0 || (transA && M % 8 != 0);
+#define SPH_DMA128_(TA_, TB_, TAIL_, PARTS_)                                                      \
     do                                                                                            \
     {                                                                                             \
         if (wide)                                                                                 \
-            hipLaunchKernelGGL((GemmF16Dma128<TA_, TB_, TAIL_, 8>), g, dim3(512), 0, stream,      \
-                               args, strips);                                                             \
+            hipLaunchKernelGGL((GemmF16Dma128<TA_, TB_, TAIL_, 8, PARTS_>), g, dim3(512), 0,      \
+                               stream, args, strips);                                             \
         else                                                                                      \
-            hipLaunchKernelGGL((GemmF16Dma128<TA_, TB_, TAIL_, 4>), g, dim3(256), 0, stream,      \
-                               args, strips);                                                             \
+            hipLaunchKernelGGL((GemmF16Dma128<TA_, TB_, TAIL_, 4, PARTS_>), g, dim3(256), 0,      \
+                               stream, args, strips);                                             \
     } while (0)
 #define SPH_DMA128(TA_, TB_)                                                                      \
     do                                                                                            \
     {                                                                                             \
-        if (tail)                                                                                 \
-            SPH_DMA128_(TA_, TB_, true);                                                          \
+        if (tail && parts)                                                                        \
+            SPH_DMA128_(TA_, TB_, true, true);                                                    \
+        else if (tail)                                                                            \
+            SPH_DMA128_(TA_, TB_, true, false);                                                   \
+        else if (parts)                                                                           \
+            SPH_DMA128_(TA_, TB_, false, true);                                                   \
         else                                                                                      \
-            SPH_DMA128_(TA_, TB_, false);                                                         \
+            SPH_DMA128_(TA_, TB_, false, false);                                                  \
     } while (0)
         if (transA && transB)
             SPH_DMA128(true, true);

@@ -46,3 +46,13 @@ def check(shape, chains):
                                    (130, 1000, 1001), (900, 901, 903)])
 def test_64_tiles(dev, shape):
     check(shape, 4)
+
+
+@pytest.mark.parametrize("shape", [(2048, 1533, 1024), (2001, 1507, 999)])
+def test_128_tiles_eight_wavefronts(dev, shape):
+    check(shape, 4)
+
+
+@pytest.mark.parametrize("shape", [(2561, 1701, 1001), (2500, 1803, 640)])
+def test_128_tiles_four_wavefronts(dev, shape):
+    check(shape, 2)
