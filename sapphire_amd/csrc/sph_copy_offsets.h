@@ -1,0 +1,53 @@
+// Where the tiled GEMM kernels copy the chunks of an operand stored k-major from, when its rows are no
+// whole number of chunks.  One definition for the kernels and for the host, so that the CPU tests
+// see that no copy reaches past an operand: what it would bring feeds no output and shows in none.
+//
+// A row's last chunk reaches into the next row, whose values only feed outputs that are not
+// stored.  In the last row of the matrix there is none; the chunk begins earlier there, so that it
+// ends with the row.  Chunks past a row's end copy its last whole chunk.
+#ifndef SPH_COPY_OFFSETS_H
+#define SPH_COPY_OFFSETS_H
+
+#include <cstdint>
+
+#if defined(__HIPCC__)
+#define SPH_COPY_INLINE __host__ __device__ inline __attribute__((always_inline))
+#else
+#define SPH_COPY_INLINE inline
+#endif
+
+namespace sph
+{
+struct KMajorPlace
+{
+    uint32_t k, column;
+};
+
+// fp32, chunks of 4: where the chunk for column x of row k of a slab is copied from.  `valid` rows of
+// the slab exist (those past them copy the first one); `ending`: its last one is the matrix's.
+// limit >= 4 columns.
+SPH_COPY_INLINE KMajorPlace QuadPlace(uint32_t k, uint32_t x, uint32_t limit, uint32_t valid,
+                                      bool ending)
+{
+    if (k >= valid)
+        k = 0;
+    const uint32_t last = limit - 4;
+    const bool clamp = x >= limit || (ending && k + 1 == valid);
+    return { k, clamp && x > last ? last : x };
+}
+
+// fp16, chunks of 8 (x a multiple of 8, limit >= 8): the first column a chunk is copied from, in every
+// row but the last of the matrix
+SPH_COPY_INLINE uint32_t ChunkColumn(uint32_t x, uint32_t limit)
+{
+    return x < limit ? x : limit - 8;
+}
+
+// ... and the bytes by which it has to begin earlier there
+SPH_COPY_INLINE uint32_t LastChunkBack(uint32_t x, uint32_t limit)
+{
+    return x < limit && x + 8 > limit ? (x + 8 - limit) * 2 : 0u;
+}
+}  // namespace sph
+
+#endif

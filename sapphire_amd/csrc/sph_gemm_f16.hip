@@ -55,6 +55,7 @@
 // kernel, whose copies' 8 columns have to lie inside the row, the last N % 8 columns (M % 8 rows of
 // an A stored K x M) go to the code of GemmF16Few, as do up to 16 rows or columns just past a tile
 // edge: as strips on the last workgroups of the body's own launch (LaunchF16).
+#include "sph_copy_offsets.h"
 #include "sph_internal.h"
 #include "sph_k_partition.h"
 
@@ -871,19 +872,6 @@ constexpr int kD = 128;
 constexpr int kDStages = 4;
 constexpr int kDStageBytes = 2 * kD * kTK * 2;  // A + B
 
-// First of the 8 columns a lane copies for chunk `x` (a multiple of 8) of a k-major row of `limit`
-// >= 8 columns: chunks past the edge copy the row's last 8.
-__device__ __forceinline__ uint32_t ChunkColumn(uint32_t x, uint32_t limit)
-{
-    return x < limit ? x : limit - 8;
-}
-
-// Bytes by which that chunk, in the last row of the matrix, has to begin earlier.
-__device__ __forceinline__ uint32_t LastChunkBack(uint32_t x, uint32_t limit)
-{
-    return x < limit && x + 8 > limit ? (x + 8 - limit) * 2 : 0u;
-}
-
 // What was copied `back` bytes too early to its place; what follows belongs to no column.
 __device__ __forceinline__ void MoveLastChunk(char* chunk, uint32_t back)
 {
@@ -974,14 +962,14 @@ __global__ __launch_bounds__(WAVES * 64, PARTS ? 2 : 1) void GemmF16Dma128(
         const uint32_t k = j * 4 + (lane >> 4);
         const uint32_t phys16 = lane & 15;
         const uint32_t logical16 = (((phys16 >> 1) ^ (2 * (k & 3))) << 1) | (phys16 & 1);
-        return (k * pitch + ChunkColumn(xBase + logical16 * 8, limit)) * 2u;
+        return (k * pitch + sph::ChunkColumn(xBase + logical16 * 8, limit)) * 2u;
     };
     // ... and what its chunk of the last k-row begins earlier by
     auto laneBack = [&](uint32_t j, uint32_t xBase, uint32_t limit) {
         const uint32_t k = j * 4 + (lane >> 4);
         const uint32_t phys16 = lane & 15;
         const uint32_t logical16 = (((phys16 >> 1) ^ (2 * (k & 3))) << 1) | (phys16 & 1);
-        return k == kTK - 1 ? LastChunkBack(xBase + logical16 * 8, limit) : 0u;
+        return k == kTK - 1 ? sph::LastChunkBack(xBase + logical16 * 8, limit) : 0u;
     };
     uint32_t aLane[kCopiesPer], bLane[kCopiesPer], aDst[kCopiesPer], bDst[kCopiesPer];
 #pragma unroll
@@ -1333,12 +1321,12 @@ __global__ __launch_bounds__(256, 2) void GemmF16Dma64(const GemmF16Args args,
     auto laneKMajor = [&](uint32_t j, uint32_t xBase, uint32_t limit, uint32_t pitch) {
         const uint32_t k = j * 8 + (lane >> 3);
         const uint32_t logical16 = (lane & 7) ^ (((k >> 1) & 1) << 2);
-        return (k * pitch + ChunkColumn(xBase + logical16 * 8, limit)) * 2u;
+        return (k * pitch + sph::ChunkColumn(xBase + logical16 * 8, limit)) * 2u;
     };
     auto laneBack = [&](uint32_t j, uint32_t xBase, uint32_t limit) {
         const uint32_t k = j * 8 + (lane >> 3);
         const uint32_t logical16 = (lane & 7) ^ (((k >> 1) & 1) << 2);
-        return k == kSK - 1 ? LastChunkBack(xBase + logical16 * 8, limit) : 0u;
+        return k == kSK - 1 ? sph::LastChunkBack(xBase + logical16 * 8, limit) : 0u;
     };
     const uint32_t pitchB = TB ? K : args.ldb;
     uint32_t aLane[kCopiesPer], bLane[kCopiesPer], aDst[kCopiesPer], bDst[kCopiesPer];

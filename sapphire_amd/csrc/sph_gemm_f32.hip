@@ -35,6 +35,7 @@
 // result may overwrite out or take a bias row and a ReLU in the epilogue, and units come from
 // (batch, stride) arithmetic -- stride 0 repeats an operand -- or from a table of element
 // offsets in device memory.
+#include "sph_copy_offsets.h"
 #include "sph_internal.h"
 #include "sph_k_partition.h"
 
@@ -812,15 +813,9 @@ GemmF32DmaKernel(const GemmF32Args args, const GemmF32Strips strips)
                                  uint32_t rowBytes, uint32_t valid, bool ending,
                                  auto rowAtPosition) {
         const uint32_t b = j * 1024 + lane * 16;  // byte inside the unpadded slab
-        uint32_t k = rowAtPosition(b / rowBytes);
-        if (k >= valid)
-            k = 0;
-        uint32_t gx = xBase + (b % rowBytes) / 4;
-        // chunks past the edge copy the row's last 4 floats; so does one that reaches past it in
-        // the last row of the matrix
-        if (gx >= limit || (ending && k + 1 == valid))
-            gx = min(gx, limit - 4);
-        return (k * pitch + gx) * 4u + kTailBias;
+        const sph::KMajorPlace from = sph::QuadPlace(
+            rowAtPosition(b / rowBytes), xBase + (b % rowBytes) / 4, limit, valid, ending);
+        return (from.k * pitch + from.column) * 4u + kTailBias;
     };
     auto locate = [&](uint32_t logicalTile, Place& p) {
         uint32_t tm, tn, unit;

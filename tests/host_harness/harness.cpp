@@ -18,6 +18,7 @@
 
 #include <sapphire_hip.h>
 #include <sph_column_walk.h>
+#include <sph_copy_offsets.h>
 #include <sph_k_partition.h>
 #include <sph_spgemm_plan.h>
 
@@ -282,6 +283,55 @@ unsigned sphh_k_partition_slot(unsigned K, unsigned groupK, unsigned waves, unsi
 {
     const sph::KPartition p = sph::PartitionK(K, groupK, waves, wave, depth);
     return g == 0xffffffffu ? sph::KPartitionFirst(p, d) : sph::KPartitionNext(p, g, depth, d);
+}
+
+// The copies of an operand stored k-major, K rows of `limit` columns (sapphire_amd/csrc/
+// sph_copy_offsets.h): how far past its end the farthest one reaches, in elements (0 or less: none
+// does), over all slabs of `bk` rows and tiles of `tile` columns.  No device is touched.
+// fp32: the last slab holds what is left of K.  `always`: its form for the matrix's last row is on.
+int sphh_quad_copies_reach(unsigned K, unsigned limit, unsigned bk, unsigned tile, int always,
+                           long long* out)
+{
+    const std::uint32_t steps = (K + bk - 1) / bk;
+    const bool tail = always != 0 || K % bk != 0;
+    const long long end = static_cast<long long>(K) * limit;
+    long long most = -end;
+    for (std::uint32_t s = 0; s < steps; ++s)
+        for (std::uint32_t k = 0; k < bk; ++k)
+            for (std::uint32_t x = 0; x < (limit + tile - 1) / tile * tile; x += 4)
+            {
+                const bool last = tail && s + 1 == steps;
+                const sph::KMajorPlace p =
+                    sph::QuadPlace(k, x, limit, last ? K - s * bk : bk, last);
+                const long long at = static_cast<long long>(s * bk + p.k) * limit + p.column;
+                most = std::max(most, at + 4 - end);
+                // what feeds an output comes from its own place, or ends with the row
+                if (s * bk + k < K && x < limit && (p.k != k || (p.column != x && !last)))
+                    return 1;
+            }
+    *out = most;
+    return 0;
+}
+
+// fp16: the last slab is the window [K - bk, K), whose last row is the matrix's.
+int sphh_chunk_copies_reach(unsigned K, unsigned limit, unsigned bk, unsigned tile, long long* out)
+{
+    const std::uint32_t steps = (K + bk - 1) / bk;
+    const long long end = static_cast<long long>(K) * limit;
+    long long most = -end;
+    for (std::uint32_t s = 0; s < steps; ++s)
+        for (std::uint32_t k = 0; k < bk; ++k)
+            for (std::uint32_t x = 0; x < (limit + tile - 1) / tile * tile; x += 8)
+            {
+                const bool last = s + 1 == steps;
+                const std::uint32_t row = (last ? K - bk : s * bk) + k;
+                long long at = static_cast<long long>(row) * limit + sph::ChunkColumn(x, limit);
+                if (last && k + 1 == bk)
+                    at -= sph::LastChunkBack(x, limit) / 2;
+                most = std::max(most, at + 8 - end);
+            }
+    *out = most;
+    return 0;
 }
 
 // The walk over a row's columns (sapphire_amd/csrc/sph_column_walk.h): out receives the columns

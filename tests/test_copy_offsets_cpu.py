@@ -1,0 +1,34 @@
+"""Where the tiled GEMM kernels copy the chunks of an operand stored k-major from
+(sapphire_amd/csrc/sph_copy_offsets.h, reached through the host harness): no copy of any slab reaches
+past the operand, whatever its width; no device is needed."""
+import ctypes
+
+import pytest
+
+from tests import host_layer as hl
+
+
+def reach(name, *args):
+    out = ctypes.c_longlong()
+    assert getattr(hl.lib(), name)(*args, ctypes.byref(out)) == 0
+    return out.value
+
+
+# fp32 kernels: (K step, tile edge)
+@pytest.mark.parametrize("bk,tile", [(32, 64), (32, 32), (16, 128)])
+def test_fp32_quads_end_with_the_operand(bk, tile):
+    for limit in [4, 5, 6, 7, 8, 9, 31, 33, 61, 63, 64, 65, 66, 67, 127, 128, 129, 130, 131, 255]:
+        for K in [16, 17, 19, 31, 32, 33, 47, 48, 63, 64, 65, 95, 96, 97, 100]:
+            got = reach("sphh_quad_copies_reach", K, limit, bk, tile, 1)
+            # exactly to the end: the last row's last chunk is there
+            assert got == 0, (limit, K)
+            if limit % 4 == 0:  # the kernels without a last step of its own
+                assert reach("sphh_quad_copies_reach", K, limit, bk, tile, 0) == 0, (limit, K)
+
+
+# fp16 kernels: (K step, tile edge, fewest slabs of broken rows)
+@pytest.mark.parametrize("bk,tile", [(64, 64), (32, 128)])
+def test_fp16_chunks_end_with_the_operand(bk, tile):
+    for limit in list(range(8, 26)) + [57, 63, 64, 65, 121, 127, 128, 129, 135, 255]:
+        for K in [2 * bk, 2 * bk + 1, 3 * bk - 1, 3 * bk, 3 * bk + 7, 5 * bk + 33]:
+            assert reach("sphh_chunk_copies_reach", K, limit, bk, tile) == 0, (limit, K)

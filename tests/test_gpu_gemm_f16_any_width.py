@@ -1,8 +1,10 @@
 """fp16-input GEMM on the 64- and 128-tile kernels with rows that are no whole number of 8 halves:
-the last chunk of a k-major operand's last row must not be read past the matrix.
+the last chunk of a k-major operand's last row is copied early and moved to its place.
 
 Integer-valued operands make every product and partial sum exact, so the result is compared bit
 for bit with the CPU loop; out lies between guard words, and in one test NaN behind the operands.
+That no copy reaches past an operand is not visible here (what it would bring feeds no output):
+test_copy_offsets_cpu.py checks the offsets.
 """
 import numpy as np
 import pytest

@@ -1,8 +1,10 @@
 """fp32 GEMM on the straight-to-LDS kernels with rows that are no whole number of 4 floats: the
-last chunk of a k-major operand's last row must not be read past the matrix.
+last chunk of a k-major operand's last row is copied early and its values are read from there.
 
 Integer-valued operands make every product and partial sum exact, so the result is compared bit
 for bit with the CPU loop; out lies between guard words, and in one test NaN behind the operands.
+That no copy reaches past an operand is not visible here (what it would bring feeds no output):
+test_copy_offsets_cpu.py checks the offsets.
 """
 import numpy as np
 import pytest
