@@ -24,9 +24,10 @@
 //   GemmF32SkinnyKernel  few output tiles: 16 x 16 or 32 x 32 tiles with K split over the
 //                        wavefronts of a workgroup;
 //   GemvRowKernel        a single output row.
-// A product for the tiled kernels is cut by the launcher into a body and up to two thin strips of
-// up to 16 rows or columns just past a tile edge where that saves a round of tiles.  The strips are computed by the few-tile kernel's code on the last
-// workgroups of the body's own launch (GemmF32Strips), or by launches of their own beside a
+// A product for the tiled kernels is cut by the launcher into a body and up to two thin strips
+// where that saves a round of tiles (up to 16 rows or columns just past a tile edge) or, beside
+// idle compute units, the last step.  The strips are computed by the few-tile kernel's code on the
+// last workgroups of the body's own launch (GemmF32Strips), or by launches of their own beside a
 // register-staged body.
 // The first two share one decomposition: a workgroup (4 wavefronts, 2 x 2) owns a BM x BN tile
 // of one M x N unit, BM = BN = 128 or 64 (whichever loads the busiest compute unit less),
@@ -77,7 +78,6 @@ struct GemmF32Args
     uint32_t tilesTotal;  // tilesM * tilesN * units
     uint32_t perXcd;      // ceil(tilesTotal / 8): the grid has 8 * perXcd workgroups
     uint32_t band;        // tile rows per band of the in-unit ordering
-    uint32_t outVec;     // 16-byte accesses to out are possible
     uint32_t overwrite;  // out = A*B instead of out += A*B
     uint32_t relu;       // out = max(., 0) applied to the value that is stored
     const float* bias;   // when set: out = (0 + bias[column]) + A*B, out is not read
@@ -1711,7 +1711,7 @@ __global__ __launch_bounds__(WAVES * 64) void GemmF32SkinnyKernel(const GemmF32A
 // more stay on 16 x 16 tiles.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kThin = 16;
-constexpr uint32_t kThinShortK = 1024;  // up to here 4 wavefronts, else 8
+constexpr uint32_t kThinShortK = 1024;  // up to here one round of four wavefronts, else of eight
 constexpr uint32_t kThinColumns = 8, kThinColumnsK = 1024;  // few columns instead (LaunchPart)
 
 // Sum over the 64 lanes of 16 values per lane; lane l ends up with the sum of value l / 4.
@@ -2432,18 +2432,14 @@ int LaunchStrip(const GemmF32Args& strip, uint32_t blocks, bool transA, bool tra
 // A thin strip of a product's last rows or columns: 16 x 16 tiles of the few-tile kernel on four
 // wavefronts, whether it then rides along with the body's launch (`pending` has room) or is
 // launched on its own, so that its bits do not depend on which.
-int AddStrip(GemmF32Args strip, uint32_t units, bool outOffsetsAligned, bool transA, bool transB,
-             GemmF32Strips* pending, hipStream_t stream)
+int AddStrip(GemmF32Args strip, uint32_t units, bool transA, bool transB, GemmF32Strips* pending,
+             hipStream_t stream)
 {
     strip.tilesM = (strip.M + 15) / 16;
     strip.tilesN = (strip.N + 15) / 16;
     const uint64_t blocks = static_cast<uint64_t>(strip.tilesM) * strip.tilesN * units;
     if (blocks >= (1ull << 30))
         return sph::Fail(SPH_ERR_INVALID, "sph_gemm_f32 - too many tiles for one launch");
-    strip.outVec = (outOffsetsAligned && (strip.N % 4 == 0) && (strip.ldc % 4 == 0) &&
-                    (reinterpret_cast<uintptr_t>(strip.out) & 15u) == 0)
-                       ? 1u
-                       : 0u;
     for (int i = 0; i < 2 && pending != nullptr; ++i)
         if (pending->blocks[i] == 0)
         {
@@ -2457,8 +2453,8 @@ int AddStrip(GemmF32Args strip, uint32_t units, bool outOffsetsAligned, bool tra
 // `transA`: A is stored K x M; `transB`: B is stored N x K.
 // `pending`: strips waiting for a launch to ride along with; a launch that takes them empties
 // the list.
-int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool outOffsetsAligned,
-               bool transA, bool transB, GemmF32Strips* pending, hipStream_t stream)
+int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool transA, bool transB,
+               GemmF32Strips* pending, hipStream_t stream)
 {
     GemmF32Args args = base;
     if (args.split == 0)
@@ -2494,7 +2490,8 @@ int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool o
     // from anywhere); every output element is still computed once.  Cut off are up to 16 rows or
     // columns past a multiple of the tile edge, when the compute unit with the most tiles then has
     // fewer of them (1025^3: 17 x 17 tiles of 64 are two per compute unit somewhere, 16 x 16 one
-    // everywhere; measured 44.8 -> 23.4 us).
+    // everywhere; measured 44.8 -> 23.4 us), and M % 4 rows or N % 4 columns where that is free
+    // (CutCost).
     // The cut depends on M, N, K and the batch only, not on how the operands are stored or
     // aligned, so a product's bits do not depend on that either.
     if (whole && (args.split & 4u) != 0 && args.M > 1 && args.K >= kBK)
@@ -2543,8 +2540,7 @@ int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool o
                 bottom.M = peelM;
                 bottom.A = args.A + (transA ? body.M : static_cast<size_t>(body.M) * args.K);
                 bottom.out = args.out + static_cast<size_t>(body.M) * args.ldc;
-                const int rc = AddStrip(bottom, units, outOffsetsAligned, transA, transB, pending,
-                                        stream);
+                const int rc = AddStrip(bottom, units, transA, transB, pending, stream);
                 if (rc != SPH_OK)
                     return rc;
             }
@@ -2559,13 +2555,11 @@ int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool o
                 right.out = args.out + body.N;
                 if (args.bias != nullptr)
                     right.bias = args.bias + body.N;
-                const int rc = AddStrip(right, units, outOffsetsAligned, transA, transB, pending,
-                                        stream);
+                const int rc = AddStrip(right, units, transA, transB, pending, stream);
                 if (rc != SPH_OK)
                     return rc;
             }
-            return LaunchPart(body, units, allowVector, outOffsetsAligned, transA, transB, pending,
-                              stream);
+            return LaunchPart(body, units, allowVector, transA, transB, pending, stream);
         }
     }
     // few 64 x 64 tiles and a long K: the kernel that splits K inside the workgroup (decided on
@@ -2575,10 +2569,6 @@ int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool o
     const bool fewTiles = (args.split & 4u) == 0 &&
                           tiles64 * 2 <= static_cast<uint64_t>(sph::ComputeUnits()) &&
                           args.K >= 64;
-    args.outVec = (outOffsetsAligned && (args.N % 4 == 0) && (args.ldc % 4 == 0) &&
-                   (reinterpret_cast<uintptr_t>(args.out) & 15u) == 0)
-                      ? 1u
-                      : 0u;
     // (of this launch: a part of a wider product may start anywhere)
     const bool basesAligned =
         ((reinterpret_cast<uintptr_t>(args.A) | reinterpret_cast<uintptr_t>(args.B)) & 15u) == 0;
@@ -2755,12 +2745,11 @@ int LaunchPart(const GemmF32Args& base, uint32_t units, bool allowVector, bool o
     return SPH_OK;
 }
 
-int Launch(const GemmF32Args& base, uint32_t units, bool allowVector, bool outOffsetsAligned,
-           bool transA, bool transB, hipStream_t stream)
+int Launch(const GemmF32Args& base, uint32_t units, bool allowVector, bool transA, bool transB,
+           hipStream_t stream)
 {
     GemmF32Strips pending{};
-    int rc = LaunchPart(base, units, allowVector, outOffsetsAligned, transA, transB, &pending,
-                        stream);
+    int rc = LaunchPart(base, units, allowVector, transA, transB, &pending, stream);
     // strips no launch has taken along: each on its own
     for (int i = 0; i < 2 && rc == SPH_OK; ++i)
         if (pending.blocks[i] != 0)
@@ -2834,8 +2823,8 @@ int sph_gemm_f32_ex(float* out, const float* A, const float* B, uint32_t M, uint
     args.strideA = strideA;
     args.strideB = strideB;
     const bool stridesAligned = batch == 1 || ((strideA % 4 == 0) && (strideB % 4 == 0));
-    return Launch(args, batch, stridesAligned, strideOut % 4 == 0 || batch == 1,
-                  (flags & SPH_GEMM_TRANS_A) != 0, (flags & SPH_GEMM_TRANS_B) != 0, stream);
+    return Launch(args, batch, stridesAligned, (flags & SPH_GEMM_TRANS_A) != 0,
+                  (flags & SPH_GEMM_TRANS_B) != 0, stream);
 }
 
 int sph_gemm_f32_sgd(float* out, const float* A, const float* B, uint32_t M, uint32_t N,
@@ -2862,8 +2851,8 @@ int sph_gemm_f32_sgd(float* out, const float* A, const float* B, uint32_t M, uin
     args.sgd = 1u;
     args.sgdScale = scale;
     args.sgdRate = rate;
-    return Launch(args, 1, true, true, (flags & SPH_GEMM_TRANS_A) != 0,
-                  (flags & SPH_GEMM_TRANS_B) != 0, stream);
+    return Launch(args, 1, true, (flags & SPH_GEMM_TRANS_A) != 0, (flags & SPH_GEMM_TRANS_B) != 0,
+                  stream);
 }
 
 int sph_linear_forward_f32(float* y, const float* x, const float* W, const float* bias,
@@ -2889,7 +2878,7 @@ int sph_linear_forward_f32(float* y, const float* x, const float* W, const float
     args.overwrite = 1u;
     args.bias = bias;
     args.relu = (flags & SPH_LINEAR_RELU) ? 1u : 0u;
-    return Launch(args, 1, true, true, false, false, stream);
+    return Launch(args, 1, true, false, false, stream);
 }
 
 int sph_gemm_f32(float* out, const float* A, const float* B, uint32_t M, uint32_t N, uint32_t K,
@@ -2914,12 +2903,9 @@ int sph_gemm_f32_grouped(const SphGemmEntry* entries, uint32_t count, float* out
     const int device = sph::CurrentDevice();
     SPH_REQUIRE(device >= 0 && device < 16, "device id out of range");
 
-    bool offsetsAligned = true, outAligned = true;
+    bool offsetsAligned = true;
     for (uint32_t i = 0; i < count; ++i)
-    {
         offsetsAligned = offsetsAligned && ((entries[i].aOff | entries[i].bOff) % 4) == 0;
-        outAligned = outAligned && (entries[i].outOff % 4) == 0;
-    }
 
     EntryTable& t = ThreadTable(device);
     {
@@ -2960,7 +2946,7 @@ int sph_gemm_f32_grouped(const SphGemmEntry* entries, uint32_t count, float* out
         args.M = M;
         args.N = N;
         args.K = K;
-        rc = Launch(args, end - begin, offsetsAligned, outAligned, false, false, stream);
+        rc = Launch(args, end - begin, offsetsAligned, false, false, stream);
         begin = end;
     }
     SPH_HIP_TRY(hipEventRecord(t.consumed, stream));
@@ -2989,7 +2975,7 @@ int sph_gemm_f32_grouped_device(const SphGemmEntry* deviceEntries, uint32_t coun
     args.M = M;
     args.N = N;
     args.K = K;
-    return Launch(args, count, aligned, aligned, false, false, stream);
+    return Launch(args, count, aligned, false, false, stream);
 }
 
 }  // extern "C"
