@@ -163,7 +163,8 @@ def f16_few_tiles(M, N, batch, K=None):
     b32 = -(-M // 32) * -(-N // 32) * batch
     b16 = -(-M // 16) * -(-N // 16) * batch
     limit = F16_FEW_TILE_CUS
-    if K is not None and M % 8 == 0 and N % 8 == 0 and K >= 64:
+    whole = M % 8 == 0 and N % 8 == 0
+    if K is not None and (K >= 64 if whole else min(M, N) >= 8 and 256 <= K <= 1536):
         limit = F16_FEW_TILE_CUS // 2 - 1     # the 64 x 64-tile kernel takes these from here up
     return b32 <= limit or (min(M, N) <= 16 and b16 <= 4 * F16_FEW_TILE_CUS)
 

@@ -21,7 +21,9 @@ CUS = 256
 
 def _in_range(M, N, K, batch):
     tiles128 = -(-M // 128) * -(-N // 128) * batch
-    return tiles128 <= CUS // 2 and not h.f16_few_tiles(M, N, batch, K) and K >= 64 and N % 8 == 0
+    # (N no multiple of 8: at least two slabs, in whichever order the operands are stored)
+    return (tiles128 <= CUS // 2 and not h.f16_few_tiles(M, N, batch, K) and M >= 8 and N >= 8 and
+            K >= (64 if M % 8 == 0 and N % 8 == 0 else 128))
 
 
 def _oracle(C, A16, B16, M, N, K, batch=1):

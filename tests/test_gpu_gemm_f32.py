@@ -169,7 +169,7 @@ def test_partial_last_k_step(dev, dims, flags):
 
 
 # N = 4 q + r, r != 0: the first 4 q columns on the tiled kernels with the
-# row pitches left at N, the last r on the kernel for narrow products.  Guard floats behind
+# row pitches left at N, and the last, broken chunk of a row reaching into the next.  Guard floats behind
 # every unit of out catch a store past column N - 1.
 @pytest.mark.parametrize("flags", [0, capi.SPH_GEMM_TRANS_A, capi.SPH_GEMM_TRANS_B,
                                    capi.SPH_GEMM_OVERWRITE])

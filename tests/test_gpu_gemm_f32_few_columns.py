@@ -39,3 +39,37 @@ def test_few_columns_grouped(dev):
     b = B[1].reshape(K, N)
     assert np.array_equal(got[0], C[0].reshape(M, N) + A[1].reshape(M, K) @ b)
     assert np.array_equal(got[1], C[1].reshape(M, N) + A[0].reshape(M, K) @ b)
+
+
+@pytest.mark.parametrize("flags", [0, rows.TA, rows.TB, rows.TA | rows.TB])
+@pytest.mark.parametrize("shape", [(1023, 7, 1030), (70, 3, 1024), (130, 8, 2049)])
+def test_few_columns_optimizer_step(dev, shape, flags):
+    """A weight of few outputs: scale and rate are powers of two, so the step adds no rounding of its
+    own but that of the subtraction."""
+    M, N, K = shape
+    scale, rate = 0.25, 0.5
+    h.announce("sph_gemm_f32_sgd few columns", shape, "flags", flags)
+    A, B, W = synth.uniform(871, (M, K)), synth.uniform(872, (K, N)), synth.uniform(873, (M, N))
+    stored = [np.ascontiguousarray(x.T) if flags & f else x
+              for x, f in ((A, rows.TA), (B, rows.TB))]
+    dW, dA, dB = (rows.capi.DeviceBuffer.from_array(v) for v in (W, *stored))
+    rows.capi.call("sph_gemm_f32_sgd", dW.ptr, dA.ptr, dB.ptr, M, N, K, scale, rate, flags)
+    got = dW.download(np.float32, (M, N))
+    for d in (dW, dA, dB):
+        d.release()
+    a, b = A.astype(np.float64), B.astype(np.float64)
+    assert np.all(np.abs(got - (W - scale * rate * (a @ b))) <= rows.bound(K, W, a, b))
+
+
+@pytest.mark.parametrize("shared", ["A", "B"])
+def test_few_columns_shared_operand(dev, shared):
+    """One operand for all units of a batch: its stride is 0 (integers: every sum is exact)."""
+    M, N, K, batch = 66, 5, 1029, 3
+    h.announce("sph_gemm_f32_ex few columns, shared", shared)
+    A = synth.small_integers(881, (1 if shared == "A" else batch, M, K), span=4)
+    B = synth.small_integers(882, (1 if shared == "B" else batch, K, N), span=4)
+    C = synth.small_integers(883, (batch, M, N), span=100)
+    got = h.gpu_gemm_f32_ex(C, A, B, M, N, K, 0, batch=batch,
+                            stride_a=0 if shared == "A" else None,
+                            stride_b=0 if shared == "B" else None)
+    assert np.array_equal(got, C + A @ B)
