@@ -90,6 +90,50 @@ __device__ __forceinline__ float Combine(const GemmF32Args& args, float old, flo
     return old + sum;
 }
 
+// Stores acc combined with the old values (or bias terms) `old` for the TM x TN blocks of 32 x 32 one
+// wavefront owns, register quad q of block (i, j) at old[(i * TN + j) * 4 + q].
+template <int TM, int TN>
+__device__ __forceinline__ void FinishTile(const floatx16 (&acc)[TM][TN], float4 (&old)[TM * TN * 4],
+                                           float* __restrict__ out, uint32_t rowBase,
+                                           uint32_t colBase, uint32_t M, uint32_t N, uint32_t l32,
+                                           uint32_t khalf, const GemmF32Args& args)
+{
+    const bool relu = args.relu != 0;
+    const bool inside = rowBase + TM * 32 <= M && colBase + TN * 32 <= N;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+            {
+                const uint32_t r = rowBase + i * 32 + l32, c = colBase + j * 32 + 8 * q + 4 * khalf;
+                float4 v = old[(i * TN + j) * 4 + q];
+                if (!inside && (r >= M || c >= N))
+                    continue;
+                v.x = Combine(args, v.x, acc[i][j][4 * q + 0]);
+                v.y = Combine(args, v.y, acc[i][j][4 * q + 1]);
+                v.z = Combine(args, v.z, acc[i][j][4 * q + 2]);
+                v.w = Combine(args, v.w, acc[i][j][4 * q + 3]);
+                if (relu)
+                {
+                    v.x = v.x > 0 ? v.x : 0;
+                    v.y = v.y > 0 ? v.y : 0;
+                    v.z = v.z > 0 ? v.z : 0;
+                    v.w = v.w > 0 ? v.w : 0;
+                }
+                float* p = out + static_cast<size_t>(r) * args.ldc + c;
+                if (inside || c + 4 <= N)
+                    *reinterpret_cast<floatx4a4*>(p) = floatx4{ v.x, v.y, v.z, v.w };
+                else
+                {
+                    p[0] = v.x;
+                    if (c + 1 < N) p[1] = v.y;
+                    if (c + 2 < N) p[2] = v.z;
+                }
+            }
+}
+
 // out (+)= acc for the TM x TN blocks of 32 x 32 one wavefront owns; rowBase / colBase are
 // the wavefront's first row and column.  Four consecutive columns that all exist are accessed
 // 16 bytes at a time, whatever the alignment of the row.
@@ -101,7 +145,6 @@ __device__ __forceinline__ void StoreTile(const floatx16 (&acc)[TM][TN], float* 
 {
     const bool accumulate = args.overwrite == 0;
     const float* __restrict__ bias = args.bias;
-    const bool relu = args.relu != 0;
     // ---- out += acc ---------------------------------------------------------
     // With the operands swapped, register v of lane l holds row l%32 and column
     // 8*(v/4) + 4*(l/32) + v%4 of its 32x32 block: registers 4q..4q+3 are 4
@@ -166,30 +209,7 @@ __device__ __forceinline__ void StoreTile(const floatx16 (&acc)[TM][TN], float* 
                                 row[min(c + 2, N - 1)], 0.f);
             });
     }
-    each([&](int i, int j, int q, uint32_t r, uint32_t c, float4& v) {
-        if (!inside && (r >= M || c >= N))
-            return;
-        v.x = Combine(args, v.x, acc[i][j][4 * q + 0]);
-        v.y = Combine(args, v.y, acc[i][j][4 * q + 1]);
-        v.z = Combine(args, v.z, acc[i][j][4 * q + 2]);
-        v.w = Combine(args, v.w, acc[i][j][4 * q + 3]);
-        if (relu)
-        {
-            v.x = v.x > 0 ? v.x : 0;
-            v.y = v.y > 0 ? v.y : 0;
-            v.z = v.z > 0 ? v.z : 0;
-            v.w = v.w > 0 ? v.w : 0;
-        }
-        float* p = out + static_cast<size_t>(r) * args.ldc + c;
-        if (inside || c + 4 <= N)
-            *reinterpret_cast<floatx4a4*>(p) = floatx4{ v.x, v.y, v.z, v.w };
-        else
-        {
-            p[0] = v.x;
-            if (c + 1 < N) p[1] = v.y;
-            if (c + 2 < N) p[2] = v.z;
-        }
-    });
+    FinishTile<TM, TN>(acc, old, out, rowBase, colBase, M, N, l32, khalf, args);
 }
 
 // The kernel that takes its operands apart into fp16 planes (sph_gemm_f32_split.hip).  Whether it is the
