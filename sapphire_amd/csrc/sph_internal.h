@@ -48,8 +48,11 @@ void CountAllocation();
 // Takes a stream-ordered scratch block for one call of the library (counted; given back with
 // hipFreeAsync on the same stream), from a pool that keeps up to 512 MiB of freed blocks.
 int AllocScratch(void** ptr, size_t bytes, hipStream_t stream);
-// The same for a caller that can do with less: SPH_OK and a null *ptr when the device is full.
-int AllocScratchIfFree(void** ptr, size_t bytes, hipStream_t stream);
+// The same for the staging of CSR x CSR: the block that the stream has kept, or one from the pool
+// (counted); SPH_OK and a null *ptr when the device is full, for a caller that can do with less.  Given
+// back with GiveStaging on the same stream.
+int TakeStaging(void** ptr, size_t bytes, hipStream_t stream);
+int GiveStaging(void* ptr, hipStream_t stream);
 
 // True between sph_graph_begin_capture and sph_graph_end_capture on this thread.  Entry
 // points that must wait for the device or allocate refuse to run while it is set.

@@ -8,8 +8,8 @@
 // ends, so no stream is destroyed while the runtime may be shutting down.
 #include "sph_internal.h"
 
+#include <algorithm>
 #include <atomic>
-
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -20,8 +20,17 @@ constexpr int kMaxDevices = 16;
 
 thread_local std::string tlsLastError;
 
+// A stream of the library's own, with the staging block that calls on it have left behind
+struct OwnStream
+{
+    hipStream_t stream = nullptr;
+    void* block = nullptr;
+    size_t bytes = 0;
+    bool taken = false;  // by the call that runs
+};
+
 std::mutex gPoolMutex;
-std::vector<hipStream_t> gIdleStreams[kMaxDevices];
+std::vector<OwnStream> gIdleStreams[kMaxDevices];
 int gComputeUnits[kMaxDevices] = {};
 bool gPoolRetains[kMaxDevices] = {};
 // (same mutex) the devices' default pools, and the library's own pools for the scratch blocks of
@@ -32,7 +41,7 @@ hipMemPool_t gScratchPools[kMaxDevices] = {};
 struct ThreadSlots
 {
     int device = 0;
-    hipStream_t own[kMaxDevices] = {};
+    OwnStream own[kMaxDevices] = {};
     hipStream_t borrowed[kMaxDevices] = {};
     hipStream_t capturing = nullptr;  // stream under capture, if any
 
@@ -40,7 +49,7 @@ struct ThreadSlots
     {
         std::lock_guard<std::mutex> lock(gPoolMutex);
         for (int d = 0; d < kMaxDevices; ++d)
-            if (own[d] != nullptr)
+            if (own[d].stream != nullptr)
                 gIdleStreams[d].push_back(own[d]);
     }
 };
@@ -104,9 +113,24 @@ int ScratchPool(hipMemPool_t* pool)
     return SPH_OK;
 }
 
+// The calling thread's idle block goes back to its pool.
+hipError_t DropKeptBlock()
+{
+    OwnStream& own = tlsSlots.own[tlsSlots.device];
+    if (own.block == nullptr || own.taken)
+        return hipSuccess;
+    const hipError_t err = hipFreeAsync(own.block, own.stream);
+    own.block = nullptr;
+    own.bytes = 0;
+    return err;
+}
+
 // Idle blocks of the library's own pool go back to the driver.
 hipError_t TrimScratch()
 {
+    const hipError_t dropped = DropKeptBlock();
+    if (dropped != hipSuccess)
+        return dropped;
     std::lock_guard<std::mutex> lock(gPoolMutex);
     hipMemPool_t own = gScratchPools[tlsSlots.device];
     return own != nullptr ? hipMemPoolTrimTo(own, 0) : hipSuccess;
@@ -120,7 +144,11 @@ hipError_t AllocWithTrim(Alloc&& alloc)
     if (err != hipErrorOutOfMemory)
         return err;
     (void)hipGetLastError();  // not the next launch's error
-    if (TrimScratch() == hipSuccess)
+    // (a block is idle when the work before it has gone)
+    const OwnStream& own = tlsSlots.own[tlsSlots.device];
+    const bool kept = own.block != nullptr && !own.taken;
+    if (TrimScratch() == hipSuccess &&
+        (!kept || (hipStreamSynchronize(own.stream) == hipSuccess && TrimScratch() == hipSuccess)))
         err = alloc();
     if (err == hipErrorOutOfMemory)
         (void)hipGetLastError();
@@ -128,7 +156,10 @@ hipError_t AllocWithTrim(Alloc&& alloc)
 }
 }  // namespace
 
-int AllocScratchIfFree(void** ptr, size_t bytes, hipStream_t stream)
+namespace
+{
+// SPH_OK and a null *ptr when the device is full
+int BlockFromPool(void** ptr, size_t bytes, hipStream_t stream)
 {
     *ptr = nullptr;
     hipMemPool_t pool = nullptr;
@@ -146,15 +177,63 @@ int AllocScratchIfFree(void** ptr, size_t bytes, hipStream_t stream)
     CountAllocation();
     return SPH_OK;
 }
+}  // namespace
 
 int AllocScratch(void** ptr, size_t bytes, hipStream_t stream)
 {
-    const int taken = AllocScratchIfFree(ptr, bytes, stream);
+    const int taken = BlockFromPool(ptr, bytes, stream);
     if (taken == SPH_OK && *ptr == nullptr)
         return Fail(SPH_ERR_DEVICE, std::string("no room for a scratch block of ") +
                                         std::to_string(bytes) + " bytes: " +
                                         hipGetErrorString(hipErrorOutOfMemory));
     return taken;
+}
+
+// Taking a block from a pool and giving it back costs the host 8 us, more than two launches, and a
+// product of a few thousand rows is over before that.  Its staging, up to 32 MiB, therefore stays with
+// the stream it was taken for, if that is one of the library's own: a later call on the stream runs behind
+// the one before, so it may use the block at once, and neither the stream (which is never destroyed) nor
+// the block is seen by another thread meanwhile.  Per thread and device that is one block; a thread that
+// ends leaves it, with the stream, to the next.  8192 rows of 64 products, calls one after the other
+// 21.3 -> 18.1 us (host 21.3 -> 13.7).
+constexpr size_t kKeptBlock = 32u << 20;
+
+int TakeStaging(void** ptr, size_t bytes, hipStream_t stream)
+{
+    OwnStream& own = tlsSlots.own[tlsSlots.device];
+    const bool keep = stream == own.stream && bytes <= kKeptBlock && !own.taken;
+    if (keep && own.block != nullptr && own.bytes >= bytes)
+    {
+        own.taken = true;
+        *ptr = own.block;
+        return SPH_OK;
+    }
+    if (keep)
+    {
+        SPH_HIP_TRY(DropKeptBlock());
+        // the next call may need a little more
+        bytes = std::min(kKeptBlock, bytes + bytes / 4);
+    }
+    const int taken = BlockFromPool(ptr, bytes, stream);
+    if (taken == SPH_OK && keep && *ptr != nullptr)
+    {
+        own.block = *ptr;
+        own.bytes = bytes;
+        own.taken = true;
+    }
+    return taken;
+}
+
+int GiveStaging(void* ptr, hipStream_t stream)
+{
+    OwnStream& own = tlsSlots.own[tlsSlots.device];
+    if (own.taken && ptr == own.block)
+    {
+        own.taken = false;
+        return SPH_OK;
+    }
+    SPH_HIP_TRY(hipFreeAsync(ptr, stream));
+    return SPH_OK;
 }
 
 int Fail(int status, const std::string& msg)
@@ -173,7 +252,7 @@ hipStream_t CurrentStream()
     const int d = tlsSlots.device;
     if (tlsSlots.borrowed[d] != nullptr)
         return tlsSlots.borrowed[d];
-    if (tlsSlots.own[d] == nullptr)
+    if (tlsSlots.own[d].stream == nullptr)
     {
         {
             std::lock_guard<std::mutex> lock(gPoolMutex);
@@ -183,7 +262,7 @@ hipStream_t CurrentStream()
                 gIdleStreams[d].pop_back();
             }
         }
-        if (tlsSlots.own[d] == nullptr)
+        if (tlsSlots.own[d].stream == nullptr)
         {
             hipStream_t s = nullptr;
             hipError_t err = hipSetDevice(d);
@@ -195,10 +274,10 @@ hipStream_t CurrentStream()
                                          hipGetErrorString(err));
                 return nullptr;
             }
-            tlsSlots.own[d] = s;
+            tlsSlots.own[d].stream = s;
         }
     }
-    return tlsSlots.own[d];
+    return tlsSlots.own[d].stream;
 }
 
 bool Capturing()
@@ -352,10 +431,10 @@ int sph_allocation_count(uint64_t* count)
 int sph_mem_pool_trim(void)
 {
     SPH_REFUSE_WHILE_CAPTURING();
+    SPH_HIP_TRY(sph::TrimScratch());  // (first: the thread's idle block may be of either pool)
     hipMemPool_t pool = nullptr;
     SPH_HIP_TRY(hipDeviceGetDefaultMemPool(&pool, tlsSlots.device));
     SPH_HIP_TRY(hipMemPoolTrimTo(pool, 0));
-    SPH_HIP_TRY(sph::TrimScratch());
     return SPH_OK;
 }
 

@@ -1320,7 +1320,7 @@ int sph_spgemm_f32(float* VC, uint32_t* COLC, uint32_t* ROWC, uint32_t capacity,
     float* stageV = nullptr;
     int taken = SPH_OK;
     const uint32_t slot = sph::TakeStagingSlot(M, N, capacity, [&](uint32_t entries) {
-        taken = sph::AllocScratchIfFree(reinterpret_cast<void**>(&stageV),
+        taken = sph::TakeStaging(reinterpret_cast<void**>(&stageV),
                                         counts * 4 + static_cast<size_t>(entries) * M * 8 + 4, stream);
         return taken != SPH_OK || stageV != nullptr;  // a full device: with less
     });
@@ -1373,8 +1373,9 @@ int sph_spgemm_f32(float* VC, uint32_t* COLC, uint32_t* ROWC, uint32_t capacity,
             LaunchFill(args, stream);
         launched = hipGetLastError();
     }
-    if (stageV != nullptr)
-        SPH_HIP_TRY(hipFreeAsync(stageV, stream));
+    const int given = stageV != nullptr ? sph::GiveStaging(stageV, stream) : SPH_OK;
+    if (given != SPH_OK)
+        return given;
     if (launched != hipSuccess)
         return sph::Fail(SPH_ERR_DEVICE, std::string("sph_spgemm_f32 - launch failed with ") +
                                              hipGetErrorString(launched));
