@@ -179,7 +179,12 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
     const char* src;  // of k = 0
     uint32_t off[4];  // bytes
     const uint32_t start = min(first, limit - 4);
-    uint32_t cut = 0;  // k-major: places by which a quad at the edge starts earlier
+    // K-major, a quad that the edge cuts: the last 4 that exist, `cut` earlier.  Each goes to its own row of
+    // the planes all the same, and those that another quad has too to the rows past the edge.  (Put in their
+    // places in the registers, at every step, 2048 x 2045 x 2048 took 88 us, this 72.)
+    uint32_t cut = 0;
+    // (of a group with fewer than 4 that exist: the first ones are another group's, and no matter of this scale)
+    const uint32_t strays = kMajor && limit < first + 4 ? min(first + 4 - limit, 4u) : 0;
     if (kMajor)
     {
         const uint32_t row = first + 4 * q, from = min(row, limit - 4);
@@ -196,7 +201,7 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
         for (uint32_t r = 0; r < 4; ++r)
             off[r] = ((min(first + 4 * q + r, limit - 1) - start) * ld + 4 * g) * 4;
     }
-    const bool anyCut = __ballot(cut != 0) != 0;
+    auto rowOf = [&](uint32_t r) __attribute__((always_inline)) { return 4 * q + ((r - cut) & 3u); };
 
     auto load = [&](floatx4 (&raw)[4], uint32_t s) __attribute__((always_inline)) {
         // (steps past the last copy it again: a load that may not be there makes every wait one for all)
@@ -235,6 +240,11 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
         else
             f(KMajorB{});
     };
+    // whether value r of this lane's is of a row that exists, and no other lane's
+    auto exists = [&](auto kMajorTag, uint32_t r) __attribute__((always_inline)) {
+        const uint32_t row = first + 4 * q;
+        return decltype(kMajorTag)::value ? r >= cut && row < limit : row + r < limit;
+    };
     auto rare = [&](auto kMajorTag, floatx4 (&raw)[4], uint32_t s, float most) __attribute__((always_inline)) {
         if (__ballot(most >= atMost) != 0)
         {
@@ -248,7 +258,7 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
             if (!scaled)
                 firstN = n;
             scaled = true;
-            if ((firstN - n > 30 || e == 255) && lane == 0)
+            if ((firstN - n > 30 || e == 255) && first < limit && lane == 0)
                 marks[s % 2].unfit = s + 1;
             s0 = __builtin_bit_cast(float, static_cast<uint32_t>(127 + n) << 23);
             s11 = s0 * 2048.f;
@@ -270,7 +280,7 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
                 const float a = at(kMajorTag, raw, r, e);
                 const bool small = Size(a) < atLeast;
                 put(kMajorTag, raw, r, e, small ? 0.f : a);
-                any |= small;
+                any |= small && exists(kMajorTag, r);
             }
         if (any)
         {
@@ -285,19 +295,17 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
     // puts right what is at an edge
     auto mend = [&](auto kMajorTag, floatx4 (&raw)[4], uint32_t s) __attribute__((always_inline)) {
         const uint32_t end = s * kChunk + kChunk;
-        if (!anyCut && end <= K)
-            return;
-        if (decltype(kMajorTag)::value)
+        if (decltype(kMajorTag)::value && strays != 0)
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-            {
-                const floatx4 v = raw[e];
-                raw[e][0] = cut == 0 ? v[0] : cut == 1 ? v[1] : cut == 2 ? v[2] : v[3];
-                raw[e][1] = cut == 0 ? v[1] : cut == 1 ? v[2] : v[3];
-                raw[e][2] = cut == 0 ? v[2] : v[3];
-            }
+            for (uint32_t r = 0; r < 4; ++r)
+                if (r < strays)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        raw[e][r] = 0.f;
+        if (end <= K)
+            return;
         // the last chunk ends with K: what the one before it has had counts as zero
-        const uint32_t had = end > K ? end - K : 0;
+        const uint32_t had = end - K;
 #pragma unroll
         for (uint32_t e = 0; e < 4; ++e)
             if (4 * g + e < had)
@@ -345,7 +353,7 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
                     uint32_t, __builtin_convertvector(
                                   (floatx2{ Rest(pair[0], a * s11), Rest(pair[1], b * s11) }), half2v));
             }
-            char* place = to + ChunkAt(4 * q + r, g / 2) + g % 2 * 8;
+            char* place = to + ChunkAt(rowOf(r), g / 2) + g % 2 * 8;
             *reinterpret_cast<uintx2*>(place) = high;
             *reinterpret_cast<uintx2*>(place + kPlane) = low;
         }
@@ -535,6 +543,25 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
         unfit = __builtin_amdgcn_readfirstlane(notFinite) != 0;
     }
     const uint32_t count = __builtin_amdgcn_readfirstlane(listed);
+    if (!unfit && count > 1)
+    {
+        // in an order that does not depend on who came first
+        if (threadIdx.x < count)
+        {
+            const Listed mine = list[threadIdx.x];
+            auto key = [](const Listed& e) {
+                return static_cast<uint64_t>(e.from) << 32 | e.place;
+            };
+            uint32_t rank = 0;
+            for (uint32_t o = 0; o < count; ++o)
+            {
+                const Listed e = list[o];
+                rank += e.k < mine.k || (e.k == mine.k && key(e) < key(mine));
+            }
+            list[rank] = mine;  // (one wavefront: all have read)
+        }
+        publish();
+    }
     if (unfit)
     {
         // The same loop with the values as they are, on the fp32 matrix cores.  A stage holds 32 rows of 32
@@ -554,7 +581,7 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                 {
-                    const uint32_t row = 4 * q + r;
+                    const uint32_t row = rowOf(r);
                     *reinterpret_cast<floatx4*>(stage + wave * 2 * kPlane + row * 128 +
                                                 (g ^ (row / 2 % 8)) * 16) =
                         floatx4{ at(tag, raw[0], r, 0), at(tag, raw[0], r, 1), at(tag, raw[0], r, 2),

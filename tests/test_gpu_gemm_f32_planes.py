@@ -71,6 +71,27 @@ def test_storage_changes_no_bit(dev, shape, offset):
         assert np.array_equal(bits(got), bits(first)), flags
 
 
+@pytest.mark.parametrize("shape", [(1921, 2047, 350), (2046, 1923, 333), (2042, 1954, 321)])
+def test_large_neighbours_of_the_last_rows(dev, shape):
+    """One to three rows and columns past a multiple of 32 share their scale with nothing else, however they
+    are stored: those before them, 2^20 larger, would make all of theirs too small for the planes."""
+    m, n, k = shape
+    A, B = synth.uniform(904, (1, m, k)), synth.uniform(905, (1, k, n))
+    A[:, m // 32 * 32 - 4:m // 32 * 32] *= 2.0 ** 20
+    B[:, :, n // 32 * 32 - 4:n // 32 * 32] *= 2.0 ** 20
+    A[:, -1, ::3] *= 2.0 ** -12
+    B[:, ::5, -1] *= 2.0 ** -12
+    C = np.zeros((1, m, n), np.float32)
+    first = None
+    for flags in (0, TA, TB, TA | TB):
+        h.announce("sph_gemm_f32_ex planes, large neighbours", shape, "flags", flags)
+        got = run(C, A, B, flags)
+        if first is None:
+            first = got
+            check(got, A, B)
+        assert np.array_equal(bits(got), bits(first)), flags
+
+
 def spread(seed, shape, low, high):
     """Signs and mantissas of U(-1, 1), exponents spread evenly over low .. high."""
     e = np.random.default_rng(seed).integers(low, high + 1, shape)
