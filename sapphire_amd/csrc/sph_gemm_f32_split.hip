@@ -26,12 +26,18 @@
 // Every value is taken apart once per tile it takes part in, about 6 vector instructions, and they bound
 // the loop beside the LDS: per step and SIMD 258 vector instructions and 24 of the matrix cores, 2000
 // clocks (the matrix cores alone 770, everything but the split 940).
-//   4096^3 920 -> 545 us (252 TFLOP/s), 2048^3 125 -> 71, 3001 x 2687 x 1000 133 -> 89, 16 x 512^3 36 -> 26.
+//   4096^3 920 -> 545 us (252 TFLOP/s), 2048^3 125 -> 69, 3001 x 2687 x 1000 133 -> 88, 16 x 512^3 36 -> 26.
+// Where such tiles leave too many compute units idle, the 8 wavefronts take a 64 x 64 tile as two teams
+// (2 x 2, 32 x 32 each): each has 32 values of k of the 64 of a step, and their sums are added up at the
+// end.  A step takes 1600 clocks, 12 instructions of the matrix cores per SIMD among as many vector ones.
+//   1024^3 18.7 -> 17.3 us (relative error 5.7e-7 -> 1.6e-7), 1024 x 1024 x 4096 63 -> 54; 5 us of these do
+//   not depend on K, 3 of them up to the first step: code comes from memory as it is first run.
 // Operands that do not fit the planes: 2048^3 125 -> 150 us, 4096^3 920 -> 1110 (exponents spread over 60
 // binades, an infinity in every row).
-// Tried: 64 x 64 tiles of 4 wavefronts on the same loop (1024^3 23 us, on the fp32 kernels 19); 4 wavefronts
-// of 64 x 64 (4096^3 660: one wavefront per SIMD waits out every barrier); three bf16 parts and six
-// products, which need no scale (4096^3 780: the energy of twice the products).
+// Tried: 64 x 64 tiles by one team (1024^3 23 us, on the fp32 kernels 19), by three (19.3: spills where the
+// operands are stored in two ways, no faster where they are not) and four (83); 4 wavefronts of 64 x 64
+// (4096^3 660: one wavefront per SIMD waits out every barrier); three bf16 parts and six products, which need
+// no scale (4096^3 780: the energy of twice the products).
 #include "sph_gemm_f32.h"
 
 #include <algorithm>
@@ -53,7 +59,6 @@ typedef _Float16 half8v __attribute__((ext_vector_type(8)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
 
-constexpr int kTile = 128;
 constexpr uint32_t kChunk = 32;      // values of k per step
 constexpr uint32_t kGroup = 32;      // rows (columns) that one wavefront splits
 constexpr uint32_t kPlane = 2048;    // bytes: 32 rows x 32 halves
@@ -102,15 +107,28 @@ __device__ __forceinline__ float Rest(_Float16 h, float c)
     return __builtin_fmaf(static_cast<float>(h), -2048.f, c);
 }
 
+// the largest of the 64 lanes' x.  (With six shuffles the first scale of a tile took 430 clocks longer.)
+__device__ __forceinline__ uint32_t LargestOfAll(uint32_t x)
+{
+    x = max(x, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true)));  // row_shr:1
+    x = max(x, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true)));  // row_shr:2
+    x = max(x, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true)));  // row_shr:4
+    x = max(x, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true)));  // row_shr:8
+    // (the last lane of 16 has what is the largest of them)
+    return max(max(__builtin_amdgcn_readlane(x, 15), __builtin_amdgcn_readlane(x, 31)),
+               max(__builtin_amdgcn_readlane(x, 47), __builtin_amdgcn_readlane(x, 63)));
+}
+
+// KS: teams of wavefronts, which take the chunks of k in turn and add up their sums at the end
 // DEPTH: steps by which the loads are ahead
-template <int BM, int BN, int WM, int WN, int DEPTH, bool TA, bool TB>
-__global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
+template <int BM, int BN, int KS, int WM, int WN, int DEPTH, bool TA, bool TB>
+__global__ __launch_bounds__(KS * WM * WN * 64) void GemmF32SplitKernel(
     const GemmF32Args args)
 {
-    constexpr int NW = WM * WN;
+    constexpr int PER = WM * WN, NW = KS * PER;
     constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
     constexpr uint32_t kGroupsA = BM / kGroup, kGroupsB = BN / kGroup;
-    static_assert(kGroupsA + kGroupsB == NW, "a wavefront splits one group");
+    static_assert(kGroupsA + kGroupsB == PER, "a wavefront splits one group");
     constexpr uint32_t kStage = NW * 2 * kPlane;
     __shared__ __attribute__((aligned(1024))) char lds[2 * kStage];
     struct Scale
@@ -133,7 +151,8 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
         return;
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t wm = wave / WN, wn = wave % WN;
+    const uint32_t team = wave / PER, member = wave % PER;
+    const uint32_t wm = member / WN, wn = member % WN;
     const uint32_t x = lane % 32, h = lane / 32;
     const uint32_t M = args.M, N = args.N, K = args.K;
     if (threadIdx.x < 2 * NW)
@@ -164,12 +183,14 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
     const float* __restrict__ srcB = args.B + offB;
     const uint32_t lda = TA ? M : K, ldb = TB ? K : N;
     const uint32_t baseM = tm * BM, baseN = tn * BN;
-    const uint32_t steps = (K + kChunk - 1) / kChunk;
+    const uint32_t steps = (K + KS * kChunk - 1) / (KS * kChunk);
+    // where the chunk of this team begins
+    auto chunkOf = [&](uint32_t s) __attribute__((always_inline)) { return (s * KS + team) * kChunk; };
 
     // ---- what this wavefront splits: rows 4 q .. 4 q + 3, k 4 g .. 4 g + 3 of its group ---------------
-    const bool ofA = wave < kGroupsA;
+    const bool ofA = member < kGroupsA;
     const bool kMajor = ofA ? TA : !TB;
-    const uint32_t group = ofA ? wave : wave - kGroupsA;
+    const uint32_t group = ofA ? member : member - kGroupsA;
     const uint32_t p8 = lane / 8;
     const uint32_t q = kMajor ? lane % 8 : p8;
     const uint32_t g = kMajor ? (p8 & 1) | (p8 & 2) << 1 | (p8 & 4) >> 1 : lane % 8;
@@ -205,7 +226,7 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
 
     auto load = [&](floatx4 (&raw)[4], uint32_t s) __attribute__((always_inline)) {
         // (steps past the last copy it again: a load that may not be there makes every wait one for all)
-        const char* base = src + min(s * kChunk, K - kChunk) * perK;
+        const char* base = src + min(chunkOf(s), K - kChunk) * perK;
         // (made opaque, or the compiler adds them up as 64-bit addresses: 2048^3 71.4 -> 69.2 us)
         asm("" : "+v"(off[0]), "+v"(off[1]), "+v"(off[2]), "+v"(off[3]));
 #pragma unroll
@@ -245,15 +266,11 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
         const uint32_t row = first + 4 * q;
         return decltype(kMajorTag)::value ? r >= cut && row < limit : row + r < limit;
     };
-    auto rare = [&](auto kMajorTag, floatx4 (&raw)[4], uint32_t s, float most) __attribute__((always_inline)) {
+    auto rare = [&](auto kMajorTag, floatx4 (&raw)[4], uint32_t s, float most, uint32_t least)
+                    __attribute__((always_inline)) {
         if (__ballot(most >= atMost) != 0)
         {
-            float all = most;
-#pragma unroll
-            for (int d = 32; d > 0; d /= 2)
-                all = fmaxf(all, __shfl_xor(all, d));
-            const int e = static_cast<int>(
-                __builtin_amdgcn_readfirstlane(__builtin_bit_cast(uint32_t, all)) >> 23);
+            const int e = static_cast<int>(LargestOfAll(__builtin_bit_cast(uint32_t, most)) >> 23);
             n = min(140 - min(max(e, 1), 254), 110);
             if (!scaled)
                 firstN = n;
@@ -271,6 +288,8 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
                 scaleOf[s % 2][wave] = { s + 1, n };
             }
         }
+        if (__ballot(least < atLeast) == 0)
+            return;
         bool any = false;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
@@ -286,15 +305,15 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
         {
             const uint32_t slot = atomicAdd(&listed, 1u);
             if (slot < kListed)
-                list[slot] = { min(s * kChunk, K - kChunk) + 4 * g,
-                               group * kGroup + 4 * q + (ofA ? 0u : 1u << 31), s * kChunk, atLeast };
+                list[slot] = { min(chunkOf(s), K - kChunk) + 4 * g,
+                               group * kGroup + 4 * q + (ofA ? 0u : 1u << 31), chunkOf(s), atLeast };
             else
                 marks[s % 2].unfit = s + 1;
         }
     };
     // puts right what is at an edge
     auto mend = [&](auto kMajorTag, floatx4 (&raw)[4], uint32_t s) __attribute__((always_inline)) {
-        const uint32_t end = s * kChunk + kChunk;
+        const uint32_t end = chunkOf(s) + kChunk;
         if (decltype(kMajorTag)::value && strays != 0)
 #pragma unroll
             for (uint32_t r = 0; r < 4; ++r)
@@ -304,7 +323,7 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
                         raw[e][r] = 0.f;
         if (end <= K)
             return;
-        // the last chunk ends with K: what the one before it has had counts as zero
+        // the last chunk ends with K: what the one before it has had counts as zero (all of one past the last)
         const uint32_t had = end - K;
 #pragma unroll
         for (uint32_t e = 0; e < 4; ++e)
@@ -335,7 +354,7 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
         const float most = MaxSize(mostOf[0], mostOf[1], MaxSize(mostOf[2], mostOf[3], 0.f));
         const uint32_t least = min(min(leastOf[0], leastOf[1]), min(leastOf[2], leastOf[3]));
         if (__ballot((most >= atMost) | (least < atLeast)) != 0)
-            rare(kMajorTag, raw, s, most);
+            rare(kMajorTag, raw, s, most, least);
     };
     auto convert = [&](auto kMajorTag, const floatx4 (&raw)[4], uint32_t parity) __attribute__((always_inline)) {
         char* to = lds + parity * kStage + wave * 2 * kPlane;
@@ -378,21 +397,21 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
     for (int j = 0; j < TN; ++j)
         nB[j] = 0;
     const uint32_t fragment = ChunkAt(x, h);
-    const char* planesA = lds + wm * TM * 2 * kPlane;
-    const char* planesB = lds + (kGroupsA + wn * TN) * 2 * kPlane;
+    const char* planesA = lds + (team * PER + wm * TM) * 2 * kPlane;
+    const char* planesB = lds + (team * PER + kGroupsA + wn * TN) * 2 * kPlane;
 
     auto rescale = [&](uint32_t s) __attribute__((always_inline)) {
         int a[TM], b[TN];
 #pragma unroll
         for (int i = 0; i < TM; ++i)
         {
-            const Scale c = scaleOf[s % 2][wm * TM + i];
+            const Scale c = scaleOf[s % 2][team * PER + wm * TM + i];
             a[i] = __builtin_amdgcn_readfirstlane(c.step == s + 1 ? c.n : nA[i]);
         }
 #pragma unroll
         for (int j = 0; j < TN; ++j)
         {
-            const Scale c = scaleOf[s % 2][kGroupsA + wn * TN + j];
+            const Scale c = scaleOf[s % 2][team * PER + kGroupsA + wn * TN + j];
             b[j] = __builtin_amdgcn_readfirstlane(c.step == s + 1 ? c.n : nB[j]);
         }
 #pragma unroll
@@ -449,8 +468,8 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
     };
 
     const uint32_t rowBase = baseM + wm * TM * 32, colBase = baseN + wn * TN * 32;
-    static_assert(TM == DEPTH && TN == 1, "the old values of block i fit raw[i]");
-    const bool early = args.overwrite == 0 && args.bias == nullptr && baseM + BM <= M && baseN + BN <= N;
+    static_assert(KS > 1 || (TM == DEPTH && TN == 1), "the old values of block i fit raw[i]");
+    const bool early = KS == 1 && args.overwrite == 0 && args.bias == nullptr && baseM + BM <= M && baseN + BN <= N;
     const float* oldAt = out + static_cast<size_t>(rowBase + x) * args.ldc + colBase + 4 * h;
 
     floatx4 raw[DEPTH][4];
@@ -476,11 +495,15 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
         convert(kMajorTag, next, 1 - parity);
         multiply(f0);
         multiply(f1);
+        // (few matrix instructions start later: their operands are under way when the barrier is passed)
+        constexpr bool kFew = TM * TN == 1;
+        if (kFew)
+            __builtin_amdgcn_sched_group_barrier(0x2, 24, 0);
 #pragma unroll
         for (int n = 0; n < 6 * TM * TN; ++n)
         {
             __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x2, 66 / (6 * TM * TN), 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, kFew ? 8 : 5, 0);
         }
         // The last two of these steps have nothing more to load and ask for what a whole tile is added to:
         // with one workgroup per compute unit nothing else runs beside the round trip (16 x 512^3 26.8 ->
@@ -596,12 +619,12 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
                     floatx4 a[TM], b[TN];
 #pragma unroll
                     for (int i = 0; i < TM; ++i)
-                        a[i] = *reinterpret_cast<const floatx4*>(stage + (wm * TM + i) * 2 * kPlane +
+                        a[i] = *reinterpret_cast<const floatx4*>(stage + (team * PER + wm * TM + i) * 2 * kPlane +
                                                                  chunk);
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
                         b[j] = *reinterpret_cast<const floatx4*>(
-                            stage + (kGroupsA + wn * TN + j) * 2 * kPlane + chunk);
+                            stage + (team * PER + kGroupsA + wn * TN + j) * 2 * kPlane + chunk);
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -614,7 +637,46 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
             }
         });
     }
-    else
+    if (KS > 1)
+    {
+        // the first team adds up the teams' sums, in their order
+        static_assert((KS - 1) * PER * TM * TN * 4096 <= 2 * kStage, "the sums fit the stages");
+        auto place = [&](uint32_t t, int block, int q) __attribute__((always_inline)) {
+            return reinterpret_cast<floatx4*>(
+                lds + (((t - 1) * PER + member) * (TM * TN * 4) + block * 4 + q) * 1024 + lane * 16);
+        };
+        publish();  // nobody reads the stages any more
+        if (team != 0)
+        {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        *place(team, i * TN + j, q) =
+                            floatx4{ acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
+                                     acc[i][j][4 * q + 3] };
+        }
+        publish();
+        if (team != 0)
+            return;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (uint32_t t = 1; t < KS; ++t)
+                    {
+                        const floatx4 sum = *place(t, i * TN + j, q);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            acc[i][j][4 * q + e] += sum[e];
+                    }
+    }
+    if (!unfit)
         // 16 values of every block, those that were left out
         for (uint32_t n = 0; n < count * 16; ++n)
         {
@@ -674,7 +736,7 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
         }
     if (early && !unfit)
     {
-        float4 old[TM * 4];
+        float4 old[TM * TN * 4];
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -686,39 +748,71 @@ __global__ __launch_bounds__(WM * WN * 64) void GemmF32SplitKernel(
         StoreTile<TM, TN>(acc, out, rowBase, colBase, M, N, x, h, args);
 }
 
-template <bool TA, bool TB>
-void LaunchAs(const GemmF32Args& args, dim3 grid, hipStream_t stream)
+template <int BM, int BN, int KS, int WM, int WN>
+void LaunchAs(const GemmF32Args& args, dim3 grid, bool transA, bool transB, hipStream_t stream)
 {
-    hipLaunchKernelGGL((GemmF32SplitKernel<kTile, kTile, 2, 4, 2, TA, TB>), grid, dim3(512), 0,
-                       stream, args);
+    auto launch = [&](auto ta, auto tb) {
+        hipLaunchKernelGGL((GemmF32SplitKernel<BM, BN, KS, WM, WN, 2, decltype(ta)::value, decltype(tb)::value>),
+                           grid, dim3(KS * WM * WN * 64), 0, stream, args);
+    };
+    if (transA && transB)
+        launch(std::true_type{}, std::true_type{});
+    else if (transA)
+        launch(std::true_type{}, std::false_type{});
+    else if (transB)
+        launch(std::false_type{}, std::true_type{});
+    else
+        launch(std::false_type{}, std::false_type{});
+}
+
+uint64_t TilesOf(const GemmF32Args& args, uint32_t units, uint32_t edge)
+{
+    return static_cast<uint64_t>((args.M + edge - 1) / edge) * ((args.N + edge - 1) / edge) * units;
+}
+
+// In the unit of the other kernels' cost (107: 14.5 us per 1000 values of k; a round is one tile per compute
+// unit) a round of 128 x 128 tiles costs 210, and 6.8 us that do not depend on K: the first loads, the first
+// scale, reading and writing out with nothing beside it.  It replaces three rounds of 64 x 64 tiles
+// (1536 x 2048 x 1024 51 -> 38 us; where it would replace two, 1501 x 1203 x 1001, both take 35).
+uint64_t Cost128(const GemmF32Args& args, uint32_t units)
+{
+    const uint64_t cus = static_cast<uint64_t>(sph::ComputeUnits());
+    return (TilesOf(args, units, 128) + cus - 1) / cus * (210 + 50000 / args.K);
+}
+
+// A round of 64 x 64 tiles by two teams costs 88, and 2.2 us more than on the fp32 matrix cores, whose
+// workgroups go on from tile to tile, so that a second round costs these 3.8 us more: 1024^3 18.7 -> 17.4 us,
+// 1024 x 1024 x 4096 63 -> 52, K = 900 17.6 -> 16.8, but K = 784 15.0 -> 15.6; in two rounds 1408^3 45 -> 42.6,
+// 1280 x 1280 x 4096 117 -> 98, but 1100^3 (both operands transposed) 36.4 -> 37.1.
+uint64_t Cost64(const GemmF32Args& args, uint32_t units)
+{
+    const uint64_t cus = static_cast<uint64_t>(sph::ComputeUnits());
+    const uint64_t rounds = (TilesOf(args, units, 64) + cus - 1) / cus;
+    return rounds * 88 + (rounds * 28000 - 12000) / args.K;
 }
 }  // namespace
 
 namespace sph
 {
-// In the unit of the other kernels' cost (107: 14.5 us per 1000 values of k) a round of 128 x 128 tiles costs
-// 210, and 6.8 us that do not depend on K: the first loads, the first scale, reading and writing out with
-// nothing beside it.  The line is where a round replaces three rounds of 64 x 64 tiles (1536 x 2048 x 1024
-// 51 -> 38 us; where it replaces two, 1501 x 1203 x 1001, both take 35).  Below K = 320 the fixed part
-// decides (2048 x 2048 x 320 30 -> 20 us), and a product's bits there do not depend on the batch.
+// Below K = 320 the fixed part decides (2048 x 2048 x 320 30 -> 20 us), and a product's bits there do not
+// depend on the batch.
 bool SplitsF32(const GemmF32Args& args, uint32_t units, uint64_t otherCost, bool transA, bool transB)
 {
-    // (lane offsets of 32 rows fit 32 bits)
-    if (args.K < 320 || args.M < 4 || args.N < 4 ||
+    // (lane offsets of 32 rows fit 32 bits, and so do the k of chunks past the last)
+    if (args.K < 320 || args.K >= (1u << 31) || args.M < 4 || args.N < 4 ||
         std::max(transA ? args.M : args.K, transB ? args.K : args.N) >= (1u << 24))
         return false;
-    const uint64_t cus = static_cast<uint64_t>(ComputeUnits());
-    const uint64_t tiles = static_cast<uint64_t>((args.M + kTile - 1) / kTile) *
-                           ((args.N + kTile - 1) / kTile) * units;
-    return (tiles + cus - 1) / cus * (210 + 50000 / args.K) < otherCost;
+    return std::min(Cost128(args, units), Cost64(args, units)) < otherCost;
 }
 
 int LaunchGemmF32Split(GemmF32Args args, uint32_t units, bool transA, bool transB,
                        hipStream_t stream)
 {
-    args.tilesM = (args.M + kTile - 1) / kTile;
-    args.tilesN = (args.N + kTile - 1) / kTile;
-    const uint64_t blocks = static_cast<uint64_t>(args.tilesM) * args.tilesN * units;
+    const bool small = Cost64(args, units) < Cost128(args, units);
+    const uint32_t edge = small ? 64 : 128;
+    args.tilesM = (args.M + edge - 1) / edge;
+    args.tilesN = (args.N + edge - 1) / edge;
+    const uint64_t blocks = TilesOf(args, units, edge);
     if (blocks >= (1ull << 31) - 8)
         return Fail(SPH_ERR_INVALID, "sph_gemm_f32 - too many tiles for one launch");
     args.tilesTotal = static_cast<uint32_t>(blocks);
@@ -730,14 +824,10 @@ int LaunchGemmF32Split(GemmF32Args args, uint32_t units, bool transA, bool trans
         band *= 2;
     args.band = std::min(band, args.tilesM);
     const dim3 grid(args.perXcd * 8);
-    if (transA && transB)
-        LaunchAs<true, true>(args, grid, stream);
-    else if (transA)
-        LaunchAs<true, false>(args, grid, stream);
-    else if (transB)
-        LaunchAs<false, true>(args, grid, stream);
+    if (small)
+        LaunchAs<64, 64, 2, 2, 2>(args, grid, transA, transB, stream);
     else
-        LaunchAs<false, false>(args, grid, stream);
+        LaunchAs<128, 128, 1, 2, 4>(args, grid, transA, transB, stream);
     SPH_CHECK_LAUNCH();
     return SPH_OK;
 }

@@ -16,10 +16,18 @@ pytestmark = pytest.mark.gpu
 TA, TB, OW = capi.SPH_GEMM_TRANS_A, capi.SPH_GEMM_TRANS_B, capi.SPH_GEMM_OVERWRITE
 
 # (batch, M, N, K): whole tiles; edges that cut a quad, K that ends within a chunk and within 4 values;
-# a batch; the smallest K
+# a batch; the smallest K.  Then 64 x 64 tiles, whose K is shared out to two teams: K that ends with the
+# first team's chunk, with the second's and within either; two rounds
 SHAPES = [(1, 2048, 2048, 352), (1, 2046, 2045, 333), (1, 1921, 2047, 350), (16, 509, 511, 322),
-          (1, 2048, 2047, 320)]
+          (1, 2048, 2047, 320), (1, 1024, 1024, 1024), (1, 1024, 1018, 992), (1, 1022, 961, 1007),
+          (1, 1021, 1023, 1025), (3, 510, 509, 1050), (1, 1280, 1270, 1300)]
 M, N, K = 2046, 2045, 333
+
+
+@pytest.fixture(params=[(2046, 2045, 333), (1022, 1021, 1003)], ids=["tiles of 128", "of 64"])
+def sizes(request, monkeypatch):
+    for name, value in zip("MNK", request.param):
+        monkeypatch.setitem(globals(), name, value)
 
 
 def bits(x):
@@ -71,7 +79,8 @@ def test_storage_changes_no_bit(dev, shape, offset):
         assert np.array_equal(bits(got), bits(first)), flags
 
 
-@pytest.mark.parametrize("shape", [(1921, 2047, 350), (2046, 1923, 333), (2042, 1954, 321)])
+@pytest.mark.parametrize("shape", [(1921, 2047, 350), (2046, 1923, 333), (2042, 1954, 321), (961, 1023, 1001),
+                                   (1022, 963, 1030)])
 def test_large_neighbours_of_the_last_rows(dev, shape):
     """One to three rows and columns past a multiple of 32 share their scale with nothing else, however they
     are stored: those before them, 2^20 larger, would make all of theirs too small for the planes."""
@@ -123,10 +132,10 @@ def growing():
 def a_few_small():
     """Rows and columns that hold nothing but one small value, next to ordinary ones."""
     A, B = synth.uniform(919, (1, M, K)), synth.uniform(920, (1, K, N))
-    for i, (row, k) in enumerate([(5, 7), (6, 7), (130, 332), (2045, 331), (2044, 0), (64, 31)]):
+    for i, (row, k) in enumerate([(5, 7), (6, 7), (130, 332), (M - 1, 331), (M - 2, 0), (64, 31)]):
         A[0, row] = 0
         A[0, row, k] = 2.0 ** -(30 + 3 * i) * 1.1
-    for i, (col, k) in enumerate([(3, 7), (4, 7), (131, 332), (2044, 330), (2043, 1)]):
+    for i, (col, k) in enumerate([(3, 7), (4, 7), (131, 332), (N - 1, 330), (N - 2, 1)]):
         B[0, :, col] = 0
         B[0, k, col] = -(2.0 ** -(31 + 3 * i)) * 1.3
     return A, B
@@ -146,8 +155,8 @@ RANGES = {"rows and columns": lambda: rows_and_columns(-12, 13),
 
 @pytest.mark.parametrize("flags", [0, TA | TB])
 @pytest.mark.parametrize("name", RANGES)
-def test_ranges(dev, name, flags):
-    h.announce("sph_gemm_f32_ex planes,", name, "flags", flags)
+def test_ranges(dev, sizes, name, flags):
+    h.announce("sph_gemm_f32_ex planes,", name, (M, N, K), "flags", flags)
     A, B = (x.astype(np.float32) for x in RANGES[name]())
     check(run(np.zeros((1, M, N), np.float32), A, B, flags), A, B)
 
@@ -166,9 +175,9 @@ def test_zeros_and_ones(dev):
 
 
 @pytest.mark.parametrize("values", [(np.inf,), (-np.inf, np.nan), (3e38, -3e38), (np.nan,)])
-def test_specials(dev, values):
+def test_specials(dev, sizes, values):
     """Infinities, NaN and sums past the largest number, as the CPU loop has them."""
-    h.announce("sph_gemm_f32_ex planes, specials", values)
+    h.announce("sph_gemm_f32_ex planes, specials", values, (M, N, K))
     A, B = synth.uniform(941, (M, K)), synth.uniform(942, (K, N))
     for i, v in enumerate(values * 3):
         A[3 + 50 * i, 5 * i] = v
@@ -187,9 +196,9 @@ def test_specials(dev, values):
     assert np.all(np.abs(got[ok].astype(np.float64) - ref[ok]) <= 1e-4 * scale[ok])
 
 
-def test_linear_and_sgd_epilogues(dev):
+def test_linear_and_sgd_epilogues(dev, sizes):
     """Bias, ReLU and the optimizer's step after the same sums."""
-    h.announce("sph_linear_forward_f32 and sph_gemm_f32_sgd planes")
+    h.announce("sph_linear_forward_f32 and sph_gemm_f32_sgd planes", (M, N, K))
     x, W = synth.uniform(951, (M, K)), synth.uniform(952, (K, N))
     bias, old = synth.uniform(953, (N,)), synth.uniform(954, (M, N))
     dx, dW, db = (capi.DeviceBuffer.from_array(v) for v in (x, W, bias))
