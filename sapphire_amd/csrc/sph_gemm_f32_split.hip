@@ -24,7 +24,7 @@
 // values travel global -> registers two steps ahead, are looked over (largest, smallest), taken apart
 // and written to one of two LDS stages while the matrix cores work on the other; one barrier per step.
 // Every value is taken apart once per tile it takes part in, about 6 vector instructions, and they bound
-// the loop beside the LDS: per step and SIMD 258 vector instructions and 24 of the matrix cores, 2000
+// the loop beside the LDS: per step and SIMD 232 vector instructions and 24 of the matrix cores, 2000
 // clocks (the matrix cores alone 770, everything but the split 940).
 //   4096^3 920 -> 545 us (252 TFLOP/s), 2048^3 125 -> 69, 3001 x 2687 x 1000 133 -> 88, 16 x 512^3 36 -> 26.
 // Where such tiles leave too many compute units idle, the 8 wavefronts take a 64 x 64 tile as two teams
