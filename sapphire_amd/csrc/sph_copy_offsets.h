@@ -1,8 +1,8 @@
-// Where the tiled GEMM kernels copy the chunks of an operand stored k-major from, when its rows are no
-// whole number of chunks.  One definition for the kernels and for the host, so that the CPU tests
+// Where the tiled GEMM kernels copy the chunks of an operand from, when its rows are no whole number of
+// chunks or steps.  One definition for the kernels and for the host, so that the CPU tests
 // see that no copy reaches past an operand: what it would bring feeds no output and shows in none.
 //
-// A row's last chunk reaches into the next row, whose values only feed outputs that are not
+// Operand stored k-major: a row's last chunk reaches into the next row, whose values only feed outputs that are not
 // stored.  In the last row of the matrix there is none; the chunk begins earlier there, so that it
 // ends with the row.  Chunks past a row's end copy its last whole chunk.
 #ifndef SPH_COPY_OFFSETS_H
@@ -34,6 +34,15 @@ SPH_COPY_INLINE KMajorPlace QuadPlace(uint32_t k, uint32_t x, uint32_t limit, ui
     const uint32_t last = limit - 4;
     const bool clamp = x >= limit || (ending && k + 1 == valid);
     return { k, clamp && x > last ? last : x };
+}
+
+// fp32, an operand stored with K contiguous: chunk c of a row of a slab that has `valid` values of k ends
+// with this one.  Chunks that reach past `valid`, and those that begin past it, are the row's last four
+// values, whatever `valid` is (K >= 4): up to three of them lie before the slab.
+SPH_COPY_INLINE uint32_t RowChunkEnd(uint32_t c, uint32_t valid)
+{
+    const uint32_t end = c * 4 + 4;
+    return end < valid ? end : valid;
 }
 
 // fp16, chunks of 8 (x a multiple of 8, limit >= 8): the first column a chunk is copied from, in every

@@ -500,8 +500,8 @@ struct DmaTile
 // per tile fixed.  Per element the arithmetic is the same as without WALK.
 //
 // TAIL: K = BK q + r with 0 < r < BK.  The last of the q + 1 steps copies only the r values of
-// k that exist - a lane whose 16-byte chunk (K-contiguous operand) or row (k-major operand)
-// lies past K copies the slab's first chunk or row instead, one whose chunk reaches past K the
+// k that exist - a lane whose row (k-major operand) lies past K copies the slab's first row instead,
+// one whose 16-byte chunk (K-contiguous operand) reaches or lies past K the
 // 4 values that end at K - and the fragments are put right where they are used (zeros for
 // k >= K, for A and B alike), so the step adds what a zero-padded slab would: the same sum,
 // in the same order, as the register-staged kernel.
@@ -627,12 +627,10 @@ GemmF32DmaKernel(const GemmF32Args args, const GemmF32Strips strips)
         using T = TileA;  // chunk geometry depends on BK only
         const uint32_t x = j * T::kRowsPerCopyK + lane / T::kChunks;  // row inside the tile
         const uint32_t c = (lane % T::kChunks) ^ T::Swizzle(x);
-        // float offset of the chunk inside the slab's row, + 4: a chunk that reaches past
-        // `valid` copies the last 4 values of the row (its LDS slot then holds k = valid - 4
-        // .. valid - 1), one that begins past it the row's first chunk
-        uint32_t k4 = c * 4 + 4;
-        if (k4 > valid)
-            k4 = k4 - 4 < valid ? valid : 4;
+        // float offset of the chunk inside the slab's row, + 4: a chunk that reaches or begins
+        // past `valid` copies the last 4 values of the row (its LDS slot then holds
+        // k = valid - 4 .. valid - 1)
+        const uint32_t k4 = sph::RowChunkEnd(c, valid);
         const uint32_t gx = min(xBase + x, limit - 1);
         return (gx * K + k4) * 4u - 16u + kTailBias;
     };

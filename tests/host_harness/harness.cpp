@@ -313,6 +313,29 @@ int sphh_quad_copies_reach(unsigned K, unsigned limit, unsigned bk, unsigned til
     return 0;
 }
 
+// The same for an operand of `rows` rows of K floats: the last slab has the values of k that are left.
+int sphh_row_chunks_reach(unsigned K, unsigned rows, unsigned bk, long long* out)
+{
+    const std::uint32_t steps = (K + bk - 1) / bk;
+    const long long end = static_cast<long long>(K) * rows;
+    long long most = -end;
+    for (std::uint32_t s = 0; s < steps; ++s)
+        for (std::uint32_t c = 0; c < bk / 4; ++c)
+            for (std::uint32_t r = 0; r < rows; ++r)
+            {
+                const std::uint32_t valid = s + 1 == steps ? K - s * bk : bk;
+                const std::uint32_t last = sph::RowChunkEnd(c, valid);
+                const long long at = static_cast<long long>(r) * K + s * bk + last - 4;
+                most = std::max(most, at + 4 - end);
+                // not ahead of the operand; what is whole comes from its own place, what K ends in ends
+                // with it
+                if (at < 0 || (c * 4 < valid && last != std::min(c * 4 + 4, valid)))
+                    return 1;
+            }
+    *out = most;
+    return 0;
+}
+
 // fp16: the last slab is the window [K - bk, K), whose last row is the matrix's.
 int sphh_chunk_copies_reach(unsigned K, unsigned limit, unsigned bk, unsigned tile, long long* out)
 {

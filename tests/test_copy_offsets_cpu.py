@@ -1,6 +1,6 @@
-"""Where the tiled GEMM kernels copy the chunks of an operand stored k-major from
-(sapphire_amd/csrc/sph_copy_offsets.h, reached through the host harness): no copy of any slab reaches
-past the operand, whatever its width; no device is needed."""
+"""Where the tiled GEMM kernels copy the chunks of an operand from (sapphire_amd/csrc/sph_copy_offsets.h,
+reached through the host harness): no copy of any slab reaches past the operand, whatever its width
+and depth; no device is needed."""
 import ctypes
 
 import pytest
@@ -24,6 +24,14 @@ def test_fp32_quads_end_with_the_operand(bk, tile):
             assert got == 0, (limit, K)
             if limit % 4 == 0:  # the kernels without a last step of its own
                 assert reach("sphh_quad_copies_reach", K, limit, bk, tile, 0) == 0, (limit, K)
+
+
+# an operand stored with K contiguous: a last slab of every number of values, one to three among them
+@pytest.mark.parametrize("bk", [16, 32])
+def test_fp32_row_chunks_end_with_the_operand(bk):
+    for K in list(range(16, 100)) + [1025, 1026, 1027]:
+        for rows in [1, 3]:
+            assert reach("sphh_row_chunks_reach", K, rows, bk) == 0, (K, rows)
 
 
 # fp16 kernels: (K step, tile edge, fewest slabs of broken rows)
