@@ -45,6 +45,19 @@ SPH_COPY_INLINE uint32_t RowChunkEnd(uint32_t c, uint32_t valid)
     return end < valid ? end : valid;
 }
 
+// fp32, few rows of an operand stored k-major: `floats` values that lie one behind the other, in pieces of
+// 4.  Of `slots` pieces that are asked for at once those past the end are the last whole one again;
+// where there is none, no piece is asked for.
+SPH_COPY_INLINE uint32_t PiecesAsked(uint32_t floats, uint32_t slots)
+{
+    return floats < 4 ? 0 : slots;
+}
+
+SPH_COPY_INLINE uint32_t PieceBegin(uint32_t piece, uint32_t floats)
+{
+    return piece * 4 < floats - 4 ? piece * 4 : floats - 4;
+}
+
 // fp16, chunks of 8 (x a multiple of 8, limit >= 8): the first column a chunk is copied from, in every
 // row but the last of the matrix
 SPH_COPY_INLINE uint32_t ChunkColumn(uint32_t x, uint32_t limit)

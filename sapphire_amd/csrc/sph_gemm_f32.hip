@@ -1733,25 +1733,25 @@ __global__ __launch_bounds__(KW * GROUPS * 64) void GemmF32ThinKernel(const Gemm
             // Rows of M floats that lie one behind the other: read as they lie (pieces of a row per
             // lane would be 64 lines per access), and taken apart by the reads from LDS.
             // All pieces are requested before the first is put down; those past the end are
-            // the last one again.
+            // the last one again (a round of K that has less than one has the broken one only).
             const uint32_t floats = min(256u * KW, K - base) * M;
             const uint32_t perM = ((1u << 20) + M - 1) / M;  // x / M below
             const float* from = A + static_cast<size_t>(base) * M;
             // float 4 q + u goes here: q / M is the lane whose four rows the piece is of
             auto place = [&](uint32_t q) { return slab + q * 4 + (q * perM >> 20); };
             constexpr int kPieces = kRows < 8 ? kRows : 8;  // (more do not fit the registers)
+            const uint32_t asked = sph::PiecesAsked(floats, kRows * 64 * KW * GROUPS);
             if (base != 0)
                 __syncthreads();
 #pragma unroll 1
-            for (uint32_t first = threadIdx.x; first < kRows * 64 * KW * GROUPS;
-                 first += kPieces * 64 * KW * GROUPS)
+            for (uint32_t first = threadIdx.x; first < asked; first += kPieces * 64 * KW * GROUPS)
             {
                 floatx4 piece[kPieces];
 #pragma unroll
                 for (int i = 0; i < kPieces; ++i)
                 {
                     const uint32_t q = first + i * 64 * KW * GROUPS;
-                    piece[i] = load4(from + min(q * 4, floats - 4));
+                    piece[i] = load4(from + sph::PieceBegin(q, floats));
                 }
 #pragma unroll
                 for (int i = 0; i < kPieces; ++i)

@@ -336,6 +336,27 @@ int sphh_row_chunks_reach(unsigned K, unsigned rows, unsigned bk, long long* out
     return 0;
 }
 
+// The pieces of an operand of K rows of M floats that a workgroup asks for, `round` values of k at a
+// time: how far past the operand's end they reach, and whether every value is in one of them or in the
+// broken piece after the last.
+int sphh_pieces_reach(unsigned K, unsigned M, unsigned round, unsigned slots, long long* out)
+{
+    const long long end = static_cast<long long>(K) * M;
+    long long most = -end;
+    for (std::uint32_t base = 0; base < K; base += round)
+    {
+        const std::uint32_t floats = std::min(round, K - base) * M;
+        const std::uint32_t asked = sph::PiecesAsked(floats, slots);
+        for (std::uint32_t q = 0; q < asked; ++q)
+            most = std::max(most, static_cast<long long>(base) * M + sph::PieceBegin(q, floats) + 4 - end);
+        for (std::uint32_t q = 0; q * 4 + 4 <= floats; ++q)
+            if (q >= asked || sph::PieceBegin(q, floats) != q * 4)
+                return 1;
+    }
+    *out = most;
+    return 0;
+}
+
 // fp16: the last slab is the window [K - bk, K), whose last row is the matrix's.
 int sphh_chunk_copies_reach(unsigned K, unsigned limit, unsigned bk, unsigned tile, long long* out)
 {

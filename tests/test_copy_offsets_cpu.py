@@ -34,6 +34,16 @@ def test_fp32_row_chunks_end_with_the_operand(bk):
             assert reach("sphh_row_chunks_reach", K, rows, bk) == 0, (K, rows)
 
 
+# few rows of an operand stored k-major: (values of k a round, most rows, pieces a round)
+@pytest.mark.parametrize("wavefronts,rows", [(1, 4), (4, 4), (8, 4), (1, 8), (2, 8), (4, 8), (8, 8),
+                                             (1, 16), (2, 16), (4, 16), (8, 16)])
+def test_fp32_pieces_end_with_the_operand(wavefronts, rows):
+    step = 256 * wavefronts
+    for M in range(1, rows + 1):
+        for K in [64, 65, 66, 67, 255, step - 1, step, step + 1, step + 2, step + 3, 2 * step + 1]:
+            assert reach("sphh_pieces_reach", K, M, step, rows * 64 * wavefronts) <= 0, (K, M)
+
+
 # fp16 kernels: (K step, tile edge, fewest slabs of broken rows)
 @pytest.mark.parametrize("bk,tile", [(64, 64), (32, 128)])
 def test_fp16_chunks_end_with_the_operand(bk, tile):

@@ -43,3 +43,12 @@ def check(M, N, K, flags):
                                    (1022, 1022, 258), (2046, 2046, 290), (1024, 1020, 1025)])
 def test_last_step_of_less_than_a_chunk(dev, shape, flags):
     check(*shape, flags)
+
+
+# few rows of an A stored K x M, and few columns of a B stored K x N: a last round of K that has less than
+# four values
+@pytest.mark.parametrize("shape", [(1, 1024, 2049), (2, 1024, 2049), (3, 1024, 4097), (1, 512, 2051),
+                                   (1024, 1, 2049), (1024, 1, 2050), (512, 2, 2049), (1024, 3, 4097)])
+def test_last_round_of_less_than_a_piece(dev, shape):
+    for flags in (0, TA, TB, TA | TB):
+        check(*shape, flags)
