@@ -39,7 +39,6 @@ if ROOT not in sys.path:
 
 PEAK_FP16_TFLOPS = 2500.0   # MI355X dense fp16 MFMA, vendor figure
 PEAK_FP32_TFLOPS = 157.3    # MI355X dense fp32 MFMA
-PEAK_SPLIT_TFLOPS = PEAK_FP16_TFLOPS / 3  # an fp32 product made of three fp16 ones
 PEAK_HBM_GBS = 8000.0       # MI355X HBM3E
 
 
@@ -734,13 +733,13 @@ def bench_mfma_ceiling(settle_ms, timed):
     return {"flop_per_launch": flop, "settle_ms": settle_ms, "timed_launches": timed, "rows": rows}
 
 
-def f32_roofline(workload, entry, kernel, ms, flops, alg_bytes, peak=PEAK_FP32_TFLOPS):
+def f32_roofline(workload, entry, kernel, ms, flops, alg_bytes):
     tf = flops / (ms * 1e-3) / 1e12
     return {"workload": workload, "entry_point": entry, "launch_ms": ms, "value": tf,
             "unit": "TFLOP/s",
             "roofline": {"bound": "mfma", "kernel": kernel, "achieved": tf,
-                         "peak": peak, "unit": "TFLOP/s",
-                         "frac": tf / peak, "flop_per_step": flops,
+                         "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
+                         "frac": tf / PEAK_FP32_TFLOPS, "flop_per_step": flops,
                          "algorithmic_bytes_per_step": alg_bytes,
                          "hbm_gbs_on_algorithmic_bytes": alg_bytes / (ms * 1e-3) / 1e9}}
 
@@ -925,7 +924,7 @@ def main():
         tf = 16 * 2 * 512 ** 3 / (ms * 1e-3) / 1e12
         result["gemm_f32"] = {"workload": "configuration 2: A[16,512,512] x B[1,512,512] fp32",
                               "launch_ms": ms, "tflops": tf,
-                              "frac_split_mfma_peak": tf / PEAK_SPLIT_TFLOPS}
+                              "frac_fp32_mfma_peak": tf / PEAK_FP32_TFLOPS}
 
     if args.only == "shapes":
         result["off_grid_shapes"] = bench_off_grid(capi, synth, min(args.steps, 20), 3)
@@ -975,7 +974,7 @@ def main():
         result["spmm"] = spmm
 
     if args.only is None:
-        # configurations 1, 2 and 4, each against its MFMA peak (configuration 1 is a
+        # configurations 1, 2 and 4, each against the fp32 MFMA peak (configuration 1 is a
         # single 33.6 MFLOP launch and is bound by launch latency, not by any roofline)
         configs = {}
         c1 = synth.config1()
@@ -987,8 +986,8 @@ def main():
         ms = bench_f32(capi, c2["A"], c2["B"], c2["C"], 512, 512, 512, 16, 0, 200, 20)
         configs["config2_f32_batched"] = f32_roofline(
             "configuration 2: out[16,512,512] += A[16,512,512] * B[1,512,512] fp32, B shared "
-            "(stride 0), one launch", "sph_gemm_f32", "GemmF32SplitKernel<128>", ms,
-            16 * 2.0 * 512 ** 3, 4 * 512 * 512 * (16 + 1 + 16 + 16), peak=PEAK_SPLIT_TFLOPS)
+            "(stride 0), one launch", "sph_gemm_f32", "GemmF32DmaKernel<64>", ms,
+            16 * 2.0 * 512 ** 3, 4 * 512 * 512 * (16 + 1 + 16 + 16))
         c4 = synth.config4()
         sizes = [c4["x"].shape[1]] + [w.shape[1] for w in c4["W"]]
         batch = c4["x"].shape[0]
@@ -1000,7 +999,7 @@ def main():
         configs["config4_mlp_forward"] = f32_roofline(
             "configuration 4: 3-layer MLP forward 784-1024-1024-10 on x[1024,784] fp32, bias and "
             "ReLU fused into each layer's launch (3 launches per step)",
-            "sph_linear_forward_f32 x 3", "GemmF32DmaKernel / GemmF32SplitKernel<64> / GemmF32SkinnyKernel (fused epilogue)",
+            "sph_linear_forward_f32 x 3", "GemmF32DmaKernel / GemmF32SkinnyKernel (fused epilogue)",
             ms, fl, mlp_bytes)
         ms, fl = bench_mlp(capi, synth, 100, 10)
         configs["config4_mlp_forward"]["reference_call_sequence"] = {

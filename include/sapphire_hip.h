@@ -204,8 +204,7 @@ int sph_sgd_step_f32(float* z, const float* dz, float learningRate, size_t count
 #define SPH_GEMM_TRANS_B 4u    /* B is stored N x K (the transpose of K x N) */
 
 /* out[b] += A[b] * B[b] for b < batch; row-major; A is M x K, B is K x N,
- * out is M x N; fp32 storage and accumulation, products exact to fp32 (of many tiles: on the fp16 matrix
- * cores, every value as two fp16 numbers that hold it to 2^-23, whatever its size).
+ * out is M x N; fp32 storage, fp32 MFMA products and accumulation.
  * Strides are in elements between consecutive matrices; 0 repeats the
  * operand for every b (batch broadcast).
  *
