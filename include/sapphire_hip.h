@@ -81,9 +81,11 @@ int sph_free(void* ptr);                               /* Memory.cpp:38-44 */
  * device's pool, where its release threshold is at least that, as it is once
  * sph_malloc_async has been called); one block of up to 32 MiB, the staging of
  * sph_spgemm_f32, stays with each thread's stream (not with one set by
- * sph_set_stream).  sph_mem_pool_trim hands the idle memory of both pools and the
- * calling thread's block back; sph_malloc and sph_malloc_async do so with the
- * block and the library's own pool before they report that the device is full. */
+ * sph_set_stream).  These blocks are 512 MiB at most together, and
+ * a thread that ends leaves its own to the next.  sph_mem_pool_trim, on any thread,
+ * hands back the idle memory of both pools and the blocks of the calling thread and
+ * of all streams that have nothing to do; sph_malloc and sph_malloc_async do so with
+ * the blocks and the library's own pool before they report that the device is full. */
 int sph_malloc_async(void** ptr, size_t bytes);
 int sph_free_async(void* ptr);
 int sph_mem_pool_trim(void);

@@ -4,7 +4,7 @@
 // per-thread default stream (Sources/Sapphire/compute/dense/cuda/Gemm.cu:24-30,
 // CMake/CompileOptions.cmake:227).  Here the same slot holds a HIP stream:
 // every thread gets its own non-blocking stream per device, created on first
-// use at the default priority and handed back to a free list when the thread
+// use at the default priority and free for another thread when the thread
 // ends, so no stream is destroyed while the runtime may be shutting down.
 #include "sph_internal.h"
 
@@ -12,7 +12,7 @@
 #include <atomic>
 #include <cstring>
 #include <mutex>
-#include <vector>
+#include <new>
 
 namespace
 {
@@ -20,17 +20,23 @@ constexpr int kMaxDevices = 16;
 
 thread_local std::string tlsLastError;
 
-// A stream of the library's own, with the staging block that calls on it have left behind
+// A stream of the library's own, with the staging block that calls on it have left behind.  Made once
+// and never destroyed; the thread that has the stream takes and gives back the block, any thread may
+// hand an idle one back to its pool.
 struct OwnStream
 {
     hipStream_t stream = nullptr;
+    // (the rest under the mutex below)
+    OwnStream* next = nullptr;  // of the device
+    bool used = true;           // a thread has it
     void* block = nullptr;
     size_t bytes = 0;
     bool taken = false;  // by the call that runs
 };
 
 std::mutex gPoolMutex;
-std::vector<OwnStream> gIdleStreams[kMaxDevices];
+OwnStream* gStreams[kMaxDevices] = {};
+size_t gBlockBytes[kMaxDevices] = {};  // of their blocks
 int gComputeUnits[kMaxDevices] = {};
 bool gPoolRetains[kMaxDevices] = {};
 // (same mutex) the devices' default pools, and the library's own pools for the scratch blocks of
@@ -41,7 +47,7 @@ hipMemPool_t gScratchPools[kMaxDevices] = {};
 struct ThreadSlots
 {
     int device = 0;
-    OwnStream own[kMaxDevices] = {};
+    OwnStream* own[kMaxDevices] = {};
     hipStream_t borrowed[kMaxDevices] = {};
     hipStream_t capturing = nullptr;  // stream under capture, if any
 
@@ -49,8 +55,8 @@ struct ThreadSlots
     {
         std::lock_guard<std::mutex> lock(gPoolMutex);
         for (int d = 0; d < kMaxDevices; ++d)
-            if (own[d].stream != nullptr)
-                gIdleStreams[d].push_back(own[d]);
+            if (own[d] != nullptr)
+                own[d]->used = false;
     }
 };
 
@@ -113,22 +119,58 @@ int ScratchPool(hipMemPool_t* pool)
     return SPH_OK;
 }
 
-// The calling thread's idle block goes back to its pool.
-hipError_t DropKeptBlock()
+// The mutex is held: the stream's block goes back to its pool, behind the work that has used it.
+hipError_t DropBlock(OwnStream& own)
 {
-    OwnStream& own = tlsSlots.own[tlsSlots.device];
-    if (own.block == nullptr || own.taken)
-        return hipSuccess;
     const hipError_t err = hipFreeAsync(own.block, own.stream);
+    gBlockBytes[tlsSlots.device] -= own.bytes;
     own.block = nullptr;
     own.bytes = 0;
     return err;
 }
 
-// Idle blocks of the library's own pool go back to the driver.
-hipError_t TrimScratch()
+// The idle blocks of the device go back to their pools: the calling thread's own, and those of streams
+// that have nothing to do, whether another thread has them or none.  (A stream under capture is
+// left alone: what is asked of it would become a part of the graph.)  `wait`: for the work that has
+// used the thread's own block.
+hipError_t DropIdleBlocks(bool wait)
 {
-    const hipError_t dropped = DropKeptBlock();
+    std::lock_guard<std::mutex> lock(gPoolMutex);
+    for (OwnStream* s = gStreams[tlsSlots.device]; s != nullptr; s = s->next)
+    {
+        if (s->block == nullptr || s->taken)
+            continue;
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        hipError_t err = hipStreamIsCapturing(s->stream, &status);
+        if (err != hipSuccess)
+            return err;
+        if (status != hipStreamCaptureStatusNone)
+            continue;
+        const bool mine = s == tlsSlots.own[tlsSlots.device];
+        if (!mine)
+        {
+            err = hipStreamQuery(s->stream);
+            if (err != hipSuccess)
+            {
+                (void)hipGetLastError();  // not the next launch's error
+                if (err == hipErrorNotReady)
+                    continue;
+                return err;
+            }
+        }
+        err = DropBlock(*s);
+        if (err == hipSuccess && (wait || !mine))
+            err = hipStreamSynchronize(s->stream);  // (the pool has it back when the stream has come to that)
+        if (err != hipSuccess)
+            return err;
+    }
+    return hipSuccess;
+}
+
+// Idle blocks go back to the pools, those of the library's own pool to the driver.
+hipError_t TrimScratch(bool wait)
+{
+    const hipError_t dropped = DropIdleBlocks(wait);
     if (dropped != hipSuccess)
         return dropped;
     std::lock_guard<std::mutex> lock(gPoolMutex);
@@ -144,11 +186,7 @@ hipError_t AllocWithTrim(Alloc&& alloc)
     if (err != hipErrorOutOfMemory)
         return err;
     (void)hipGetLastError();  // not the next launch's error
-    // (a block is idle when the work before it has gone)
-    const OwnStream& own = tlsSlots.own[tlsSlots.device];
-    const bool kept = own.block != nullptr && !own.taken;
-    if (TrimScratch() == hipSuccess &&
-        (!kept || (hipStreamSynchronize(own.stream) == hipSuccess && TrimScratch() == hipSuccess)))
+    if (TrimScratch(true) == hipSuccess)
         err = alloc();
     if (err == hipErrorOutOfMemory)
         (void)hipGetLastError();
@@ -192,45 +230,61 @@ int AllocScratch(void** ptr, size_t bytes, hipStream_t stream)
 // Taking a block from a pool and giving it back costs the host 8 us, more than two launches, and a
 // product of a few thousand rows is over before that.  Its staging, up to 32 MiB, therefore stays with
 // the stream it was taken for, if that is one of the library's own: a later call on the stream runs behind
-// the one before, so it may use the block at once, and neither the stream (which is never destroyed) nor
-// the block is seen by another thread meanwhile.  Per thread and device that is one block; a thread that
-// ends leaves it, with the stream, to the next.  8192 rows of 64 products, calls one after the other
-// 21.3 -> 18.1 us (host 21.3 -> 13.7).
+// the one before, so it may use the block at once.  Per thread and device that is one block, for all
+// of them together as much as the pool keeps; a thread that ends leaves it, with the stream, to the
+// next.  8192 rows of 64 products, calls one after the other 21.3 -> 18.1 us (host 21.3 -> 13.7).
 constexpr size_t kKeptBlock = 32u << 20;
 
 int TakeStaging(void** ptr, size_t bytes, hipStream_t stream)
 {
-    OwnStream& own = tlsSlots.own[tlsSlots.device];
-    const bool keep = stream == own.stream && bytes <= kKeptBlock && !own.taken;
-    if (keep && own.block != nullptr && own.bytes >= bytes)
-    {
-        own.taken = true;
-        *ptr = own.block;
-        return SPH_OK;
-    }
+    const int d = tlsSlots.device;
+    OwnStream* own = tlsSlots.own[d];
+    bool keep = own != nullptr && stream == own->stream && bytes <= kKeptBlock;
     if (keep)
     {
-        SPH_HIP_TRY(DropKeptBlock());
+        std::lock_guard<std::mutex> lock(gPoolMutex);
+        keep = !own->taken;
+        if (keep && own->block != nullptr && own->bytes >= bytes)
+        {
+            own->taken = true;
+            *ptr = own->block;
+            return SPH_OK;
+        }
+        if (keep && own->block != nullptr)
+            SPH_HIP_TRY(DropBlock(*own));
         // the next call may need a little more
-        bytes = std::min(kKeptBlock, bytes + bytes / 4);
+        const size_t more = std::min(kKeptBlock, bytes + bytes / 4);
+        keep = keep && gBlockBytes[d] + more <= kScratchKept;
+        if (keep)
+            gBlockBytes[d] += bytes = more;
     }
     const int taken = BlockFromPool(ptr, bytes, stream);
-    if (taken == SPH_OK && keep && *ptr != nullptr)
+    if (keep)
     {
-        own.block = *ptr;
-        own.bytes = bytes;
-        own.taken = true;
+        std::lock_guard<std::mutex> lock(gPoolMutex);
+        if (taken == SPH_OK && *ptr != nullptr)
+        {
+            own->block = *ptr;
+            own->bytes = bytes;
+            own->taken = true;
+        }
+        else
+            gBlockBytes[d] -= bytes;
     }
     return taken;
 }
 
 int GiveStaging(void* ptr, hipStream_t stream)
 {
-    OwnStream& own = tlsSlots.own[tlsSlots.device];
-    if (own.taken && ptr == own.block)
+    OwnStream* own = tlsSlots.own[tlsSlots.device];
+    if (own != nullptr)
     {
-        own.taken = false;
-        return SPH_OK;
+        std::lock_guard<std::mutex> lock(gPoolMutex);
+        if (own->taken && ptr == own->block)
+        {
+            own->taken = false;
+            return SPH_OK;
+        }
     }
     SPH_HIP_TRY(hipFreeAsync(ptr, stream));
     return SPH_OK;
@@ -252,32 +306,37 @@ hipStream_t CurrentStream()
     const int d = tlsSlots.device;
     if (tlsSlots.borrowed[d] != nullptr)
         return tlsSlots.borrowed[d];
-    if (tlsSlots.own[d].stream == nullptr)
+    if (tlsSlots.own[d] == nullptr)
     {
         {
             std::lock_guard<std::mutex> lock(gPoolMutex);
-            if (!gIdleStreams[d].empty())
+            OwnStream* idle = gStreams[d];
+            while (idle != nullptr && idle->used)
+                idle = idle->next;
+            if (idle != nullptr)
             {
-                tlsSlots.own[d] = gIdleStreams[d].back();
-                gIdleStreams[d].pop_back();
+                idle->used = true;
+                tlsSlots.own[d] = idle;
+                return idle->stream;
             }
         }
-        if (tlsSlots.own[d].stream == nullptr)
+        OwnStream* own = new (std::nothrow) OwnStream;
+        hipError_t err = own != nullptr ? hipSetDevice(d) : hipErrorOutOfMemory;
+        if (err == hipSuccess)
+            err = hipStreamCreateWithFlags(&own->stream, hipStreamNonBlocking);
+        if (err != hipSuccess)
         {
-            hipStream_t s = nullptr;
-            hipError_t err = hipSetDevice(d);
-            if (err == hipSuccess)
-                err = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-            if (err != hipSuccess)
-            {
-                Fail(SPH_ERR_DEVICE, std::string("stream creation failed with ") +
-                                         hipGetErrorString(err));
-                return nullptr;
-            }
-            tlsSlots.own[d].stream = s;
+            delete own;
+            Fail(SPH_ERR_DEVICE,
+                 std::string("stream creation failed with ") + hipGetErrorString(err));
+            return nullptr;
         }
+        std::lock_guard<std::mutex> lock(gPoolMutex);
+        own->next = gStreams[d];
+        gStreams[d] = own;
+        tlsSlots.own[d] = own;
     }
-    return tlsSlots.own[d].stream;
+    return tlsSlots.own[d]->stream;
 }
 
 bool Capturing()
@@ -431,7 +490,7 @@ int sph_allocation_count(uint64_t* count)
 int sph_mem_pool_trim(void)
 {
     SPH_REFUSE_WHILE_CAPTURING();
-    SPH_HIP_TRY(sph::TrimScratch());  // (first: the thread's idle block may be of either pool)
+    SPH_HIP_TRY(sph::TrimScratch(false));  // (first: an idle block may be of either pool)
     hipMemPool_t pool = nullptr;
     SPH_HIP_TRY(hipDeviceGetDefaultMemPool(&pool, tlsSlots.device));
     SPH_HIP_TRY(hipMemPoolTrimTo(pool, 0));
@@ -598,7 +657,11 @@ int sph_graph_begin_capture(void)
             return rc;
     }
     SPH_STREAM_OR_FAIL(stream);
-    SPH_HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+    {
+        // (no other thread hands this stream's block back meanwhile)
+        std::lock_guard<std::mutex> lock(gPoolMutex);
+        SPH_HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+    }
     tlsSlots.capturing = stream;
     return SPH_OK;
 }
