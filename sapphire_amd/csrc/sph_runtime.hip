@@ -7,8 +7,8 @@
 // use at the default priority and free for another thread when the thread
 // ends, so no stream is destroyed while the runtime may be shutting down.
 #include "sph_internal.h"
+#include "sph_spgemm_plan.h"
 
-#include <algorithm>
 #include <atomic>
 #include <cstring>
 #include <mutex>
@@ -252,24 +252,25 @@ int TakeStaging(void** ptr, size_t bytes, hipStream_t stream)
         }
         if (keep && own->block != nullptr)
             SPH_HIP_TRY(DropBlock(*own));
-        // the next call may need a little more
-        const size_t more = std::min(kKeptBlock, bytes + bytes / 4);
-        keep = keep && gBlockBytes[d] + more <= kScratchKept;
+        keep = keep && gBlockBytes[d] + kKeptBlock <= kScratchKept;
         if (keep)
-            gBlockBytes[d] += bytes = more;
+            gBlockBytes[d] += kKeptBlock;  // until it is known what the block is
     }
-    const int taken = BlockFromPool(ptr, bytes, stream);
-    if (keep)
+    if (!keep)
+        return BlockFromPool(ptr, bytes, stream);
+    int taken = SPH_OK;
+    const size_t got = TakeWithRoom(bytes, kKeptBlock, [&](size_t size) {
+        taken = BlockFromPool(ptr, size, stream);
+        return taken != SPH_OK || *ptr != nullptr;
+    });
+    std::lock_guard<std::mutex> lock(gPoolMutex);
+    gBlockBytes[d] -= kKeptBlock;
+    if (taken == SPH_OK && *ptr != nullptr)
     {
-        std::lock_guard<std::mutex> lock(gPoolMutex);
-        if (taken == SPH_OK && *ptr != nullptr)
-        {
-            own->block = *ptr;
-            own->bytes = bytes;
-            own->taken = true;
-        }
-        else
-            gBlockBytes[d] -= bytes;
+        own->block = *ptr;
+        own->bytes = got;
+        own->taken = true;
+        gBlockBytes[d] += got;
     }
     return taken;
 }

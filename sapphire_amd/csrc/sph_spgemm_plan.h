@@ -3,6 +3,7 @@
 #ifndef SPH_SPGEMM_PLAN_H
 #define SPH_SPGEMM_PLAN_H
 
+#include <cstddef>
 #include <cstdint>
 
 #if defined(__HIPCC__)
@@ -39,6 +40,18 @@ uint32_t TakeStagingSlot(uint32_t M, uint32_t N, uint32_t capacity, Take&& take)
             return static_cast<uint32_t>(slot);
     }
     return 0;
+}
+
+// Bytes of a staging block that is to stay for the next call, which may need a little more: a quarter
+// on top, up to `most`, where `take(bytes)` finds memory for that, else just `bytes` (<= most).  Returns
+// what was taken, 0 for nothing.
+template <typename Take>
+std::size_t TakeWithRoom(std::size_t bytes, std::size_t most, Take&& take)
+{
+    const std::size_t more = bytes + bytes / 4 < most ? bytes + bytes / 4 : most;
+    if (take(more))
+        return more;
+    return more != bytes && take(bytes) ? bytes : 0;
 }
 }  // namespace sph
 

@@ -426,6 +426,19 @@ unsigned sphh_staging_slot(unsigned M, unsigned N, unsigned capacity, unsigned l
     });
 }
 
+// The staging block of up to `most` bytes that a call for `bytes` takes when `room` bytes are free, and in
+// tried[0 .. *tries) the sizes it asked for.  No device is touched.
+unsigned long long sphh_take_with_room(unsigned long long bytes, unsigned long long most,
+                                       unsigned long long room, unsigned long long* tried,
+                                       unsigned* tries)
+{
+    *tries = 0;
+    return sph::TakeWithRoom(bytes, most, [&](std::size_t size) {
+        tried[(*tries)++] = size;
+        return size <= room;
+    });
+}
+
 // Compute::Gemm into a FRESH y (never filled, never read): the operator sees the deferred zero
 // state of the new buffer and stores the product.  yOut receives the result.
 int sphh_compute_gemm_fresh_y(float* yOut, const int* y, int yn, const float* aData, const int* a,

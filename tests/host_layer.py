@@ -37,6 +37,9 @@ def lib():
         h.sphh_staging_slot.argtypes = [ctypes.c_uint] * 3 + [
             ctypes.c_ulonglong, ctypes.POINTER(ctypes.c_uint), ctypes.POINTER(ctypes.c_uint)]
         h.sphh_staging_slot.restype = ctypes.c_uint
+        h.sphh_take_with_room.argtypes = [ctypes.c_ulonglong] * 3 + [
+            ctypes.POINTER(ctypes.c_ulonglong), ctypes.POINTER(ctypes.c_uint)]
+        h.sphh_take_with_room.restype = ctypes.c_ulonglong
         h.sphh_column_walk.argtypes = [ctypes.c_uint] * 3 + [ctypes.POINTER(ctypes.c_ulonglong)]
         h.sphh_spgemm_turns.argtypes = [ctypes.c_uint] * 2
         h.sphh_spgemm_turns.restype = ctypes.c_uint
@@ -174,6 +177,13 @@ def staging_slot(M, N, capacity, room):
     tried, tries = (ctypes.c_uint * 8)(), ctypes.c_uint(0)
     slot = int(lib().sphh_staging_slot(M, N, capacity, room, tried, ctypes.byref(tries)))
     return slot, [int(tried[i]) for i in range(tries.value)]
+
+
+def take_with_room(bytes, most, room):
+    """(size taken, sizes asked for)"""
+    tried, tries = (ctypes.c_ulonglong * 8)(), ctypes.c_uint(0)
+    got = int(lib().sphh_take_with_room(bytes, most, room, tried, ctypes.byref(tries)))
+    return got, [int(tried[i]) for i in range(tries.value)]
 
 
 def spgemm_turns(M, rows_per_turn):

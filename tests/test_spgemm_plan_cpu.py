@@ -23,6 +23,14 @@ def test_staging_asks_for_less_when_the_device_is_full():
         assert hl.staging_slot(*empty, 2**40) == (0, [])
 
 
+def test_a_kept_block_is_larger_only_where_there_is_room():
+    for bytes, room, want in [(1000, 1250, (1250, [1250])), (1000, 1249, (1000, [1250, 1000])),
+                              (1000, 1000, (1000, [1250, 1000])), (1000, 999, (0, [1250, 1000])),
+                              (1800, 2000, (2000, [2000])), (1800, 1999, (1800, [2000, 1800])),
+                              (2000, 1999, (0, [2000])), (2000, 2000, (2000, [2000])), (1, 1, (1, [1]))]:
+        assert hl.take_with_room(bytes, 2000, room) == want, (bytes, room)
+
+
 def test_staging_stays_below_the_limit_of_its_indexes():
     room = 2**60
     # one row: 3 * capacity + 64 against 2^31
