@@ -583,7 +583,7 @@ __device__ __forceinline__ uint32_t LightRowOfAnyLength(const SpgemmArgs& args, 
 // chain of four dependent loads; seven wavefronts per SIMD are resident (five left 8192 rows in
 // two rounds; eight spill scalars and are level).  Against a sort by compares and selects, shuffles
 // through the LDS crossbar and a search of every product's entry of A one entry after the other:
-// 65536 rows with 8 entries on both sides 63 -> 38 us for the pass, the whole call 86 -> 59 us;
+// 65536 rows with 8 entries on both sides 63 -> 35 us for the pass, the whole call 86 -> 59 us;
 // 8192 rows 15.8 -> 9.4 us.
 template <int MODE, typename Key>
 __global__ __launch_bounds__(kLightWaves * 64, 7) void SpgemmLightKernel(const SpgemmArgs args)
